@@ -1,6 +1,7 @@
 // Set handles: constructors (Star(V, C, d, lb, ub), Star(lb, ub) for arrays of boxes, the reduceMem box), reference
 // counting, property reads and the estimateRanges entry points.
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -8,6 +9,75 @@
 #include "internal.h"
 
 using namespace nnvhip;
+
+namespace {
+
+// Read-back of lb / ub: the kernel stores them straight into pinned host memory in the caller's layout (lb of all
+// sets, then ub of all sets, N entries each) and the host watches one flag per block.  What bounds it is latency, not
+// bytes: a device-to-host copy into pageable memory costs the host some 20 us each (two per call: 36-40 us for a
+// ten-row set), the kernel plus the host's last look at the flag about 10 us.  A block ends with a system-scope fence
+// behind its stores and then its flag, so whoever sees the flag sees the block's values.
+struct PostSet {
+  const double* lb;
+  const double* ub;
+};
+constexpr int kPostBlock = 4096;  // values per block: 32 KB of stores over PCIe
+__global__ __launch_bounds__(256) void post_ranges_kernel(const PostSet* __restrict__ table, PostSet one, int64_t N, int64_t total,
+                                                           double* __restrict__ dst, uint32_t* __restrict__ flags) {
+  const int64_t half = total / 2;
+  const int64_t e1 = min(total, (int64_t)(blockIdx.x + 1) * kPostBlock);
+  for (int64_t e = (int64_t)blockIdx.x * kPostBlock + threadIdx.x; e < e1; e += 256) {
+    const int64_t q = e < half ? e : e - half;
+    const int64_t i = q / N;
+    const PostSet s = table ? table[i] : one;
+    dst[e] = (e < half ? s.lb : s.ub)[q - i * N];
+  }
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(flags + blockIdx.x, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// lb / ub of all sets (known on the device) to the host; either pointer may be null.
+int post_ranges(nnvhip_ctx* c, int64_t count, nnvhip_star* const* s, double* lb, double* ub) {
+  const int64_t N = s[0]->N, total = 2 * N * count, blocks = ceil_div(total, kPostBlock);
+  const PostSet* table = nullptr;
+  BufRef tab;
+  if (count > 1) {
+    std::vector<PostSet> ps((size_t)count);
+    for (int64_t i = 0; i < count; ++i) ps[(size_t)i] = PostSet{s[i]->lb, s[i]->ub};
+    NNV_TRY(c->upload_table(ps.data(), sizeof(PostSet) * count, &tab));
+    table = tab->as<PostSet>();
+  }
+  void* slot = nullptr;
+  const size_t flag_bytes = ((size_t)blocks * sizeof(uint32_t) + 255) & ~size_t(255);
+  NNV_TRY(c->stage(flag_bytes + sizeof(double) * (size_t)total, &slot));
+  uint32_t* flags = static_cast<uint32_t*>(slot);
+  double* vals = reinterpret_cast<double*>(static_cast<char*>(slot) + flag_bytes);
+  for (int64_t b = 0; b < blocks; ++b) reinterpret_cast<volatile uint32_t*>(flags)[b] = 0;
+  std::atomic_thread_fence(std::memory_order_seq_cst);
+  hipLaunchKernelGGL(post_ranges_kernel, dim3((unsigned)blocks), dim3(256), 0, c->stream, table, PostSet{s[0]->lb, s[0]->ub}, N, total, vals,
+                     flags);
+  NNV_HIP_TRY(hipGetLastError());
+  const auto t0 = std::chrono::steady_clock::now();
+  long spins = 0;
+  for (int64_t b = 0; b < blocks; ++b)
+    while (__atomic_load_n(flags + b, __ATOMIC_ACQUIRE) == 0) {
+      if (!c->deferred.empty()) c->drain_deferred(16);  // something useful to do while the device works
+      if ((++spins & 0xfff) == 0 && std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count() > 10.0) {
+        NNV_HIP_TRY(hipStreamSynchronize(c->stream));  // surfaces a launch failure, if any
+        if (__atomic_load_n(flags + b, __ATOMIC_ACQUIRE) == 0) NNV_FAIL(NNVHIP_ERR_HIP, "the ranges did not arrive");
+      }
+    }
+  if (lb) memcpy(lb, vals, sizeof(double) * (size_t)(total / 2));
+  if (ub) memcpy(ub, vals + total / 2, sizeof(double) * (size_t)(total / 2));
+  return NNVHIP_OK;
+}
+
+// Above this many values the copy engine is the better way: the blocks' stores reach some 20 GB/s, and a call that
+// large no longer notices 20 us.
+constexpr int64_t kPostMax = int64_t(1) << 17;
+
+}  // namespace
 
 extern "C" {
 
@@ -493,6 +563,7 @@ int nnvhip_estimate_ranges_batch(nnvhip_ctx* c, int64_t count, nnvhip_star* cons
   NNV_TRY(c->end_op());
   if (lb || ub) {
     int64_t N = s[0]->N;
+    if (2 * N * count <= kPostMax) return post_ranges(c, count, s, lb, ub);
     // ranges computed by one call sit at a fixed stride in one buffer
     const int64_t stride = count > 1 ? s[1]->lb - s[0]->lb : 0;
     bool regular = count > 1 && stride >= N;
