@@ -45,9 +45,11 @@ struct ChainLayer {
 };
 
 struct ChainSet {
-  const double* V;    // the input set, fully in memory
-  const double* plb;
+  const double* V;    // the input set, fully in memory - or, with idx, a box of which only the centre is (the first layer
+  const double* plb;  // is an FC layer then): column 1 + t is scale[idx[t]] at row idx[t]
   const double* pub;
+  const int32_t* idx;
+  const double* scale;
   int64_t ld;
   int32_t N, n;
 };
@@ -192,7 +194,14 @@ __global__ __launch_bounds__(kChainThreads) void reach_chain_kernel(const ChainS
         for (int tc = wc; tc < CT; tc += WC) {
           const int col_a = tc * 16 + l16;  // the column this lane feeds
           const bool col_ok = col_a < nd;
-          const double* vcol = Vsrc + (int64_t)(col_ok ? col_a : 0) * ld;
+          const bool box = l == 0 && S.idx != nullptr;  // (uniform)
+          const double* vcol = Vsrc + (int64_t)(col_ok && !box ? col_a : 0) * ld;
+          int hot = -1;  // a box's generator column: its one row and the value there
+          double hot_v = 0.0;
+          if (box && col_ok && col_a > 0) {
+            hot = S.idx[col_a - 1];
+            hot_v = S.scale[hot];
+          }
           double pl[4], pu[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {  // predicate bounds of the lane's four result columns
@@ -215,7 +224,8 @@ __global__ __launch_bounds__(kChainThreads) void reach_chain_kernel(const ChainS
               if (k < Kk) {
                 const int kk = n_keep >= 0 ? s_keep[k] : k;
                 bv[u] = wrow[(int64_t)kk * ldw];
-                if (col_ok) av[u] = vcol[kk];
+                if (hot >= 0) av[u] = kk == hot ? hot_v : 0.0;
+                else if (col_ok) av[u] = vcol[kk];
               }
             }
 #pragma unroll
@@ -564,7 +574,17 @@ int reach_small_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, cons
   if ((double)plan.doubles * (double)count > 5.0e8) return NNVHIP_OK;  // 4 GB of worst-case buffers
   *taken = true;
 
-  NNV_TRY(ensure_dense_batch(c, count, in, true, true));
+  // boxes go in as they are where the first layer is an FC layer
+  auto as_box = [&](const nnvhip_star* s) {
+    return kind[0] == NNVHIP_LAYER_FC && !s->rows_pending && !s->cs.any_pending() && s->n > 0 && s->stored_cols() == 1 && s->oh_from == 1 &&
+           s->oh_idx != nullptr && s->oh_scale != nullptr;
+  };
+  {
+    std::vector<nnvhip_star*> full;
+    for (int64_t i = 0; i < count; ++i)
+      if (!as_box(in[i])) full.push_back(in[i]);
+    if (!full.empty()) NNV_TRY(ensure_dense_batch(c, (int64_t)full.size(), full.data(), true, true));
+  }
   BufRef arena, iarena, cnt;
   NNV_TRY(c->alloc(sizeof(double) * plan.doubles * count, &arena));
   NNV_TRY(c->alloc(sizeof(int32_t) * plan.ints * count, &iarena));
@@ -588,7 +608,11 @@ int reach_small_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, cons
     a.mailbox_seq = (int32_t)(c->mailbox_seq & 0xffffu);
   }
   std::vector<ChainSet> sets((size_t)count);
-  for (int64_t i = 0; i < count; ++i) sets[i] = ChainSet{in[i]->V, in[i]->plb, in[i]->pub, in[i]->ld, (int32_t)in[i]->N, (int32_t)in[i]->n};
+  for (int64_t i = 0; i < count; ++i) {
+    const bool box = as_box(in[i]);
+    sets[i] = ChainSet{in[i]->V, in[i]->plb, in[i]->pub, box ? in[i]->oh_idx : nullptr, box ? in[i]->oh_scale : nullptr, in[i]->ld,
+                       (int32_t)in[i]->N, (int32_t)in[i]->n};
+  }
   const ChainSet* table = nullptr;
   BufRef tab;
   if (count > 1) {

@@ -182,6 +182,14 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
     for (int64_t i = 0; i < count; ++i)
       if (dense[i] > in[i]->stored_cols() || (dense_only && (in[i]->rows_pending || in[i]->cs.any_pending()))) full.push_back(in[i]);
     if (!full.empty()) {
+      // (boxes of one array move together: the array stays back to back)
+      if ((int64_t)full.size() < count) {
+        full.clear();
+        for (int64_t i = 0; i < count; ++i)
+          if (dense[i] > in[i]->stored_cols() || (dense_only && (in[i]->rows_pending || in[i]->cs.any_pending())) ||
+              (in[i]->oh_scale != nullptr && in[i]->stored_cols() < in[i]->n + 1))
+            full.push_back(in[i]);
+      }
       st = ensure_dense_batch(c, (int64_t)full.size(), full.data());
       contig = true;  // the sets moved: look again
       for (int64_t i = 1; i < count; ++i)
@@ -448,9 +456,13 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
           any_fill = true;
         }
       }
-      bool all_stored = true;
-      for (int64_t i = 0; i < count; ++i) all_stored = all_stored && in[i]->stored_cols() == in[i]->n + 1;
-      if (any_onehot && !any_rows && all_stored) {
+      // (boxes keep their centres only, back to back; a set with nothing but its centre counts either way)
+      bool all_stored = true, centres_only = true;
+      for (int64_t i = 0; i < count; ++i) {
+        all_stored = all_stored && in[i]->stored_cols() == in[i]->n + 1;
+        centres_only = centres_only && in[i]->stored_cols() == 1 && dense[i] == 1;
+      }
+      if (any_onehot && !any_rows && (all_stored || centres_only)) {
         // all sets contract over every row: their dense columns are simply listed (tiles may span sets)
         if (cols >= (int64_t(1) << 31)) st = NNVHIP_ERR_SHAPE;
         std::vector<int32_t> map;
@@ -458,13 +470,14 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
         int64_t off = 0;
         for (int64_t i = 0; i < count; ++i) {
           for (int64_t j = 0; j < dense[i]; ++j) map.push_back((int32_t)(off + j));
-          off += in[i]->n + 1;  // box stars: all columns stored, input and output arenas laid out alike
+          off += in[i]->n + 1;  // all columns stored: input and output arenas are laid out alike
         }
         BufRef cmap;
         if (st == NNVHIP_OK) st = c->upload_table(map.data(), sizeof(int32_t) * map.size(), &cmap);
         if (st == NNVHIP_OK) {
           GemmRows rows;
           rows.colmap = cmap->as<int32_t>();
+          rows.b_plain = centres_only;
           st = launch_gemm(c, Wd, fc->Mp, in[0]->V, in[0]->ld, outs[0]->V, outs[0]->ld, fc->Mp, total_dense, fc->Kp, bias,
                            nullptr, &rows);
         }

@@ -31,6 +31,7 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void gemm_f64_kernel(const doubl
                                                         const int32_t* __restrict__ kmap,
                                                         const GemmSeg* __restrict__ segs,
                                                         const int32_t* __restrict__ colmap,
+                                                        const int32_t* __restrict__ bmap,
                                                         const double* __restrict__ Bk, int64_t ldbk) {
   constexpr int NT = 64 * WR * WC;  // threads per block
   constexpr int FM = TM / WR / 16;
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void gemm_f64_kernel(const doubl
   for (int p = 0; p < B_PASS; ++p) {
     const int64_t jl = (tid + p * NT) / (KT / 2);
     const int64_t col = col_base + jl;
-    bcol[p] = col < col_end ? ((MAPPED && colmap != nullptr) ? (int64_t)colmap[col] : b_col_base + jl) : -1;
+    bcol[p] = col < col_end ? ((MAPPED && bmap != nullptr) ? (int64_t)bmap[col] : b_col_base + jl) : -1;
   }
 
   auto load_tiles = [&](int k0) {
@@ -359,12 +360,12 @@ static int launch_cfg(nnvhip_ctx* ctx, const double* A, int64_t lda, const doubl
                        dim3(64 * WR * WC), 0, A, lda, B, ldb, C, ldc, (int)Mp, ncols, (int)Kp, bias, (int)tiles_m,
                        (int)tiles_n, (int)best_xr, (int)local_m, (int)ksplit, ws ? ws->as<double>() : nullptr,
                        fuse ? fuse->plb : nullptr, fuse ? fuse->pub : nullptr, rpart, rows->kmap, rows->segs, rows->colmap,
-                       rows->Bk, rows->ldbk);
+                       rows->b_plain ? nullptr : rows->colmap, rows->Bk, rows->ldbk);
   } else
     NNV_LAUNCH(ctx, timed, (gemm_f64_kernel<TM, TN, WR, WC, KT, false>), dim3((unsigned)grid_x, (unsigned)ksplit),
                        dim3(64 * WR * WC), 0, A, lda, B, ldb, C, ldc, (int)Mp, ncols, (int)Kp, bias, (int)tiles_m,
                        (int)tiles_n, (int)best_xr, (int)local_m, (int)ksplit, ws ? ws->as<double>() : nullptr,
-                       fuse ? fuse->plb : nullptr, fuse ? fuse->pub : nullptr, rpart, nullptr, nullptr, nullptr, nullptr, 0);
+                       fuse ? fuse->plb : nullptr, fuse ? fuse->pub : nullptr, rpart, nullptr, nullptr, nullptr, nullptr, nullptr, 0);
   NNV_TRY(ctx->kernel_timer_end(timed, 0, rows && rows->flop > 0.0 ? rows->flop : 2.0 * (double)Mp * (double)Kp * (double)ncols));
   if (defer != nullptr) {
     defer->ws = ws;

@@ -622,8 +622,10 @@ struct GemmRows {
   int64_t ldbk = 0;
   const GemmSeg* segs = nullptr;
   // without segs: product column t reads column colmap[t] of B and writes column colmap[t] of C
-  // (columns picked from an arena of sets that share the row list)
+  // (columns picked from an arena of sets that share the row list); with b_plain the product's columns are B's own
+  // and only C's are mapped (centres that lie back to back)
   const int32_t* colmap = nullptr;
+  bool b_plain = false;
   int32_t seg_cols = 128;
   double flop = 0.0;  // flop actually executed (for the kernel timers)
   // 64: take the 64 x 64 tile whatever the shape model says (short products of a few hundred tiles, whose blocks

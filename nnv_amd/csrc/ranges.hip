@@ -1120,16 +1120,98 @@ static bool scan_in_windows(const nnvhip_star* t) {
   return 2 * (int64_t)t->box_eh * t->box_ew <= P;
 }
 
+// Ranges of boxes whose generator columns exist as a list of scaled unit vectors only (nnvhip_star_from_box): row r has
+// at most one generator, column t with idx[t] = r (idx ascends: found by bisection), so its four sums are single
+// products - the values a scan of the written matrix gives, without writing it.  One thread per row.
+struct BoxRange {
+  const double* centre;
+  const int32_t* idx;
+  const double* scale;
+  const double* plb;
+  const double* pub;
+  double* lb;
+  double* ub;
+  int32_t n, N;
+};
+__global__ __launch_bounds__(256) void box_ranges_kernel(const BoxRange* __restrict__ table, BoxRange one) {
+  const BoxRange d = table ? table[blockIdx.y] : one;
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r >= d.N) return;
+  int a = 0, b = d.n;  // first t with idx[t] >= r
+  if (d.n == d.N) a = b = r;
+  while (a < b) {
+    const int m = (a + b) >> 1;
+    if (d.idx[m] < r) a = m + 1;
+    else b = m;
+  }
+  double x1 = 0.0, x2 = 0.0, y1 = 0.0, y2 = 0.0;
+  if (a < d.n && d.idx[a] == r) {
+    const double v = d.scale[r], pl = d.plb[a], pu = d.pub[a];
+    const double vp = fmax(v, 0.0), vn = fmin(v, 0.0);
+    x1 = fma(vp, pl, x1);  // xmin1
+    x2 = fma(vn, pu, x2);  // xmin2
+    y1 = fma(vp, pu, y1);  // xmax1
+    y2 = fma(vn, pl, y2);  // xmax2
+  }
+  const double c = d.centre[r];
+  d.lb[r] = (c + x1) + x2;  // set/Star.m:1098-1104, left to right
+  d.ub[r] = (c + y1) + y2;
+}
+
+static bool is_unwritten_box(const nnvhip_star* t) {
+  return !t->rows_pending && t->n > 0 && t->stored_cols() == 1 && t->oh_from == 1 && t->oh_idx != nullptr && t->oh_scale != nullptr &&
+         !t->cs.any_pending();
+}
+
+static BoxRange box_range_of(const nnvhip_star* t, double* lb, double* ub) {
+  return BoxRange{t->V, t->oh_idx, t->oh_scale, t->plb, t->pub, lb, ub, (int32_t)t->n, (int32_t)t->N};
+}
+
+static int compute_box_ranges(nnvhip_ctx* ctx, const std::vector<nnvhip_star*>& sets) {
+  int64_t doubles = 0, max_N = 0;
+  for (auto* t : sets) {
+    if (t->N >= (int64_t(1) << 31)) NNV_FAIL(NNVHIP_ERR_SHAPE, "set dimension too large");
+    doubles += 2 * t->ld;
+    max_N = std::max(max_N, t->N);
+  }
+  BufRef rb, tab;
+  NNV_TRY(ctx->alloc(sizeof(double) * doubles, &rb));
+  std::vector<BoxRange> br;
+  br.reserve(sets.size());
+  double* at = rb->as<double>();
+  for (auto* t : sets) {
+    br.push_back(box_range_of(t, at, at + t->ld));
+    at += 2 * t->ld;
+  }
+  for (size_t i0 = 0; i0 < br.size(); i0 += 65535) {
+    const size_t cnt = std::min<size_t>(65535, br.size() - i0);
+    const BoxRange* table = nullptr;
+    if (cnt > 1) {
+      NNV_TRY(ctx->upload_table(br.data() + i0, sizeof(BoxRange) * cnt, &tab));
+      table = tab->as<BoxRange>();
+    }
+    hipLaunchKernelGGL(box_ranges_kernel, dim3((unsigned)ceil_div(max_N, 256), (unsigned)cnt), dim3(256), 0, ctx->stream, table, br[i0]);
+    NNV_HIP_TRY(hipGetLastError());
+  }
+  for (size_t i = 0; i < sets.size(); ++i) {
+    sets[i]->rbuf = rb;
+    sets[i]->lb = br[i].lb;
+    sets[i]->ub = br[i].ub;
+  }
+  return NNVHIP_OK;
+}
+
 int compute_ranges(nnvhip_ctx* ctx, int64_t count, nnvhip_star* const* s, RangeCounts* counts) {
-  // sets that already carry ranges are skipped
-  std::vector<nnvhip_star*> todo;
+  // sets that already carry ranges are skipped, boxes with nothing but a centre in memory go by a kernel of their own
+  std::vector<nnvhip_star*> todo, boxes;
   todo.reserve((size_t)count);
   const uint64_t visit = ++ctx->visit_seq;  // (a handle may be listed twice)
   for (int64_t i = 0; i < count; ++i)
     if (!s[i]->lb && s[i]->visit != visit) {
       s[i]->visit = visit;
-      todo.push_back(s[i]);
+      (is_unwritten_box(s[i]) ? boxes : todo).push_back(s[i]);
     }
+  if (!boxes.empty()) NNV_TRY(compute_box_ranges(ctx, boxes));
   if (todo.empty()) return NNVHIP_OK;
   // Sets whose generator images are in memory inside their windows only are scanned inside the windows (all
   // sets of the call, or none: one launch serves them all; the same sums to the bit either way).
@@ -1402,6 +1484,19 @@ int ranges_into_static(nnvhip_ctx* ctx, const nnvhip_star* s, double* lb_dev, do
     return NNVHIP_OK;
   }
   if (ctx->device < 0 || ctx->device >= kMaxDevices) NNV_FAIL(NNVHIP_ERR_ARG, "device number %d is out of range", ctx->device);
+  if (is_unwritten_box(s) && s->N < (int64_t(1) << 31)) {  // a box: a row has one generator, nothing to combine
+    if (2 * s->ld > ctx->static_scratch_doubles) NNV_FAIL(NNVHIP_ERR_SHAPE, "nnvhip_estimate_ranges_static: a set of dimension %lld does not fit the static workspace", (long long)s->N);
+    std::lock_guard<std::mutex> lock(g_static_use_mutex);
+    StaticUse& use = g_static_use[ctx->device];
+    if (use.last != nullptr && use.last != ctx) NNV_HIP_TRY(hipStreamWaitEvent(ctx->stream, use.done, 0));
+    double* lb = ctx->static_scratch;
+    hipLaunchKernelGGL(box_ranges_kernel, dim3((unsigned)ceil_div(s->N, 256)), dim3(256), 0, ctx->stream, nullptr, box_range_of(s, lb, lb + s->ld));
+    hipLaunchKernelGGL(copy_ranges_kernel, dim3((unsigned)ceil_div(s->N, 256)), dim3(256), 0, ctx->stream, lb, lb + s->ld, lb_dev, ub_dev, s->N);
+    NNV_HIP_TRY(hipGetLastError());
+    NNV_HIP_TRY(hipEventRecord(use.done, ctx->stream));
+    use.last = ctx;
+    return NNVHIP_OK;
+  }
   // the set must be a plain stored matrix: writing pending columns or rows would need a buffer
   if (s->rows_pending || s->cs.any_pending() || s->stored_cols() != s->n + 1)
     NNV_FAIL(NNVHIP_ERR_ARG, "nnvhip_estimate_ranges_static: parts of this set are not in memory yet (read it once, or use "

@@ -482,12 +482,33 @@ __global__ __launch_bounds__(64 * kApplyWaves) void relu_apply_kernel(const Relu
   }
 }
 
-// unit-vector columns of a set: column j (of ncols) = e_idx[j]
-__global__ void onehot_columns_kernel(double* __restrict__ V, int64_t ld, const int32_t* __restrict__ idx, int ncols) {
-  for (int j = blockIdx.y; j < ncols; j += gridDim.y) {
-    const int hot = idx[j];
-    for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < ld; r += (int64_t)gridDim.x * blockDim.x)
-      V[r + (int64_t)j * ld] = r == hot ? 1.0 : 0.0;
+// Whole matrices of sets whose trailing columns exist as a list of scaled unit vectors only: the stored columns are
+// copied, column have + t is scale[idx[t]] (1 without scales) at row idx[t] and zero elsewhere.  Bound by its writes;
+// lane = two rows (16-byte streaming stores), the waves of a block interleave columns.
+struct TailSet {
+  const double* V;
+  double* out;
+  const int32_t* idx;
+  const double* scale;
+  int64_t ld;
+  int32_t have, ncols;
+};
+__global__ __launch_bounds__(512) void write_tail_kernel(const TailSet* __restrict__ table, TailSet one, int cols_per_chunk) {
+  const TailSet d = table ? table[blockIdx.z] : one;
+  const int64_t r0 = (int64_t)blockIdx.x * 128 + 2 * (threadIdx.x & 63);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j0 = blockIdx.y * cols_per_chunk, j1 = min(d.ncols, j0 + cols_per_chunk);
+  if (r0 >= d.ld) return;
+  typedef double dd2 __attribute__((ext_vector_type(2)));
+  for (int j = j0 + wave; j < j1; j += 8) {
+    dd2 v = dd2{0.0, 0.0};
+    if (j < d.have) {
+      v = *reinterpret_cast<const dd2*>(d.V + r0 + (int64_t)j * d.ld);
+    } else {
+      const int hot = d.idx[j - d.have];
+      if ((hot >> 1) == (int)(r0 >> 1)) v[hot & 1] = d.scale != nullptr ? d.scale[hot] : 1.0;
+    }
+    __builtin_nontemporal_store(v, reinterpret_cast<dd2*>(d.out + r0 + (int64_t)j * d.ld));
   }
 }
 
@@ -535,21 +556,46 @@ static int launch_apply(nnvhip_ctx* ctx, int64_t count, std::vector<ReluDesc>& d
   return NNVHIP_OK;
 }
 
-// implicit unit-vector columns of a set whose rows are in place: copy and append
-static int write_tail_columns(nnvhip_ctx* ctx, nnvhip_star* s) {
-  const int64_t have = s->stored_cols();
-  if (s->oh_idx == nullptr || s->oh_from != have || s->oh_scale != nullptr)
-    NNV_FAIL(NNVHIP_ERR_ARG, "internal: implicit columns without their description");
+// implicit unit-vector columns of sets whose rows are in place: copies with the columns appended, in one arena
+static int write_tail_columns(nnvhip_ctx* ctx, const std::vector<nnvhip_star*>& sets) {
+  int64_t total = 0, max_cols = 0, max_ld = 0;
+  for (auto* s : sets) {
+    if (s->oh_idx == nullptr || s->oh_from != s->stored_cols()) NNV_FAIL(NNVHIP_ERR_ARG, "internal: implicit columns without their description");
+    if (s->n + 1 >= (int64_t(1) << 31)) NNV_FAIL(NNVHIP_ERR_SHAPE, "too many predicate variables");
+    total += s->ld * (s->n + 1);
+    max_cols = std::max(max_cols, s->n + 1);
+    max_ld = std::max(max_ld, s->ld);
+  }
   BufRef full;
-  NNV_TRY(ctx->alloc(sizeof(double) * s->ld * (s->n + 1), &full));
-  NNV_HIP_TRY(hipMemcpyAsync(full->ptr, s->V, sizeof(double) * s->ld * have, hipMemcpyDeviceToDevice, ctx->stream));
-  const int m = (int)(s->n + 1 - have);
-  hipLaunchKernelGGL(onehot_columns_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(s->ld, 256), 64), (unsigned)std::min(m, 4096)),
-                     dim3(256), 0, ctx->stream, full->as<double>() + have * s->ld, s->ld, s->oh_idx, m);
-  NNV_HIP_TRY(hipGetLastError());
-  s->Vbuf = full;
-  s->V = full->as<double>();
-  s->vcols = -1;
+  NNV_TRY(ctx->alloc(sizeof(double) * total, &full));
+  std::vector<TailSet> ts(sets.size());
+  int64_t off = 0;
+  for (size_t i = 0; i < sets.size(); ++i) {
+    nnvhip_star* s = sets[i];
+    ts[i] = TailSet{s->V, full->as<double>() + off, s->oh_idx, s->oh_scale, s->ld, (int32_t)s->stored_cols(), (int32_t)(s->n + 1)};
+    off += s->ld * (s->n + 1);
+  }
+  const int64_t row_blocks = ceil_div(max_ld, 128);
+  int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(ceil_div(8192, row_blocks * (int64_t)sets.size()), ceil_div(max_cols, 16)));
+  const int64_t cpc = ceil_div(max_cols, chunks);
+  chunks = ceil_div(max_cols, cpc);
+  for (size_t i0 = 0; i0 < sets.size(); i0 += 65535) {
+    const size_t cnt = std::min<size_t>(65535, sets.size() - i0);
+    const TailSet* table = nullptr;
+    BufRef tab;
+    if (cnt > 1) {
+      NNV_TRY(ctx->upload_table(ts.data() + i0, sizeof(TailSet) * cnt, &tab));
+      table = tab->as<TailSet>();
+    }
+    hipLaunchKernelGGL(write_tail_kernel, dim3((unsigned)row_blocks, (unsigned)chunks, (unsigned)cnt), dim3(512), 0, ctx->stream, table,
+                       ts[i0], (int)cpc);
+    NNV_HIP_TRY(hipGetLastError());
+  }
+  for (size_t i = 0; i < sets.size(); ++i) {
+    sets[i]->Vbuf = full;
+    sets[i]->V = ts[i].out;
+    sets[i]->vcols = -1;
+  }
   return NNVHIP_OK;
 }
 
@@ -564,19 +610,18 @@ int ensure_dense_batch(nnvhip_ctx* ctx, int64_t count, nnvhip_star* const* sets,
     if (!cols.empty()) NNV_TRY(write_pending_columns(ctx, (int64_t)cols.size(), cols.data()));
   }
   // sets with a pending row reset: one arena and one apply launch per leading dimension
-  std::vector<nnvhip_star*> pend;
+  std::vector<nnvhip_star*> pend, tails;
   const uint64_t visit = ++ctx->visit_seq;  // (a handle may be listed twice)
   for (int64_t i = 0; i < count; ++i) {
     nnvhip_star* s = sets[i];
-    if (s->rows_pending) {
-      if (s->visit != visit) {
-        s->visit = visit;
-        pend.push_back(s);
-      }
-    } else if (need_tail && s->stored_cols() != s->n + 1) {
-      NNV_TRY(write_tail_columns(ctx, s));
-    }
+    if (s->visit == visit) continue;
+    s->visit = visit;
+    if (s->rows_pending)
+      pend.push_back(s);
+    else if (need_tail && s->stored_cols() != s->n + 1)
+      tails.push_back(s);
   }
+  if (!tails.empty()) NNV_TRY(write_tail_columns(ctx, tails));
   while (!pend.empty()) {
     std::vector<nnvhip_star*> grp, rest;
     for (auto* s : pend) (s->ld == pend[0]->ld ? grp : rest).push_back(s);

@@ -5,6 +5,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <map>
 
 #include "internal.h"
 
@@ -149,158 +150,155 @@ int nnvhip_star_create(nnvhip_ctx* c, int64_t N, int64_t n, const double* V, con
   return NNVHIP_OK;
 }
 
-__global__ void box_fill_kernel(double* __restrict__ V, int64_t ld, int N, const double* __restrict__ center,
-                                const double* __restrict__ vec, const int32_t* __restrict__ gen_dim,
-                                const int64_t* __restrict__ col_off, const int64_t* __restrict__ gen_off) {
-  // one block column per (set, column); rows across threads.  Column 0 is the centre; column
-  // 1+g holds vec(dim_g) at row dim_g and zeros elsewhere (diag(vec) with empty columns removed).
-  int set = blockIdx.z;
-  int64_t ncols = col_off[set + 1] - col_off[set];
-  for (int64_t j = blockIdx.y; j < ncols; j += gridDim.y) {
-    double* col = V + (col_off[set] + j) * ld;
-    int dim = j == 0 ? -1 : gen_dim[gen_off[set] + j - 1];
-    // two rows per thread, one 16-byte store (ld is even and every column starts on a 16-byte boundary)
-    for (int r = 2 * (blockIdx.x * blockDim.x + threadIdx.x); r < ld; r += 2 * gridDim.x * blockDim.x) {
-      double v[2] = {0.0, 0.0};
-#pragma unroll
-      for (int e = 0; e < 2; ++e)
-        if (r + e < N) {
-          if (j == 0) v[e] = center[(int64_t)set * N + r + e];
-          else if (r + e == dim) v[e] = vec[(int64_t)set * N + r + e];
-        }
-      *reinterpret_cast<double2*>(col + r) = make_double2(v[0], v[1]);
-    }
-  }
-}
-
-// info[2s] = offset of set s in the bounds buffer, info[2s+1] = its padded predicate count
-__global__ void fill_pm_one_kernel(double* __restrict__ bounds, const int64_t* __restrict__ info) {
-  const int64_t off = info[2 * blockIdx.y], n = info[2 * blockIdx.y + 1];
-  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) {
-    bounds[off + i] = -1.0;
-    bounds[off + n + i] = 1.0;
-  }
-}
-
+// Star(lb, ub) for every column of two N x count matrices.  A box's generators are scaled unit vectors, and the handle
+// says which (oh_idx, oh_scale): only the centres go to memory (vcols = 1), back to back, and whoever reads the whole
+// matrix has the columns written then (ensure_dense).  Everything the call puts on the device - centres, half-widths,
+// predicate bounds, index lists - is laid out in pinned memory and travels in one copy; no kernel runs.  (Writing the
+// matrices took 133 us for 100 boxes of 784 dimensions, 1.54 ms for 1024 of them, 6.4 GB nobody read; seven small
+// copies and kernels took 60 us of a single set's reach.)
 int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* lb, const double* ub,
                          nnvhip_star** out) {
   CHECK_CTX(c);
   if (!lb || !ub || !out) NNV_FAIL(NNVHIP_ERR_ARG, "null argument");
   if (N <= 0 || count <= 0 || count > 65535) NNV_FAIL(NNVHIP_ERR_SHAPE, "Inconsistent dimensions between lb and ub");
-  // Box constructor arithmetic on the host (set/Box.m:35-45): it decides the column count.
-  std::vector<double> center(N * count), vec(N * count);
-  std::vector<int32_t> gen_dim;
-  std::vector<int64_t> col_off(count + 1, 0), gen_off(count + 1, 0);
-  std::vector<char> neg_scale((size_t)count, 0);
+  const int64_t ld = round_up(N, kLdAlign);
   // Sets with the same half-widths, bit for bit (the boxes of a regular partition), share one scale vector and one
   // index list on the device: layers downstream recognise by the pointers that such sets gather the same scaled
   // weight columns.  shape_of[s] = the first set with set s's half-widths (among the first few distinct shapes).
-  std::vector<int64_t> shape_of((size_t)count);
-  std::vector<int64_t> shapes;
-  std::vector<uint64_t> shape_hash;
+  // Every shape that is not another set's has a record here.
+  struct Shape {
+    int64_t n = 0;        // dimensions with a width: generator columns
+    int64_t idx_of = -1;  // the shape whose index list it uses (its own, or the first one with all dimensions)
+    int64_t idx_off = 0, pb_off = 0;
+    bool neg = false;
+  };
+  std::vector<int64_t> shape_of((size_t)count);  // index into shapes
+  std::vector<Shape> shapes;
+  std::vector<double> vecs;  // half-widths of the shapes, ld apart
+  int64_t kept_shapes = 0;   // how many of them later sets are compared with
+  std::vector<double> vec((size_t)ld, 0.0);
+  // first pass: half-widths only (they decide the sizes); the centres are formed below, in their place
   for (int64_t s = 0; s < count; ++s) {
-    int64_t n = 0;
-    uint64_t hash = 0x9E3779B97F4A7C15ull;  // of the half-widths' bit patterns: vectors are compared only when it matches
-    for (int64_t i = 0; i < N; ++i) {
-      double l = lb[s * N + i], u = ub[s * N + i];
-      center[s * N + i] = 0.5 * (l + u);
-      double v = 0.5 * (u - l);
-      vec[s * N + i] = v;
-      uint64_t bits;
-      memcpy(&bits, &v, sizeof bits);
-      hash = (hash ^ bits) * 0x100000001B3ull;
-      hash ^= hash >> 29;
-      if (v < 0.0) neg_scale[s] = 1;
-      // zero columns are deleted only when the generator matrix has more than one element
-      if (v != 0.0 || N == 1) {
-        gen_dim.push_back((int32_t)i);
-        ++n;
+    const double *l = lb + s * N, *u = ub + s * N;
+    for (int64_t i = 0; i < N; ++i) vec[(size_t)i] = 0.5 * (u[i] - l[i]);  // Box constructor, set/Box.m:36
+    int64_t found = -1;
+    for (int64_t k = 0; k < kept_shapes && found < 0; ++k)
+      if (memcmp(&vecs[(size_t)(k * ld)], vec.data(), sizeof(double) * N) == 0) found = k;
+    if (found < 0) {
+      found = (int64_t)shapes.size();
+      Shape sh;
+      if (N == 1) {
+        sh.n = 1;  // zero columns are deleted only when the generator matrix has more than one element (set/Box.m:41-43)
+      } else {
+        for (int64_t i = 0; i < N; ++i) sh.n += vec[(size_t)i] != 0.0;
       }
+      for (int64_t i = 0; i < N; ++i) sh.neg = sh.neg || vec[(size_t)i] < 0.0;
+      shapes.push_back(sh);
+      vecs.insert(vecs.end(), vec.begin(), vec.end());
+      if (kept_shapes < 16 && found == kept_shapes) ++kept_shapes;
     }
-    gen_off[s + 1] = gen_off[s] + n;
-    col_off[s + 1] = col_off[s] + n + 1;
-    shape_of[s] = s;
-    for (size_t k = 0; k < shapes.size(); ++k)
-      if (shape_hash[k] == hash && memcmp(&vec[shapes[k] * N], &vec[s * N], sizeof(double) * N) == 0) {
-        shape_of[s] = shapes[k];
-        break;
-      }
-    if (shape_of[s] == s && shapes.size() < 16) {
-      shapes.push_back(s);
-      shape_hash.push_back(hash);
+    shape_of[(size_t)s] = found;
+  }
+  // layout of the one device block, in doubles: centres | half-widths by shape | predicate bounds by column count | lists
+  const int64_t vec_off = ld * count;
+  int64_t doubles = vec_off + ld * (int64_t)shapes.size();
+  std::map<int64_t, int64_t> pb_at;  // column count -> offset of its -1 / +1 vectors
+  for (Shape& sh : shapes) {
+    auto at = pb_at.find(sh.n);
+    if (at == pb_at.end()) {
+      at = pb_at.emplace(sh.n, doubles).first;
+      doubles += 2 * round_up(std::max<int64_t>(sh.n, 1), kLdAlign);
     }
+    sh.pb_off = at->second;
   }
-  int64_t ld = round_up(N, kLdAlign);
-  int64_t total_cols = col_off[count];
-  BufRef arena, dcenter, dvec, dgen, dcol, dgoff;
-  NNV_TRY(c->alloc(sizeof(double) * ld * total_cols, &arena));
-  NNV_TRY(c->upload(center.data(), sizeof(double) * center.size(), &dcenter));
-  NNV_TRY(c->upload(vec.data(), sizeof(double) * vec.size(), &dvec));
-  if (gen_dim.empty()) gen_dim.push_back(0);
-  NNV_TRY(c->upload(gen_dim.data(), sizeof(int32_t) * gen_dim.size(), &dgen));
-  NNV_TRY(c->upload(col_off.data(), sizeof(int64_t) * col_off.size(), &dcol));
-  NNV_TRY(c->upload(gen_off.data(), sizeof(int64_t) * gen_off.size(), &dgoff));
-  int64_t max_cols = 0;
-  for (int64_t s = 0; s < count; ++s) max_cols = std::max(max_cols, col_off[s + 1] - col_off[s]);
-  dim3 grid((unsigned)std::min<int64_t>(ceil_div(ld, 512), 64), (unsigned)std::min<int64_t>(max_cols, 4096),
-            (unsigned)count);
-  hipLaunchKernelGGL(box_fill_kernel, grid, dim3(256), 0, c->stream, arena->as<double>(), ld, (int)N,
-                     dcenter->as<double>(), dvec->as<double>(), dgen->as<int32_t>(), dcol->as<int64_t>(),
-                     dgoff->as<int64_t>());
-  NNV_HIP_TRY(hipGetLastError());
-  // predicate bounds -1/+1 for all sets in one buffer
-  int64_t npad_total = 0;
-  std::vector<int64_t> poff(count);
-  for (int64_t s = 0; s < count; ++s) {
-    poff[s] = npad_total;
-    npad_total += 2 * round_up(std::max<int64_t>(gen_off[s + 1] - gen_off[s], 1), kLdAlign);
+  int64_t ints = 0, full = -1;
+  for (size_t k = 0; k < shapes.size(); ++k) {
+    Shape& sh = shapes[k];
+    if (sh.n == N && full >= 0) {
+      sh.idx_of = full;
+      continue;
+    }
+    sh.idx_of = (int64_t)k;
+    sh.idx_off = ints;
+    ints += round_up(std::max<int64_t>(sh.n, 1), kLdAlign);
+    if (sh.n == N) full = (int64_t)k;
   }
-  BufRef pb;
-  NNV_TRY(c->alloc(sizeof(double) * npad_total, &pb));
+  // (sets whose whole matrices no reader could ever be given are refused here, as they were when they were written)
+  double whole = 0.0;
+  for (int64_t s = 0; s < count; ++s) whole += 8.0 * (double)ld * (double)(shapes[(size_t)shape_of[(size_t)s]].n + 1);
+  if (whole > (double)c->device_bytes) NNV_FAIL(NNVHIP_ERR_OOM, "out of device memory allocating %.0f bytes", whole);
+  const size_t bytes = sizeof(double) * (size_t)doubles + sizeof(int32_t) * (size_t)ints;
+  void* st = nullptr;
+  NNV_TRY(c->stage(bytes, &st));
+  BufRef buf;
+  NNV_TRY(c->alloc(bytes, &buf));
+  double* h = static_cast<double*>(st);
+  int32_t* hi = reinterpret_cast<int32_t*>(h + doubles);
   for (int64_t s = 0; s < count; ++s) {
-    nnvhip_star* st = new_star(c);
-    st->N = N;
-    st->n = gen_off[s + 1] - gen_off[s];
-    st->ld = ld;
-    st->Vbuf = arena;
-    st->V = arena->as<double>() + col_off[s] * ld;
-    st->pbuf = pb;
-    int64_t npad = round_up(std::max<int64_t>(st->n, 1), kLdAlign);
-    st->plb = pb->as<double>() + poff[shape_of[s]];  // (the same -1 / +1 for every set of the shape)
-    st->pub = st->plb + npad;
+    const double *l = lb + s * N, *u = ub + s * N;
+    double* col = h + s * ld;
+    for (int64_t i = 0; i < N; ++i) col[i] = 0.5 * (l[i] + u[i]);  // set/Box.m:35
+    for (int64_t i = N; i < ld; ++i) col[i] = 0.0;
+  }
+  memcpy(h + vec_off, vecs.data(), sizeof(double) * vecs.size());
+  for (const auto& pb : pb_at) {
+    const int64_t npad = round_up(std::max<int64_t>(pb.first, 1), kLdAlign);
+    std::fill(h + pb.second, h + pb.second + npad, -1.0);
+    std::fill(h + pb.second + npad, h + pb.second + 2 * npad, 1.0);
+  }
+  for (size_t k = 0; k < shapes.size(); ++k) {
+    const Shape& sh = shapes[k];
+    if (sh.idx_of != (int64_t)k) continue;
+    int32_t* list = hi + sh.idx_off;
+    int64_t t = 0;
+    for (int64_t i = 0; i < N; ++i)
+      if (N == 1 || vecs[k * ld + i] != 0.0) list[t++] = (int32_t)i;
+    for (const int64_t end = round_up(std::max<int64_t>(sh.n, 1), kLdAlign); t < end; ++t) list[t] = 0;
+  }
+  NNV_HIP_TRY(hipMemcpyAsync(buf->ptr, st, bytes, hipMemcpyHostToDevice, c->stream));
+  c->h2d_bytes += (int64_t)bytes;
+  double* d = buf->as<double>();
+  const int32_t* di = reinterpret_cast<const int32_t*>(d + doubles);
+  for (int64_t s = 0; s < count; ++s) {
+    const int64_t k = shape_of[(size_t)s];
+    const Shape& sh = shapes[(size_t)k];
+    nnvhip_star* o = new_star(c);
+    o->N = N;
+    o->n = sh.n;
+    o->ld = ld;
+    o->Vbuf = buf;
+    o->V = d + s * ld;
+    o->pbuf = buf;
+    o->plb = d + sh.pb_off;
+    o->pub = o->plb + round_up(std::max<int64_t>(sh.n, 1), kLdAlign);
     // C = zeros(1, n), d = 0 (set/Star.m:226-227): a base node with one all-zero row
     auto base = make_ref<ConsNode>();
     base->p_total = 1;
-    base->n_total = st->n;
-    st->cons = base;  // C0/d0 left null = all zeros
-    st->has_zono = true;  // Z = Zono(center, gens), set/Star.m:230-236
-    if (st->n > 0) {  // every generator column is vec(dim) * e_dim
-      st->oh_from = 1;
-      st->oh_idx_buf = dgen;
-      st->oh_idx = dgen->as<int32_t>() + gen_off[shape_of[s]];
-      st->oh_scale_buf = dvec;
-      st->oh_scale = dvec->as<double>() + shape_of[s] * N;
-      st->oh_scale_neg = neg_scale[s] != 0;
+    base->n_total = o->n;
+    o->cons = base;  // C0/d0 left null = all zeros
+    o->has_zono = true;  // Z = Zono(center, gens), set/Star.m:230-236
+    if (o->n > 0) {  // every generator column is vec(dim) * e_dim
+      o->vcols = 1;
+      o->oh_from = 1;
+      o->oh_idx_buf = buf;
+      o->oh_idx = di + shapes[(size_t)sh.idx_of].idx_off;
+      o->oh_scale_buf = buf;
+      o->oh_scale = d + vec_off + k * ld;
+      o->oh_scale_neg = sh.neg;
     }
-    out[s] = st;
+    out[s] = o;
   }
-  // one launch fills every set's bounds: lb half gets -1, ub half +1
-  {
-    std::vector<int64_t> pinfo((size_t)(2 * count));
-    int64_t max_npad = 0;
-    for (int64_t s = 0; s < count; ++s) {
-      pinfo[2 * s] = poff[s];
-      pinfo[2 * s + 1] = round_up(std::max<int64_t>(out[s]->n, 1), kLdAlign);
-      max_npad = std::max(max_npad, pinfo[2 * s + 1]);
-    }
-    BufRef dinfo;
-    NNV_TRY(c->upload(pinfo.data(), sizeof(int64_t) * pinfo.size(), &dinfo));
-    hipLaunchKernelGGL(fill_pm_one_kernel, dim3((unsigned)ceil_div(max_npad, 256), (unsigned)count), dim3(256), 0, c->stream,
-                       pb->as<double>(), dinfo->as<int64_t>());
-  }
-  NNV_HIP_TRY(hipGetLastError());
   return NNVHIP_OK;
+}
+
+// info[2k] = offset (in doubles) of block k, info[2k+1] = npad: lb half := -1, ub half := +1
+__global__ void fill_pm_one_kernel(double* __restrict__ bounds, const int64_t* __restrict__ info) {
+  const int64_t off = info[2 * blockIdx.y], npad = info[2 * blockIdx.y + 1];
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i < npad) {
+    bounds[off + i] = -1.0;
+    bounds[off + npad + i] = 1.0;
+  }
 }
 
 // Columns of the set the reduceMem suffix of the ReLU layer builds: column 0 the centre, column 1 + g the value
