@@ -347,6 +347,10 @@ enum { NNVHIP_LAYER_FC = 0, NNVHIP_LAYER_CONV2D = 1, NNVHIP_LAYER_RELU = 2 };
 NNVHIP_API int nnvhip_reach_layers(nnvhip_ctx* ctx, int64_t n_layers, const int32_t* kind, const void* const* layer,
                         const int64_t* hw, int order, double relax_factor, int64_t count, nnvhip_star* const* in,
                         nnvhip_star** out);
+/* *yes = 1 if nnvhip_reach_layers would run this layer list for these sets as one launch (a small FC / ReLU
+ * network), 0 if as the layer loop. */
+NNVHIP_API int nnvhip_reach_is_one_launch(nnvhip_ctx* ctx, int64_t n_layers, const int32_t* kind, const void* const* layer,
+                                          int order, int64_t count, nnvhip_star* const* in, int32_t* yes);
 /* PosLin.multipleStepReachStarApprox_at_one(I.resetRow(reset_rows), index, lb, ub),
  * nn/funcs/PosLin.m:685-742 and set/Star.m:1442-1461: the step with the lists handed in instead of
  * derived from estimateRanges -- what the relaxFactor < 1 branches call once the host LPs

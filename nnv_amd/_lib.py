@@ -28,7 +28,7 @@ SYMBOLS = [
     "nnvhip_avgpool2d_output_size", "nnvhip_affine_avgpool2d", "nnvhip_permute_rows",
     "nnvhip_star_fetch_rows", "nnvhip_relu_apply_lists", "nnvhip_probe_mfma_peak",
     "nnvhip_estimate_ranges_static", "nnvhip_debug_mailbox_pack", "nnvhip_debug_mailbox_unpack",
-    "nnvhip_debug_set_relu_call_number", "nnvhip_reach_layers", "nnvhip_relu_reduce_mem",
+    "nnvhip_debug_set_relu_call_number", "nnvhip_reach_layers", "nnvhip_reach_is_one_launch", "nnvhip_relu_reduce_mem",
     "nnvhip_set_switch", "nnvhip_hint_next_fc", "nnvhip_debug_counters", "nnvhip_debug_relu_bounds", "nnvhip_weight_cache_stats", "nnvhip_weight_cache_release", "nnvhip_debug_weak_weight_hash",
 ]
 
@@ -121,6 +121,7 @@ def load():
                                         C.POINTER(C.c_int32)],
         "nnvhip_debug_set_relu_call_number": [p, i64],
         "nnvhip_reach_layers": [p, i64, p, p, p, C.c_int, dbl, i64, pp, pp],
+        "nnvhip_reach_is_one_launch": [p, i64, p, p, C.c_int, i64, pp, C.POINTER(C.c_int32)],
         "nnvhip_relu_reduce_mem": [p, p, i64, i64, i64, pp, p, p],
         "nnvhip_set_switch": [p, C.c_char_p, C.c_int],
         "nnvhip_hint_next_fc": [p, p],

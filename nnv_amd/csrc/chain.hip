@@ -559,19 +559,31 @@ static bool plan_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, con
   return true;
 }
 
+// Whether the layer list runs as one launch for these sets, and the layout of its arenas if so.
+static bool chain_takes(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, int order, int64_t count,
+                        nnvhip_star* const* in, ChainPlan* plan) {
+  if (!c->small_chain || c->dense_affine || count < 1 || count > 65535) return false;
+  if (order != NNVHIP_ORDER_INDEX && order != NNVHIP_ORDER_AREA && order != NNVHIP_ORDER_RANGE) return false;
+  int64_t n0_max = 0;
+  for (int64_t i = 0; i < count; ++i) {
+    if (!in[i] || in[i]->ctx != c || in[i]->N != in[0]->N) return false;  // the layer loop reports it
+    n0_max = std::max(n0_max, in[i]->n);
+  }
+  if (!plan_chain(c, n_layers, kind, layer, in[0]->N, n0_max, plan)) return false;
+  return (double)plan->doubles * (double)count <= 5.0e8;  // 4 GB of worst-case buffers
+}
+
+bool small_chain_takes(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, int order, int64_t count,
+                       nnvhip_star* const* in) {
+  ChainPlan plan;
+  return chain_takes(c, n_layers, kind, layer, order, count, in, &plan);
+}
+
 int reach_small_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, int order, int64_t count,
                       nnvhip_star* const* in, nnvhip_star** out, bool* taken) {
   *taken = false;
-  if (!c->small_chain || c->dense_affine || count > 65535) return NNVHIP_OK;
-  if (order != NNVHIP_ORDER_INDEX && order != NNVHIP_ORDER_AREA && order != NNVHIP_ORDER_RANGE) return NNVHIP_OK;
-  int64_t n0_max = 0;
-  for (int64_t i = 0; i < count; ++i) {
-    if (!in[i] || in[i]->ctx != c || in[i]->N != in[0]->N) return NNVHIP_OK;  // the layer loop reports it
-    n0_max = std::max(n0_max, in[i]->n);
-  }
   ChainPlan plan;
-  if (!plan_chain(c, n_layers, kind, layer, in[0]->N, n0_max, &plan)) return NNVHIP_OK;
-  if ((double)plan.doubles * (double)count > 5.0e8) return NNVHIP_OK;  // 4 GB of worst-case buffers
+  if (!chain_takes(c, n_layers, kind, layer, order, count, in, &plan)) return NNVHIP_OK;
   *taken = true;
 
   // boxes go in as they are where the first layer is an FC layer
@@ -621,6 +633,10 @@ int reach_small_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, cons
   }
   NNV_LAUNCH(c, c->kernel_timing, reach_chain_kernel, dim3((unsigned)count), dim3(kChainThreads), 0, table, sets[0], a);
   NNV_HIP_TRY(hipGetLastError());
+  // Handles of earlier arrays that were released but not let go yet go now, all of them, while the kernel runs: their
+  // arenas are what the next call of this size takes (a thousand sets come to a gigabyte, and a queue that grows from
+  // call to call would have the pool ask the driver for another one each time).
+  c->drain_deferred();
 
   // the crossing counts: all the host needs to know to fill in the handles
   std::vector<int32_t> counts((size_t)(2 * n_layers * count), 0);

@@ -904,6 +904,8 @@ int materialize_constraints(const nnvhip_star* s, double* C_host, double* d_host
 
 // chain.hip: the layer loop of a small FC / ReLU network as one launch (one block per set).  *taken = false:
 // not applicable (nothing was done; the caller runs the layer loop).  out: n_layers x count handles.
+bool small_chain_takes(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, int order, int64_t count,
+                       nnvhip_star* const* in);
 int reach_small_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, int order, int64_t count,
                       nnvhip_star* const* in, nnvhip_star** out, bool* taken);
 

@@ -201,6 +201,14 @@ int nnvhip_relu_relax(nnvhip_ctx* c, int order, double relax_factor, int64_t cou
   return c->end_op();
 }
 
+int nnvhip_reach_is_one_launch(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, int order, int64_t count,
+                               nnvhip_star* const* in, int32_t* yes) {
+  if (!c) NNV_FAIL(NNVHIP_ERR_ARG, "null context");
+  if (n_layers < 1 || count <= 0 || !in || !kind || !layer || !yes) NNV_FAIL(NNVHIP_ERR_ARG, "null argument");
+  *yes = small_chain_takes(c, n_layers, kind, layer, order, count, in) ? 1 : 0;
+  return NNVHIP_OK;
+}
+
 int nnvhip_reach_layers(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, const int64_t* hw,
                         int order, double relax_factor, int64_t count, nnvhip_star* const* in, nnvhip_star** out) {
   if (!c) NNV_FAIL(NNVHIP_ERR_ARG, "null context");

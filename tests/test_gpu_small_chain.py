@@ -178,3 +178,16 @@ def test_networks_beyond_the_limits_take_the_layer_loop(nnv, oracle):
     c = rs.rand(20) - 0.5
     _check_against_oracle(nnv, oracle, layers, nnv.Star(c - 0.01, c + 0.01), oracle.star_from_box(c - 0.01, c + 0.01),
                           "relax-star-area", expect_chain=False)
+
+
+@pytest.mark.parametrize("count", [63, 64, 65, 300])
+def test_arrays_of_any_size_take_the_one_launch(nnv, oracle, count):
+    """64 sets and more (where larger networks leave the one-call path), 256 and more (whose handles are released
+    later); partly boxes without width in some dimensions, so that the sets have different predicate counts."""
+    rs = np.random.RandomState(count)
+    layers = _net(rs, [6, 24, 17, 5])
+    lbs = rs.randn(6, count) * 0.3
+    ubs = lbs + 0.4 * rs.rand(6, count) * (rs.rand(6, count) < 0.8)
+    for _ in range(2):
+        _check_against_oracle(nnv, oracle, layers, nnv.Star.from_boxes(lbs, ubs), [oracle.star_from_box(lbs[:, i], ubs[:, i]) for i in range(count)],
+                              "relax-star-area")
