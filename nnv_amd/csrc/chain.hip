@@ -725,6 +725,7 @@ int reach_small_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, cons
         o->n_crossing = m;
         o->pre_ub_buf = arena;
         o->pre_ub = prev_ub ? prev_ub : A + L.rng_off + L.ld;
+        o->pre_lb = o->pre_ub - L.ld;  // (lb in front of ub, ld apart)
         o->n_kept = L.M - m - inact;
         o->kept_buf = iarena;
         o->kept_idx = IA + L.idx_off + L.ld;

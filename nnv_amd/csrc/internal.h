@@ -458,9 +458,10 @@ struct nnvhip_star {
   nnvhip::BufRef rbuf;
   double* lb = nullptr;
   double* ub = nullptr;
-  // set by the ReLU step: the estimated upper bounds of its input, by neuron (the range buffer is kept alive)
+  // set by the ReLU step: the estimated bounds of its input, by neuron (the range buffer is kept alive)
   nnvhip::BufRef pre_ub_buf;
   const double* pre_ub = nullptr;
+  const double* pre_lb = nullptr;
   // filled for sets produced by the ReLU step
   int64_t n_inactive = -1;
   int64_t n_crossing = -1;

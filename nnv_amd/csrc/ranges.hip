@@ -1201,16 +1201,72 @@ static int compute_box_ranges(nnvhip_ctx* ctx, const std::vector<nnvhip_star*>& 
   return NNVHIP_OK;
 }
 
+// Ranges of a ReLU step's output from the ranges it classified by: an inactive row is zero, a crossing row is the unit
+// vector of its own predicate (bounds 0 and ub), every other row is the input's row with the input's bounds.  So the
+// output's matrix is not asked for: no row reset, no appended columns, no scan (CNN 28x28x1, bounds of all layers: 120 us
+// of kernels that wrote and read two 90 MB matrices).
+struct ReluRange {
+  const double* lb_in;
+  const double* ub_in;
+  double* lb;
+  double* ub;
+  int32_t N;
+};
+__global__ __launch_bounds__(256) void relu_ranges_kernel(const ReluRange* __restrict__ table, ReluRange one) {
+  const ReluRange d = table ? table[blockIdx.y] : one;
+  const int r = blockIdx.x * 256 + threadIdx.x;
+  if (r >= d.N) return;
+  const double lo = d.lb_in[r], up = d.ub_in[r];
+  const bool inactive = up <= 0.0, crossing = lo < 0.0 && up > 0.0;
+  d.lb[r] = inactive || crossing ? 0.0 : lo;
+  d.ub[r] = inactive ? 0.0 : up;
+}
+
+static int compute_relu_ranges(nnvhip_ctx* ctx, const std::vector<nnvhip_star*>& sets) {
+  int64_t doubles = 0, max_N = 0;
+  for (auto* t : sets) {
+    doubles += 2 * t->ld;
+    max_N = std::max(max_N, t->N);
+  }
+  BufRef rb, tab;
+  NNV_TRY(ctx->alloc(sizeof(double) * doubles, &rb));
+  std::vector<ReluRange> rr;
+  rr.reserve(sets.size());
+  double* at = rb->as<double>();
+  for (auto* t : sets) {
+    rr.push_back(ReluRange{t->pre_lb, t->pre_ub, at, at + t->ld, (int32_t)t->N});
+    at += 2 * t->ld;
+  }
+  for (size_t i0 = 0; i0 < rr.size(); i0 += 65535) {
+    const size_t cnt = std::min<size_t>(65535, rr.size() - i0);
+    const ReluRange* table = nullptr;
+    if (cnt > 1) {
+      NNV_TRY(ctx->upload_table(rr.data() + i0, sizeof(ReluRange) * cnt, &tab));
+      table = tab->as<ReluRange>();
+    }
+    hipLaunchKernelGGL(relu_ranges_kernel, dim3((unsigned)ceil_div(max_N, 256), (unsigned)cnt), dim3(256), 0, ctx->stream, table, rr[i0]);
+    NNV_HIP_TRY(hipGetLastError());
+  }
+  for (size_t i = 0; i < sets.size(); ++i) {
+    sets[i]->rbuf = rb;
+    sets[i]->lb = rr[i].lb;
+    sets[i]->ub = rr[i].ub;
+  }
+  return NNVHIP_OK;
+}
+
 int compute_ranges(nnvhip_ctx* ctx, int64_t count, nnvhip_star* const* s, RangeCounts* counts) {
-  // sets that already carry ranges are skipped, boxes with nothing but a centre in memory go by a kernel of their own
-  std::vector<nnvhip_star*> todo, boxes;
+  // sets that already carry ranges are skipped; boxes with nothing but a centre in memory and outputs of a ReLU step go
+  // by kernels of their own
+  std::vector<nnvhip_star*> todo, boxes, relus;
   todo.reserve((size_t)count);
   const uint64_t visit = ++ctx->visit_seq;  // (a handle may be listed twice)
   for (int64_t i = 0; i < count; ++i)
     if (!s[i]->lb && s[i]->visit != visit) {
       s[i]->visit = visit;
-      (is_unwritten_box(s[i]) ? boxes : todo).push_back(s[i]);
+      (is_unwritten_box(s[i]) ? boxes : s[i]->pre_lb != nullptr ? relus : todo).push_back(s[i]);
     }
+  if (!relus.empty()) NNV_TRY(compute_relu_ranges(ctx, relus));
   if (!boxes.empty()) NNV_TRY(compute_box_ranges(ctx, boxes));
   if (todo.empty()) return NNVHIP_OK;
   // Sets whose generator images are in memory inside their windows only are scanned inside the windows (all
@@ -1503,6 +1559,7 @@ int ranges_into_static(nnvhip_ctx* ctx, const nnvhip_star* s, double* lb_dev, do
                              "nnvhip_estimate_ranges)");
   const int64_t ld = s->ld, n = s->n;
   if (n >= (int64_t(1) << 31)) NNV_FAIL(NNVHIP_ERR_SHAPE, "too many predicate variables");
+  const bool relu_out = s->pre_lb != nullptr && 2 * ld <= ctx->static_scratch_doubles;  // (the same values nnvhip_estimate_ranges gives)
   // workspace: lb (ld), ub (ld), then chunks x [4][ld] partial sums
   if (6 * ld > ctx->static_scratch_doubles)
     NNV_FAIL(NNVHIP_ERR_SHAPE, "nnvhip_estimate_ranges_static: a set of dimension %lld does not fit the static workspace "
@@ -1526,9 +1583,13 @@ int ranges_into_static(nnvhip_ctx* ctx, const nnvhip_star* s, double* lb_dev, do
   std::lock_guard<std::mutex> lock(g_static_use_mutex);
   StaticUse& use = g_static_use[ctx->device];
   if (use.last != nullptr && use.last != ctx) NNV_HIP_TRY(hipStreamWaitEvent(ctx->stream, use.done, 0));
-  hipLaunchKernelGGL((ranges_partial_kernel<8, 4>), dim3((unsigned)row_blocks, (unsigned)chunks, 1), dim3(64 * kRangeWaves), 0,
-                     ctx->stream, nullptr, d);
-  if (chunks > 1)
+  if (relu_out)
+    hipLaunchKernelGGL(relu_ranges_kernel, dim3((unsigned)ceil_div(s->N, 256)), dim3(256), 0, ctx->stream, nullptr,
+                       ReluRange{s->pre_lb, s->pre_ub, d.lb, d.ub, (int32_t)s->N});
+  else
+    hipLaunchKernelGGL((ranges_partial_kernel<8, 4>), dim3((unsigned)row_blocks, (unsigned)chunks, 1), dim3(64 * kRangeWaves), 0,
+                       ctx->stream, nullptr, d);
+  if (chunks > 1 && !relu_out)
     hipLaunchKernelGGL(ranges_final_kernel<1>, dim3((unsigned)ceil_div(ld, 64), 1, 1), dim3(256), 0, ctx->stream, nullptr, d);
   hipLaunchKernelGGL(copy_ranges_kernel, dim3((unsigned)ceil_div(s->N, 256)), dim3(256), 0, ctx->stream, d.lb, d.ub, lb_dev, ub_dev,
                      s->N);

@@ -1079,9 +1079,10 @@ int relu_relax(nnvhip_ctx* ctx, int order, int64_t count, nnvhip_star* const* in
     o->pub = d.pub_out;
     o->n_inactive = counts[2 * i + 1];
     o->n_crossing = d.m;
-    if (given == nullptr) {  // the input's estimated upper bounds, by neuron
+    if (given == nullptr) {  // the input's estimated bounds, by neuron
       o->pre_ub_buf = in[i]->rbuf;
       o->pre_ub = in[i]->ub;
+      o->pre_lb = in[i]->lb;
     }
     if (ahead_mm) {
       o->ahead_mm_buf = ahead_mm;

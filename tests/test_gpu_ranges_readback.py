@@ -57,3 +57,35 @@ def test_a_box_is_written_when_its_matrix_is_read(N, count, all_wide):
         assert np.array_equal(sets[i].V, exp[i].V) and np.array_equal(fresh[i].V, exp[i].V)
         assert_close(mapped[i].V, oracle.affine_map(exp[i], W, b).V, "W * box")
         assert np.array_equal(relu[i].V, oracle.reach_relaxed_star(exp[i], "relax-star-area").V)
+
+
+@pytest.mark.parametrize("N,count", [(1, 1), (255, 1), (257, 3), (2500, 1)])
+@pytest.mark.parametrize("eager", [False, True])
+def test_ranges_of_a_relu_output_come_from_its_input(N, count, eager):
+    """Ranges of a ReLU step's output without its matrix: against the scan of that matrix by the oracle, with the matrix
+    written by the step or not, one-block and multi-block classification."""
+    import nnv_amd as nnv
+    from oracle import nnv_oracle as oracle
+    from tests.gpu_util import assert_close_elementwise
+    rs = np.random.RandomState(N + count)
+    ctx = nnv.default_context()
+    n = 9
+    sets, exp = [], []
+    for _ in range(count):
+        V = rs.randn(N, n + 1)
+        V[rs.rand(N) < 0.1] = 0.0                    # rows with lb = ub = 0
+        V[:, 1:] *= 0.3
+        C, d, pl, pu = np.zeros((1, n)), np.zeros(1), -rs.rand(n), rs.rand(n)
+        sets.append(nnv.Star(V, C, d, pl, pu))
+        exp.append(oracle.reach_relaxed_star(oracle.OStar(V, C, d, pl, pu), "relax-star-area"))
+    ctx.set_eager_relu(eager)
+    try:
+        out = nnv.ReluLayer().reach(sets, "relax-star-area", [], 1)
+    finally:
+        ctx.set_eager_relu(False)
+    lb, ub = nnv.Star.estimateRanges_array(out)
+    for i in range(count):
+        ol, ou = oracle.estimate_ranges(exp[i])
+        assert_close_elementwise(lb[:, i], ol, "lb")
+        assert_close_elementwise(ub[:, i], ou, "ub")
+        assert np.array_equal(out[i].V, exp[i].V)
