@@ -588,8 +588,7 @@ int reach_small_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, cons
 
   // boxes go in as they are where the first layer is an FC layer
   auto as_box = [&](const nnvhip_star* s) {
-    return kind[0] == NNVHIP_LAYER_FC && !s->rows_pending && !s->cs.any_pending() && s->n > 0 && s->stored_cols() == 1 && s->oh_from == 1 &&
-           s->oh_idx != nullptr && s->oh_scale != nullptr;
+    return kind[0] == NNVHIP_LAYER_FC && is_unwritten_box(s);
   };
   {
     std::vector<nnvhip_star*> full;

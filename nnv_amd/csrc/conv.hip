@@ -933,6 +933,28 @@ int launch_conv_boxes(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int64
   return NNVHIP_OK;
 }
 
+int launch_pool_boxes(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t Wo, const int64_t pool[2], const int64_t stride[2],
+                      int64_t pad_top, int64_t pad_left, const ColBox* in_box, int64_t dense, const int32_t* onehot_idx, int64_t m,
+                      ColBox* out_box) {
+  ConvGeom g{};
+  g.H = (int)H;
+  g.W = (int)W;
+  g.Ho = (int)Ho;
+  g.Wo = (int)Wo;
+  g.FH = (int)pool[0];
+  g.FW = (int)pool[1];
+  g.sh = (int)stride[0];
+  g.sw = (int)stride[1];
+  g.dh = g.dw = 1;
+  g.pt = (int)pad_top;
+  g.pl = (int)pad_left;
+  g.HW = (int)(H * W);
+  hipLaunchKernelGGL(conv_boxes_kernel, dim3((unsigned)ceil_div(dense + m, 256)), dim3(256), 0, ctx->stream, in_box, dense, onehot_idx, m,
+                     out_box, g);
+  NNV_HIP_TRY(hipGetLastError());
+  return NNVHIP_OK;
+}
+
 bool conv2d_in_windows(const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldin, int64_t ncols,
                        const ColBox* out_box, int eh, int ew) {
   ConvGeom g;

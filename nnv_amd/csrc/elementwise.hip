@@ -10,16 +10,22 @@
 // Geometry of every kernel: a lane owns two adjacent rows, the eight waves of a block interleave
 // columns; grid = (row blocks, column chunks, sets).
 #include <algorithm>
+#include <cmath>
+#include <map>
 #include <memory>
 #include <vector>
 
 #include "internal.h"
+#include "relu_sort.h"
 
 struct nnvhip_rowmap {
   nnvhip_ctx* ctx = nullptr;
   int64_t N = 0, ld = 0;
   int32_t n_steps = 0;
   int32_t op[8] = {0}, scope[8] = {0};
+  bool keeps_zeros = true;   // the steps on all columns leave a zero generator entry zero (products and quotients by finite
+                             // numbers, divisors not zero)
+  bool may_flip = false;     // ... and some of them are negative
   nnvhip::BufRef params;  // ld x n_steps, zero padded rows
 };
 
@@ -96,6 +102,69 @@ __global__ __launch_bounds__(64 * kEwWaves) void rowmap_kernel(const SetDesc* __
   }
 }
 
+// ---- generators that are known to be sparse --------------------------------------------------------------------
+// The generator images behind a normalisation or an average pooling are as sparse as the ones in front of it: a row map
+// scales them where they are, a pooling moves a window to the positions whose cells reach it.  The kernels below work
+// inside the windows (nnvhip_star::box) and leave the zeros around them to a reader of whole columns (ColSource::win_*),
+// as a convolution does.  A block takes a few columns and its threads their window places (position and channel), so a
+// column costs eh * ew * C elements instead of the image; column 0, the centre, is a whole image and has the first blocks.
+// What bounds them is the latency of scattered 16-40 byte pieces, not bytes.  A 32x32x3 CNN with
+// normalisation and pooling (3073-3362 columns): batch normalisation 63 -> 9 us, row reset and pooling 48 + 51 -> 13 and
+// 30 + 41 -> 22 us, and the convolutions in between stay inside windows too (162 -> 24, 83 -> 14 us).
+struct WinArgs {
+  const double* in;
+  double* out;
+  const ColBox* box;       // windows of the output's columns
+  int64_t ldin, ldout;
+  int32_t eh, area;        // bound on a window: eh rows, area = eh * ew positions
+  int32_t C;
+  int32_t ncols;           // columns of the output
+  int32_t centre_blocks;   // the first blocks do column 0, 256 rows each ...
+  int32_t cols_per_block;  // ... the others so many generator columns each
+};
+
+__global__ __launch_bounds__(256) void rowmap_window_kernel(WinArgs w, RowmapArgs a, int H, int HW) {
+  if ((int)blockIdx.x < w.centre_blocks) {
+    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (r >= w.ldout) return;
+    double x = w.in[r];
+    for (int s = 0; s < a.n_steps; ++s) x = apply_op(a.op[s], x, a.params[(int64_t)s * a.ld + r]);
+    w.out[r] = x;
+    return;
+  }
+  const int j0 = 1 + ((int)blockIdx.x - w.centre_blocks) * w.cols_per_block;
+  const int per = w.area * w.C, items = per * min(w.cols_per_block, w.ncols - j0);
+  for (int f = threadIdx.x; f < items; f += 256) {
+    const int jj = f / per, e = f - jj * per, j = j0 + jj;
+    const int c = e / w.area, t = e - c * w.area;
+    const int dw = t / w.eh, dh = t - dw * w.eh;
+    const ColBox b = w.box[j];
+    const int h = b.h0 + dh, x = b.w0 + dw;
+    if (h > b.h1 || x > b.w1) continue;
+    const int64_t r = (int64_t)c * HW + x * H + h;
+    double v = w.in[r + (int64_t)j * w.ldin];
+    for (int s = 0; s < a.n_steps; ++s)
+      if (a.scope[s] == NNVHIP_SCOPE_ALL) v = apply_op(a.op[s], v, a.params[(int64_t)s * a.ld + r]);
+    w.out[r + (int64_t)j * w.ldout] = v;
+  }
+}
+
+// Centre and scales of boxes of which nothing else is in memory: blockIdx.y = vector (sets' centres, then scale vectors).
+struct VecMap {
+  const double* in;
+  double* out;
+  int32_t centre;  // 1: every step applies
+};
+__global__ __launch_bounds__(256) void rowmap_vectors_kernel(const VecMap* __restrict__ table, RowmapArgs a) {
+  const VecMap d = table[blockIdx.y];
+  const int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (r >= a.ld) return;
+  double x = d.in[r];
+  for (int s = 0; s < a.n_steps; ++s)
+    if (d.centre || a.scope[s] == NNVHIP_SCOPE_ALL) x = apply_op(a.op[s], x, a.params[(int64_t)s * a.ld + r]);
+  d.out[r] = x;
+}
+
 struct PoolArgs {
   int64_t ldin, ldout;
   int32_t H, W, C, Ho, Wo;
@@ -159,6 +228,71 @@ __global__ __launch_bounds__(64 * kEwWaves) void avgpool_kernel(const SetDesc* _
       for (int u = 0; u < 4; ++u) acc[u] = __dmul_rn(acc[u], scale);
     }
     for (int u = 0; u < nu; ++u) d.out[r + (int64_t)(jb + u) * a.ldout] = acc[u];  // padding rows stay zero
+  }
+}
+
+// What the pooling reads besides whole columns: windows of the input's dense columns, the classes of a pending row reset
+// (rows other than kKeep read as zero), the list of unit-vector columns.
+struct PoolIn {
+  const ColBox* box;       // by input column, for 1 <= j < dense; or null (dense == 1)
+  const int32_t* cls;      // or null
+  const int32_t* idx;      // column dense + t is scale[idx[t]] (1 without scales) at row idx[t]
+  const double* scale;
+  int32_t dense;
+};
+
+// Sums run as in avgpool_kernel (window columns outer, rows inner); what lies outside an input window adds an exact zero
+// and is left out.
+__global__ __launch_bounds__(256) void avgpool_window_kernel(WinArgs w, PoolArgs a, PoolIn s) {
+  const int HW = a.H * a.W, P = a.Ho * a.Wo;
+  auto cell = [&](int ho, int wo, int& y1, int& y2, int& x1, int& x2) {
+    y1 = ho * a.sh - a.pt;
+    x1 = wo * a.sw - a.pl;
+    y2 = min(y1 + a.ph, a.H);
+    x2 = min(x1 + a.pw, a.W);
+    y1 = max(y1, 0);
+    x1 = max(x1, 0);
+    return 1.0 / (double)((y2 - y1) * (x2 - x1));
+  };
+  if ((int)blockIdx.x < w.centre_blocks) {
+    const int r = (int)blockIdx.x * 256 + (int)threadIdx.x;
+    if (r >= P * w.C) return;
+    const int c = r / P, p = r - c * P, wo = p / a.Ho, ho = p - wo * a.Ho;
+    int y1, y2, x1, x2;
+    const double scale = cell(ho, wo, y1, y2, x1, x2);
+    double acc = 0.0;
+    for (int x = x1; x < x2; ++x)
+      for (int y = y1; y < y2; ++y) {
+        const int64_t q = (int64_t)c * HW + x * a.H + y;
+        acc = __dadd_rn(acc, s.cls == nullptr || s.cls[q] == kKeep ? w.in[q] : 0.0);
+      }
+    w.out[r] = __dmul_rn(acc, scale);
+    return;
+  }
+  const int j0 = 1 + ((int)blockIdx.x - w.centre_blocks) * w.cols_per_block;
+  const int per = w.area * w.C, items = per * min(w.cols_per_block, w.ncols - j0);
+  for (int f = threadIdx.x; f < items; f += 256) {
+    const int jj = f / per, e = f - jj * per, j = j0 + jj;
+    const int c = e / w.area, t = e - c * w.area;
+    const int dw = t / w.eh, dh = t - dw * w.eh;
+    const ColBox b = w.box[j];
+    const int ho = b.h0 + dh, wo = b.w0 + dw;
+    if (ho > b.h1 || wo > b.w1) continue;
+    int y1, y2, x1, x2;
+    const double scale = cell(ho, wo, y1, y2, x1, x2);
+    double acc = 0.0;
+    if (j < s.dense) {
+      const ColBox q = s.box[j];
+      const double* col = w.in + (int64_t)j * w.ldin + (int64_t)c * HW;
+      for (int x = max(x1, (int)q.w0); x < min(x2, q.w1 + 1); ++x)
+        for (int y = max(y1, (int)q.h0); y < min(y2, q.h1 + 1); ++y)
+          acc = __dadd_rn(acc, s.cls == nullptr || s.cls[(int64_t)c * HW + x * a.H + y] == kKeep ? col[x * a.H + y] : 0.0);
+    } else {
+      const int src = s.idx[j - s.dense];
+      const int sc = src / HW, sp = src - sc * HW, sx = sp / a.H, sy = sp - sx * a.H;
+      if (sc == c && sx >= x1 && sx < x2 && sy >= y1 && sy < y2) acc = s.scale != nullptr ? s.scale[src] : 1.0;
+    }
+    w.out[(int64_t)c * P + wo * a.Ho + ho + (int64_t)j * w.ldout] = __dmul_rn(acc, scale);
   }
 }
 
@@ -284,6 +418,212 @@ static int run_row_layer(nnvhip_ctx* c, int64_t count, nnvhip_star* const* in, n
   return NNVHIP_OK;
 }
 
+// Marks a set's generator columns as written inside their windows only and launches nothing; the padding rows are zeroed.
+static int leave_outside_windows(nnvhip_ctx* c, nnvhip_star* o, int64_t H, int64_t W) {
+  const int64_t ncols = o->n;  // columns 1 .. n
+  o->cs.win_box_buf = o->box_buf;
+  o->cs.win_box = o->box;
+  o->cs.win_from = 1;
+  o->cs.win_to = o->n + 1;
+  o->cs.win_rows = o->N;
+  o->cs.win_H = (int32_t)H;
+  o->cs.win_W = (int32_t)W;
+  if (c->poison_pending)  // debugging aid: NaNs where nothing will be written
+    NNV_HIP_TRY(hipMemsetAsync(o->V + o->ld, 0xff, sizeof(double) * o->ld * ncols, c->stream));
+  if (o->ld != o->N) NNV_TRY(launch_zero_pad_rows(c, o->V, o->ld, o->N, ncols + 1));
+  return NNVHIP_OK;
+}
+
+static WinArgs win_args(const nnvhip_star* in, const nnvhip_star* o, int64_t C, dim3* grid) {
+  WinArgs w{};
+  w.in = in->V;
+  w.out = o->V;
+  w.box = o->box;
+  w.ldin = in->ld;
+  w.ldout = o->ld;
+  w.eh = o->box_eh;
+  w.area = o->box_eh * o->box_ew;
+  w.C = (int32_t)C;
+  w.ncols = (int32_t)(o->n + 1);
+  // a block: the columns that make two to four elements a thread, one column at least
+  w.cols_per_block = (int32_t)std::max<int64_t>(1, 1024 / std::max<int64_t>(1, (int64_t)w.area * C));
+  w.centre_blocks = (int32_t)ceil_div(o->ld, 256);
+  *grid = dim3((unsigned)(w.centre_blocks + ceil_div(o->n, w.cols_per_block)));
+  return w;
+}
+
+static bool small_windows(int64_t eh, int64_t ew, int64_t P) { return eh > 0 && ew > 0 && 2 * eh * ew <= P; }
+static bool windows_allowed(const nnvhip_ctx* c) { return !c->eager_cols && !c->dense_affine && !c->no_conv_boxes; }
+
+// Row map of an image set whose generator images are zero outside small windows, every column of which is in memory there.
+static bool rowmap_in_windows(const nnvhip_ctx* c, const nnvhip_rowmap* m, const nnvhip_star* s) {
+  if (!windows_allowed(c) || !m->keeps_zeros || s->rows_pending || s->stored_cols() != s->n + 1 || s->n < 1) return false;
+  if (s->box == nullptr || s->box_cols < s->n + 1 || s->box_H <= 0 || s->box_W <= 0) return false;
+  const int64_t P = (int64_t)s->box_H * s->box_W;
+  return s->N % P == 0 && small_windows(s->box_eh, s->box_ew, P) && !s->cs.pending && s->cs.zero_to <= 1 && !s->cs.delta_pending() &&
+         s->n < 1000000;
+}
+
+static int rowmap_windows(nnvhip_ctx* c, const RowmapArgs& a, int64_t N, int64_t count, nnvhip_star* const* in, nnvhip_star** out) {
+  std::vector<nnvhip_star*> outs;
+  bool contig = false;
+  int64_t cols = 0;
+  NNV_TRY(c->begin_op());
+  int st = make_affine_outputs(c, count, in, N, &outs, &contig, &cols);
+  for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i) {
+    nnvhip_star* o = outs[i];
+    o->box_buf = in[i]->box_buf;
+    o->box = in[i]->box;
+    o->box_cols = in[i]->box_cols;
+    o->box_H = in[i]->box_H;
+    o->box_W = in[i]->box_W;
+    o->box_eh = in[i]->box_eh;
+    o->box_ew = in[i]->box_ew;
+    const int64_t HW = (int64_t)o->box_H * o->box_W;
+    st = leave_outside_windows(c, o, o->box_H, o->box_W);
+    dim3 grid;
+    const WinArgs w = win_args(in[i], o, N / HW, &grid);
+    if (st == NNVHIP_OK) {
+      NNV_LAUNCH(c, c->kernel_timing, rowmap_window_kernel, grid, dim3(256), 0, w, a, (int)o->box_H, (int)HW);
+      st = c->kernel_timer_end(c->kernel_timing, 4, 16.0 * ((double)w.area * w.C * (double)o->n + (double)N));
+    }
+    if (st == NNVHIP_OK && hipGetLastError() != hipSuccess) {
+      set_error("kernel launch failed");
+      st = NNVHIP_ERR_HIP;
+    }
+  }
+  if (st == NNVHIP_OK) st = c->end_op();
+  if (st != NNVHIP_OK) {
+    release_all(outs);
+    return st;
+  }
+  for (int64_t i = 0; i < count; ++i) out[i] = outs[i];
+  return NNVHIP_OK;
+}
+
+// Row map of boxes of which only the centres are in memory: the same boxes with mapped centres and scales (a scale vector
+// shared by several sets is mapped once and stays shared).
+static int rowmap_boxes(nnvhip_ctx* c, const RowmapArgs& a, bool may_flip, int64_t N, int64_t count, nnvhip_star* const* in,
+                        nnvhip_star** out) {
+  const int64_t ld = a.ld;
+  NNV_TRY(c->begin_op());
+  std::map<const double*, int64_t> scale_at;
+  for (int64_t i = 0; i < count; ++i) scale_at.emplace(in[i]->oh_scale, (int64_t)scale_at.size());
+  BufRef buf, tab;
+  NNV_TRY(c->alloc(sizeof(double) * ld * (count + (int64_t)scale_at.size()), &buf));
+  std::vector<VecMap> vm((size_t)(count + (int64_t)scale_at.size()));
+  for (int64_t i = 0; i < count; ++i) vm[(size_t)i] = VecMap{in[i]->V, buf->as<double>() + i * ld, 1};
+  for (const auto& sc : scale_at) vm[(size_t)(count + sc.second)] = VecMap{sc.first, buf->as<double>() + (count + sc.second) * ld, 0};
+  NNV_TRY(c->upload_table(vm.data(), sizeof(VecMap) * vm.size(), &tab));
+  for (size_t v0 = 0; v0 < vm.size(); v0 += 65535) {
+    const unsigned cnt = (unsigned)std::min<size_t>(65535, vm.size() - v0);
+    NNV_LAUNCH(c, c->kernel_timing, rowmap_vectors_kernel, dim3((unsigned)ceil_div(ld, 256), cnt), dim3(256), 0, tab->as<VecMap>() + v0, a);
+    NNV_TRY(c->kernel_timer_end(c->kernel_timing, 4, 16.0 * (double)ld * cnt));
+  }
+  NNV_HIP_TRY(hipGetLastError());
+  for (int64_t i = 0; i < count; ++i) {
+    nnvhip_star* o = new_star(c);
+    o->N = N;
+    o->n = in[i]->n;
+    o->ld = ld;
+    o->Vbuf = buf;
+    o->V = vm[(size_t)i].out;
+    o->vcols = 1;
+    o->pbuf = in[i]->pbuf;
+    o->plb = in[i]->plb;
+    o->pub = in[i]->pub;
+    o->ptails = in[i]->ptails;
+    o->pslot = in[i]->pslot;
+    o->pcap = in[i]->pcap;
+    o->cons = in[i]->cons;
+    o->oh_from = 1;
+    o->oh_idx_buf = in[i]->oh_idx_buf;
+    o->oh_idx = in[i]->oh_idx;
+    o->oh_scale_buf = buf;
+    o->oh_scale = vm[(size_t)(count + scale_at[in[i]->oh_scale])].out;
+    o->oh_scale_neg = in[i]->oh_scale_neg || may_flip;
+    o->oh_inv_buf = in[i]->oh_inv_buf;
+    o->oh_inv = in[i]->oh_inv;
+    out[i] = o;
+  }
+  return c->end_op();
+}
+
+// Average pooling inside windows: the input's dense images have small windows (or there is nothing dense but the centre),
+// its other columns are unit vectors by list, and the output's windows are small.
+struct PoolPlan {
+  int64_t dense = 0, m = 0, eh = 0, ew = 0;
+};
+static bool pool_in_windows(const nnvhip_ctx* c, const nnvhip_avgpool2d* p, const nnvhip_star* s, int64_t H, int64_t W, int64_t Ho, int64_t Wo,
+                            PoolPlan* pl) {
+  if (!windows_allowed(c) || s->n < 1 || H >= 32768 || W >= 32768) return false;
+  const int64_t nc = s->n + 1;
+  pl->dense = (s->oh_from > 0 && s->oh_from < nc) ? s->oh_from : nc;
+  pl->m = nc - pl->dense;
+  if (pl->dense > s->stored_cols() || (pl->m > 0 && s->oh_idx == nullptr)) return false;
+  if (s->cs.pending || s->cs.zero_to > 1 || s->cs.delta_pending() || (s->rows_pending && s->cls == nullptr)) return false;
+  if (pl->dense > 1 && !(s->box != nullptr && s->box_H == H && s->box_W == W && s->box_cols >= pl->dense)) return false;
+  auto extent = [&](int d, int64_t e, int64_t size) { return std::min<int64_t>(size, (e - 1 + p->pool[d] - 1) / p->stride[d] + 1); };
+  pl->eh = pl->ew = 0;
+  if (pl->dense > 1) {
+    pl->eh = extent(0, s->box_eh, Ho);
+    pl->ew = extent(1, s->box_ew, Wo);
+  }
+  if (pl->m > 0) {
+    pl->eh = std::max(pl->eh, extent(0, 1, Ho));
+    pl->ew = std::max(pl->ew, extent(1, 1, Wo));
+  }
+  return small_windows(pl->eh, pl->ew, Ho * Wo) && s->n < 1000000;
+}
+
+static int pool_windows(nnvhip_ctx* c, const nnvhip_avgpool2d* p, PoolArgs a, int64_t count, nnvhip_star* const* in, const PoolPlan* plans,
+                        nnvhip_star** out) {
+  const int64_t Nout = (int64_t)a.Ho * a.Wo * a.C;
+  std::vector<nnvhip_star*> outs;
+  bool contig = false;
+  int64_t cols = 0;
+  NNV_TRY(c->begin_op());
+  int st = make_affine_outputs(c, count, in, Nout, &outs, &contig, &cols);
+  for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i) {
+    nnvhip_star* o = outs[i];
+    const PoolPlan& pl = plans[i];
+    st = c->alloc(sizeof(ColBox) * (size_t)(o->n + 1), &o->box_buf);
+    if (st != NNVHIP_OK) break;
+    ColBox* tab = o->box_buf->as<ColBox>();
+    st = launch_pool_boxes(c, a.H, a.W, a.Ho, a.Wo, p->pool, p->stride, p->pad[0], p->pad[2], pl.dense > 1 ? in[i]->box : nullptr, pl.dense,
+                           in[i]->oh_idx, pl.m, tab);
+    o->box = tab;
+    o->box_cols = o->n + 1;
+    o->box_H = a.Ho;
+    o->box_W = a.Wo;
+    o->box_eh = (int32_t)pl.eh;
+    o->box_ew = (int32_t)pl.ew;
+    if (st == NNVHIP_OK) st = leave_outside_windows(c, o, a.Ho, a.Wo);
+    if (st != NNVHIP_OK) break;
+    dim3 grid;
+    const WinArgs w = win_args(in[i], o, a.C, &grid);
+    PoolIn s{};
+    s.box = pl.dense > 1 ? in[i]->box : nullptr;
+    s.cls = in[i]->rows_pending ? in[i]->cls : nullptr;
+    s.idx = in[i]->oh_idx;
+    s.scale = in[i]->oh_scale;
+    s.dense = (int32_t)pl.dense;
+    NNV_LAUNCH(c, c->kernel_timing, avgpool_window_kernel, grid, dim3(256), 0, w, a, s);
+    st = c->kernel_timer_end(c->kernel_timing, 4, 8.0 * ((double)w.area * w.C * (double)o->n * 2.0 + (double)(in[i]->N + Nout)));
+    if (st == NNVHIP_OK && hipGetLastError() != hipSuccess) {
+      set_error("kernel launch failed");
+      st = NNVHIP_ERR_HIP;
+    }
+  }
+  if (st == NNVHIP_OK) st = c->end_op();
+  if (st != NNVHIP_OK) {
+    release_all(outs);
+    return st;
+  }
+  for (int64_t i = 0; i < count; ++i) out[i] = outs[i];
+  return NNVHIP_OK;
+}
+
 }  // namespace nnvhip
 
 using namespace nnvhip;
@@ -306,6 +646,15 @@ int nnvhip_rowmap_create(nnvhip_ctx* c, int64_t N, int32_t n_steps, const int32_
       NNV_FAIL(NNVHIP_ERR_ARG, "invalid step %d", s);
     m->op[s] = op[s];
     m->scope[s] = scope[s];
+  }
+  for (int s = 0; s < n_steps; ++s) {
+    if (m->scope[s] != NNVHIP_SCOPE_ALL) continue;
+    if (m->op[s] != NNVHIP_OP_MUL && m->op[s] != NNVHIP_OP_DIV) m->keeps_zeros = false;
+    for (int64_t r = 0; r < N; ++r) {
+      const double v = params[s * N + r];
+      if (!std::isfinite(v) || (m->op[s] == NNVHIP_OP_DIV && v == 0.0)) m->keeps_zeros = false;
+      if (std::signbit(v)) m->may_flip = true;
+    }
   }
   // padding rows get the neutral operand of their step so that they stay exactly zero
   std::vector<double> host((size_t)(m->ld * n_steps));
@@ -342,6 +691,15 @@ int nnvhip_affine_rowmap(nnvhip_ctx* c, const nnvhip_rowmap* m, int64_t count, n
   for (int s = 0; s < kMaxSteps; ++s) {
     a.op[s] = m->op[s];
     a.scope[s] = m->scope[s];
+  }
+  {
+    bool windows = true, boxes = m->keeps_zeros && windows_allowed(c);
+    for (int64_t i = 0; i < count; ++i) {
+      windows = windows && rowmap_in_windows(c, m, in[i]);
+      boxes = boxes && is_unwritten_box(in[i]) && in[i]->ld == m->ld;
+    }
+    if (windows) return rowmap_windows(c, a, m->N, count, in, out);
+    if (boxes) return rowmap_boxes(c, a, m->may_flip, m->N, count, in, out);
   }
   return run_row_layer(c, count, in, out, m->N, kEwRows, 4 * kEwWaves,
                        [&](dim3 grid, const SetDesc* table, const SetDesc& one, int32_t cpc, int64_t) {
@@ -415,6 +773,12 @@ int nnvhip_affine_avgpool2d(nnvhip_ctx* c, const nnvhip_avgpool2d* p, int64_t H,
   a.sw = (int32_t)p->stride[1];
   a.pt = (int32_t)p->pad[0];
   a.pl = (int32_t)p->pad[2];
+  {
+    std::vector<PoolPlan> plans((size_t)count);
+    bool windows = true;
+    for (int64_t i = 0; i < count && windows; ++i) windows = in[i]->N == in[0]->N && pool_in_windows(c, p, in[i], H, W, Ho, Wo, &plans[(size_t)i]);
+    if (windows) return pool_windows(c, p, a, count, in, plans.data(), out);
+  }
   return run_row_layer(c, count, in, out, Ho * Wo * C, 64, 4 * kEwWaves,
                        [&](dim3 grid, const SetDesc* table, const SetDesc& one, int32_t cpc, int64_t ldout) {
                          a.cols_per_chunk = cpc;

@@ -793,6 +793,10 @@ bool conv2d_in_windows(const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t 
 // windows (in_box null: whole image); the `m` columns from `dense` on from the pixels onehot_idx names.
 int launch_conv_boxes(nnvhip_ctx* ctx, const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo,
                       const ColBox* in_box, int64_t dense, const int32_t* onehot_idx, int64_t m, ColBox* out_box);
+// The same for an average pooling (windows of positions whose pooling cells reach the input's window).
+int launch_pool_boxes(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t Wo, const int64_t pool[2], const int64_t stride[2],
+                      int64_t pad_top, int64_t pad_left, const ColBox* in_box, int64_t dense, const int32_t* onehot_idx, int64_t m,
+                      ColBox* out_box);
 // Bound on the extent of an output window whose input window spans at most `e` rows (dim 0) or columns (dim 1).
 int64_t conv_box_extent(const nnvhip_conv2d* conv, int dim, int64_t e, int64_t out_size);
 // whether launch_conv2d takes pending_cls for such an input (H x W x Cin images, leading dimension ldin)
@@ -873,6 +877,9 @@ int launch_range_sums_mm(nnvhip_ctx* ctx, const nnvhip_fc* fc, int64_t count, co
                          std::vector<int64_t>* slot,  // slot[i]: which pair of columns of `out` holds set i's sums
                          bool plb_zero = false);      // every lower bound involved is 0: the first column of every pair is
                                                       // zero and only the second is multiplied out
+// Whether a set is a box of which only the centre is in memory (nnvhip_star_from_box, a row map of one): its generator
+// columns are the scaled unit vectors oh_scale[r] * e_r, r = oh_idx[t], t ascending with r.
+bool is_unwritten_box(const nnvhip_star* s);
 // lb / ub (and, by centre_mode, the centre column) of a fully connected layer's output for one set whose
 // gathered columns need no pass of their own, finished in one kernel (ranges.hip).
 int launch_fc_rowsum(nnvhip_ctx* ctx, const nnvhip_fc* fc, nnvhip_star* out, int mode, const double* scale, const int32_t* cls,

@@ -1158,7 +1158,7 @@ __global__ __launch_bounds__(256) void box_ranges_kernel(const BoxRange* __restr
   d.ub[r] = (c + y1) + y2;
 }
 
-static bool is_unwritten_box(const nnvhip_star* t) {
+bool is_unwritten_box(const nnvhip_star* t) {
   return !t->rows_pending && t->n > 0 && t->stored_cols() == 1 && t->oh_from == 1 && t->oh_idx != nullptr && t->oh_scale != nullptr &&
          !t->cs.any_pending();
 }
@@ -1554,7 +1554,9 @@ int ranges_into_static(nnvhip_ctx* ctx, const nnvhip_star* s, double* lb_dev, do
     return NNVHIP_OK;
   }
   // the set must be a plain stored matrix: writing pending columns or rows would need a buffer
-  if (s->rows_pending || s->cs.any_pending() || s->stored_cols() != s->n + 1)
+  // (columns that are in memory inside their windows are scanned there)
+  const bool win = s->cs.win_pending() && !s->cs.pending && s->cs.zero_to <= 1 && !s->cs.delta_pending() && scan_in_windows(s);
+  if (s->rows_pending || (s->cs.any_pending() && !win) || s->stored_cols() != s->n + 1)
     NNV_FAIL(NNVHIP_ERR_ARG, "nnvhip_estimate_ranges_static: parts of this set are not in memory yet (read it once, or use "
                              "nnvhip_estimate_ranges)");
   const int64_t ld = s->ld, n = s->n;
@@ -1586,7 +1588,14 @@ int ranges_into_static(nnvhip_ctx* ctx, const nnvhip_star* s, double* lb_dev, do
   if (relu_out)
     hipLaunchKernelGGL(relu_ranges_kernel, dim3((unsigned)ceil_div(s->N, 256)), dim3(256), 0, ctx->stream, nullptr,
                        ReluRange{s->pre_lb, s->pre_ub, d.lb, d.ub, (int32_t)s->N});
-  else
+  else if (win) {
+    d.box = s->box;
+    d.bH = s->box_H;
+    d.bW = s->box_W;
+    const int P = d.bH * d.bW, C = (int)(s->N / P);
+    hipLaunchKernelGGL(ranges_window_kernel<1>, dim3((unsigned)(ceil_div(P, 64) * ceil_div(C, 4)), (unsigned)chunks), dim3(512), 0,
+                       ctx->stream, nullptr, d, (int)ceil_div(P, 64), C);
+  } else
     hipLaunchKernelGGL((ranges_partial_kernel<8, 4>), dim3((unsigned)row_blocks, (unsigned)chunks, 1), dim3(64 * kRangeWaves), 0,
                        ctx->stream, nullptr, d);
   if (chunks > 1 && !relu_out)

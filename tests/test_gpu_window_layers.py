@@ -1,0 +1,92 @@
+"""Row maps and average pooling on generators that are known to be sparse (windows of a convolution, unit vectors of a box
+or a ReLU step): against the oracle layer by layer, with what is left unwritten poisoned, in the order written first /
+read first, and for the sizes where windows reach the border, overlap or stop paying."""
+import numpy as np
+import pytest
+
+from oracle import nnv_oracle as o
+from tests.gpu_util import assert_close, compare_sets
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def nnv():
+    import nnv_amd
+    return nnv_amd
+
+
+def _layers(rs, names, hw, cin):
+    h, w = hw
+    c, out = cin, []
+    for nm in names:
+        if nm.startswith("conv"):
+            k, s, p, co = (int(t) for t in nm[4:].split("_"))
+            out.append({"type": "conv", "W": rs.randn(k, k, c, co) / k, "b": rs.randn(co) * 0.1, "padding": [p] * 4, "stride": [s] * 2, "dilation": [1, 1]})
+            h, w, c = (h + 2 * p - k) // s + 1, (w + 2 * p - k) // s + 1, co
+        elif nm == "bn":
+            out.append({"type": "batchnorm", "mean": 0.1 * rs.randn(c), "var": rs.rand(c) + 0.5, "eps": 1e-5, "scale": rs.randn(c) * (rs.rand(c) < 0.8),
+                        "offset": 0.1 * rs.randn(c)})
+        elif nm.startswith("pool"):
+            k, s, p = (int(t) for t in nm[4:].split("_"))
+            out.append({"type": "avgpool", "pool": [k, k], "stride": [s, s], "padding": [p] * 4})
+            h, w = (h + 2 * p - k) // s + 1, (w + 2 * p - k) // s + 1
+        elif nm == "relu":
+            out.append({"type": "relu"})
+        elif nm == "norm":
+            out.append({"type": "imageinput", "normalization": "zscore", "input_size": [h, w, c], "mean": rs.rand(1, 1, c), "std": 0.5 + rs.rand(c)})
+        elif nm == "sym":
+            out.append({"type": "imageinput", "normalization": "rescale-symmetric", "input_size": [h, w, c], "min": -1.0, "max": 3.0})
+        elif nm == "flat":
+            out.append({"type": "flatten", "flatten_type": "nnet.keras.layer.FlattenCStyleLayer"})
+        else:
+            out.append({"type": "fc", "W": rs.randn(int(nm[2:]), h * w * c) / np.sqrt(h * w * c), "b": rs.randn(int(nm[2:])) * 0.1})
+    return out
+
+
+NETS = [
+    ((12, 9), 3, "norm conv3_1_1_4 bn relu pool2_2_0 conv3_1_1_5 bn relu pool3_2_1 flat fc7"),
+    ((13, 13), 1, "sym bn conv3_1_1_6 bn pool2_2_0 bn relu pool2_1_1 conv3_2_0_4 relu fc5"),
+    ((16, 16), 2, "pool2_2_0 bn conv3_1_1_3 relu bn relu fc4"),          # pooling a box; a row map behind a pending reset
+    ((17, 16), 1, "norm pool3_2_1 relu pool2_1_1 bn fc6"),
+    ((5, 5), 2, "norm conv3_1_1_3 bn relu pool2_2_0 fc3"),                 # windows as large as the image
+    ((9, 20), 3, "norm conv5_1_2_3 bn relu pool5_3_2 conv1_1_0_4 relu fc3"),
+]
+
+
+@pytest.mark.parametrize("hw,cin,names", NETS)
+@pytest.mark.parametrize("mode", ["default", "poison", "single_dims", "eager", "array"])
+def test_sparse_generators_through_row_maps_and_pooling(nnv, hw, cin, names, mode):
+    rs = np.random.RandomState(len(names) + hw[0])
+    layers = _layers(rs, names.split(), hw, cin)
+    count = 3 if mode == "array" else 1
+    ctx = nnv.default_context()
+    dev_in, ora_in = [], []
+    for _ in range(count):
+        x = rs.rand(*hw, cin)
+        eps = 0.02 * (rs.rand(*hw, cin) < 0.7) if mode == "single_dims" else 0.02
+        dev_in.append(nnv.ImageStar(x - eps, x + eps))
+        ora_in.append(o.image_star_from_bounds(x - eps, x + eps))
+    was = ctx.switch_is_on("poison_pending"), ctx.switch_is_on("eager_cols")
+    if mode == "poison":
+        ctx.set_switch("poison_pending", True)
+    if mode == "eager":
+        ctx.set_eager_columns(True)
+    try:
+        net = nnv.NN.from_config(layers)
+        out = net.reach(dev_in if count > 1 else dev_in[0], {"reachMethod": "relax-star-area", "relaxFactor": 1})
+        ranges = [(s[0] if count > 1 else s).estimateRanges() for s in net.reachSet[:-1]]   # before any matrix is read
+        for i in range(count):
+            exp, exp_sets = o.nn_reach(layers, ora_in[i], "relax-star-area", 1.0, keep=True)
+            for li, (L, ds, os_) in enumerate(zip(layers, net.reachSet, exp_sets)):
+                tag = "layer %d (%s) set %d" % (li + 1, L["type"], i)
+                ds = ds[i] if count > 1 else ds
+                if i == 0 and li < len(layers) - 1:
+                    elb, eub = o.image_star_estimate_ranges(os_) if isinstance(os_, o.OImageStar) else o.estimate_ranges(os_)
+                    assert_close(ranges[li][0], elb, tag + " lb")
+                    assert_close(ranges[li][1], eub, tag + " ub")
+                compare_sets(ds, os_, tag, check_constraints=False)
+            compare_sets(out[i] if count > 1 else out, exp, "output", check_constraints=True)
+    finally:
+        ctx.set_switch("poison_pending", was[0])
+        ctx.set_eager_columns(was[1])
