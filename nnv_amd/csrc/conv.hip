@@ -267,29 +267,82 @@ __global__ void conv_weights_kmajor_kernel(const double* __restrict__ W, double*
   Wk[idx] = co < Cout ? W[k + (int64_t)co * Kp] : 0.0;
 }
 
-struct ConvFastArgs {
-  const double* in;
-  int64_t ldin;
-  double* out;
+struct StampSet {
+  const int32_t* idx;   // input row of every one-hot column
+  const double* scale;  // by input row, or null (= 1)
+  double* out;          // first of these columns in the output set
+  const double* plb;    // predicate bounds of these columns
+  const double* pub;
+  double* part;         // [chunks][4][ldout] range sums of these columns (as the estimateRanges pass leaves them)
+  int32_t m;
+  int32_t win_only;     // 1: only the rows inside a column's window (the positions whose taps span its pixel) are written
+  const int32_t* pixel_col;  // (by-row pass) input row -> its column here, -1: none
+};
+
+struct ConvFastArgs {  // the layer
   int64_t ldout;
   const double* Wk;
   int coutp;
   const double* bias;
   ConvGeom g;
-  int64_t total_rows;
   int tiles_c;
   const FastTap* taps;
-  const uint32_t* keep;
   int keep_words;
+  int stamp_blocks;  // blocks for a set's unit-vector columns, dealt in between its tile blocks (0: none)
+};
+
+// One set of a call.  All sets of an array go into one launch (blockIdx.y = set): a convolution of one image's generators
+// has a few dozen to a few hundred blocks, and a launch per image left the chip three quarters idle and the host behind
+// (25 images of 28x28x1 through 3x3 filters to 16 and to 32 channels: 150 launches, 25 x 18 + 25 x 20 us of kernels plus
+// the gaps; now six launches, 68 + 125 us).
+struct ConvSet {
+  const double* in;
+  double* out;
+  int64_t ldin;
+  int64_t total_rows;
+  const uint32_t* keep;
   ConvRows cr;
+  int32_t blocks;  // tile blocks
+  int32_t stride;  // grid position p is stamp block (p + 1) / stride - 1 where (p + 1) % stride == 0 (and that is < stamp_blocks)
+  StampSet d;      // unit-vector columns whose stamps go into the same launch
 };
 
 // LDS of a block of the kernel below: the weight tiles [2][k][channel] first (their transfers want 1 KiB alignment),
 // then the position tiles [2][k][position]; the row mask (MASK only) sits in the dynamic part behind them.
 constexpr size_t conv_fast_lds_bytes(int tc) { return sizeof(double) * 2 * kKt * (128 + (size_t)tc); }
 
+// This block's set.  Field by field: a copy of the whole record is made through a generic pointer, which leaves the fields in
+// vector registers.
+__device__ __forceinline__ ConvSet conv_set_of_block(const ConvSet* __restrict__ table, const ConvSet& one) {
+  if (table == nullptr) return one;
+  const ConvSet* __restrict__ t = table + blockIdx.y;
+  ConvSet s;
+  s.in = t->in;
+  s.out = t->out;
+  s.ldin = t->ldin;
+  s.total_rows = t->total_rows;
+  s.keep = t->keep;
+  s.cr.box = t->cr.box;
+  s.cr.eh = t->cr.eh;
+  s.cr.area = t->cr.area;
+  s.cr.in_box = t->cr.in_box;
+  s.blocks = t->blocks;
+  s.stride = t->stride;
+  s.d.idx = t->d.idx;
+  s.d.scale = t->d.scale;
+  s.d.out = t->d.out;
+  s.d.plb = t->d.plb;
+  s.d.pub = t->d.pub;
+  s.d.part = t->d.part;
+  s.d.m = t->d.m;
+  s.d.win_only = t->d.win_only;
+  s.d.pixel_col = t->d.pixel_col;
+  return s;
+}
+
 template <int TC, int WR, int WC, bool MASK, bool COMPACT>
-__device__ __forceinline__ void conv2d_fast_block(const ConvFastArgs& a, int64_t bid, double* __restrict__ lds, uint32_t* keep_s) {
+__device__ __forceinline__ void conv2d_fast_block(const ConvFastArgs& a, const ConvSet& set, int64_t bid, double* __restrict__ lds,
+                                                  uint32_t* keep_s) {
   constexpr int TP = 128, NT = 512;
   static_assert(WR * WC == 8, "eight waves");
   constexpr int FM = TP / WR / 16;
@@ -298,20 +351,20 @@ __device__ __forceinline__ void conv2d_fast_block(const ConvFastArgs& a, int64_t
   constexpr int kRowsPerLoad = 128 / TC;   // rows of Wk per transfer
   double(*Wts)[kKt * TC] = reinterpret_cast<double(*)[kKt * TC]>(lds);                // [k][channel]
   double(*Ps)[kKt * TP] = reinterpret_cast<double(*)[kKt * TP]>(lds + 2 * kKt * TC);  // [k][position]
-  const double* __restrict__ in = a.in;
-  const int64_t ldin = a.ldin;
-  double* __restrict__ out = a.out;
+  const double* __restrict__ in = set.in;
+  const int64_t ldin = set.ldin;
+  double* __restrict__ out = set.out;
   const int64_t ldout = a.ldout;
   const double* __restrict__ Wk = a.Wk;
   const int coutp = a.coutp;
   const double* __restrict__ bias = a.bias;
   const ConvGeom& g = a.g;
-  const int64_t total_rows = a.total_rows;
+  const int64_t total_rows = set.total_rows;
   const int tiles_c = a.tiles_c;
   const FastTap* __restrict__ taps = a.taps;
-  const uint32_t* __restrict__ keep = a.keep;
+  const uint32_t* __restrict__ keep = set.keep;
   const int keep_words = a.keep_words;
-  const ConvRows& cr = a.cr;
+  const ConvRows& cr = set.cr;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -444,17 +497,45 @@ __device__ __forceinline__ void conv2d_fast_block(const ConvFastArgs& a, int64_t
 }
 
 template <int TC, int WR, int WC, bool MASK, bool COMPACT>
-__global__ __launch_bounds__(512) void conv2d_fast_kernel(ConvFastArgs a) {
+__global__ __launch_bounds__(512) void conv2d_fast_kernel(ConvFastArgs a, const ConvSet* __restrict__ table, ConvSet one) {
   __shared__ __attribute__((aligned(1024))) double lds[2 * kKt * (128 + TC)];
   extern __shared__ uint32_t keep_s[];  // row mask (MASK only)
-  conv2d_fast_block<TC, WR, WC, MASK, COMPACT>(a, blockIdx.x, lds, keep_s);
+  const ConvSet set = conv_set_of_block(table, one);
+  if ((int)blockIdx.x >= set.blocks) return;
+  conv2d_fast_block<TC, WR, WC, MASK, COMPACT>(a, set, blockIdx.x, lds, keep_s);
 }
 
-// Windows of the output columns of a convolution (see launch_conv_boxes in internal.h).
-__global__ void conv_boxes_kernel(const ColBox* __restrict__ in_box, int64_t dense, const int32_t* __restrict__ onehot_idx,
-                                  int64_t m, ColBox* __restrict__ out_box, ConvGeom g) {
-  const int64_t j = blockIdx.x * (int64_t)256 + threadIdx.x;
-  if (j >= dense + m) return;
+// What the kernels above and below look up, for every set of a call (blockIdx.y) in one launch: the windows of the output's
+// columns (ConvSetup::out_box) and, by input row, the unit-vector column that sits there (ConvSetup::inv; -1: none).  The
+// first inv_blocks blocks build kInvRows entries of the second table each: in LDS, because every entry is written whether or
+// not a column names it, then out in order.  Latency bound (a few KB); three launches before.
+constexpr int kInvRows = 4096;
+__global__ __launch_bounds__(256) void conv_setup_kernel(const ConvSetup* __restrict__ table, ConvSetup one, int inv_blocks, ConvGeom g) {
+  const ConvSetup d = table ? table[blockIdx.y] : one;
+  if ((int)blockIdx.x < inv_blocks) {
+    __shared__ int32_t rows[kInvRows];
+    const int r0 = (int)blockIdx.x * kInvRows, nr = min(kInvRows, d.n_inv - r0);
+    if (d.inv == nullptr || nr <= 0) return;
+    for (int r = threadIdx.x; r < nr; r += 256) rows[r] = -1;
+    __syncthreads();
+    for (int t0 = threadIdx.x; t0 < d.m; t0 += 4 * 256) {
+      int at[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) at[u] = t0 + u * 256 < d.m ? d.idx[t0 + u * 256] - r0 : -1;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (at[u] >= 0 && at[u] < nr) rows[at[u]] = t0 + u * 256;
+    }
+    __syncthreads();
+    for (int r = threadIdx.x; r < nr; r += 256) d.inv[r0 + r] = rows[r];
+    return;
+  }
+  const ColBox* __restrict__ in_box = d.in_box;
+  const int32_t* __restrict__ onehot_idx = d.idx;
+  ColBox* __restrict__ out_box = d.out_box;
+  const int dense = d.dense, m = d.m;
+  const int64_t j = ((int)blockIdx.x - inv_blocks) * (int64_t)256 + threadIdx.x;
+  if (out_box == nullptr || j >= (int64_t)dense + m) return;
   int h0 = 0, h1 = g.H - 1, w0 = 0, w1 = g.W - 1;  // window of the input column
   if (j >= dense) {
     const int src = onehot_idx[j - dense] % g.HW;
@@ -496,18 +577,6 @@ __global__ void zero_pad_rows_kernel(double* __restrict__ V, int64_t ld, int64_t
 // wo*sw - pl + fw*dw = w, and zero elsewhere.  The dense accumulation would add exact zeros to that
 // one product, so 0 + w*s is the same value.  One pass that writes the output columns (HBM bound);
 // lane = two adjacent output rows, the waves of a block interleave columns.
-struct StampSet {
-  const int32_t* idx;   // input row of every one-hot column
-  const double* scale;  // by input row, or null (= 1)
-  double* out;          // first of these columns in the output set
-  const double* plb;    // predicate bounds of these columns
-  const double* pub;
-  double* part;         // [chunks][4][ldout] range sums of these columns (as the estimateRanges pass leaves them)
-  int32_t m;
-  int32_t win_only;     // 1: only the rows inside a column's window (the positions whose taps span its pixel) are written
-  const int32_t* pixel_col;  // (by-row pass) input row -> its column here, -1: none
-};
-
 __global__ __launch_bounds__(512) void conv_stamp_kernel(const StampSet* __restrict__ table, StampSet one, ConvGeom g,
                                                          const double* __restrict__ Wt, int64_t ldout, int cols_per_chunk) {
   const StampSet d = table ? table[blockIdx.z] : one;
@@ -627,8 +696,14 @@ __global__ __launch_bounds__(512) void conv_stamp_kernel(const StampSet* __restr
 }
 
 // One bit per row of a set with a pending row reset: 1 where the row is kept.  Word w covers rows 32w..32w+31.
-__global__ __launch_bounds__(256) void keep_bits_kernel(const int32_t* __restrict__ cls, int64_t N, uint32_t* __restrict__ bits,
-                                                        int words) {
+struct KeepBits {
+  const int32_t* cls;
+  uint32_t* bits;
+};
+__global__ __launch_bounds__(256) void keep_bits_kernel(const KeepBits* __restrict__ table, KeepBits one, int64_t N, int words) {
+  const KeepBits set = table ? table[blockIdx.y] : one;
+  const int32_t* __restrict__ cls = set.cls;
+  uint32_t* __restrict__ bits = set.bits;
   const int64_t r = blockIdx.x * (int64_t)256 + threadIdx.x;
   const unsigned long long b = __ballot(r < N && cls[r] == kKeep);
   const int lane = threadIdx.x & 63;
@@ -642,11 +717,6 @@ __global__ __launch_bounds__(256) void keep_bits_kernel(const int32_t* __restric
 // -1: none) gets out(r, t) = 0 + W(k, co) * scale.  One thread per row writes those elements - exactly the
 // non-zero candidates, i.e. the rows inside every column's window - and adds up the row's four range sums tap
 // by tap.  Everything else in the columns is zero and is written by the caller (or left for later).
-__global__ void stamp_pixel_columns_kernel(const int32_t* __restrict__ idx, int m, int32_t* __restrict__ pixel_col) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t < m) pixel_col[idx[t]] = t;
-}
-
 // S lanes share a row, lane s taking the taps k = s, s + S, ...; their sums are combined by a butterfly (a fixed
 // order).  S = 1 for filters with few taps, 16 otherwise (a row's taps are then walked by 16 lanes at once).
 // A block first decodes the taps once into LDS (filter position and the tap's offset from the pixel under the
@@ -736,26 +806,22 @@ __global__ __launch_bounds__(256) void conv_stamp_rows_kernel(StampSet d, ConvGe
 // write different columns of the output and read nothing of each other, the first is bound by the matrix pipe and the
 // second by scattered stores, so their blocks are dealt to the chip in turn (every stride-th block of the grid is a
 // stamp block, until there are no more) and run side by side on a compute unit.
-struct ConvStampArgs {
-  StampSet d;
-  const double* Wt;
-  const int32_t* pixel_col;
-  int32_t blocks;  // stamp blocks in the grid
-  int32_t stride;  // grid position p is stamp block (p + 1) / stride - 1 where (p + 1) % stride == 0 (and that is < blocks)
-};
-
 template <int TC, int WR, int WC, bool MASK, bool COMPACT, int S>
-__global__ __launch_bounds__(512) void conv2d_fast_stamps_kernel(ConvFastArgs a, ConvStampArgs st) {
+__global__ __launch_bounds__(512) void conv2d_fast_stamps_kernel(ConvFastArgs a, const double* __restrict__ Wt,
+                                                                 const ConvSet* __restrict__ table, ConvSet one) {
   static_assert(sizeof(int2) * kStampTapTable <= conv_fast_lds_bytes(TC), "the stamp blocks' tap table fits the tiles' LDS");
   __shared__ __attribute__((aligned(1024))) double lds[2 * kKt * (128 + TC)];
   extern __shared__ uint32_t keep_s[];  // row mask (MASK only)
+  const ConvSet set = conv_set_of_block(table, one);
   const int p = blockIdx.x;
-  const int k = (p + 1) / st.stride;
-  if ((p + 1) % st.stride == 0 && k <= st.blocks) {
-    conv_stamp_rows_block<S, 512>(k - 1, reinterpret_cast<int2*>(lds), st.d, a.g, st.Wt, st.pixel_col, a.ldout);
+  const int k = (p + 1) / set.stride;
+  if ((p + 1) % set.stride == 0 && k <= a.stamp_blocks) {
+    conv_stamp_rows_block<S, 512>(k - 1, reinterpret_cast<int2*>(lds), set.d, a.g, Wt, set.d.pixel_col, a.ldout);
     return;
   }
-  conv2d_fast_block<TC, WR, WC, MASK, COMPACT>(a, p - min(st.blocks, p / st.stride), lds, keep_s);
+  const int bid = p - min(a.stamp_blocks, p / set.stride);
+  if (bid >= set.blocks) return;
+  conv2d_fast_block<TC, WR, WC, MASK, COMPACT>(a, set, bid, lds, keep_s);
 }
 
 // LDS of the convolution kernel beside its tap table and row mask: the two double-buffered operand tiles
@@ -844,69 +910,74 @@ static int conv_fast_taps(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, const ConvGe
   return NNVHIP_OK;
 }
 
-// stamp != null (a set's unit-vector columns, pixel_col and part filled in, filters undilated): their stamps go into
-// the same launch.
+// The sets of `jobs` have a row mask (keep), windows (compact) and stamps that go into the launch (stamps) all or none.
 template <int TC, int WR, int WC>
-static int launch_conv_fast(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, const ConvGeom& g, const double* in, int64_t ldin, double* out,
-                            int64_t ldout, int64_t ncols, const uint32_t* keep, int keep_words, const ConvRows& cr,
-                            const StampSet* stamp) {
-  const bool compact = cr.box != nullptr;
-  const int64_t total_rows = compact ? (int64_t)g.P + (ncols - 1) * cr.area : (int64_t)g.P * ncols;
+static int launch_conv_fast(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, const ConvGeom& g, int64_t ldout, const std::vector<ConvSet>& jobs,
+                            const std::vector<int64_t>& ncols, bool keep, int keep_words, bool compact, bool stamps) {
   const int64_t tiles_c = ceil_div(g.Cout, TC);
-  const int64_t blocks = ceil_div(total_rows, 128) * tiles_c;
   const size_t dyn = keep ? sizeof(uint32_t) * (size_t)keep_words : 0;
   if (conv_fast_static_lds(TC) + dyn > kConvLdsLimit) NNV_FAIL(NNVHIP_ERR_SHAPE, "internal: row mask too large for the convolution kernel");
   ConvFastArgs a{};
   NNV_TRY(conv_fast_taps(ctx, cv, g, &a.taps));
-  a.in = in;
-  a.ldin = ldin;
-  a.out = out;
   a.ldout = ldout;
   a.Wk = cv->Wk->as<double>();
   a.coutp = (int)cv->coutp;
   a.bias = cv->bias ? cv->bias->as<double>() : nullptr;
   a.g = g;
-  a.total_rows = total_rows;
   a.tiles_c = (int)tiles_c;
-  a.keep = keep;
   a.keep_words = keep_words;
-  a.cr = cr;
   // lanes per output row of the stamp blocks: 8 for filters with many taps (beside the tile blocks that measured best:
-  // config 4 0.747 ms against 0.752 with 16 lanes, 0.756 with 4, 0.782 with 32), else 1
+  // CNN 32x32x3 0.747 ms against 0.752 with 16 lanes, 0.756 with 4, 0.782 with 32), else 1
   const bool wide_stamps = g.K > 32;
-  ConvStampArgs sa{};
-  if (stamp != nullptr) {
-    sa.d = *stamp;
-    sa.Wt = cv->W->as<double>();
-    sa.pixel_col = stamp->pixel_col;
-    sa.blocks = (int32_t)ceil_div(ldout * (wide_stamps ? 8 : 1), 512);
-    sa.stride = (int32_t)std::max<int64_t>(1, (blocks + sa.blocks) / sa.blocks);
+  const int64_t stamp_blocks = stamps ? ceil_div(ldout * (wide_stamps ? 8 : 1), 512) : 0;
+  a.stamp_blocks = (int)stamp_blocks;
+  std::vector<ConvSet> sets = jobs;
+  double rows = 0.0;
+  for (size_t i = 0; i < sets.size(); ++i) {
+    ConvSet& s = sets[i];
+    s.total_rows = compact ? (int64_t)g.P + (ncols[i] - 1) * s.cr.area : (int64_t)g.P * ncols[i];
+    const int64_t blocks = ceil_div(s.total_rows, 128) * tiles_c;
+    if (blocks + stamp_blocks >= (int64_t(1) << 31)) NNV_FAIL(NNVHIP_ERR_SHAPE, "convolution too large for one launch");
+    s.blocks = (int32_t)blocks;
+    s.stride = stamps ? (int32_t)std::max<int64_t>(1, (blocks + stamp_blocks) / stamp_blocks) : 1;
+    rows += (double)s.total_rows;
   }
-  const int64_t grid = blocks + sa.blocks;
-  if (grid >= (int64_t(1) << 31)) NNV_FAIL(NNVHIP_ERR_SHAPE, "convolution too large for one launch");
-  NNV_TRY(ctx->kernel_timer_begin(ctx->kernel_timing));
-#define NNV_CONV_FAST(MASK, COMPACT)                                                                                                    \
-  do {                                                                                                                                  \
-    if (stamp == nullptr)                                                                                                               \
-      NNV_LAUNCH(ctx, ctx->kernel_timing, (conv2d_fast_kernel<TC, WR, WC, MASK, COMPACT>), dim3((unsigned)grid), dim3(512), dyn, a);    \
-    else if (wide_stamps)                                                                                                               \
-      NNV_LAUNCH(ctx, ctx->kernel_timing, (conv2d_fast_stamps_kernel<TC, WR, WC, MASK, COMPACT, 8>), dim3((unsigned)grid), dim3(512), \
-                 dyn, a, sa);                                                                                                           \
-    else                                                                                                                                \
-      NNV_LAUNCH(ctx, ctx->kernel_timing, (conv2d_fast_stamps_kernel<TC, WR, WC, MASK, COMPACT, 1>), dim3((unsigned)grid), dim3(512),  \
-                 dyn, a, sa);                                                                                                           \
+  for (size_t i0 = 0; i0 < sets.size(); i0 += 65535) {
+    const size_t cnt = std::min<size_t>(65535, sets.size() - i0);
+    int64_t grid_x = 0;
+    for (size_t i = i0; i < i0 + cnt; ++i) grid_x = std::max<int64_t>(grid_x, sets[i].blocks + stamp_blocks);
+    const ConvSet* table = nullptr;
+    BufRef tab;
+    if (cnt > 1) {  // (a device copy: every block reads its record)
+      NNV_TRY(ctx->upload(sets.data() + i0, sizeof(ConvSet) * cnt, &tab));
+      table = tab->as<ConvSet>();
+    }
+    const ConvSet& one = sets[i0];
+    const dim3 grid((unsigned)grid_x, (unsigned)cnt);
+    NNV_TRY(ctx->kernel_timer_begin(ctx->kernel_timing));
+#define NNV_CONV_FAST(MASK, COMPACT)                                                                                                     \
+  do {                                                                                                                                   \
+    if (!stamps)                                                                                                                         \
+      NNV_LAUNCH(ctx, ctx->kernel_timing, (conv2d_fast_kernel<TC, WR, WC, MASK, COMPACT>), grid, dim3(512), dyn, a, table, one);         \
+    else if (wide_stamps)                                                                                                                \
+      NNV_LAUNCH(ctx, ctx->kernel_timing, (conv2d_fast_stamps_kernel<TC, WR, WC, MASK, COMPACT, 8>), grid, dim3(512), dyn, a,            \
+                 cv->W->as<double>(), table, one);                                                                                       \
+    else                                                                                                                                 \
+      NNV_LAUNCH(ctx, ctx->kernel_timing, (conv2d_fast_stamps_kernel<TC, WR, WC, MASK, COMPACT, 1>), grid, dim3(512), dyn, a,            \
+                 cv->W->as<double>(), table, one);                                                                                       \
   } while (0)
-  if (keep && compact)
-    NNV_CONV_FAST(true, true);
-  else if (keep)
-    NNV_CONV_FAST(true, false);
-  else if (compact)
-    NNV_CONV_FAST(false, true);
-  else
-    NNV_CONV_FAST(false, false);
+    if (keep && compact)
+      NNV_CONV_FAST(true, true);
+    else if (keep)
+      NNV_CONV_FAST(true, false);
+    else if (compact)
+      NNV_CONV_FAST(false, true);
+    else
+      NNV_CONV_FAST(false, false);
 #undef NNV_CONV_FAST
-  NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 1, 2.0 * (double)total_rows * g.Cout * g.K));
-  NNV_HIP_TRY(hipGetLastError());
+    NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 1, 2.0 * rows * g.Cout * g.K * ((double)cnt / (double)sets.size())));
+    NNV_HIP_TRY(hipGetLastError());
+  }
   return NNVHIP_OK;
 }
 
@@ -923,14 +994,34 @@ int64_t conv_box_extent(const nnvhip_conv2d* cv, int dim, int64_t e, int64_t out
   return std::min<int64_t>(out_size, (e - 1 + (F - 1) * cv->dil[dim]) / cv->stride[dim] + 1);
 }
 
-int launch_conv_boxes(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo,
-                      const ColBox* in_box, int64_t dense, const int32_t* onehot_idx, int64_t m, ColBox* out_box) {
+static int launch_setup(nnvhip_ctx* ctx, const ConvGeom& g, int64_t count, const ConvSetup* sets) {
+  for (int64_t i0 = 0; i0 < count; i0 += 65535) {
+    const int64_t cnt = std::min<int64_t>(65535, count - i0);
+    int64_t inv_rows = 0, cols = 0;
+    for (int64_t i = i0; i < i0 + cnt; ++i) {
+      if (sets[i].inv != nullptr) inv_rows = std::max<int64_t>(inv_rows, sets[i].n_inv);
+      if (sets[i].out_box != nullptr) cols = std::max<int64_t>(cols, (int64_t)sets[i].dense + sets[i].m);
+    }
+    const int64_t inv_blocks = ceil_div(inv_rows, kInvRows), blocks = inv_blocks + ceil_div(cols, 256);
+    if (blocks == 0) continue;
+    const ConvSetup* table = nullptr;
+    BufRef tab;
+    if (cnt > 1) {
+      NNV_TRY(ctx->upload_table(sets + i0, sizeof(ConvSetup) * (size_t)cnt, &tab));
+      table = tab->as<ConvSetup>();
+    }
+    hipLaunchKernelGGL(conv_setup_kernel, dim3((unsigned)blocks, (unsigned)cnt), dim3(256), 0, ctx->stream, table, sets[i0],
+                       (int)inv_blocks, g);
+    NNV_HIP_TRY(hipGetLastError());
+  }
+  return NNVHIP_OK;
+}
+
+int launch_conv_setup(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t count,
+                      const ConvSetup* sets) {
   ConvGeom g;
   fill_geom(g, cv, H, W, Ho, Wo);
-  hipLaunchKernelGGL(conv_boxes_kernel, dim3((unsigned)ceil_div(dense + m, 256)), dim3(256), 0, ctx->stream, in_box, dense, onehot_idx, m,
-                     out_box, g);
-  NNV_HIP_TRY(hipGetLastError());
-  return NNVHIP_OK;
+  return launch_setup(ctx, g, count, sets);
 }
 
 int launch_pool_boxes(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t Wo, const int64_t pool[2], const int64_t stride[2],
@@ -949,10 +1040,8 @@ int launch_pool_boxes(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t
   g.pt = (int)pad_top;
   g.pl = (int)pad_left;
   g.HW = (int)(H * W);
-  hipLaunchKernelGGL(conv_boxes_kernel, dim3((unsigned)ceil_div(dense + m, 256)), dim3(256), 0, ctx->stream, in_box, dense, onehot_idx, m,
-                     out_box, g);
-  NNV_HIP_TRY(hipGetLastError());
-  return NNVHIP_OK;
+  const ConvSetup one{in_box, onehot_idx, out_box, nullptr, (int32_t)dense, (int32_t)m, 0};
+  return launch_setup(ctx, g, 1, &one);
 }
 
 bool conv2d_in_windows(const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldin, int64_t ncols,
@@ -963,78 +1052,104 @@ bool conv2d_in_windows(const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho
          conv_fast_ok(cv, g, ldin, (int64_t)eh * ew);
 }
 
-int launch_conv2d(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo,
-                  const double* in, int64_t ldin, double* out, int64_t ldout, int64_t ncols,
-                  const int32_t* pending_cls, const ColBox* out_box, int eh, int ew, const ColBox* in_box, bool leave_outside,
-                  const uint32_t* pending_bits, const ConvStampSet* stamp, bool* stamped) {
-  if (stamped != nullptr) *stamped = false;
+int launch_conv2d(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldout,
+                  std::vector<ConvJob>& jobs) {
   if (cv->Kp > kMaxTaps) NNV_FAIL(NNVHIP_ERR_SHAPE, "filters with more than %d taps (FH*FW*Cin) are not supported", kMaxTaps);
   if ((cv->FH - 1) * cv->dil[0] > 0xffff || (cv->FW - 1) * cv->dil[1] > 0xffff)
     NNV_FAIL(NNVHIP_ERR_SHAPE, "dilated filter extent too large");
   ConvGeom g;
   fill_geom(g, cv, H, W, Ho, Wo);
-  const int64_t Nout = Ho * Wo * cv->Cout;
-  // a pending row reset of the input is applied on load, from one bit per input row
+  // a pending row reset of an input is applied on load, from one bit per input row
   const int64_t n_in = H * W * cv->Cin;
-  const uint32_t* keep = nullptr;
-  int keep_words = 0;
-  BufRef bits;
-  if (pending_cls != nullptr) {
-    if (!conv2d_can_mask(cv, H, W, Ho, Wo, ldin)) NNV_FAIL(NNVHIP_ERR_SHAPE, "internal: row mask too large for the convolution kernel");
-    keep_words = (int)ceil_div(n_in, 32);
-    if (pending_bits != nullptr) {
-      keep = pending_bits;
-    } else {
-      NNV_TRY(ctx->alloc(sizeof(uint32_t) * (size_t)keep_words, &bits));
+  const int keep_words = (int)ceil_div(n_in, 32);
+  std::vector<const uint32_t*> keep(jobs.size(), nullptr);
+  BufRef bits, bits_tab;
+  {
+    std::vector<KeepBits> kb;
+    for (size_t i = 0; i < jobs.size(); ++i) {
+      if (jobs[i].pending_cls == nullptr) continue;
+      if (!conv2d_can_mask(cv, H, W, Ho, Wo, jobs[i].ldin)) NNV_FAIL(NNVHIP_ERR_SHAPE, "internal: row mask too large for the convolution kernel");
+      keep[i] = jobs[i].pending_bits;
+      if (keep[i] == nullptr) kb.push_back(KeepBits{jobs[i].pending_cls, nullptr});
+    }
+    if (!kb.empty()) {
+      const int64_t words = round_up((int64_t)keep_words, 16);
+      NNV_TRY(ctx->alloc(sizeof(uint32_t) * (size_t)words * kb.size(), &bits));
+      size_t k = 0;
+      for (size_t i = 0; i < jobs.size(); ++i)
+        if (jobs[i].pending_cls != nullptr && keep[i] == nullptr) {
+          kb[k].bits = bits->as<uint32_t>() + words * (int64_t)k;
+          keep[i] = kb[k++].bits;
+        }
       // whole waves only, so that every word is written by a lane that exists
-      hipLaunchKernelGGL(keep_bits_kernel, dim3((unsigned)ceil_div(n_in, 256)), dim3(256), 0, ctx->stream, pending_cls, n_in,
-                         bits->as<uint32_t>(), keep_words);
-      NNV_HIP_TRY(hipGetLastError());
-      keep = bits->as<uint32_t>();
+      for (size_t i0 = 0; i0 < kb.size(); i0 += 65535) {
+        const size_t cnt = std::min<size_t>(65535, kb.size() - i0);
+        const KeepBits* table = nullptr;
+        if (cnt > 1) {
+          NNV_TRY(ctx->upload_table(kb.data() + i0, sizeof(KeepBits) * cnt, &bits_tab));
+          table = bits_tab->as<KeepBits>();
+        }
+        hipLaunchKernelGGL(keep_bits_kernel, dim3((unsigned)ceil_div(n_in, 256), (unsigned)cnt), dim3(256), 0, ctx->stream, table, kb[i0],
+                           n_in, keep_words);
+        NNV_HIP_TRY(hipGetLastError());
+      }
     }
   }
   // 128 positions x Cout tile, eight waves per block (two per SIMD keep the MFMA pipe fed while
-  // the other wave gathers)
-  int st;
-  // Generator images with known windows are computed inside them only (the caller has zeroed the rest) when that
-  // at least halves the rows; it takes the kernel with scalar tap decoding.
-  ConvRows cr{nullptr, 0, 0, nullptr};
-  if (conv2d_in_windows(cv, H, W, Ho, Wo, ldin, ncols, out_box, eh, ew)) cr = ConvRows{out_box, eh, eh * ew, in_box};
-  if (cr.box == nullptr && (in_box != nullptr || leave_outside))
-    NNV_FAIL(NNVHIP_ERR_ARG, "internal: the convolution was to stay inside the images' windows");
-  if (cr.box != nullptr && !leave_outside)  // everything outside the windows
-    NNV_HIP_TRY(hipMemsetAsync(out + ldout, 0, sizeof(double) * (size_t)ldout * (size_t)(ncols - 1), ctx->stream));
-  if (cr.box != nullptr || conv_fast_ok(cv, g, ldin)) {
+  // the other wave gathers).  Sets that take the same instantiation share a launch.
+  std::vector<ConvSet> group[8];
+  std::vector<int64_t> group_cols[8];
+  for (size_t i = 0; i < jobs.size(); ++i) {
+    ConvJob& jb = jobs[i];
+    // Generator images with known windows are computed inside them only (the caller has zeroed the rest) when that
+    // at least halves the rows; it takes the kernel with scalar tap decoding.
+    ConvSet set{};
+    if (conv2d_in_windows(cv, H, W, Ho, Wo, jb.ldin, jb.ncols, jb.out_box, jb.eh, jb.ew))
+      set.cr = ConvRows{jb.out_box, jb.eh, jb.eh * jb.ew, jb.in_box};
+    const bool compact = set.cr.box != nullptr;
+    if (!compact && (jb.in_box != nullptr || jb.leave_outside))
+      NNV_FAIL(NNVHIP_ERR_ARG, "internal: the convolution was to stay inside the images' windows");
+    if (compact && !jb.leave_outside)  // everything outside the windows
+      NNV_HIP_TRY(hipMemsetAsync(jb.out + ldout, 0, sizeof(double) * (size_t)ldout * (size_t)(jb.ncols - 1), ctx->stream));
+    if (!compact && !conv_fast_ok(cv, g, jb.ldin)) {
+      int st;
+      if (cv->Cout <= 16)
+        st = launch_conv_cfg<128, 16, 8, 1>(ctx, cv, g, jb.in, jb.ldin, jb.out, ldout, jb.ncols, keep[i], keep_words);
+      else if (cv->Cout <= 32)
+        st = launch_conv_cfg<128, 32, 4, 2>(ctx, cv, g, jb.in, jb.ldin, jb.out, ldout, jb.ncols, keep[i], keep_words);
+      else
+        st = launch_conv_cfg<128, 64, 4, 2>(ctx, cv, g, jb.in, jb.ldin, jb.out, ldout, jb.ncols, keep[i], keep_words);
+      NNV_TRY(st);
+      continue;
+    }
     // the stamps of the set's unit-vector columns ride along where they are made row by row and come with their
     // pixel table and a place for their range sums
     static_assert(sizeof(ConvStampSet) == sizeof(StampSet), "same layout");
-    StampSet one;
-    const StampSet* merge = nullptr;
-    if (stamp != nullptr && stamped != nullptr && stamp->m > 0 && stamp->pixel_col != nullptr && stamp->part != nullptr &&
-        cv->dil[0] == 1 && cv->dil[1] == 1 && g.K <= kStampTapTable) {
-      memcpy(&one, stamp, sizeof one);
-      merge = &one;
-      if (!one.win_only)  // whole columns: the zeros first
-        NNV_HIP_TRY(hipMemsetAsync(one.out, 0, sizeof(double) * (size_t)ldout * (size_t)one.m, ctx->stream));
-      *stamped = true;
+    const ConvStampSet* stamp = jb.stamp;
+    jb.stamped = stamp != nullptr && stamp->m > 0 && stamp->pixel_col != nullptr && stamp->part != nullptr && cv->dil[0] == 1 &&
+                 cv->dil[1] == 1 && g.K <= kStampTapTable;
+    if (jb.stamped) {
+      memcpy(&set.d, stamp, sizeof set.d);
+      if (!set.d.win_only)  // whole columns: the zeros first
+        NNV_HIP_TRY(hipMemsetAsync(set.d.out, 0, sizeof(double) * (size_t)ldout * (size_t)set.d.m, ctx->stream));
     }
-    if (cv->Cout <= 16)
-      st = launch_conv_fast<16, 8, 1>(ctx, cv, g, in, ldin, out, ldout, ncols, keep, keep_words, cr, merge);
-    else if (cv->Cout <= 32)
-      st = launch_conv_fast<32, 4, 2>(ctx, cv, g, in, ldin, out, ldout, ncols, keep, keep_words, cr, merge);
-    else
-      st = launch_conv_fast<64, 4, 2>(ctx, cv, g, in, ldin, out, ldout, ncols, keep, keep_words, cr, merge);
-  } else if (cv->Cout <= 16) {
-    st = launch_conv_cfg<128, 16, 8, 1>(ctx, cv, g, in, ldin, out, ldout, ncols, keep, keep_words);
-  } else if (cv->Cout <= 32) {
-    st = launch_conv_cfg<128, 32, 4, 2>(ctx, cv, g, in, ldin, out, ldout, ncols, keep, keep_words);
-  } else {
-    st = launch_conv_cfg<128, 64, 4, 2>(ctx, cv, g, in, ldin, out, ldout, ncols, keep, keep_words);
+    set.in = jb.in;
+    set.ldin = jb.ldin;
+    set.out = jb.out;
+    set.keep = keep[i];
+    const int key = (keep[i] != nullptr ? 1 : 0) | (compact ? 2 : 0) | (jb.stamped ? 4 : 0);
+    group[key].push_back(set);
+    group_cols[key].push_back(jb.ncols);
   }
-  NNV_TRY(st);
-  if (ldout != Nout) {  // keep the padding rows of the output at zero
-    hipLaunchKernelGGL(zero_pad_rows_kernel, dim3(256), dim3(256), 0, ctx->stream, out, ldout, Nout, ncols);
-    NNV_HIP_TRY(hipGetLastError());
+  for (int key = 0; key < 8; ++key) {
+    if (group[key].empty()) continue;
+    const bool masked = key & 1, compact = key & 2, stamps = key & 4;
+    if (cv->Cout <= 16)
+      NNV_TRY((launch_conv_fast<16, 8, 1>(ctx, cv, g, ldout, group[key], group_cols[key], masked, keep_words, compact, stamps)));
+    else if (cv->Cout <= 32)
+      NNV_TRY((launch_conv_fast<32, 4, 2>(ctx, cv, g, ldout, group[key], group_cols[key], masked, keep_words, compact, stamps)));
+    else
+      NNV_TRY((launch_conv_fast<64, 4, 2>(ctx, cv, g, ldout, group[key], group_cols[key], masked, keep_words, compact, stamps)));
   }
   return NNVHIP_OK;
 }
@@ -1062,17 +1177,6 @@ static void fill_geom(ConvGeom& g, const nnvhip_conv2d* cv, int64_t H, int64_t W
 
 static bool conv_stamps_by_row(const nnvhip_conv2d* cv) { return cv->dil[0] == 1 && cv->dil[1] == 1; }
 bool conv_stamps_by_pixel(const nnvhip_conv2d* cv) { return conv_stamps_by_row(cv); }
-
-int launch_pixel_columns(nnvhip_ctx* ctx, const int32_t* idx, int64_t m, int64_t n_in, BufRef* inv) {
-  NNV_TRY(ctx->alloc(sizeof(int32_t) * (size_t)n_in, inv));
-  NNV_HIP_TRY(hipMemsetAsync((*inv)->ptr, 0xff, sizeof(int32_t) * (size_t)n_in, ctx->stream));
-  if (m > 0) {
-    hipLaunchKernelGGL(stamp_pixel_columns_kernel, dim3((unsigned)ceil_div(m, 256)), dim3(256), 0, ctx->stream, idx, (int)m,
-                       (*inv)->as<int32_t>());
-    NNV_HIP_TRY(hipGetLastError());
-  }
-  return NNVHIP_OK;
-}
 
 int64_t conv_stamp_chunks(const nnvhip_conv2d* cv, int64_t ldout, int64_t count, int64_t max_m) {
   if (conv_stamps_by_row(cv)) return 1;
@@ -1103,20 +1207,13 @@ int launch_conv_stamps(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
   if (conv_stamps_by_row(cv)) {
     if (chunks != 1) NNV_FAIL(NNVHIP_ERR_ARG, "internal: one chunk of range sums per set");
     if (g.K > kStampTapTable) NNV_FAIL(NNVHIP_ERR_SHAPE, "internal: more taps than the stamp kernel's table holds");
-    const int64_t n_in = H * W * cv->Cin;
-    std::vector<BufRef> made;  // tables of the sets that came without one
     NNV_TRY(ctx->kernel_timer_begin(ctx->kernel_timing));
     for (int64_t i = 0; i < count; ++i) {
       if (sets[i].m == 0) continue;
       StampSet one;
       memcpy(&one, &sets[i], sizeof one);
       const int32_t* pc = one.pixel_col;
-      if (pc == nullptr) {
-        BufRef inv;
-        NNV_TRY(launch_pixel_columns(ctx, one.idx, one.m, n_in, &inv));
-        pc = inv->as<int32_t>();
-        made.push_back(inv);
-      }
+      if (pc == nullptr) NNV_FAIL(NNVHIP_ERR_ARG, "internal: stamps without their pixel table");
       if (!one.win_only)  // whole columns: the zeros first
         NNV_HIP_TRY(hipMemsetAsync(one.out, 0, sizeof(double) * (size_t)ldout * (size_t)one.m, ctx->stream));
       if (g.K <= 32)

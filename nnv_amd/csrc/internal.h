@@ -769,31 +769,44 @@ struct ConvStampSet {
   double* part;         // this set's [chunks][4][ldout] range sums
   int32_t m;
   int32_t win_only;     // 1: write the rows inside each column's window only
-  const int32_t* pixel_col;  // input row -> its one-hot column (index into idx), -1: none; or null (made by the launch)
+  const int32_t* pixel_col;  // input row -> its one-hot column (index into idx), -1: none (ConvSetup::inv); undilated filters only
 };
-int launch_conv2d(nnvhip_ctx* ctx, const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo,
-                  const double* in, int64_t ldin, double* out, int64_t ldout, int64_t ncols,
-                  const int32_t* pending_cls /* per input row, or null: rows whose class is not kKeep read as zero */,
-                  const ColBox* out_box = nullptr /* per output column, or null: with it (and conv2d_in_windows), columns
-                                                    1.. are computed inside their windows only, at most eh x ew positions */,
-                  int eh = 0, int ew = 0,
-                  const ColBox* in_box = nullptr /* windows of the input columns: taps outside them are not read (the input
-                                                    may be in memory inside its windows only); needs conv2d_in_windows */,
-                  bool leave_outside = false /* do not write the zeros outside the output windows */,
-                  const uint32_t* pending_bits = nullptr /* with pending_cls: the same as one bit per row (1 = kept), where
-                                                            the step that classified the rows left them */,
-                  const ConvStampSet* stamp = nullptr /* the set's unit-vector columns: their stamps go into the same
-                                                                 launch where that is possible ... */,
-                  bool* stamped = nullptr /* ... which this reports (launch_conv_stamps is then not needed for the set) */);
+// The dense images of one set of a call.
+struct ConvJob {
+  const double* in;
+  int64_t ldin;
+  double* out;
+  int64_t ncols;
+  const int32_t* pending_cls;    // per input row, or null: rows whose class is not kKeep read as zero ...
+  const uint32_t* pending_bits;  // ... or the same as one bit per row (1 = kept), where the step that classified the rows left them
+  const ColBox* out_box;         // per output column, or null: with it (and conv2d_in_windows), columns 1.. are computed inside
+  int eh, ew;                    // their windows only, at most eh x ew positions
+  const ColBox* in_box;          // windows of the input columns: taps outside them are not read (the input may be in memory inside
+                                 // its windows only); needs conv2d_in_windows
+  bool leave_outside;            // do not write the zeros outside the output windows
+  const ConvStampSet* stamp;     // the set's unit-vector columns: their stamps go into the same launch where that is possible ...
+  bool stamped;                  // ... which the launch reports here (launch_conv_stamps is then not needed for the set)
+};
+// Padding rows [Nout, ldout) are the caller's.
+int launch_conv2d(nnvhip_ctx* ctx, const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldout,
+                  std::vector<ConvJob>& jobs);
 int launch_zero_pad_rows(nnvhip_ctx* ctx, double* V, int64_t ld, int64_t N, int64_t ncols);  // rows [N, ld) of ncols columns := 0
 // whether launch_conv2d computes the generator images of such a call inside their windows only
 bool conv2d_in_windows(const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldin, int64_t ncols,
                        const ColBox* out_box, int eh, int ew);
-// Windows of a convolution's output columns: column 0 the whole image; columns below `dense` from the input's
-// windows (in_box null: whole image); the `m` columns from `dense` on from the pixels onehot_idx names.
-int launch_conv_boxes(nnvhip_ctx* ctx, const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo,
-                      const ColBox* in_box, int64_t dense, const int32_t* onehot_idx, int64_t m, ColBox* out_box);
-// The same for an average pooling (windows of positions whose pooling cells reach the input's window).
+// Windows of a convolution's output columns (out_box, or null: none wanted): column 0 the whole image; columns below `dense`
+// from the input's windows (in_box null: whole image); the `m` columns from `dense` on from the pixels idx names.  And
+// inv[idx[t]] = t, -1 elsewhere (n_inv entries; inv null: not wanted).
+struct ConvSetup {
+  const ColBox* in_box;
+  const int32_t* idx;
+  ColBox* out_box;
+  int32_t* inv;
+  int32_t dense, m, n_inv;
+};
+int launch_conv_setup(nnvhip_ctx* ctx, const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t count,
+                      const ConvSetup* sets);
+// The windows behind an average pooling (positions whose pooling cells reach the input's window).
 int launch_pool_boxes(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t Wo, const int64_t pool[2], const int64_t stride[2],
                       int64_t pad_top, int64_t pad_left, const ColBox* in_box, int64_t dense, const int32_t* onehot_idx, int64_t m,
                       ColBox* out_box);
@@ -803,10 +816,8 @@ int64_t conv_box_extent(const nnvhip_conv2d* conv, int dim, int64_t e, int64_t o
 bool conv2d_can_mask(const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldin);
 int conv2d_prepare_weights(nnvhip_ctx* ctx, nnvhip_conv2d* conv);  // builds conv->Wk from conv->W (at creation)
 
-// Whether the stamp launch of this layer looks columns up by pixel (ConvStampSet::pixel_col), and that table for one
-// set: inv[idx[t]] = t, -1 elsewhere (n_in entries, allocated here).
+// Whether the stamp launch of this layer looks columns up by pixel (ConvStampSet::pixel_col).
 bool conv_stamps_by_pixel(const nnvhip_conv2d* conv);
-int launch_pixel_columns(nnvhip_ctx* ctx, const int32_t* idx, int64_t m, int64_t n_in, BufRef* inv);
 // Number of column chunks (= range-sum chunks per set) the stamp launch will use.
 int64_t conv_stamp_chunks(const nnvhip_conv2d* conv, int64_t ldout, int64_t count, int64_t max_m);
 int launch_conv_stamps(nnvhip_ctx* ctx, const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo,

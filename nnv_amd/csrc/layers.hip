@@ -93,24 +93,55 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
   const int64_t sch = any_stamps && st == NNVHIP_OK ? conv_stamp_chunks(cv, outs[0]->ld, count, max_m) : 0;
   BufRef sums;
   if (sch > 0) st = c->alloc(sizeof(double) * 4 * outs[0]->ld * sch * count, &sums);
-  std::vector<char> stamped((size_t)count, 0);
+  // windows of the output's columns and the pixel tables of the unit-vector columns: one buffer each, one launch
+  std::vector<ConvSetup> setup((size_t)count);
+  BufRef boxes, invs;
+  int64_t box_cols = 0, inv_sets = 0;
+  const int64_t inv_stride = round_up(in[0]->N, kLdAlign);
+  auto wants_inv = [&](int64_t i) { return plan[i].m > 0 && in[i]->oh_inv == nullptr && conv_stamps_by_pixel(cv); };
+  for (int64_t i = 0; i < count; ++i) {
+    if (plan[i].out_boxes) box_cols += plan[i].nc;
+    if (wants_inv(i)) ++inv_sets;
+  }
+  if (st == NNVHIP_OK && box_cols > 0) st = c->alloc(sizeof(ColBox) * (size_t)box_cols, &boxes);
+  if (st == NNVHIP_OK && inv_sets > 0) st = c->alloc(sizeof(int32_t) * (size_t)(inv_stride * inv_sets), &invs);
+  if (st == NNVHIP_OK && (box_cols > 0 || inv_sets > 0)) {
+    int64_t box_at = 0, inv_at = 0;
+    for (int64_t i = 0; i < count; ++i) {
+      const Plan& pl = plan[i];
+      ConvSetup& su = setup[(size_t)i];
+      su = ConvSetup{pl.in_ok ? in[i]->box : nullptr, in[i]->oh_idx, nullptr, nullptr, (int32_t)pl.dense, (int32_t)pl.m, (int32_t)in[i]->N};
+      if (pl.out_boxes) {
+        su.out_box = boxes->as<ColBox>() + box_at;
+        box_at += pl.nc;
+      }
+      if (wants_inv(i)) {
+        su.inv = invs->as<int32_t>() + inv_at;
+        inv_at += inv_stride;
+      }
+    }
+    st = launch_conv_setup(c, cv, H, W, Ho, Wo, count, setup.data());
+    for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i)
+      if (setup[(size_t)i].inv != nullptr) {  // (kept on the input: its columns do not change, and an input set is usually mapped again)
+        in[i]->oh_inv_buf = invs;
+        in[i]->oh_inv = setup[(size_t)i].inv;
+      }
+  }
+  std::vector<ConvJob> jobs;
+  jobs.reserve((size_t)count);
   for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i) {
     const Plan& pl = plan[i];
     nnvhip_star* o = outs[i];
     const ColBox* ob = nullptr;
     if (pl.out_boxes) {
-      st = c->alloc(sizeof(ColBox) * (size_t)pl.nc, &o->box_buf);
-      if (st != NNVHIP_OK) break;
-      ColBox* tab = o->box_buf->as<ColBox>();
-      st = launch_conv_boxes(c, cv, H, W, Ho, Wo, pl.in_ok ? in[i]->box : nullptr, pl.dense, in[i]->oh_idx, pl.m, tab);
-      if (st != NNVHIP_OK) break;
       int64_t eh = pl.dense > 1 ? pl.dense_eh : 0, ew = pl.dense > 1 ? pl.dense_ew : 0;
       if (pl.m > 0) {
         eh = std::max(eh, conv_box_extent(cv, 0, 1, Ho));
         ew = std::max(ew, conv_box_extent(cv, 1, 1, Wo));
       }
-      ob = tab;
-      o->box = tab;
+      ob = setup[(size_t)i].out_box;
+      o->box_buf = boxes;
+      o->box = ob;
       o->box_cols = pl.nc;
       o->box_H = (int32_t)Ho;
       o->box_W = (int32_t)Wo;
@@ -140,31 +171,20 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
     stamps[i].pub = o->pub + (pl.dense - 1);
     stamps[i].part = sums ? sums->as<double>() + 4 * outs[0]->ld * sch * i : nullptr;
     stamps[i].m = (int32_t)pl.m;
-    if (pl.m > 0 && in[i]->oh_inv == nullptr && conv_stamps_by_pixel(cv)) {
-      // (kept on the input: its columns do not change, and an input set is usually mapped again)
-      st = launch_pixel_columns(c, in[i]->oh_idx, pl.m, in[i]->N, &in[i]->oh_inv_buf);
-      if (st != NNVHIP_OK) break;
-      in[i]->oh_inv = in[i]->oh_inv_buf->as<int32_t>();
-    }
     stamps[i].pixel_col = in[i]->oh_inv;
     stamps[i].win_only = (lazy && pl.m > 0) ? 1 : 0;
-    bool done = false;
-    st = launch_conv2d(c, cv, H, W, Ho, Wo, in[i]->V, in[i]->ld, o->V, o->ld, pl.dense,
-                       in[i]->rows_pending ? in[i]->cls : nullptr, pl.compact ? ob : nullptr, pl.dense_eh, pl.dense_ew,
-                       pl.compact ? in[i]->box : nullptr, pl.compact && lazy, in[i]->rows_pending ? in[i]->keep_bits : nullptr,
-                       sch == 1 ? &stamps[i] : nullptr, &done);
-    stamped[(size_t)i] = done ? 1 : 0;
-    // (launch_conv2d zeroes the padding rows of the columns it writes; the stamp kernel only writes them when
-    // it writes whole columns)
-    if (st == NNVHIP_OK && stamps[i].win_only && o->ld != Nout) st = launch_zero_pad_rows(c, stamps[i].out, o->ld, Nout, pl.m);
+    jobs.push_back(ConvJob{in[i]->V, in[i]->ld, o->V, pl.dense, in[i]->rows_pending ? in[i]->cls : nullptr,
+                           in[i]->rows_pending ? in[i]->keep_bits : nullptr, pl.compact ? ob : nullptr, pl.dense_eh, pl.dense_ew,
+                           pl.compact ? in[i]->box : nullptr, pl.compact && lazy, sch == 1 ? &stamps[i] : nullptr, false});
   }
+  if (st == NNVHIP_OK) st = launch_conv2d(c, cv, H, W, Ho, Wo, outs[0]->ld, jobs);
   if (st == NNVHIP_OK && any_stamps) {
     // the stamp pass also leaves the range sums of its columns on the output handles; sets whose stamps went into
     // their convolution's launch are done
     std::vector<ConvStampSet> rest = stamps;
     bool any_left = false;
     for (int64_t i = 0; i < count; ++i) {
-      if (stamped[(size_t)i]) rest[(size_t)i].m = 0;
+      if (jobs[(size_t)i].stamped) rest[(size_t)i].m = 0;
       any_left = any_left || rest[(size_t)i].m > 0;
     }
     if (any_left) st = launch_conv_stamps(c, cv, H, W, Ho, Wo, outs[0]->ld, count, rest.data(), sch);
@@ -176,6 +196,8 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
         outs[i]->rng_first_col = (in[i]->n + 1) - stamps[i].m;
       }
   }
+  // padding rows of every column of the call (they lie back to back)
+  if (st == NNVHIP_OK) st = launch_zero_pad_rows(c, outs[0]->V, outs[0]->ld, Nout, cols);
   if (st == NNVHIP_OK) st = c->end_op();
   if (st != NNVHIP_OK) {
     release_all(outs);
