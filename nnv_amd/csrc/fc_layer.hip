@@ -239,10 +239,21 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
       gs[i].fill = outs[i]->V;
       gs[i].bias = bias;
     };
+    // Images inside known windows (the output of a network's convolutional part): the contraction stays inside them
+    // (fc_window.hip) and reads nothing outside.  Calls that are launch bound take one dense launch as before; a set that
+    // keeps no row contracts over nothing.
+    int win_tile = 0;
+    if (st == NNVHIP_OK && !dense_only && (count == 1 || contig)) {
+      bool work = true;
+      for (int64_t i = 0; i < count && work; ++i)
+        work = !(in[i]->n_kept == 0 && in[i]->kept_idx != nullptr) &&
+               (double)fc->Mp * (double)fc->Kp * (double)dense[i] * (double)count >= 4.0e6;
+      if (work) win_tile = fc_window_tile(fc, count, in, dense.data());
+    }
     // Inputs with columns that are described but not in memory yet: the contraction reads them from
     // memory unless it goes over no row at all or through the packing pass (which takes such columns
     // from the weights they were gathered from).  Everybody else has them written now.
-    if (st == NNVHIP_OK) {
+    if (st == NNVHIP_OK && win_tile == 0) {
       std::vector<nnvhip_star*> cols;
       for (int64_t i = 0; i < count; ++i) {
         if (!in[i]->cs.any_pending()) continue;
@@ -281,9 +292,14 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
         // enough 128 x 128 tiles to go round: the tile kernel of gemm_seg.hip (rows packed transposed, operands
         // staged straight into LDS), as for an array of sets
         const int64_t tiles128 = ceil_div(dense[0], 128) * ceil_div(fc->Mp, 128);
-        const bool tile_kernel = compact && pack && rows.kmap != nullptr && !dense_only && tiles128 >= 128 && kp <= 2048 &&
+        const bool tile_kernel = win_tile == 0 && compact && pack && rows.kmap != nullptr && !dense_only && tiles128 >= 128 && kp <= 2048 &&
                                  dense[0] < (int64_t(1) << 24);
-        if (tile_kernel) {
+        if (win_tile > 0) {
+          fuse.chunks = ceil_div(dense[0] - 1, win_tile);
+          st = c->alloc(sizeof(double) * 4 * outs[0]->ld * fuse.chunks, &fuse.part);
+          const FcWindowSet ws{in[0], outs[0], dense[0], fuse.part ? fuse.part->as<double>() : nullptr};
+          if (st == NNVHIP_OK) st = launch_fc_window(c, fc, win_tile, 1, &ws);
+        } else if (tile_kernel) {
           const int64_t ldo = outs[0]->ld, ldt = round_up(dense[0], 128), ntiles = ceil_div(dense[0], 128);
           st = c->alloc(sizeof(double) * kp * ldt, &packed);
           if (st == NNVHIP_OK) {
@@ -332,7 +348,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
             rows.ldbk = kp;
           }
         }
-        if (st == NNVHIP_OK && !tile_kernel)
+        if (st == NNVHIP_OK && !tile_kernel && win_tile == 0)
           st = launch_gemm(c, Wd, fc->Mp, in[0]->V, in[0]->ld, outs[0]->V, outs[0]->ld, fc->Mp, dense[0], kp, bias, &fuse,
                            compact ? &rows : nullptr);
         if (st == NNVHIP_OK && fuse.chunks > 0) {
@@ -372,7 +388,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
         if (st == NNVHIP_OK && gs[0].m > 0) st = finalize_fused_ranges(c, outs[0], part, ch);
       } else {
         BufRef packed;
-        if (compact && pack) {
+        if (compact && pack && win_tile == 0) {
           st = c->alloc(sizeof(double) * kp * dense[0], &packed);
           if (st == NNVHIP_OK) {
             PackSet ps = pack_of(in[0], in[0]->kept_idx, packed->as<double>(), kp, dense[0]);
@@ -394,6 +410,11 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
             gs[0].cin = in[0]->V;
             gs[0].cpart = cpart->as<double>();
           }
+        } else if (st == NNVHIP_OK && win_tile > 0) {
+          fuse.chunks = ceil_div(dense[0] - 1, win_tile);
+          st = c->alloc(sizeof(double) * 4 * outs[0]->ld * (fuse.chunks + gch), &fuse.part);
+          const FcWindowSet ws{in[0], outs[0], dense[0], fuse.part ? fuse.part->as<double>() : nullptr};
+          if (st == NNVHIP_OK) st = launch_fc_window(c, fc, win_tile, 1, &ws);
         } else if (st == NNVHIP_OK) {
           st = launch_gemm(c, Wd, fc->Mp, in[0]->V, in[0]->ld, outs[0]->V, outs[0]->ld, fc->Mp, dense[0], kp, bias,
                            centre_only ? nullptr : &fuse, compact ? &rows : nullptr, centre_only ? &defer : nullptr);
@@ -462,7 +483,19 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
         all_stored = all_stored && in[i]->stored_cols() == in[i]->n + 1;
         centres_only = centres_only && in[i]->stored_cols() == 1 && dense[i] == 1;
       }
-      if (any_onehot && !any_rows && (all_stored || centres_only)) {
+      if (win_tile > 0) {
+        const int64_t ldo = outs[0]->ld;
+        for (int64_t i = 0; i < count; ++i) {
+          tiles_of[i] = ceil_div(dense[i] - 1, win_tile);
+          chunk_off[i + 1] = chunk_off[i] + tiles_of[i] + (gs[i].m > 0 ? gch_part : 0);
+        }
+        st = c->alloc(sizeof(double) * 4 * ldo * chunk_off[count], &sums);
+        std::vector<FcWindowSet> ws((size_t)count);
+        for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i)
+          ws[(size_t)i] = FcWindowSet{in[i], outs[i], dense[i], sums->as<double>() + 4 * ldo * chunk_off[i]};
+        if (st == NNVHIP_OK) st = launch_fc_window(c, fc, win_tile, count, ws.data());
+        bias_in_kernel = true;
+      } else if (any_onehot && !any_rows && (all_stored || centres_only)) {
         // all sets contract over every row: their dense columns are simply listed (tiles may span sets)
         if (cols >= (int64_t(1) << 31)) st = NNVHIP_ERR_SHAPE;
         std::vector<int32_t> map;

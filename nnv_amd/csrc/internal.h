@@ -901,6 +901,18 @@ int launch_fc_rowsum(nnvhip_ctx* ctx, const nnvhip_fc* fc, nnvhip_star* out, int
 int finalize_fused_ranges(nnvhip_ctx* ctx, nnvhip_star* s, const BufRef& part, int64_t chunks,
                           const double* cpart = nullptr, int64_t cchunks = 0, const double* cbias = nullptr);
 
+// fc_window.hip: the contraction of a fully connected layer over sets whose generator images are zero outside known windows
+// (nnvhip_star::box), tile by tile over the windows' union only.
+// Columns per tile where the sets of a call (all of them) take it, 0: they do not.  dense: leading columns to contract.
+int fc_window_tile(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in, const int64_t* dense);
+struct FcWindowSet {
+  const nnvhip_star* in;
+  nnvhip_star* out;   // its leading `dense` columns are written, bias included
+  int64_t dense;
+  double* rpart;      // ceil((dense - 1) / tile) chunks of [4][ld] range sums of the columns 1 .. dense - 1, or null
+};
+int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count, const FcWindowSet* sets);
+
 // relu.hip
 // Makes V a plain stored matrix: writes columns that are still pending (need_cols; always when one of
 // the other two steps reads them), runs a pending row reset and, with need_tail, writes the implicit
