@@ -13,22 +13,15 @@
 #include <cstring>
 #include <type_traits>
 
+#include "conv_stamp.h"
 #include "internal.h"
 #include "lds_dma.h"
 #include "mfma_tile.h"
 #include "relu_sort.h"
+#include "window_sort.h"
 
 namespace nnvhip {
 
-struct ConvGeom {
-  int H, W, Cin, Ho, Wo, Cout;
-  int FH, FW, sh, sw, dh, dw, pt, pl;
-  int K, Kp;
-  int P;   // Ho * Wo
-  int HW;  // H * W
-};
-
-constexpr int kMaxTaps = 4096;  // tap table held in LDS: 8 bytes per (padded) tap
 constexpr size_t kConvLdsLimit = 64 * 1024;  // LDS of one block: operand tiles + tap table + row mask
 
 // Tap k = fh + FH*(fw + FW*ci) -> packed (input offset ci*H*W : 32 | fh*dh : 16 | fw*dw : 16).
@@ -267,18 +260,6 @@ __global__ void conv_weights_kmajor_kernel(const double* __restrict__ W, double*
   Wk[idx] = co < Cout ? W[k + (int64_t)co * Kp] : 0.0;
 }
 
-struct StampSet {
-  const int32_t* idx;   // input row of every one-hot column
-  const double* scale;  // by input row, or null (= 1)
-  double* out;          // first of these columns in the output set
-  const double* plb;    // predicate bounds of these columns
-  const double* pub;
-  double* part;         // [chunks][4][ldout] range sums of these columns (as the estimateRanges pass leaves them)
-  int32_t m;
-  int32_t win_only;     // 1: only the rows inside a column's window (the positions whose taps span its pixel) are written
-  const int32_t* pixel_col;  // (by-row pass) input row -> its column here, -1: none
-};
-
 struct ConvFastArgs {  // the layer
   int64_t ldout;
   const double* Wk;
@@ -505,62 +486,69 @@ __global__ __launch_bounds__(512) void conv2d_fast_kernel(ConvFastArgs a, const 
   conv2d_fast_block<TC, WR, WC, MASK, COMPACT>(a, set, blockIdx.x, lds, keep_s);
 }
 
-// What the kernels above and below look up, for every set of a call (blockIdx.y) in one launch: the windows of the output's
-// columns (ConvSetup::out_box) and, by input row, the unit-vector column that sits there (ConvSetup::inv; -1: none).  The
-// first inv_blocks blocks build kInvRows entries of the second table each: in LDS, because every entry is written whether or
-// not a column names it, then out in order.  Latency bound (a few KB); three launches before.
-constexpr int kInvRows = 4096;
-__global__ __launch_bounds__(256) void conv_setup_kernel(const ConvSetup* __restrict__ table, ConvSetup one, int inv_blocks, ConvGeom g) {
-  const ConvSetup d = table ? table[blockIdx.y] : one;
-  if ((int)blockIdx.x < inv_blocks) {
-    __shared__ int32_t rows[kInvRows];
-    const int r0 = (int)blockIdx.x * kInvRows, nr = min(kInvRows, d.n_inv - r0);
-    if (d.inv == nullptr || nr <= 0) return;
-    for (int r = threadIdx.x; r < nr; r += 256) rows[r] = -1;
-    __syncthreads();
-    for (int t0 = threadIdx.x; t0 < d.m; t0 += 4 * 256) {
-      int at[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) at[u] = t0 + u * 256 < d.m ? d.idx[t0 + u * 256] - r0 : -1;
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (at[u] >= 0 && at[u] < nr) rows[at[u]] = t0 + u * 256;
-    }
-    __syncthreads();
-    for (int r = threadIdx.x; r < nr; r += 256) d.inv[r0 + r] = rows[r];
-    return;
-  }
-  const ColBox* __restrict__ in_box = d.in_box;
-  const int32_t* __restrict__ onehot_idx = d.idx;
-  ColBox* __restrict__ out_box = d.out_box;
-  const int dense = d.dense, m = d.m;
-  const int64_t j = ((int)blockIdx.x - inv_blocks) * (int64_t)256 + threadIdx.x;
-  if (out_box == nullptr || j >= (int64_t)dense + m) return;
+// Window of column j of the output: from the window of the input's column (in_box null: whole image) or the pixel of its
+// unit vector.
+__device__ __forceinline__ ColBox conv_out_box(const ConvSetup& d, const ConvGeom& g, int64_t j) {
   int h0 = 0, h1 = g.H - 1, w0 = 0, w1 = g.W - 1;  // window of the input column
-  if (j >= dense) {
-    const int src = onehot_idx[j - dense] % g.HW;
+  if (j >= d.dense) {
+    const int src = d.idx[j - d.dense] % g.HW;
     w0 = w1 = src / g.H;
     h0 = h1 = src - w0 * g.H;
-  } else if (j > 0 && in_box != nullptr) {
-    const ColBox b = in_box[j];
+  } else if (j > 0 && d.in_box != nullptr) {
+    const ColBox b = d.in_box[j];
     h0 = b.h0, h1 = b.h1, w0 = b.w0, w1 = b.w1;
   }
-  ColBox o;
-  if (j == 0) {
-    // the centre image is not sparse: where every tap falls into the padding it still holds the bias
-    o = ColBox{0, (int16_t)(g.Ho - 1), 0, (int16_t)(g.Wo - 1)};
-  } else if (h0 > h1 || w0 > w1) {
-    o = ColBox{1, 0, 1, 0};
-  } else {
-    // output rows whose taps ho*sh - pt + fh*dh (0 <= fh < FH) reach [h0, h1]
-    auto floordiv = [](int a, int s) { return a >= 0 ? a / s : -((-a + s - 1) / s); };
-    const int a0 = h0 + g.pt - (g.FH - 1) * g.dh, a1 = h1 + g.pt;
-    const int b0 = w0 + g.pl - (g.FW - 1) * g.dw, b1 = w1 + g.pl;
-    const int ho0 = max(0, -floordiv(-a0, g.sh)), ho1 = min(g.Ho - 1, floordiv(a1, g.sh));
-    const int wo0 = max(0, -floordiv(-b0, g.sw)), wo1 = min(g.Wo - 1, floordiv(b1, g.sw));
-    o = (ho0 > ho1 || wo0 > wo1) ? ColBox{1, 0, 1, 0} : ColBox{(int16_t)ho0, (int16_t)ho1, (int16_t)wo0, (int16_t)wo1};
+  // the centre image is not sparse: where every tap falls into the padding it still holds the bias
+  if (j == 0) return ColBox{0, (int16_t)(g.Ho - 1), 0, (int16_t)(g.Wo - 1)};
+  if (h0 > h1 || w0 > w1) return ColBox{1, 0, 1, 0};
+  // output rows whose taps ho*sh - pt + fh*dh (0 <= fh < FH) reach [h0, h1]
+  auto floordiv = [](int a, int s) { return a >= 0 ? a / s : -((-a + s - 1) / s); };
+  const int a0 = h0 + g.pt - (g.FH - 1) * g.dh, a1 = h1 + g.pt;
+  const int b0 = w0 + g.pl - (g.FW - 1) * g.dw, b1 = w1 + g.pl;
+  const int ho0 = max(0, -floordiv(-a0, g.sh)), ho1 = min(g.Ho - 1, floordiv(a1, g.sh));
+  const int wo0 = max(0, -floordiv(-b0, g.sw)), wo1 = min(g.Wo - 1, floordiv(b1, g.sw));
+  return (ho0 > ho1 || wo0 > wo1) ? ColBox{1, 0, 1, 0} : ColBox{(int16_t)ho0, (int16_t)ho1, (int16_t)wo0, (int16_t)wo1};
+}
+
+// What the kernels above and below look up, for every set of a call (blockIdx.y) in one launch: the windows of the output's
+// columns (ConvSetup::out_box), by input row the unit-vector column that sits there (ConvSetup::inv; -1: none), and the
+// order of the columns by the start of their windows (ConvSetup::order).  The first sort_blocks blocks make the order, a run
+// of columns each, the next inv_blocks build kInvRows entries of the second table each: in LDS, because every entry is written whether
+// or not a column names it, then out in order.  Latency bound (a few KB).
+constexpr int kInvRows = 4096;
+__global__ __launch_bounds__(kSortThreads) void conv_setup_kernel(const ConvSetup* __restrict__ table, ConvSetup one, int sort_blocks,
+                                                                  int inv_blocks, ConvGeom g) {
+  const ConvSetup d = table ? table[blockIdx.y] : one;
+  const int blk = (int)blockIdx.x - sort_blocks;
+  if (blk < 0) {
+    if (d.order == nullptr) return;
+    sort_windows(d.dense - 1, g.P, d.order, d.first, blockIdx.x, sort_blocks, [&](int j) {
+      const ColBox b = conv_out_box(d, g, j);
+      return b.h0 > b.h1 ? 0 : b.w0 * g.Ho + b.h0;
+    });
+    return;
   }
-  out_box[j] = o;
+  if (blk < inv_blocks) {
+    __shared__ int32_t rows[kInvRows];
+    const int r0 = blk * kInvRows, nr = min(kInvRows, d.n_inv - r0);
+    if (d.inv == nullptr || nr <= 0) return;
+    for (int r = threadIdx.x; r < nr; r += kSortThreads) rows[r] = -1;
+    __syncthreads();
+    for (int t0 = threadIdx.x; t0 < d.m; t0 += 4 * kSortThreads) {
+      int at[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) at[u] = t0 + u * kSortThreads < d.m ? d.idx[t0 + u * kSortThreads] - r0 : -1;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (at[u] >= 0 && at[u] < nr) rows[at[u]] = t0 + u * kSortThreads;
+    }
+    __syncthreads();
+    for (int r = threadIdx.x; r < nr; r += kSortThreads) d.inv[r0 + r] = rows[r];
+    return;
+  }
+  const int64_t j = (blk - inv_blocks) * (int64_t)kSortThreads + threadIdx.x;
+  if (d.out_box == nullptr || j >= (int64_t)d.dense + d.m) return;
+  d.out_box[j] = conv_out_box(d, g, j);
 }
 
 __global__ void zero_pad_rows_kernel(double* __restrict__ V, int64_t ld, int64_t N, int64_t ncols) {
@@ -711,90 +699,6 @@ __global__ __launch_bounds__(256) void keep_bits_kernel(const KeepBits* __restri
   if ((lane & 31) == 0 && w < words) bits[w] = (uint32_t)(b >> lane);
 }
 
-// ---- the stamps by output row (undilated filters) ---------------------------------------------------
-// Row r = (ho, wo, co) of the output meets the stamps of the pixels under its filter window, one per tap: for
-// tap k = (fh, fw, ci) the pixel (ho*sh - pt + fh, wo*sw - pl + fw, ci), whose unit-vector column t (pixel_col,
-// -1: none) gets out(r, t) = 0 + W(k, co) * scale.  One thread per row writes those elements - exactly the
-// non-zero candidates, i.e. the rows inside every column's window - and adds up the row's four range sums tap
-// by tap.  Everything else in the columns is zero and is written by the caller (or left for later).
-// S lanes share a row, lane s taking the taps k = s, s + S, ...; their sums are combined by a butterfly (a fixed
-// order).  S = 1 for filters with few taps, 16 otherwise (a row's taps are then walked by 16 lanes at once).
-// A block first decodes the taps once into LDS (filter position and the tap's offset from the pixel under the
-// filter's corner), so that the walk has no division in it, and looks up four taps' pixels before it handles them.
-constexpr int kStampTapTable = kMaxTaps;  // taps per output (FH * FW * Cin): no layer has more
-// Block `blk` of NT threads; taps: LDS for g.K entries.
-template <int S, int NT>
-__device__ __forceinline__ void conv_stamp_rows_block(int64_t blk, int2* taps, const StampSet& d, const ConvGeom& g,
-                                                      const double* __restrict__ Wt, const int32_t* __restrict__ pixel_col,
-                                                      int64_t ldout) {
-  for (int k = threadIdx.x; k < g.K; k += NT) {
-    const int fh = k % g.FH;
-    const int q = k / g.FH;
-    const int fw = q % g.FW;
-    const int ci = q / g.FW;
-    taps[k] = make_int2(fh | (fw << 16), fh + g.H * (fw + g.W * ci));  // x: fh | fw << 16, y: fh + H * (fw + W * ci)
-  }
-  __syncthreads();
-  const int64_t gt = blk * (int64_t)NT + threadIdx.x;
-  const int64_t r = gt / S;
-  const int s = (int)(gt % S);
-  const bool row = r < ldout;
-  const int64_t Nout = (int64_t)g.P * g.Cout;
-  double x1 = 0.0, x2 = 0.0, y1 = 0.0, y2 = 0.0;
-  if (row && r < Nout) {
-    const int co = (int)(r / g.P);
-    const int p = (int)(r - (int64_t)co * g.P);
-    const int wo = p / g.Ho, ho = p - wo * g.Ho;
-    const int hb = ho * g.sh - g.pt, wb = wo * g.sw - g.pl;
-    const int pbase = hb + g.H * wb;  // the pixel under the filter's corner (may lie outside the image)
-    const double* wcol = Wt + (int64_t)co * g.Kp;
-    for (int k0 = s; k0 < g.K; k0 += 4 * S) {
-      int t[4], pix[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int k = k0 + u * S;
-        t[u] = -1;
-        pix[u] = 0;
-        if (k < g.K) {
-          const int2 tp = taps[k];
-          const int h = hb + (tp.x & 0xffff), w = wb + (tp.x >> 16);
-          if ((unsigned)h < (unsigned)g.H && (unsigned)w < (unsigned)g.W) {
-            pix[u] = pbase + tp.y;
-            t[u] = pixel_col[pix[u]];
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        if (t[u] < 0) continue;
-        const int k = k0 + u * S;
-        const double sc = d.scale != nullptr ? d.scale[pix[u]] : 1.0;
-        const double v = __dadd_rn(0.0, __dmul_rn(wcol[k], sc));
-        d.out[r + (int64_t)t[u] * ldout] = v;
-        const double pl = d.plb[t[u]], pu = d.pub[t[u]];
-        const double vp = fmax(v, 0.0), vn = fmin(v, 0.0);
-        x1 = fma(vp, pl, x1);  // xmin1
-        x2 = fma(vn, pu, x2);  // xmin2
-        y1 = fma(vp, pu, y1);  // xmax1
-        y2 = fma(vn, pl, y2);  // xmax2
-      }
-    }
-  }
-#pragma unroll
-  for (int off = 1; off < S; off <<= 1) {
-    x1 += __shfl_xor(x1, off);
-    x2 += __shfl_xor(x2, off);
-    y1 += __shfl_xor(y1, off);
-    y2 += __shfl_xor(y2, off);
-  }
-  if (row && s == 0) {
-    d.part[r] = x1;
-    d.part[ldout + r] = x2;
-    d.part[2 * ldout + r] = y1;
-    d.part[3 * ldout + r] = y2;
-  }
-}
-
 template <int S>
 __global__ __launch_bounds__(256) void conv_stamp_rows_kernel(StampSet d, ConvGeom g, const double* __restrict__ Wt,
                                                               const int32_t* __restrict__ pixel_col, int64_t ldout) {
@@ -854,8 +758,6 @@ static int launch_conv_cfg(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, const ConvG
   NNV_HIP_TRY(hipGetLastError());
   return NNVHIP_OK;
 }
-
-static void fill_geom(ConvGeom& g, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo);
 
 // ---- which kernel, and whether it can mask rows on load --------------------------------------------
 constexpr size_t conv_fast_static_lds(int tc) { return sizeof(double) * 2 * kKt * (128 + (size_t)tc); }
@@ -998,11 +900,13 @@ static int launch_setup(nnvhip_ctx* ctx, const ConvGeom& g, int64_t count, const
   for (int64_t i0 = 0; i0 < count; i0 += 65535) {
     const int64_t cnt = std::min<int64_t>(65535, count - i0);
     int64_t inv_rows = 0, cols = 0;
+    int sort_blocks = 0;
     for (int64_t i = i0; i < i0 + cnt; ++i) {
+      if (sets[i].order != nullptr) sort_blocks = std::max(sort_blocks, sort_window_blocks(sets[i].dense - 1));
       if (sets[i].inv != nullptr) inv_rows = std::max<int64_t>(inv_rows, sets[i].n_inv);
       if (sets[i].out_box != nullptr) cols = std::max<int64_t>(cols, (int64_t)sets[i].dense + sets[i].m);
     }
-    const int64_t inv_blocks = ceil_div(inv_rows, kInvRows), blocks = inv_blocks + ceil_div(cols, 256);
+    const int64_t inv_blocks = ceil_div(inv_rows, kInvRows), blocks = sort_blocks + inv_blocks + ceil_div(cols, kSortThreads);
     if (blocks == 0) continue;
     const ConvSetup* table = nullptr;
     BufRef tab;
@@ -1010,8 +914,8 @@ static int launch_setup(nnvhip_ctx* ctx, const ConvGeom& g, int64_t count, const
       NNV_TRY(ctx->upload_table(sets + i0, sizeof(ConvSetup) * (size_t)cnt, &tab));
       table = tab->as<ConvSetup>();
     }
-    hipLaunchKernelGGL(conv_setup_kernel, dim3((unsigned)blocks, (unsigned)cnt), dim3(256), 0, ctx->stream, table, sets[i0],
-                       (int)inv_blocks, g);
+    hipLaunchKernelGGL(conv_setup_kernel, dim3((unsigned)blocks, (unsigned)cnt), dim3(kSortThreads), 0, ctx->stream, table, sets[i0],
+                       sort_blocks, (int)inv_blocks, g);
     NNV_HIP_TRY(hipGetLastError());
   }
   return NNVHIP_OK;
@@ -1040,7 +944,7 @@ int launch_pool_boxes(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t
   g.pt = (int)pad_top;
   g.pl = (int)pad_left;
   g.HW = (int)(H * W);
-  const ConvSetup one{in_box, onehot_idx, out_box, nullptr, (int32_t)dense, (int32_t)m, 0};
+  const ConvSetup one{in_box, onehot_idx, out_box, nullptr, (int32_t)dense, (int32_t)m, 0, nullptr, nullptr};
   return launch_setup(ctx, g, 1, &one);
 }
 
@@ -1154,7 +1058,7 @@ int launch_conv2d(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int64_t W
   return NNVHIP_OK;
 }
 
-static void fill_geom(ConvGeom& g, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo) {
+void fill_geom(ConvGeom& g, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo) {
   g.H = (int)H;
   g.W = (int)W;
   g.Cin = (int)cv->Cin;

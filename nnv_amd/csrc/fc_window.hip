@@ -21,6 +21,7 @@
 #include "internal.h"
 #include "mfma_tile.h"
 #include "relu_sort.h"
+#include "window_sort.h"
 
 namespace nnvhip {
 
@@ -47,11 +48,25 @@ struct FcWinArgs {
   int32_t shift;         // window starts are told apart in steps of 1 << shift positions
   int32_t buckets;
   int32_t tiles_m;
+  int32_t sort_blocks;
 };
 
-constexpr int kSortThreads = 1024;
-constexpr int kSortWaves = kSortThreads / 64;
-constexpr int kMaxBuckets = 1024;  // the waves' counts take 32 KB of LDS
+// This block's set.
+__device__ __forceinline__ FcWinSet win_set(const FcWinSet* __restrict__ table, const FcWinSet& one) {
+  FcWinSet s = table ? in_global(table)[blockIdx.y] : one;
+  s.V = in_global(s.V);
+  s.box = in_global(s.box);
+  s.keep_bits = in_global(s.keep_bits);
+  s.cls = in_global(s.cls);
+  s.kept = in_global(s.kept);
+  s.order = in_global(s.order);
+  s.cpart = in_global(s.cpart);
+  s.out = in_global(s.out);
+  s.plb = in_global(s.plb);
+  s.pub = in_global(s.pub);
+  s.rpart = in_global(s.rpart);
+  return s;
+}
 
 // Place of a window's start on a walk over strips two positions wide, up one strip and down the next, so that columns
 // next to one another in the order start next to one another.  An empty window goes first.
@@ -62,14 +77,14 @@ __device__ __forceinline__ int window_bucket(ColBox b, const FcWinArgs& a) {
   return min((strip * hs + ((strip & 1) ? hs - 1 - h : h)) * 2 + (w & 1), a.buckets - 1);
 }
 
-// Block 0 of a set: the stable counting sort of its columns by window start.  The other blocks: a share of the rows of
-// the centre's product each.  Grid: (1 + centre blocks, sets).
+// The first sort_blocks blocks of a set: the stable counting sort of its columns by window start.  The other blocks: a share
+// of the rows of the centre's product each.  Grid: (sort blocks + centre blocks, sets).
 __global__ __launch_bounds__(kSortThreads) void fc_window_setup_kernel(const FcWinSet* __restrict__ table, FcWinSet one, FcWinArgs a) {
-  const FcWinSet S = table ? table[blockIdx.y] : one;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  if (blockIdx.x > 0) {  // rows [k0, k1) of the centre's product; a row of the output per thread, groups of threads interleave
+  const FcWinSet S = win_set(table, one);
+  const int tid = threadIdx.x;
+  if ((int)blockIdx.x >= a.sort_blocks) {  // rows [k0, k1) of the centre's product; a row of the output per thread, groups of threads interleave
     __shared__ double red[kSortThreads];
-    const int chunk = blockIdx.x - 1;
+    const int chunk = blockIdx.x - a.sort_blocks;
     if (chunk >= S.cchunks) return;
     const int k0 = chunk * S.kper, k1 = min(S.nk, k0 + S.kper);
     const int rp = min(kSortThreads, (a.Mp + 63) / 64 * 64), groups = kSortThreads / rp;
@@ -101,83 +116,7 @@ __global__ __launch_bounds__(kSortThreads) void fc_window_setup_kernel(const FcW
     }
     return;
   }
-  __shared__ uint16_t cnt[kSortWaves][kMaxBuckets];
-  __shared__ int wsum[kSortWaves];
-  const int n = S.ncols - 1;
-  for (int t = tid; t < kSortWaves * kMaxBuckets / 2; t += kSortThreads) reinterpret_cast<uint32_t*>(cnt)[t] = 0;
-  __syncthreads();
-  int bits = 0;
-  while ((1 << bits) < a.buckets) ++bits;
-  // a wave owns a run of columns, 64 at a time: lanes with the same bucket find each other by one ballot per bit
-  const int seg = ((n + kSortWaves - 1) / kSortWaves + 63) / 64 * 64;
-  const int j0 = min(n, wave * seg), j1 = min(n, j0 + seg);
-  auto same_bucket = [&](int key, bool valid) {
-    unsigned long long m = __ballot(valid);
-    for (int b = 0; b < bits; ++b) {
-      const unsigned long long v = __ballot((key >> b) & 1);
-      m &= ((key >> b) & 1) ? v : ~v;
-    }
-    return m;
-  };
-  const unsigned long long below = (1ull << lane) - 1ull;
-  constexpr int kAhead = 8;  // rounds whose windows are asked for together
-  for (int jj = j0; jj < j1; jj += 64 * kAhead) {
-    int keys[kAhead];
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      const int j = jj + 64 * u + lane;
-      keys[u] = j < j1 ? window_bucket(S.box[1 + j], a) : 0;
-    }
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      if (jj + 64 * u >= j1) break;
-      const bool valid = jj + 64 * u + lane < j1;
-      const int key = keys[u];
-      const unsigned long long m = same_bucket(key, valid);
-      if (valid && (m & below) == 0) cnt[wave][key] = (uint16_t)(cnt[wave][key] + __popcll(m));
-    }
-  }
-  __syncthreads();
-  // first place of every (bucket, wave): buckets in order, a bucket's waves in order
-  int total = 0;
-  if (tid < a.buckets)
-    for (int w = 0; w < kSortWaves; ++w) {
-      const int c = cnt[w][tid];
-      cnt[w][tid] = (uint16_t)total;
-      total += c;
-    }
-  int scan = total;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int v = __shfl_up(scan, off);
-    if (lane >= off) scan += v;
-  }
-  if (lane == 63) wsum[wave] = scan;
-  __syncthreads();
-  int base = scan - total;
-  for (int w = 0; w < wave; ++w) base += wsum[w];
-  if (tid < a.buckets)
-    for (int w = 0; w < kSortWaves; ++w) cnt[w][tid] = (uint16_t)(cnt[w][tid] + base);
-  __syncthreads();
-  for (int jj = j0; jj < j1; jj += 64 * kAhead) {
-    int keys[kAhead];
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      const int j = jj + 64 * u + lane;
-      keys[u] = j < j1 ? window_bucket(S.box[1 + j], a) : 0;
-    }
-#pragma unroll
-    for (int u = 0; u < kAhead; ++u) {
-      if (jj + 64 * u >= j1) break;
-      const int j = jj + 64 * u + lane;
-      const bool valid = j < j1;
-      const int key = keys[u];
-      const unsigned long long m = same_bucket(key, valid);
-      const int at = valid ? cnt[wave][key] : 0;
-      if (valid) S.order[at + __popcll(m & below)] = 1 + j;
-      if (valid && (m & below) == 0) cnt[wave][key] = (uint16_t)(at + __popcll(m));
-    }
-  }
+  sort_windows(S.ncols - 1, a.buckets, S.order, nullptr, blockIdx.x, a.sort_blocks, [&](int j) { return window_bucket(S.box[j], a); });
 }
 
 // TM x TN output tile per block of WR x WC waves.  Column tiles are dealt to the XCDs (blockIdx.x % 8) with all their row
@@ -197,7 +136,7 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
   __shared__ double s_pl[TN], s_pu[TN];
   __shared__ int s_u[4];
   __shared__ int s_cnt[NW];
-  const FcWinSet S = table ? table[blockIdx.y] : one;
+  const FcWinSet S = win_set(table, one);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   const int mt = slot % a.tiles_m, nt = (slot / a.tiles_m) * 8 + xcd;
@@ -406,7 +345,7 @@ int fc_window_tile(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in, c
     const nnvhip_star* s = in[i];
     const ColSource& cs = s->cs;
     if (s->box == nullptr || s->box_H != H || s->box_W != W || s->box_eh != f->box_eh || s->box_ew != f->box_ew) return 0;
-    if (dense[i] < 2 || dense[i] > 65535 || dense[i] > s->box_cols || dense[i] > s->stored_cols()) return 0;
+    if (dense[i] < 2 || dense[i] > kSortColumns || dense[i] > s->box_cols || dense[i] > s->stored_cols()) return 0;
     // (unit-vector columns carry their one in a row the step has reset: they are the gather pass's)
     if (s->oh_from > 0 && dense[i] > s->oh_from) return 0;
     if (cs.pending || cs.zero_to > 1 || cs.delta_pending()) return 0;
@@ -441,7 +380,7 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
     const int64_t hs = ((a.H - 1) >> shift) + 1, ws = ((a.Wd - 1) >> shift) + 1;
     return ceil_div(ws, 2) * hs * 2;
   };
-  while (buckets(a.shift) > kMaxBuckets) ++a.shift;
+  while (buckets(a.shift) > kSortBuckets) ++a.shift;
   a.buckets = (int32_t)buckets(a.shift);
   const int tm = fc->Mp <= 32 ? 32 : 64;
   a.tiles_m = (int32_t)ceil_div(fc->Mp, tm);
@@ -462,6 +401,7 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
     parts += d.cchunks;
     max_tiles = std::max<int64_t>(max_tiles, d.tiles);
     max_chunks = std::max<int64_t>(max_chunks, d.cchunks);
+    a.sort_blocks = std::max(a.sort_blocks, sort_window_blocks(sets[i].dense - 1));
   }
   BufRef order, cpart, dev;
   NNV_TRY(ctx->alloc(sizeof(int32_t) * orders, &order));
@@ -491,7 +431,7 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
     NNV_TRY(ctx->upload_table(tab.data(), sizeof(FcWinSet) * tab.size(), &dev));
     table = dev->as<FcWinSet>();
   }
-  hipLaunchKernelGGL(fc_window_setup_kernel, dim3((unsigned)(1 + max_chunks), (unsigned)count), dim3(kSortThreads), 0, ctx->stream, table,
+  hipLaunchKernelGGL(fc_window_setup_kernel, dim3((unsigned)(a.sort_blocks + max_chunks), (unsigned)count), dim3(kSortThreads), 0, ctx->stream, table,
                      tab[0], a);
   const dim3 grid((unsigned)(round_up(max_tiles + 1, 8) * a.tiles_m), (unsigned)count);
 #define NNV_FC_WINDOW(TM, TN, WR, WC, KT) \

@@ -112,6 +112,15 @@ Ref<T> make_ref() {
   return Ref<T>(new T());
 }
 
+// The same pointer, known to the compiler to point to device memory.  A pointer that a kernel reads from a descriptor in
+// memory could point anywhere as far as the compiler knows, and its accesses become flat ones: those count as LDS operations
+// as well, so that every wait for an LDS read also waits for all of them, and loads issued ahead of the work they are for
+// are waited for at once.
+template <class T>
+__device__ __forceinline__ T* in_global(T* p) {
+  return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;  // (a direct cast there and back is folded away)
+}
+
 struct Buffer {
   int64_t ref_count = 0;
   nnvhip_ctx* ctx = nullptr;
@@ -796,13 +805,18 @@ bool conv2d_in_windows(const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t 
                        const ColBox* out_box, int eh, int ew);
 // Windows of a convolution's output columns (out_box, or null: none wanted): column 0 the whole image; columns below `dense`
 // from the input's windows (in_box null: whole image); the `m` columns from `dense` on from the pixels idx names.  And
-// inv[idx[t]] = t, -1 elsewhere (n_inv entries; inv null: not wanted).
+// inv[idx[t]] = t, -1 elsewhere (n_inv entries; inv null: not wanted).  And (order null: not wanted) the columns 1 ..
+// dense - 1 by where their output windows start: order[first[s] .. first[s + 1]) are those that start at position s = w0 * Ho
+// + h0, ascending (columns with an empty window stand anywhere); needs the input's windows, at most kSortColumns columns and
+// kSortBuckets positions.
 struct ConvSetup {
   const ColBox* in_box;
   const int32_t* idx;
   ColBox* out_box;
   int32_t* inv;
   int32_t dense, m, n_inv;
+  int32_t* order;
+  int32_t* first;
 };
 int launch_conv_setup(nnvhip_ctx* ctx, const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t count,
                       const ConvSetup* sets);
@@ -815,6 +829,24 @@ int64_t conv_box_extent(const nnvhip_conv2d* conv, int dim, int64_t e, int64_t o
 // whether launch_conv2d takes pending_cls for such an input (H x W x Cin images, leading dimension ldin)
 bool conv2d_can_mask(const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldin);
 int conv2d_prepare_weights(nnvhip_ctx* ctx, nnvhip_conv2d* conv);  // builds conv->Wk from conv->W (at creation)
+
+// conv_window.hip: the dense images 0 .. dense - 1 of sets with windows (ConvJob::in_box / out_box), by output position, with
+// their range sums.  The elements inside the output windows are written, nothing else.
+bool conv_window_takes(const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t dense, int eh, int ew);
+int conv_window_parts(const nnvhip_conv2d* conv, int64_t Ho, int64_t Wo, int64_t dense, int eh, int ew);  // chunks of range sums of such a set
+struct ConvWindowSet {
+  const nnvhip_star* in;
+  const nnvhip_star* out;  // with its windows
+  int64_t dense;
+  int eh, ew;              // bound on the output windows of its images
+  const int32_t* order;    // ConvSetup::order, first
+  const int32_t* first;
+  int64_t parts;           // conv_window_parts
+  double* part;            // [parts][4][ldout]
+  const ConvStampSet* stamp;  // its unit-vector columns, stamped in the same launch (with their pixel table; undilated filters), or null
+};
+int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldout, int64_t count,
+                       const ConvWindowSet* sets);
 
 // Whether the stamp launch of this layer looks columns up by pixel (ConvStampSet::pixel_col).
 bool conv_stamps_by_pixel(const nnvhip_conv2d* conv);

@@ -91,26 +91,39 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
     max_m = std::max<int64_t>(max_m, plan[i].m);
   }
   const int64_t sch = any_stamps && st == NNVHIP_OK ? conv_stamp_chunks(cv, outs[0]->ld, count, max_m) : 0;
+  // Images with windows go by output position (conv_window.hip), which leaves their range sums too; not when the caller
+  // wants every column in memory (the zeros around the windows are then written first).
+  std::vector<int64_t> parts((size_t)count, 0), chunk_at((size_t)count + 1, 0);  // parts > 0: by position
+  for (int64_t i = 0; i < count; ++i) {
+    const Plan& pl = plan[i];
+    if (!c->eager_cols && pl.out_boxes && pl.compact && conv_window_takes(cv, H, W, Ho, Wo, pl.dense, pl.dense_eh, pl.dense_ew))
+      parts[(size_t)i] = conv_window_parts(cv, Ho, Wo, pl.dense, pl.dense_eh, pl.dense_ew);
+    chunk_at[(size_t)i + 1] = chunk_at[(size_t)i] + parts[(size_t)i] + sch;
+  }
   BufRef sums;
-  if (sch > 0) st = c->alloc(sizeof(double) * 4 * outs[0]->ld * sch * count, &sums);
+  if (chunk_at[(size_t)count] > 0 && st == NNVHIP_OK) st = c->alloc(sizeof(double) * 4 * outs[0]->ld * chunk_at[(size_t)count], &sums);
   // windows of the output's columns and the pixel tables of the unit-vector columns: one buffer each, one launch
   std::vector<ConvSetup> setup((size_t)count);
-  BufRef boxes, invs;
-  int64_t box_cols = 0, inv_sets = 0;
+  BufRef boxes, invs, orders;
+  int64_t box_cols = 0, inv_sets = 0, order_ints = 0;
+  const int64_t first_stride = round_up(Ho * Wo + 1, kLdAlign);
   const int64_t inv_stride = round_up(in[0]->N, kLdAlign);
   auto wants_inv = [&](int64_t i) { return plan[i].m > 0 && in[i]->oh_inv == nullptr && conv_stamps_by_pixel(cv); };
   for (int64_t i = 0; i < count; ++i) {
     if (plan[i].out_boxes) box_cols += plan[i].nc;
     if (wants_inv(i)) ++inv_sets;
+    if (parts[(size_t)i] > 0) order_ints += first_stride + plan[i].dense;
   }
+  if (st == NNVHIP_OK && order_ints > 0) st = c->alloc(sizeof(int32_t) * (size_t)order_ints, &orders);
   if (st == NNVHIP_OK && box_cols > 0) st = c->alloc(sizeof(ColBox) * (size_t)box_cols, &boxes);
   if (st == NNVHIP_OK && inv_sets > 0) st = c->alloc(sizeof(int32_t) * (size_t)(inv_stride * inv_sets), &invs);
   if (st == NNVHIP_OK && (box_cols > 0 || inv_sets > 0)) {
-    int64_t box_at = 0, inv_at = 0;
+    int64_t box_at = 0, inv_at = 0, order_at = 0;
     for (int64_t i = 0; i < count; ++i) {
       const Plan& pl = plan[i];
       ConvSetup& su = setup[(size_t)i];
-      su = ConvSetup{pl.in_ok ? in[i]->box : nullptr, in[i]->oh_idx, nullptr, nullptr, (int32_t)pl.dense, (int32_t)pl.m, (int32_t)in[i]->N};
+      su = ConvSetup{pl.in_ok ? in[i]->box : nullptr, in[i]->oh_idx, nullptr, nullptr, (int32_t)pl.dense, (int32_t)pl.m, (int32_t)in[i]->N, nullptr,
+                     nullptr};
       if (pl.out_boxes) {
         su.out_box = boxes->as<ColBox>() + box_at;
         box_at += pl.nc;
@@ -118,6 +131,11 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
       if (wants_inv(i)) {
         su.inv = invs->as<int32_t>() + inv_at;
         inv_at += inv_stride;
+      }
+      if (parts[(size_t)i] > 0) {
+        su.first = orders->as<int32_t>() + order_at;
+        su.order = su.first + first_stride;
+        order_at += first_stride + pl.dense;
       }
     }
     st = launch_conv_setup(c, cv, H, W, Ho, Wo, count, setup.data());
@@ -128,6 +146,9 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
       }
   }
   std::vector<ConvJob> jobs;
+  std::vector<int64_t> job_of;
+  std::vector<ConvWindowSet> windows;
+  std::vector<char> stamped((size_t)count, 0);  // sets whose stamps go into another launch
   jobs.reserve((size_t)count);
   for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i) {
     const Plan& pl = plan[i];
@@ -169,22 +190,33 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
     stamps[i].out = o->V + pl.dense * o->ld;
     stamps[i].plb = o->plb + (pl.dense - 1);
     stamps[i].pub = o->pub + (pl.dense - 1);
-    stamps[i].part = sums ? sums->as<double>() + 4 * outs[0]->ld * sch * i : nullptr;
+    stamps[i].part = sums ? sums->as<double>() + 4 * outs[0]->ld * (chunk_at[(size_t)i] + parts[(size_t)i]) : nullptr;
     stamps[i].m = (int32_t)pl.m;
     stamps[i].pixel_col = in[i]->oh_inv;
     stamps[i].win_only = (lazy && pl.m > 0) ? 1 : 0;
-    jobs.push_back(ConvJob{in[i]->V, in[i]->ld, o->V, pl.dense, in[i]->rows_pending ? in[i]->cls : nullptr,
-                           in[i]->rows_pending ? in[i]->keep_bits : nullptr, pl.compact ? ob : nullptr, pl.dense_eh, pl.dense_ew,
-                           pl.compact ? in[i]->box : nullptr, pl.compact && lazy, sch == 1 ? &stamps[i] : nullptr, false});
+    if (parts[(size_t)i] > 0) {
+      const bool stamp = sch == 1 && pl.m > 0 && in[i]->oh_inv != nullptr && conv_stamps_by_pixel(cv);
+      windows.push_back(ConvWindowSet{in[i], o, pl.dense, pl.dense_eh, pl.dense_ew, setup[(size_t)i].order, setup[(size_t)i].first, parts[(size_t)i],
+                                      sums->as<double>() + 4 * o->ld * chunk_at[(size_t)i], stamp ? &stamps[i] : nullptr});
+      if (stamp) stamped[(size_t)i] = 1;
+    } else {
+      job_of.push_back(i);
+      jobs.push_back(ConvJob{in[i]->V, in[i]->ld, o->V, pl.dense, in[i]->rows_pending ? in[i]->cls : nullptr,
+                             in[i]->rows_pending ? in[i]->keep_bits : nullptr, pl.compact ? ob : nullptr, pl.dense_eh, pl.dense_ew,
+                             pl.compact ? in[i]->box : nullptr, pl.compact && lazy, sch == 1 ? &stamps[i] : nullptr, false});
+    }
   }
   if (st == NNVHIP_OK) st = launch_conv2d(c, cv, H, W, Ho, Wo, outs[0]->ld, jobs);
+  for (size_t k = 0; k < jobs.size(); ++k) stamped[(size_t)job_of[k]] = jobs[k].stamped ? 1 : 0;
+  if (st == NNVHIP_OK)
+    st = launch_conv_window(c, cv, H, W, Ho, Wo, outs[0]->ld, (int64_t)windows.size(), windows.data());
   if (st == NNVHIP_OK && any_stamps) {
     // the stamp pass also leaves the range sums of its columns on the output handles; sets whose stamps went into
     // their convolution's launch are done
     std::vector<ConvStampSet> rest = stamps;
     bool any_left = false;
     for (int64_t i = 0; i < count; ++i) {
-      if (jobs[(size_t)i].stamped) rest[(size_t)i].m = 0;
+      if (stamped[(size_t)i]) rest[(size_t)i].m = 0;
       any_left = any_left || rest[(size_t)i].m > 0;
     }
     if (any_left) st = launch_conv_stamps(c, cv, H, W, Ho, Wo, outs[0]->ld, count, rest.data(), sch);
@@ -195,6 +227,13 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
         outs[i]->rng_chunks = sch;
         outs[i]->rng_first_col = (in[i]->n + 1) - stamps[i].m;
       }
+  }
+  for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i) {  // ... and with the images' own, every column has its sums
+    if (parts[(size_t)i] == 0) continue;
+    outs[i]->rng_buf = sums;
+    outs[i]->rng_part = sums->as<double>() + 4 * outs[0]->ld * chunk_at[(size_t)i];
+    outs[i]->rng_chunks = parts[(size_t)i] + (stamps[i].m > 0 ? sch : 0);
+    outs[i]->rng_first_col = 1;
   }
   // padding rows of every column of the call (they lie back to back)
   if (st == NNVHIP_OK) st = launch_zero_pad_rows(c, outs[0]->V, outs[0]->ld, Nout, cols);
