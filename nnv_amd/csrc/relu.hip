@@ -355,40 +355,40 @@ __global__ __launch_bounds__(256) void relu_rank_kernel(const ReluDesc* __restri
       d.pub_out[j] = d.pub_in[j];
     }
   }
-  const int i0 = blockIdx.x * kRankI;
-  if (i0 >= m) return;
   const int il = tid & (kRankI - 1), slice = tid / kRankI;  // 256 / kRankI = 16 slices
-  const int i = i0 + il;
-  const double ki = i < m ? d.key[i] : 0.0;
   __shared__ double keys[kRankStage];
   __shared__ int part[16][kRankI];
-  int cnt = 0;
-  for (int base = 0; base < m; base += kRankStage) {
-    const int n = min(kRankStage, m - base);
-    if (base > 0) __syncthreads();  // everybody is done with the previous piece
-    for (int t = tid; t < n; t += 256) keys[t] = d.key[base + t];
-    __syncthreads();
+  for (int i0 = blockIdx.x * kRankI; i0 < m; i0 += gridDim.x * kRankI) {
+    const int i = i0 + il;
+    const double ki = i < m ? d.key[i] : 0.0;
+    int cnt = 0;
+    for (int base = 0; base < m; base += kRankStage) {
+      const int n = min(kRankStage, m - base);
+      __syncthreads();  // everybody is done with the previous piece
+      for (int t = tid; t < n; t += 256) keys[t] = d.key[base + t];
+      __syncthreads();
 #pragma unroll 8
-    for (int t = slice; t < n; t += 16) {
-      const double kj = keys[t];
-      cnt += (kj > ki || (kj == ki && (base + t) < i)) ? 1 : 0;
+      for (int t = slice; t < n; t += 16) {
+        const double kj = keys[t];
+        cnt += (kj > ki || (kj == ki && (base + t) < i)) ? 1 : 0;
+      }
     }
-  }
-  part[slice][il] = cnt;
-  __syncthreads();
-  if (slice != 0 || i >= m) return;
-  int r = 0;
+    part[slice][il] = cnt;
+    __syncthreads();
+    if (slice != 0 || i >= m) continue;
+    int r = 0;
 #pragma unroll
-  for (int q = 0; q < 16; ++q) r += part[q][il];
-  const int neuron = d.asc_idx[i];
-  d.cross_idx[r] = neuron;
-  if (d.col_of != nullptr) d.col_of[neuron] = r;
-  if (flags & kRankNewBounds) {
-    const double ub = d.ub[neuron];
-    d.plb_out[n_in + r] = 0.0;
-    d.pub_out[n_in + r] = ub;
-    d.lbub[r] = d.lb[neuron];
-    d.lbub[d.ld_lbub + r] = ub;
+    for (int q = 0; q < 16; ++q) r += part[q][il];
+    const int neuron = d.asc_idx[i];
+    d.cross_idx[r] = neuron;
+    if (d.col_of != nullptr) d.col_of[neuron] = r;
+    if (flags & kRankNewBounds) {
+      const double ub = d.ub[neuron];
+      d.plb_out[n_in + r] = 0.0;
+      d.pub_out[n_in + r] = ub;
+      d.lbub[r] = d.lb[neuron];
+      d.lbub[d.ld_lbub + r] = ub;
+    }
   }
 }
 
@@ -856,8 +856,10 @@ int relu_relax(nnvhip_ctx* ctx, int order, int64_t count, nnvhip_star* const* in
     NNV_LAUNCH(ctx, tk, relu_compact_kernel, grid, dim3(1024), 0, table, descs[0]);
     NNV_TRY(ctx->kernel_timer_end(tk, 6, 0.5 * cls_bytes));
     if (early_rank)
-      hipLaunchKernelGGL(relu_rank_kernel, dim3((unsigned)ceil_div(N, kRankI), 1, (unsigned)count), dim3(256), 0, ctx->stream, table,
-                         descs[0], kRankNewBounds | kRankOldBounds | kRankCountOnDevice);
+      // (the host does not know m yet: enough blocks to fill the chip once, which walk the list; a block for every 16 neurons
+      // that might cross were 19 600 for 25 sets of 12 544 neurons, most of them idle: 39 us, now 11)
+      hipLaunchKernelGGL(relu_rank_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(N, kRankI), std::max<int64_t>(64, 1024 / count)), 1, (unsigned)count),
+                         dim3(256), 0, ctx->stream, table, descs[0], kRankNewBounds | kRankOldBounds | kRankCountOnDevice);
   }
   NNV_HIP_TRY(hipGetLastError());
 
