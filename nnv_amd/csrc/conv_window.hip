@@ -194,8 +194,7 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
     for (int q = 0; q < 4; ++q) x[i][q] = 0.0;
 
   const int lo = (int)((int64_t)total * part / S.parts), hi = (int)((int64_t)total * (part + 1) / S.parts);
-  // (the first part's first stretch starts with the centre, which covers every position; its bounds are zero: it adds
-  // nothing to the sums)
+  // (the first part's first stretch starts with the centre, which covers every position)
   for (int i0 = lo; i0 < hi || (part == 0 && i0 == lo); i0 += kConvWinCols - 1) {
     // the columns of this stretch whose window covers the position
     int n = 0;
@@ -331,14 +330,15 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
           for (int r = 0; r < 4; ++r) {
             const int c = c0 + wc * (TN / WC) + j * 16 + lcol + 4 * r;
             if (c >= n) continue;
+            const int col = s_col[c];
             const double v = acc[i][j][r], pl = s_pl[c], pu = s_pu[c];
-            const double vp = fmax(v, 0.0), vn = fmin(v, 0.0);
+            // (the centre takes no part in the sums: an infinite one would leave 0 * Inf there)
+            const double vp = col > 0 ? fmax(v, 0.0) : 0.0, vn = col > 0 ? fmin(v, 0.0) : 0.0;
             x[i][0] = fma(vp, pl, x[i][0]);
             x[i][1] = fma(vn, pu, x[i][1]);
             x[i][2] = fma(vp, pu, x[i][2]);
             x[i][3] = fma(vn, pl, x[i][3]);
             if (co < a.g.Cout) {
-              const int col = s_col[c];
               S.out[(int64_t)col * a.ldo + (int64_t)co * a.g.P + p] = col == 0 && a.bias != nullptr ? v + bias[i] : v;
             }
           }

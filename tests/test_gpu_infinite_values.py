@@ -1,0 +1,55 @@
+"""Infinite bounds, centres and weights through the kernels that leave products with exact zeros out: 0 * Inf is NaN, so
+what may be left out with finite numbers may not be with infinite ones, and a sum that does not take part in the reference
+(the centre's, in Star.estimateRanges) may not turn into one."""
+import numpy as np
+import pytest
+
+from oracle import nnv_oracle as o
+from tests.gpu_util import assert_close
+
+pytestmark = pytest.mark.gpu
+
+OPTS = {"reachMethod": "relax-star-area", "relaxFactor": 1}
+
+
+@pytest.fixture(scope="module")
+def nnv():
+    import nnv_amd
+    return nnv_amd
+
+
+def _same_where_not_finite(got, exp, what):
+    got, exp = np.asarray(got), np.asarray(exp)
+    assert got.shape == exp.shape, what
+    assert np.array_equal(np.isnan(got), np.isnan(exp)), what + ": NaN in other places"
+    inf = np.isinf(exp)
+    assert np.array_equal(np.isinf(got), inf) and np.array_equal(got[inf], exp[inf]), what + ": other infinities"
+    fin = np.isfinite(exp)
+    assert_close(got[fin], exp[fin], what)
+
+
+@pytest.mark.parametrize("channels", [16, 33])
+def test_an_infinite_centre_behind_a_convolution_by_position(nnv, channels):
+    """An infinite bias makes one channel of the first layer's centre infinite; the second layer's centre is +-Inf all
+    over.  Its generators are finite: the bounds are +-Inf, not NaN."""
+    rs = np.random.RandomState(channels)
+    W1, W2 = rs.randn(3, 3, 1, 16) / 3, rs.randn(3, 3, 16, channels) / 12
+    W2[:, :, 3, :] = np.abs(W2[:, :, 3, :]) * np.where(np.arange(channels) % 2 == 0, 1.0, -1.0)
+    b1 = rs.randn(16) * 0.1
+    b1[3] = np.inf
+    conv = lambda W, b: {"type": "conv", "W": W, "b": b, "padding": [1] * 4, "stride": [1, 1], "dilation": [1, 1]}
+    layers = [conv(W1, b1), {"type": "relu"}, conv(W2, rs.randn(channels) * 0.1), {"type": "relu"}]
+    x = rs.rand(10, 11, 1)
+    net = nnv.NN.from_config(layers)
+    with np.errstate(invalid="ignore"):
+        _, exp = o.nn_reach(layers, o.image_star_from_bounds(x - 0.02, x + 0.02), "relax-star-area", 1.0, keep=True)
+        net.reach(nnv.ImageStar(x - 0.02, x + 0.02), OPTS)
+        for li in (0, 2):
+            lb, ub = net.reachSet[li].estimateRanges()
+            elb, eub = o.image_star_estimate_ranges(exp[li])
+            assert np.isinf(elb).any() and not np.isnan(elb).any()
+            _same_where_not_finite(lb, elb, "layer %d lb" % (li + 1))
+            _same_where_not_finite(ub, eub, "layer %d ub" % (li + 1))
+        # the step classifies by these bounds: what lies at -Inf is reset, what lies at +Inf is kept
+        V = net.reachSet[3].V
+        assert not V[np.isneginf(eub)].any() and np.isposinf(V[..., 0][np.isposinf(elb)]).all()
