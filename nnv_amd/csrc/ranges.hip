@@ -5,6 +5,7 @@
 // column chunk, eight loads in flight per wave; partial sums of the chunks are combined in a fixed order by a second tiny kernel,
 // so results are bit-reproducible from run to run (no floating-point atomics).
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 #include "internal.h"
@@ -1204,22 +1205,46 @@ static int compute_box_ranges(nnvhip_ctx* ctx, const std::vector<nnvhip_star*>& 
 // Ranges of a ReLU step's output from the ranges it classified by: an inactive row is zero, a crossing row is the unit
 // vector of its own predicate (bounds 0 and ub), every other row is the input's row with the input's bounds.  So the
 // output's matrix is not asked for: no row reset, no appended columns, no scan (CNN 28x28x1, bounds of all layers: 120 us
-// of kernels that wrote and read two 90 MB matrices).
+// of kernels that wrote and read two 90 MB matrices).  An infinite upper bound among the appended predicates makes 0 * Inf
+// of every zero in its column, so a block looks through them first: lb is NaN then, ub too except in the row of the only
+// infinite one.
 struct ReluRange {
   const double* lb_in;
   const double* ub_in;
+  const double* new_ub;  // upper bounds of the appended predicates
   double* lb;
   double* ub;
-  int32_t N;
+  int32_t N, m;
 };
 __global__ __launch_bounds__(256) void relu_ranges_kernel(const ReluRange* __restrict__ table, ReluRange one) {
   const ReluRange d = table ? table[blockIdx.y] : one;
   const int r = blockIdx.x * 256 + threadIdx.x;
+  const double lo = r < d.N ? d.lb_in[r] : 0.0, up = r < d.N ? d.ub_in[r] : 0.0;
+  int infinite = 0;
+  for (int t = threadIdx.x; t < d.m; t += 4 * 256) {
+    double v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = t + u * 256 < d.m ? d.new_ub[t + u * 256] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) infinite += v[u] == HUGE_VAL ? 1 : 0;
+  }
+  const int some = __syncthreads_or(infinite);
+  const int threads = some != 0 ? __syncthreads_count(infinite > 0) : 0;
+  const bool several = some > 1 || threads > 1;
   if (r >= d.N) return;
-  const double lo = d.lb_in[r], up = d.ub_in[r];
   const bool inactive = up <= 0.0, crossing = lo < 0.0 && up > 0.0;
-  d.lb[r] = inactive || crossing ? 0.0 : lo;
-  d.ub[r] = inactive ? 0.0 : up;
+  double l = inactive || crossing ? 0.0 : lo, h = inactive ? 0.0 : up;
+  if (some != 0) {
+    l = __longlong_as_double(0x7ff8000000000000ll);
+    if (several || !(crossing && up == HUGE_VAL)) h = l;
+  }
+  d.lb[r] = l;
+  d.ub[r] = h;
+}
+
+static ReluRange relu_range_of(const nnvhip_star* t, double* lb, double* ub) {
+  const int64_t m = std::max<int64_t>(t->n_crossing, 0);
+  return ReluRange{t->pre_lb, t->pre_ub, t->pub + (t->n - m), lb, ub, (int32_t)t->N, (int32_t)m};
 }
 
 static int compute_relu_ranges(nnvhip_ctx* ctx, const std::vector<nnvhip_star*>& sets) {
@@ -1234,7 +1259,7 @@ static int compute_relu_ranges(nnvhip_ctx* ctx, const std::vector<nnvhip_star*>&
   rr.reserve(sets.size());
   double* at = rb->as<double>();
   for (auto* t : sets) {
-    rr.push_back(ReluRange{t->pre_lb, t->pre_ub, at, at + t->ld, (int32_t)t->N});
+    rr.push_back(relu_range_of(t, at, at + t->ld));
     at += 2 * t->ld;
   }
   for (size_t i0 = 0; i0 < rr.size(); i0 += 65535) {
@@ -1587,7 +1612,7 @@ int ranges_into_static(nnvhip_ctx* ctx, const nnvhip_star* s, double* lb_dev, do
   if (use.last != nullptr && use.last != ctx) NNV_HIP_TRY(hipStreamWaitEvent(ctx->stream, use.done, 0));
   if (relu_out)
     hipLaunchKernelGGL(relu_ranges_kernel, dim3((unsigned)ceil_div(s->N, 256)), dim3(256), 0, ctx->stream, nullptr,
-                       ReluRange{s->pre_lb, s->pre_ub, d.lb, d.ub, (int32_t)s->N});
+                       relu_range_of(s, d.lb, d.ub));
   else if (win) {
     d.box = s->box;
     d.bH = s->box_H;

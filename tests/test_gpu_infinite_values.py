@@ -53,3 +53,24 @@ def test_an_infinite_centre_behind_a_convolution_by_position(nnv, channels):
         # the step classifies by these bounds: what lies at -Inf is reset, what lies at +Inf is kept
         V = net.reachSet[3].V
         assert not V[np.isneginf(eub)].any() and np.isposinf(V[..., 0][np.isposinf(elb)]).all()
+
+
+@pytest.mark.parametrize("N", [20, 300, 3000])      # one block, several, beyond the one-block classification
+@pytest.mark.parametrize("rows", [(4,), (4, 9), ()])
+def test_an_infinite_upper_bound_in_front_of_a_relu(nnv, N, rows):
+    """A neuron with bounds -Inf .. Inf gets a predicate with upper bound Inf: in Star.estimateRanges of the output every
+    other row meets it as 0 * Inf."""
+    rs = np.random.RandomState(N + len(rows))
+    n = 2
+    V = rs.randn(N, n + 1)
+    for r in rows:
+        V[r] = [0.5, 1.5e308, 1.5e308]              # (finite entries whose sum is not)
+    C, d, pl, pu = np.zeros((1, n)), np.zeros(1), -np.ones(n), np.ones(n)
+    with np.errstate(invalid="ignore", over="ignore"):
+        exp = o.reach_relaxed_star(o.OStar(V, C, d, pl, pu), "relax-star-area")
+        elb, eub = o.estimate_ranges(exp)
+    out = nnv.ReluLayer().reach(nnv.Star(V, C, d, pl, pu), "relax-star-area", [], 1)
+    lb, ub = out.estimateRanges()
+    assert np.isnan(elb).all() == (len(rows) > 0)
+    _same_where_not_finite(lb, elb, "lb")
+    _same_where_not_finite(ub, eub, "ub")
