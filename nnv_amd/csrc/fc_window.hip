@@ -337,7 +337,7 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
 
 int fc_window_tile(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in, const int64_t* dense) {
   const nnvhip_star* f = in[0];
-  if (f->box == nullptr || f->box_H < 1 || f->box_W < 1) return 0;
+  if (!fc->finite || f->box == nullptr || f->box_H < 1 || f->box_W < 1) return 0;  // (0 * Inf is NaN: the rows the union leaves out count then)
   const int64_t H = f->box_H, W = f->box_W;
   if (H > 8192 || W > 8192 || fc->K % (H * W) != 0 || fc->K >= (int64_t(1) << 31) || fc->Mp >= (int64_t(1) << 20)) return 0;
   int64_t cols = 0;

@@ -547,6 +547,9 @@ struct nnvhip_fc {
   std::atomic<int> refs{1};
   nnvhip_ctx* ctx = nullptr;
   int64_t M = 0, K = 0, Mp = 0, Kp = 0;
+  // no weight is infinite or NaN: products with entries that are known to be zero may be left out (0 * Inf is NaN).  (The
+  // products with structural zeros of unit vectors and reset rows are left out either way.)
+  bool finite = true;
   uint64_t uid = 0;     // of this context's layers, never reused (a set remembers which layer a product made ahead is for)
   nnvhip::BufRef W;     // Mp x Kp, zero padded, ld = Mp
   nnvhip::BufRef bias;  // Mp entries (zero padded) or null
@@ -563,6 +566,7 @@ struct nnvhip_conv2d {
   int64_t FH = 0, FW = 0, Cin = 0, Cout = 0;
   int64_t pad[4] = {0, 0, 0, 0}, stride[2] = {1, 1}, dil[2] = {1, 1};
   int64_t K = 0, Kp = 0;  // K = FH*FW*Cin taps, Kp = padded
+  bool finite = true;     // as nnvhip_fc::finite
   nnvhip::BufRef W;       // Kp x Cout, zero padded rows, ld = Kp (MATLAB layout is already K x Cout)
   nnvhip::BufRef bias;    // Cout entries or null
   // the same weights k-major for the kernel that brings its weight tiles straight into LDS: Kp rows of

@@ -51,6 +51,16 @@ void hash_bytes(const void* data, size_t bytes, uint64_t* h0, uint64_t* h1) {
 
 using namespace nnvhip;
 
+static bool all_finite(const double* v, int64_t n) {
+  uint64_t bad = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    uint64_t bits;
+    memcpy(&bits, v + i, sizeof bits);
+    bad |= ((bits >> 52) & 0x7ff) == 0x7ff;
+  }
+  return bad == 0;
+}
+
 // Frees the cache's references: every entry (all), or least recently used entries that nobody else holds
 // until the cache is back under its budget.
 void nnvhip_ctx::drop_weight_cache(bool all) {
@@ -176,6 +186,7 @@ int nnvhip_fc_create(nnvhip_ctx* c, const double* W, const double* b, int64_t M,
   fc->K = K;
   fc->Mp = round_up(M, kLdAlign);
   fc->Kp = round_up(K, kLdAlign);
+  fc->finite = all_finite(W, M * K);
   // (128 doubles of slack: the tile kernel of gemm_seg.hip reads whole 128-row pieces of a column)
   NNV_TRY(c->alloc(sizeof(double) * (fc->Mp * fc->Kp + 128), &fc->W));
   NNV_HIP_TRY(hipMemsetAsync(fc->W->ptr, 0, sizeof(double) * fc->Mp * fc->Kp, c->stream));
@@ -274,6 +285,7 @@ int nnvhip_conv2d_create(nnvhip_ctx* c, const double* W, const double* bias, int
   }
   cv->K = FH * FW * Cin;
   cv->Kp = round_up(cv->K, kLdAlign);
+  cv->finite = all_finite(W, cv->K * Cout);
   // MATLAB's FH x FW x Cin x Cout array is a (FH*FW*Cin) x Cout column-major matrix already
   NNV_TRY(c->alloc(sizeof(double) * cv->Kp * Cout, &cv->W));
   NNV_HIP_TRY(hipMemsetAsync(cv->W->ptr, 0, sizeof(double) * cv->Kp * Cout, c->stream));

@@ -55,6 +55,49 @@ def test_an_infinite_centre_behind_a_convolution_by_position(nnv, channels):
         assert not V[np.isneginf(eub)].any() and np.isposinf(V[..., 0][np.isposinf(elb)]).all()
 
 
+def test_an_infinite_weight_in_an_fc_layer_behind_a_convolution(nnv):
+    """Every generator image times an infinite weight: NaN where the image is zero at that weight's row, as in the
+    product over whole images."""
+    rs = np.random.RandomState(3)
+    W1, Wf = rs.randn(3, 3, 1, 6) / 3, rs.randn(33, 16 * 16 * 6) / 40
+    Wf[5, 700] = np.inf
+    layers = [{"type": "conv", "W": W1, "b": 20.0 + rs.randn(6), "padding": [1] * 4, "stride": [1, 1], "dilation": [1, 1]},
+              {"type": "relu"}, {"type": "fc", "W": Wf, "b": rs.randn(33)}]
+    x = rs.rand(16, 16, 1)
+    net = nnv.NN.from_config(layers)
+    with np.errstate(invalid="ignore"):
+        _, exp = o.nn_reach(layers, o.image_star_from_bounds(x - 0.02, x + 0.02), "relax-star-area", 1.0, keep=True)
+        out = net.reach(nnv.ImageStar(x - 0.02, x + 0.02), OPTS)
+        V = exp[2].V.reshape(33, -1)
+        assert np.isnan(V[5]).any()
+        _same_where_not_finite(np.asarray(out.V).reshape(33, -1), V, "V")
+
+
+def test_an_infinite_weight_in_a_convolution_by_position(nnv):
+    """The same for a convolution whose images have windows: the rows a ReLU step has reset count as zeros inside a
+    window, so an infinite weight over them is NaN, whatever way the images are computed."""
+    rs = np.random.RandomState(4)
+    W1, W2 = rs.randn(3, 3, 1, 16) / 3, rs.randn(3, 3, 16, 32) / 12
+    W2[1, 1, 2, 7] = np.inf
+    conv = lambda W, b: {"type": "conv", "W": W, "b": b, "padding": [1] * 4, "stride": [1, 1], "dilation": [1, 1]}
+    net = nnv.NN.from_config([conv(W1, rs.randn(16) * 0.1), {"type": "relu"}, conv(W2, rs.randn(32) * 0.1), {"type": "relu"}])
+    x = rs.rand(12, 12, 1)
+    ctx = nnv.default_context()
+    got = []
+    for eager in (True, False):                     # (with every column in memory the images go by the implicit GEMM)
+        ctx.set_eager_columns(eager)
+        try:
+            net.reach(nnv.ImageStar(x - 0.02, x + 0.02), OPTS)
+            out = net.reachSet[2]
+            got.append((out.estimateRanges(), np.array(out.V)))
+        finally:
+            ctx.set_eager_columns(False)
+    assert np.isnan(got[0][1]).any()
+    _same_where_not_finite(got[1][1], got[0][1], "V")
+    _same_where_not_finite(got[1][0][0], got[0][0][0], "lb")
+    _same_where_not_finite(got[1][0][1], got[0][0][1], "ub")
+
+
 @pytest.mark.parametrize("N", [20, 300, 3000])      # one block, several, beyond the one-block classification
 @pytest.mark.parametrize("rows", [(4,), (4, 9), ()])
 def test_an_infinite_upper_bound_in_front_of_a_relu(nnv, N, rows):
