@@ -149,6 +149,18 @@ NNVHIP_API int nnvhip_debug_counters(nnvhip_ctx* ctx, int64_t* device_mallocs, i
  * many through one that copied the input's bounds into arrays of its own (new_pred_lb = [predicate_lb; zeros(m,1)],
  * nn/funcs/PosLin.m:737-738, either way).  Either pointer may be NULL. */
 NNVHIP_API int nnvhip_debug_relu_bounds(nnvhip_ctx* ctx, int64_t* appended_in_place, int64_t* copied);
+/* Which way the sets of the layer calls went since the context was created, for tests of the dispatch rules: sets[r] =
+ * how many took route r (NNVHIP_ROUTES entries).  A set counts where a kernel of the route was launched for it. */
+enum {
+  NNVHIP_ROUTE_CONV_WINDOW = 0,    /* convolution by output position */
+  NNVHIP_ROUTE_CONV_WINDOW_PARTS,  /* ... with a position's columns in several parts */
+  NNVHIP_ROUTE_FC_WINDOW,          /* FC layer inside its images' windows */
+  NNVHIP_ROUTE_ROWMAP_WINDOW,      /* row map inside windows */
+  NNVHIP_ROUTE_ROWMAP_BOX,         /* row map of a box of which only the centre is in memory */
+  NNVHIP_ROUTE_POOL_WINDOW,        /* average pooling inside windows */
+  NNVHIP_ROUTES
+};
+NNVHIP_API int nnvhip_debug_routes(nnvhip_ctx* ctx, int64_t* sets);
 /* Host-to-device traffic of the context since it was created (no counterpart in the reference, whose arrays
  * never leave the host): the number of layers whose weights were uploaded (nnvhip_fc_create /
  * nnvhip_conv2d_create calls that did not find their arrays resident), the bytes of those uploads, and all

@@ -29,7 +29,7 @@ SYMBOLS = [
     "nnvhip_star_fetch_rows", "nnvhip_relu_apply_lists", "nnvhip_probe_mfma_peak",
     "nnvhip_estimate_ranges_static", "nnvhip_debug_mailbox_pack", "nnvhip_debug_mailbox_unpack",
     "nnvhip_debug_set_relu_call_number", "nnvhip_reach_layers", "nnvhip_reach_is_one_launch", "nnvhip_relu_reduce_mem",
-    "nnvhip_set_switch", "nnvhip_hint_next_fc", "nnvhip_debug_counters", "nnvhip_debug_relu_bounds", "nnvhip_weight_cache_stats", "nnvhip_weight_cache_release", "nnvhip_debug_weak_weight_hash",
+    "nnvhip_set_switch", "nnvhip_hint_next_fc", "nnvhip_debug_counters", "nnvhip_debug_relu_bounds", "nnvhip_debug_routes", "nnvhip_weight_cache_stats", "nnvhip_weight_cache_release", "nnvhip_debug_weak_weight_hash",
 ]
 
 
@@ -127,6 +127,7 @@ def load():
         "nnvhip_hint_next_fc": [p, p],
         "nnvhip_debug_counters": [p, pi64, pi64, pi64, pi64],
         "nnvhip_debug_relu_bounds": [p, pi64, pi64],
+        "nnvhip_debug_routes": [p, C.POINTER(i64)],
         "nnvhip_weight_cache_stats": [p, pi64, pi64, pi64],
         "nnvhip_weight_cache_release": [p, pi64],
         "nnvhip_debug_weak_weight_hash": [C.c_int],
@@ -268,6 +269,13 @@ class Context:
         a, b = C.c_int64(), C.c_int64()
         check(self.lib.nnvhip_debug_relu_bounds(self.handle, C.byref(a), C.byref(b)))
         return a.value, b.value
+
+    def routes(self):
+        """{route: sets that took it} since the context was created (nnvhip_debug_routes)."""
+        names = ("conv_window", "conv_window_parts", "fc_window", "rowmap_window", "rowmap_box", "pool_window")
+        v = (C.c_int64 * len(names))()
+        check(self.lib.nnvhip_debug_routes(self.handle, v))
+        return dict(zip(names, v))
 
     def hint_next_fc(self, weights):
         """nnvhip_hint_next_fc: the FC layer (its device weights, or None) that will follow the next ReLU step."""

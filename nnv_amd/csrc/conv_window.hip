@@ -418,6 +418,8 @@ int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
       any_stamps = true;
     }
     max_parts = std::max<int64_t>(max_parts, s.parts);
+    ++ctx->routes[NNVHIP_ROUTE_CONV_WINDOW];
+    if (s.parts > 1) ++ctx->routes[NNVHIP_ROUTE_CONV_WINDOW_PARTS];
     // (as the implicit GEMM over the windows counts them; the rows a block leaves out are known on the device only)
     flop += 2.0 * ((double)(s.dense - 1) * s.eh * s.ew + (double)a.g.P) * (double)cv->Cout * (double)cv->K;
   }

@@ -493,6 +493,12 @@ int nnvhip_debug_relu_bounds(nnvhip_ctx* c, int64_t* appended_in_place, int64_t*
   return NNVHIP_OK;
 }
 
+int nnvhip_debug_routes(nnvhip_ctx* c, int64_t* sets) {
+  if (!c || !sets) NNV_FAIL(NNVHIP_ERR_ARG, "null argument");
+  std::copy(c->routes, c->routes + NNVHIP_ROUTES, sets);
+  return NNVHIP_OK;
+}
+
 int nnvhip_pool_stats(nnvhip_ctx* c, int64_t* in_use, int64_t* cached) {
   if (!c) NNV_FAIL(NNVHIP_ERR_ARG, "null context");
   c->drain_deferred();

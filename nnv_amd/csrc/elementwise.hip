@@ -484,6 +484,7 @@ static int rowmap_windows(nnvhip_ctx* c, const RowmapArgs& a, int64_t N, int64_t
     dim3 grid;
     const WinArgs w = win_args(in[i], o, N / HW, &grid);
     if (st == NNVHIP_OK) {
+      ++c->routes[NNVHIP_ROUTE_ROWMAP_WINDOW];
       NNV_LAUNCH(c, c->kernel_timing, rowmap_window_kernel, grid, dim3(256), 0, w, a, (int)o->box_H, (int)HW);
       st = c->kernel_timer_end(c->kernel_timing, 4, 16.0 * ((double)w.area * w.C * (double)o->n + (double)N));
     }
@@ -521,6 +522,7 @@ static int rowmap_boxes(nnvhip_ctx* c, const RowmapArgs& a, bool may_flip, int64
     NNV_TRY(c->kernel_timer_end(c->kernel_timing, 4, 16.0 * (double)ld * cnt));
   }
   NNV_HIP_TRY(hipGetLastError());
+  c->routes[NNVHIP_ROUTE_ROWMAP_BOX] += count;
   for (int64_t i = 0; i < count; ++i) {
     nnvhip_star* o = new_star(c);
     o->N = N;
@@ -608,6 +610,7 @@ static int pool_windows(nnvhip_ctx* c, const nnvhip_avgpool2d* p, PoolArgs a, in
     s.idx = in[i]->oh_idx;
     s.scale = in[i]->oh_scale;
     s.dense = (int32_t)pl.dense;
+    ++c->routes[NNVHIP_ROUTE_POOL_WINDOW];
     NNV_LAUNCH(c, c->kernel_timing, avgpool_window_kernel, grid, dim3(256), 0, w, a, s);
     st = c->kernel_timer_end(c->kernel_timing, 4, 8.0 * ((double)w.area * w.C * (double)o->n * 2.0 + (double)(in[i]->N + Nout)));
     if (st == NNVHIP_OK && hipGetLastError() != hipSuccess) {

@@ -443,6 +443,7 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
   else NNV_FC_WINDOW(64, 64, 2, 4, 16);
 #undef NNV_FC_WINDOW
   NNV_HIP_TRY(hipGetLastError());
+  ctx->routes[NNVHIP_ROUTE_FC_WINDOW] += count;
   return NNVHIP_OK;
 }
 

@@ -385,6 +385,7 @@ struct nnvhip_ctx {
   // group's shared product and contracting over the rows in which they differ (environment NNVHIP_NO_ROW_DELTAS)
   bool no_row_deltas = false;
   int64_t n_bounds_in_place = 0, n_bounds_copied = 0;  // sets through ReLU steps, by where their predicate bounds went
+  int64_t routes[NNVHIP_ROUTES] = {0};                 // sets by the way they went (nnvhip_debug_routes)
   bool no_sum_shortcuts = false;  // the pass that sums unwritten pieces: every set in full, with both bounds of every predicate
   // debugging aid (environment NNVHIP_POISON_PENDING): columns left unwritten are filled with NaNs
   bool poison_pending = false;

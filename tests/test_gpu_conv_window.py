@@ -1,6 +1,7 @@
 """Convolutions that go by output position (images with windows): against the oracle, with what is left unwritten poisoned, at
 the edges of the channel tiles (16, 32, 64), with more columns per position than one list holds and more than one part,
-with strides, dilation, borders, empty windows and without a kept row; in an array and by itself (to the bit, without dilation)."""
+with strides, dilation, borders, empty windows and without a kept row; in an array and by itself (to the bit, without dilation).  Every case asserts which
+layers went by position."""
 import numpy as np
 import pytest
 
@@ -26,24 +27,25 @@ def _layers(rs, hw, cin, convs, bias):
     return out
 
 
-# (filter, stride, padding, dilation, channels) per layer; bias of the first layer: -20 leaves no row, +20 every row
+# (filter, stride, padding, dilation, channels) per layer; bias of the first layer: -20 leaves no row, +20 every row; how many
+# layers go by position; whether a position's columns come in several parts there
 NETS = [
-    ((9, 11), 1, [(3, 1, 1, 1, 16), (3, 1, 1, 1, 16)], 0.0),
-    ((9, 11), 1, [(3, 1, 1, 1, 14), (3, 2, 1, 1, 17)], 0.0),
-    ((12, 10), 1, [(3, 1, 1, 1, 8), (3, 1, 1, 1, 33), (3, 2, 0, 1, 64)], 0.0),
-    ((10, 10), 2, [(3, 1, 1, 1, 6), (3, 1, 1, 1, 65)], 0.0),
-    ((12, 13), 3, [(5, 2, 2, 1, 16), (3, 1, 1, 1, 32), (3, 1, 0, 1, 20)], 0.0),
-    ((14, 12), 1, [(3, 1, 1, 1, 16), (3, 1, 2, 2, 32)], 0.0),
-    ((11, 11), 1, [(1, 2, 0, 1, 40), (1, 1, 0, 1, 60)], 0.0),
-    ((8, 8), 40, [(1, 1, 0, 1, 20), (3, 1, 1, 1, 16)], 0.0),      # 360 columns per position
-    ((9, 9), 1, [(3, 1, 1, 1, 16), (3, 1, 1, 1, 16)], -20.0),
-    ((9, 9), 1, [(3, 1, 1, 1, 16), (3, 1, 1, 1, 16)], 20.0),
+    ((9, 11), 1, [(3, 1, 1, 1, 16), (3, 1, 1, 1, 16)], 0.0, 1, False),
+    ((9, 11), 1, [(3, 1, 1, 1, 14), (3, 2, 1, 1, 17)], 0.0, 1, False),
+    ((12, 10), 1, [(3, 1, 1, 1, 8), (3, 1, 1, 1, 33), (3, 2, 0, 1, 64)], 0.0, 1, False),
+    ((10, 10), 2, [(3, 1, 1, 1, 6), (3, 1, 1, 1, 65)], 0.0, 1, False),
+    ((24, 26), 3, [(5, 2, 2, 1, 16), (3, 1, 1, 1, 32), (3, 1, 0, 1, 20)], 0.0, 2, True),
+    ((14, 12), 1, [(3, 1, 1, 1, 16), (3, 1, 2, 2, 32)], 0.0, 1, False),
+    ((11, 11), 1, [(1, 2, 0, 1, 40), (1, 1, 0, 1, 60)], 0.0, 1, False),
+    ((8, 8), 40, [(1, 1, 0, 1, 20), (3, 1, 1, 1, 16)], 0.0, 1, True),      # 360 columns per position
+    ((9, 9), 1, [(3, 1, 1, 1, 16), (3, 1, 1, 1, 16)], -20.0, 1, False),
+    ((9, 9), 1, [(3, 1, 1, 1, 16), (3, 1, 1, 1, 16)], 20.0, 1, False),
 ]
 
 
-@pytest.mark.parametrize("hw,cin,convs,bias", NETS)
+@pytest.mark.parametrize("hw,cin,convs,bias,by_position,parts", NETS)
 @pytest.mark.parametrize("poison", [False, True])
-def test_convolution_by_position(nnv, hw, cin, convs, bias, poison):
+def test_convolution_by_position(nnv, hw, cin, convs, bias, by_position, parts, poison):
     rs = np.random.RandomState(hw[0] + 31 * cin + len(convs))
     layers = _layers(rs, hw, cin, convs, bias)
     opts = {"reachMethod": "relax-star-area", "relaxFactor": 1}
@@ -57,7 +59,10 @@ def test_convolution_by_position(nnv, hw, cin, convs, bias, poison):
     ctx.set_switch("poison_pending", poison)
     try:
         net = nnv.NN.from_config(layers)
+        before = ctx.routes()
         net.reach([nnv.ImageStar(*b) for b in boxes], opts)
+        took = {k: v - before[k] for k, v in ctx.routes().items()}
+        assert took["conv_window"] == 2 * by_position and (took["conv_window_parts"] > 0) == parts, took
         arr = [[(s.estimateRanges(), np.array(s.V)) for s in layer] for layer in net.reachSet]
         for i, b in enumerate(boxes):
             net.reach(nnv.ImageStar(*b), opts)

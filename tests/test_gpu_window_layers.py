@@ -1,6 +1,6 @@
 """Row maps and average pooling on generators that are known to be sparse (windows of a convolution, unit vectors of a box
 or a ReLU step): against the oracle layer by layer, with what is left unwritten poisoned, in the order written first /
-read first, and for the sizes where windows reach the border, overlap or stop paying."""
+read first, and for the sizes where windows reach the border, overlap or stop paying.  Every case asserts which layers stayed inside windows."""
 import numpy as np
 import pytest
 
@@ -44,19 +44,20 @@ def _layers(rs, names, hw, cin):
     return out
 
 
+# the last: sets per image that go through a row map in windows, a row map of a box, a pooling in windows
 NETS = [
-    ((12, 9), 3, "norm conv3_1_1_4 bn relu pool2_2_0 conv3_1_1_5 bn relu pool3_2_1 flat fc7"),
-    ((13, 13), 1, "sym bn conv3_1_1_6 bn pool2_2_0 bn relu pool2_1_1 conv3_2_0_4 relu fc5"),
-    ((16, 16), 2, "pool2_2_0 bn conv3_1_1_3 relu bn relu fc4"),          # pooling a box; a row map behind a pending reset
-    ((17, 16), 1, "norm pool3_2_1 relu pool2_1_1 bn fc6"),
-    ((5, 5), 2, "norm conv3_1_1_3 bn relu pool2_2_0 fc3"),                 # windows as large as the image
-    ((9, 20), 3, "norm conv5_1_2_3 bn relu pool5_3_2 conv1_1_0_4 relu fc3"),
+    ((12, 9), 3, "norm conv3_1_1_4 bn relu pool2_2_0 conv3_1_1_5 bn relu pool3_2_1 flat fc7", (1, 1, 1)),
+    ((13, 13), 1, "sym bn conv3_1_1_6 bn pool2_2_0 bn relu pool2_1_1 conv3_2_0_4 relu fc5", (2, 2, 2)),
+    ((16, 16), 2, "pool2_2_0 bn conv3_1_1_3 relu bn relu fc4", (1, 0, 1)),          # pooling a box; a row map behind a pending reset
+    ((17, 16), 1, "norm pool3_2_1 relu pool2_1_1 bn fc6", (1, 1, 2)),
+    ((5, 5), 2, "norm conv3_1_1_3 bn relu pool2_2_0 fc3", (1, 1, 0)),                 # windows as large as the image
+    ((9, 20), 3, "norm conv5_1_2_3 bn relu pool5_3_2 conv1_1_0_4 relu fc3", (1, 1, 1)),
 ]
 
 
-@pytest.mark.parametrize("hw,cin,names", NETS)
+@pytest.mark.parametrize("hw,cin,names,inside", NETS)
 @pytest.mark.parametrize("mode", ["default", "poison", "single_dims", "eager", "array"])
-def test_sparse_generators_through_row_maps_and_pooling(nnv, hw, cin, names, mode):
+def test_sparse_generators_through_row_maps_and_pooling(nnv, hw, cin, names, inside, mode):
     rs = np.random.RandomState(len(names) + hw[0])
     layers = _layers(rs, names.split(), hw, cin)
     count = 3 if mode == "array" else 1
@@ -74,7 +75,10 @@ def test_sparse_generators_through_row_maps_and_pooling(nnv, hw, cin, names, mod
         ctx.set_eager_columns(True)
     try:
         net = nnv.NN.from_config(layers)
+        before = ctx.routes()
         out = net.reach(dev_in if count > 1 else dev_in[0], {"reachMethod": "relax-star-area", "relaxFactor": 1})
+        took = {k: v - before[k] for k, v in ctx.routes().items()}
+        assert (took["rowmap_window"], took["rowmap_box"], took["pool_window"]) == tuple(0 if mode == "eager" else count * k for k in inside), took
         ranges = [(s[0] if count > 1 else s).estimateRanges() for s in net.reachSet[:-1]]   # before any matrix is read
         for i in range(count):
             exp, exp_sets = o.nn_reach(layers, ora_in[i], "relax-star-area", 1.0, keep=True)
