@@ -928,9 +928,8 @@ int launch_conv_setup(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int64
   return launch_setup(ctx, g, count, sets);
 }
 
-int launch_pool_boxes(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t Wo, const int64_t pool[2], const int64_t stride[2],
-                      int64_t pad_top, int64_t pad_left, const ColBox* in_box, int64_t dense, const int32_t* onehot_idx, int64_t m,
-                      ColBox* out_box) {
+int launch_pool_setup(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t Wo, const int64_t pool[2], const int64_t stride[2],
+                      int64_t pad_top, int64_t pad_left, int64_t count, const ConvSetup* sets) {
   ConvGeom g{};
   g.H = (int)H;
   g.W = (int)W;
@@ -944,8 +943,7 @@ int launch_pool_boxes(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t
   g.pt = (int)pad_top;
   g.pl = (int)pad_left;
   g.HW = (int)(H * W);
-  const ConvSetup one{in_box, onehot_idx, out_box, nullptr, (int32_t)dense, (int32_t)m, 0, nullptr, nullptr};
-  return launch_setup(ctx, g, 1, &one);
+  return launch_setup(ctx, g, count, sets);
 }
 
 bool conv2d_in_windows(const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldin, int64_t ncols,

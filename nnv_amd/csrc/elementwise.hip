@@ -111,28 +111,38 @@ __global__ __launch_bounds__(64 * kEwWaves) void rowmap_kernel(const SetDesc* __
 // What bounds them is the latency of scattered 16-40 byte pieces, not bytes.  A 32x32x3 CNN with
 // normalisation and pooling (3073-3362 columns): batch normalisation 63 -> 9 us, row reset and pooling 48 + 51 -> 13 and
 // 30 + 41 -> 22 us, and the convolutions in between stay inside windows too (162 -> 24, 83 -> 14 us).
-struct WinArgs {
+struct WinSet {            // one set of a call (blockIdx.y)
   const double* in;
   double* out;
   const ColBox* box;       // windows of the output's columns
-  int64_t ldin, ldout;
   int32_t eh, area;        // bound on a window: eh rows, area = eh * ew positions
-  int32_t C;
+  int32_t C, H, HW;        // channels; the input's image
   int32_t ncols;           // columns of the output
-  int32_t centre_blocks;   // the first blocks do column 0, 256 rows each ...
-  int32_t cols_per_block;  // ... the others so many generator columns each
+  int32_t cols_per_block;  // generator columns of a block
+  // What a pooling reads besides whole columns: windows of the input's dense columns, the classes of a pending row reset
+  // (rows other than kKeep read as zero), the list of unit-vector columns.
+  int32_t dense;
+  const ColBox* in_box;    // by input column, for 1 <= j < dense; or null (dense == 1)
+  const int32_t* cls;      // or null
+  const int32_t* idx;      // column dense + t is scale[idx[t]] (1 without scales) at row idx[t]
+  const double* scale;
+};
+struct WinArgs {
+  int64_t ldin, ldout;
+  int32_t centre_blocks;   // the first blocks of a set do column 0, 256 rows each, the others a few generator columns each
 };
 
-__global__ __launch_bounds__(256) void rowmap_window_kernel(WinArgs w, RowmapArgs a, int H, int HW) {
-  if ((int)blockIdx.x < w.centre_blocks) {
+__global__ __launch_bounds__(256) void rowmap_window_kernel(const WinSet* __restrict__ table, WinSet one, WinArgs g, RowmapArgs a) {
+  const WinSet w = table ? table[blockIdx.y] : one;
+  if ((int)blockIdx.x < g.centre_blocks) {
     const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (r >= w.ldout) return;
+    if (r >= g.ldout) return;
     double x = w.in[r];
     for (int s = 0; s < a.n_steps; ++s) x = apply_op(a.op[s], x, a.params[(int64_t)s * a.ld + r]);
     w.out[r] = x;
     return;
   }
-  const int j0 = 1 + ((int)blockIdx.x - w.centre_blocks) * w.cols_per_block;
+  const int j0 = 1 + ((int)blockIdx.x - g.centre_blocks) * w.cols_per_block;
   const int per = w.area * w.C, items = per * min(w.cols_per_block, w.ncols - j0);
   for (int f = threadIdx.x; f < items; f += 256) {
     const int jj = f / per, e = f - jj * per, j = j0 + jj;
@@ -141,11 +151,11 @@ __global__ __launch_bounds__(256) void rowmap_window_kernel(WinArgs w, RowmapArg
     const ColBox b = w.box[j];
     const int h = b.h0 + dh, x = b.w0 + dw;
     if (h > b.h1 || x > b.w1) continue;
-    const int64_t r = (int64_t)c * HW + x * H + h;
-    double v = w.in[r + (int64_t)j * w.ldin];
+    const int64_t r = (int64_t)c * w.HW + x * w.H + h;
+    double v = w.in[r + (int64_t)j * g.ldin];
     for (int s = 0; s < a.n_steps; ++s)
       if (a.scope[s] == NNVHIP_SCOPE_ALL) v = apply_op(a.op[s], v, a.params[(int64_t)s * a.ld + r]);
-    w.out[r + (int64_t)j * w.ldout] = v;
+    w.out[r + (int64_t)j * g.ldout] = v;
   }
 }
 
@@ -231,19 +241,10 @@ __global__ __launch_bounds__(64 * kEwWaves) void avgpool_kernel(const SetDesc* _
   }
 }
 
-// What the pooling reads besides whole columns: windows of the input's dense columns, the classes of a pending row reset
-// (rows other than kKeep read as zero), the list of unit-vector columns.
-struct PoolIn {
-  const ColBox* box;       // by input column, for 1 <= j < dense; or null (dense == 1)
-  const int32_t* cls;      // or null
-  const int32_t* idx;      // column dense + t is scale[idx[t]] (1 without scales) at row idx[t]
-  const double* scale;
-  int32_t dense;
-};
-
 // Sums run as in avgpool_kernel (window columns outer, rows inner); what lies outside an input window adds an exact zero
 // and is left out.
-__global__ __launch_bounds__(256) void avgpool_window_kernel(WinArgs w, PoolArgs a, PoolIn s) {
+__global__ __launch_bounds__(256) void avgpool_window_kernel(const WinSet* __restrict__ table, WinSet one, WinArgs g, PoolArgs a) {
+  const WinSet w = table ? table[blockIdx.y] : one;
   const int HW = a.H * a.W, P = a.Ho * a.Wo;
   auto cell = [&](int ho, int wo, int& y1, int& y2, int& x1, int& x2) {
     y1 = ho * a.sh - a.pt;
@@ -254,7 +255,7 @@ __global__ __launch_bounds__(256) void avgpool_window_kernel(WinArgs w, PoolArgs
     x1 = max(x1, 0);
     return 1.0 / (double)((y2 - y1) * (x2 - x1));
   };
-  if ((int)blockIdx.x < w.centre_blocks) {
+  if ((int)blockIdx.x < g.centre_blocks) {
     const int r = (int)blockIdx.x * 256 + (int)threadIdx.x;
     if (r >= P * w.C) return;
     const int c = r / P, p = r - c * P, wo = p / a.Ho, ho = p - wo * a.Ho;
@@ -264,12 +265,12 @@ __global__ __launch_bounds__(256) void avgpool_window_kernel(WinArgs w, PoolArgs
     for (int x = x1; x < x2; ++x)
       for (int y = y1; y < y2; ++y) {
         const int64_t q = (int64_t)c * HW + x * a.H + y;
-        acc = __dadd_rn(acc, s.cls == nullptr || s.cls[q] == kKeep ? w.in[q] : 0.0);
+        acc = __dadd_rn(acc, w.cls == nullptr || w.cls[q] == kKeep ? w.in[q] : 0.0);
       }
     w.out[r] = __dmul_rn(acc, scale);
     return;
   }
-  const int j0 = 1 + ((int)blockIdx.x - w.centre_blocks) * w.cols_per_block;
+  const int j0 = 1 + ((int)blockIdx.x - g.centre_blocks) * w.cols_per_block;
   const int per = w.area * w.C, items = per * min(w.cols_per_block, w.ncols - j0);
   for (int f = threadIdx.x; f < items; f += 256) {
     const int jj = f / per, e = f - jj * per, j = j0 + jj;
@@ -281,18 +282,18 @@ __global__ __launch_bounds__(256) void avgpool_window_kernel(WinArgs w, PoolArgs
     int y1, y2, x1, x2;
     const double scale = cell(ho, wo, y1, y2, x1, x2);
     double acc = 0.0;
-    if (j < s.dense) {
-      const ColBox q = s.box[j];
-      const double* col = w.in + (int64_t)j * w.ldin + (int64_t)c * HW;
+    if (j < w.dense) {
+      const ColBox q = w.in_box[j];
+      const double* col = w.in + (int64_t)j * g.ldin + (int64_t)c * HW;
       for (int x = max(x1, (int)q.w0); x < min(x2, q.w1 + 1); ++x)
         for (int y = max(y1, (int)q.h0); y < min(y2, q.h1 + 1); ++y)
-          acc = __dadd_rn(acc, s.cls == nullptr || s.cls[(int64_t)c * HW + x * a.H + y] == kKeep ? col[x * a.H + y] : 0.0);
+          acc = __dadd_rn(acc, w.cls == nullptr || w.cls[(int64_t)c * HW + x * a.H + y] == kKeep ? col[x * a.H + y] : 0.0);
     } else {
-      const int src = s.idx[j - s.dense];
+      const int src = w.idx[j - w.dense];
       const int sc = src / HW, sp = src - sc * HW, sx = sp / a.H, sy = sp - sx * a.H;
-      if (sc == c && sx >= x1 && sx < x2 && sy >= y1 && sy < y2) acc = s.scale != nullptr ? s.scale[src] : 1.0;
+      if (sc == c && sx >= x1 && sx < x2 && sy >= y1 && sy < y2) acc = w.scale != nullptr ? w.scale[src] : 1.0;
     }
-    w.out[(int64_t)c * P + wo * a.Ho + ho + (int64_t)j * w.ldout] = __dmul_rn(acc, scale);
+    w.out[(int64_t)c * P + wo * a.Ho + ho + (int64_t)j * g.ldout] = __dmul_rn(acc, scale);
   }
 }
 
@@ -418,38 +419,65 @@ static int run_row_layer(nnvhip_ctx* c, int64_t count, nnvhip_star* const* in, n
   return NNVHIP_OK;
 }
 
-// Marks a set's generator columns as written inside their windows only and launches nothing; the padding rows are zeroed.
-static int leave_outside_windows(nnvhip_ctx* c, nnvhip_star* o, int64_t H, int64_t W) {
-  const int64_t ncols = o->n;  // columns 1 .. n
-  o->cs.win_box_buf = o->box_buf;
-  o->cs.win_box = o->box;
-  o->cs.win_from = 1;
-  o->cs.win_to = o->n + 1;
-  o->cs.win_rows = o->N;
-  o->cs.win_H = (int32_t)H;
-  o->cs.win_W = (int32_t)W;
-  if (c->poison_pending)  // debugging aid: NaNs where nothing will be written
-    NNV_HIP_TRY(hipMemsetAsync(o->V + o->ld, 0xff, sizeof(double) * o->ld * ncols, c->stream));
-  if (o->ld != o->N) NNV_TRY(launch_zero_pad_rows(c, o->V, o->ld, o->N, ncols + 1));
-  return NNVHIP_OK;
+// Marks the generator columns of a call's outputs as written inside their windows only; the padding rows are zeroed (the
+// outputs lie back to back: one launch).
+static int leave_outside_windows(nnvhip_ctx* c, const std::vector<nnvhip_star*>& outs, int64_t total_cols) {
+  for (auto* o : outs) {
+    o->cs.win_box_buf = o->box_buf;
+    o->cs.win_box = o->box;
+    o->cs.win_from = 1;
+    o->cs.win_to = o->n + 1;
+    o->cs.win_rows = o->N;
+    o->cs.win_H = o->box_H;
+    o->cs.win_W = o->box_W;
+    if (c->poison_pending)  // debugging aid: NaNs where nothing will be written
+      NNV_HIP_TRY(hipMemsetAsync(o->V + o->ld, 0xff, sizeof(double) * o->ld * o->n, c->stream));
+  }
+  return launch_zero_pad_rows(c, outs[0]->V, outs[0]->ld, outs[0]->N, total_cols);
 }
 
-static WinArgs win_args(const nnvhip_star* in, const nnvhip_star* o, int64_t C, dim3* grid) {
-  WinArgs w{};
-  w.in = in->V;
-  w.out = o->V;
-  w.box = o->box;
-  w.ldin = in->ld;
-  w.ldout = o->ld;
-  w.eh = o->box_eh;
-  w.area = o->box_eh * o->box_ew;
-  w.C = (int32_t)C;
-  w.ncols = (int32_t)(o->n + 1);
-  // a block: the columns that make two to four elements a thread, one column at least
-  w.cols_per_block = (int32_t)std::max<int64_t>(1, 1024 / std::max<int64_t>(1, (int64_t)w.area * C));
-  w.centre_blocks = (int32_t)ceil_div(o->ld, 256);
-  *grid = dim3((unsigned)(w.centre_blocks + ceil_div(o->n, w.cols_per_block)));
+// The sets of a call (all but the pooling's own fields), its arguments and its grid.
+struct WinCall {
+  std::vector<WinSet> sets;
+  WinArgs g{};
+  dim3 grid;
+  double places = 0.0;  // window places of all generator columns
+  const WinSet* table = nullptr;
+  BufRef tab;
+};
+static WinCall win_call(int64_t count, nnvhip_star* const* in, const std::vector<nnvhip_star*>& outs, int64_t HW) {
+  WinCall w;
+  w.g.ldin = in[0]->ld;
+  w.g.ldout = outs[0]->ld;
+  w.g.centre_blocks = (int32_t)ceil_div(outs[0]->ld, 256);
+  int64_t column_blocks = 0;
+  w.sets.resize((size_t)count);
+  for (int64_t i = 0; i < count; ++i) {
+    const nnvhip_star* o = outs[(size_t)i];
+    WinSet& s = w.sets[(size_t)i];
+    s = WinSet{};
+    s.in = in[i]->V;
+    s.out = o->V;
+    s.box = o->box;
+    s.eh = o->box_eh;
+    s.area = o->box_eh * o->box_ew;
+    s.H = o->box_H;
+    s.HW = (int32_t)(HW > 0 ? HW : (int64_t)o->box_H * o->box_W);
+    s.C = (int32_t)(in[i]->N / s.HW);
+    s.ncols = (int32_t)(o->n + 1);
+    // a block: the columns that make two to four elements a thread, one column at least
+    s.cols_per_block = (int32_t)std::max<int64_t>(1, 1024 / std::max<int64_t>(1, (int64_t)s.area * s.C));
+    column_blocks = std::max<int64_t>(column_blocks, ceil_div(o->n, s.cols_per_block));
+    w.places += (double)s.area * s.C * (double)o->n;
+  }
+  w.grid = dim3((unsigned)(w.g.centre_blocks + column_blocks), (unsigned)count);
   return w;
+}
+static int upload_sets(nnvhip_ctx* c, WinCall* w) {
+  if (w->sets.size() < 2) return NNVHIP_OK;
+  NNV_TRY(c->upload_table(w->sets.data(), sizeof(WinSet) * w->sets.size(), &w->tab));
+  w->table = w->tab->as<WinSet>();
+  return NNVHIP_OK;
 }
 
 static bool small_windows(int64_t eh, int64_t ew, int64_t P) { return eh > 0 && ew > 0 && 2 * eh * ew <= P; }
@@ -464,29 +492,35 @@ static bool rowmap_in_windows(const nnvhip_ctx* c, const nnvhip_rowmap* m, const
          s->n < 1000000;
 }
 
+// One launch for all sets of a call, here and in pool_windows.  (With a launch or three per image, 100 images of 12 x 12
+// through two poolings, a batch normalisation, a convolution and two FC layers took 5.9 ms a pass, 4.7 ms over whole columns;
+// now 2.7 ms.  64 images of 28 x 28: 4.2, 4.3 and 1.8 ms.)
 static int rowmap_windows(nnvhip_ctx* c, const RowmapArgs& a, int64_t N, int64_t count, nnvhip_star* const* in, nnvhip_star** out) {
+  if (count > 65535) NNV_FAIL(NNVHIP_ERR_SHAPE, "at most 65535 sets per call");
   std::vector<nnvhip_star*> outs;
   bool contig = false;
   int64_t cols = 0;
   NNV_TRY(c->begin_op());
   int st = make_affine_outputs(c, count, in, N, &outs, &contig, &cols);
-  for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i) {
-    nnvhip_star* o = outs[i];
-    o->box_buf = in[i]->box_buf;
-    o->box = in[i]->box;
-    o->box_cols = in[i]->box_cols;
-    o->box_H = in[i]->box_H;
-    o->box_W = in[i]->box_W;
-    o->box_eh = in[i]->box_eh;
-    o->box_ew = in[i]->box_ew;
-    const int64_t HW = (int64_t)o->box_H * o->box_W;
-    st = leave_outside_windows(c, o, o->box_H, o->box_W);
-    dim3 grid;
-    const WinArgs w = win_args(in[i], o, N / HW, &grid);
+  if (st == NNVHIP_OK) {
+    for (int64_t i = 0; i < count; ++i) {
+      nnvhip_star* o = outs[(size_t)i];
+      o->box_buf = in[i]->box_buf;
+      o->box = in[i]->box;
+      o->box_cols = in[i]->box_cols;
+      o->box_H = in[i]->box_H;
+      o->box_W = in[i]->box_W;
+      o->box_eh = in[i]->box_eh;
+      o->box_ew = in[i]->box_ew;
+    }
+    st = leave_outside_windows(c, outs, cols);
+  }
+  if (st == NNVHIP_OK) {
+    WinCall w = win_call(count, in, outs, 0);
+    st = upload_sets(c, &w);
     if (st == NNVHIP_OK) {
-      ++c->routes[NNVHIP_ROUTE_ROWMAP_WINDOW];
-      NNV_LAUNCH(c, c->kernel_timing, rowmap_window_kernel, grid, dim3(256), 0, w, a, (int)o->box_H, (int)HW);
-      st = c->kernel_timer_end(c->kernel_timing, 4, 16.0 * ((double)w.area * w.C * (double)o->n + (double)N));
+      NNV_LAUNCH(c, c->kernel_timing, rowmap_window_kernel, w.grid, dim3(256), 0, w.table, w.sets[0], w.g, a);
+      st = c->kernel_timer_end(c->kernel_timing, 4, 16.0 * (w.places + (double)N * (double)count));
     }
     if (st == NNVHIP_OK && hipGetLastError() != hipSuccess) {
       set_error("kernel launch failed");
@@ -498,7 +532,8 @@ static int rowmap_windows(nnvhip_ctx* c, const RowmapArgs& a, int64_t N, int64_t
     release_all(outs);
     return st;
   }
-  for (int64_t i = 0; i < count; ++i) out[i] = outs[i];
+  c->routes[NNVHIP_ROUTE_ROWMAP_WINDOW] += count;
+  for (int64_t i = 0; i < count; ++i) out[i] = outs[(size_t)i];
   return NNVHIP_OK;
 }
 
@@ -580,39 +615,50 @@ static bool pool_in_windows(const nnvhip_ctx* c, const nnvhip_avgpool2d* p, cons
 
 static int pool_windows(nnvhip_ctx* c, const nnvhip_avgpool2d* p, PoolArgs a, int64_t count, nnvhip_star* const* in, const PoolPlan* plans,
                         nnvhip_star** out) {
+  if (count > 65535) NNV_FAIL(NNVHIP_ERR_SHAPE, "at most 65535 sets per call");
   const int64_t Nout = (int64_t)a.Ho * a.Wo * a.C;
   std::vector<nnvhip_star*> outs;
   bool contig = false;
   int64_t cols = 0;
   NNV_TRY(c->begin_op());
   int st = make_affine_outputs(c, count, in, Nout, &outs, &contig, &cols);
-  for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i) {
-    nnvhip_star* o = outs[i];
-    const PoolPlan& pl = plans[i];
-    st = c->alloc(sizeof(ColBox) * (size_t)(o->n + 1), &o->box_buf);
-    if (st != NNVHIP_OK) break;
-    ColBox* tab = o->box_buf->as<ColBox>();
-    st = launch_pool_boxes(c, a.H, a.W, a.Ho, a.Wo, p->pool, p->stride, p->pad[0], p->pad[2], pl.dense > 1 ? in[i]->box : nullptr, pl.dense,
-                           in[i]->oh_idx, pl.m, tab);
-    o->box = tab;
-    o->box_cols = o->n + 1;
-    o->box_H = a.Ho;
-    o->box_W = a.Wo;
-    o->box_eh = (int32_t)pl.eh;
-    o->box_ew = (int32_t)pl.ew;
-    if (st == NNVHIP_OK) st = leave_outside_windows(c, o, a.Ho, a.Wo);
-    if (st != NNVHIP_OK) break;
-    dim3 grid;
-    const WinArgs w = win_args(in[i], o, a.C, &grid);
-    PoolIn s{};
-    s.box = pl.dense > 1 ? in[i]->box : nullptr;
-    s.cls = in[i]->rows_pending ? in[i]->cls : nullptr;
-    s.idx = in[i]->oh_idx;
-    s.scale = in[i]->oh_scale;
-    s.dense = (int32_t)pl.dense;
-    ++c->routes[NNVHIP_ROUTE_POOL_WINDOW];
-    NNV_LAUNCH(c, c->kernel_timing, avgpool_window_kernel, grid, dim3(256), 0, w, a, s);
-    st = c->kernel_timer_end(c->kernel_timing, 4, 8.0 * ((double)w.area * w.C * (double)o->n * 2.0 + (double)(in[i]->N + Nout)));
+  BufRef boxes;
+  if (st == NNVHIP_OK) st = c->alloc(sizeof(ColBox) * (size_t)cols, &boxes);
+  if (st == NNVHIP_OK) {
+    std::vector<ConvSetup> setup((size_t)count);
+    ColBox* at = boxes->as<ColBox>();
+    for (int64_t i = 0; i < count; ++i) {
+      nnvhip_star* o = outs[(size_t)i];
+      const PoolPlan& pl = plans[i];
+      setup[(size_t)i] = ConvSetup{pl.dense > 1 ? in[i]->box : nullptr, in[i]->oh_idx, at, nullptr, (int32_t)pl.dense, (int32_t)pl.m, 0, nullptr, nullptr};
+      o->box_buf = boxes;
+      o->box = at;
+      o->box_cols = o->n + 1;
+      o->box_H = a.Ho;
+      o->box_W = a.Wo;
+      o->box_eh = (int32_t)pl.eh;
+      o->box_ew = (int32_t)pl.ew;
+      at += o->n + 1;
+    }
+    st = launch_pool_setup(c, a.H, a.W, a.Ho, a.Wo, p->pool, p->stride, p->pad[0], p->pad[2], count, setup.data());
+  }
+  if (st == NNVHIP_OK) st = leave_outside_windows(c, outs, cols);
+  if (st == NNVHIP_OK) {
+    WinCall w = win_call(count, in, outs, (int64_t)a.H * a.W);
+    for (int64_t i = 0; i < count; ++i) {
+      WinSet& s = w.sets[(size_t)i];
+      s.H = a.H;
+      s.in_box = plans[i].dense > 1 ? in[i]->box : nullptr;
+      s.cls = in[i]->rows_pending ? in[i]->cls : nullptr;
+      s.idx = in[i]->oh_idx;
+      s.scale = in[i]->oh_scale;
+      s.dense = (int32_t)plans[i].dense;
+    }
+    st = upload_sets(c, &w);
+    if (st == NNVHIP_OK) {
+      NNV_LAUNCH(c, c->kernel_timing, avgpool_window_kernel, w.grid, dim3(256), 0, w.table, w.sets[0], w.g, a);
+      st = c->kernel_timer_end(c->kernel_timing, 4, 8.0 * (w.places * 2.0 + (double)(in[0]->N + Nout) * (double)count));
+    }
     if (st == NNVHIP_OK && hipGetLastError() != hipSuccess) {
       set_error("kernel launch failed");
       st = NNVHIP_ERR_HIP;
@@ -623,7 +669,8 @@ static int pool_windows(nnvhip_ctx* c, const nnvhip_avgpool2d* p, PoolArgs a, in
     release_all(outs);
     return st;
   }
-  for (int64_t i = 0; i < count; ++i) out[i] = outs[i];
+  c->routes[NNVHIP_ROUTE_POOL_WINDOW] += count;
+  for (int64_t i = 0; i < count; ++i) out[i] = outs[(size_t)i];
   return NNVHIP_OK;
 }
 
@@ -698,7 +745,7 @@ int nnvhip_affine_rowmap(nnvhip_ctx* c, const nnvhip_rowmap* m, int64_t count, n
   {
     bool windows = true, boxes = m->keeps_zeros && windows_allowed(c);
     for (int64_t i = 0; i < count; ++i) {
-      windows = windows && rowmap_in_windows(c, m, in[i]);
+      windows = windows && in[i]->ld == in[0]->ld && rowmap_in_windows(c, m, in[i]);
       boxes = boxes && is_unwritten_box(in[i]) && in[i]->ld == m->ld;
     }
     if (windows) return rowmap_windows(c, a, m->N, count, in, out);
@@ -779,7 +826,8 @@ int nnvhip_affine_avgpool2d(nnvhip_ctx* c, const nnvhip_avgpool2d* p, int64_t H,
   {
     std::vector<PoolPlan> plans((size_t)count);
     bool windows = true;
-    for (int64_t i = 0; i < count && windows; ++i) windows = in[i]->N == in[0]->N && pool_in_windows(c, p, in[i], H, W, Ho, Wo, &plans[(size_t)i]);
+    for (int64_t i = 0; i < count && windows; ++i)
+      windows = in[i]->N == in[0]->N && in[i]->ld == in[0]->ld && pool_in_windows(c, p, in[i], H, W, Ho, Wo, &plans[(size_t)i]);
     if (windows) return pool_windows(c, p, a, count, in, plans.data(), out);
   }
   return run_row_layer(c, count, in, out, Ho * Wo * C, 64, 4 * kEwWaves,

@@ -825,10 +825,9 @@ struct ConvSetup {
 };
 int launch_conv_setup(nnvhip_ctx* ctx, const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t count,
                       const ConvSetup* sets);
-// The windows behind an average pooling (positions whose pooling cells reach the input's window).
-int launch_pool_boxes(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t Wo, const int64_t pool[2], const int64_t stride[2],
-                      int64_t pad_top, int64_t pad_left, const ColBox* in_box, int64_t dense, const int32_t* onehot_idx, int64_t m,
-                      ColBox* out_box);
+// The same for an average pooling (positions whose pooling cells reach the input's window; out_box only).
+int launch_pool_setup(nnvhip_ctx* ctx, int64_t H, int64_t W, int64_t Ho, int64_t Wo, const int64_t pool[2], const int64_t stride[2],
+                      int64_t pad_top, int64_t pad_left, int64_t count, const ConvSetup* sets);
 // Bound on the extent of an output window whose input window spans at most `e` rows (dim 0) or columns (dim 1).
 int64_t conv_box_extent(const nnvhip_conv2d* conv, int dim, int64_t e, int64_t out_size);
 // whether launch_conv2d takes pending_cls for such an input (H x W x Cin images, leading dimension ldin)

@@ -94,3 +94,39 @@ def test_sparse_generators_through_row_maps_and_pooling(nnv, hw, cin, names, ins
     finally:
         ctx.set_switch("poison_pending", was[0])
         ctx.set_eager_columns(was[1])
+
+
+def test_an_array_goes_in_one_launch_per_layer(nnv):
+    """Twenty images with different numbers of predicates, one of them listed twice: one launch per row map and pooling, the
+    same sets to the bit as every image gives by itself."""
+    rs = np.random.RandomState(5)
+    hw, cin, names = (12, 11), 3, "norm conv3_1_1_4 bn relu pool2_2_0 pool2_1_0 relu".split()
+    layers = _layers(rs, names, hw, cin)
+    ctx = nnv.default_context()
+    net = nnv.NN.from_config(layers)
+    opts = {"reachMethod": "relax-star-area", "relaxFactor": 1}
+    bounds = []
+    for i in range(20):
+        x, eps = rs.rand(*hw, cin), 0.02 * (rs.rand(*hw, cin) < 0.2 + 0.04 * i)
+        bounds.append((x - eps, x + eps))
+    sets = [nnv.ImageStar(*b) for b in bounds]
+    before = ctx.routes()
+    ctx.set_timing(2)
+    try:
+        ctx.kernel_time(4)
+        net.reach(sets + [sets[3]], opts)
+        _, launches, _ = ctx.kernel_time(4)
+    finally:
+        ctx.set_timing(0)
+    took = {k: v - before[k] for k, v in ctx.routes().items()}
+    assert (took["rowmap_box"], took["rowmap_window"], took["pool_window"]) == (21, 21, 42), took
+    assert launches == 4, "one launch per row map and pooling layer"
+    got = [[(s.estimateRanges(), np.array(s.V)) for s in layer] for layer in net.reachSet]
+    for i, b in list(enumerate(bounds)) + [(20, bounds[3])]:
+        net.reach(nnv.ImageStar(*b), opts)
+        for li, out in enumerate(net.reachSet):
+            (lb, ub), V = got[li][i]
+            assert np.array_equal(V, np.array(out.V)), (li, i)
+            elb, eub = out.estimateRanges()
+            assert_close(lb, elb, "lb")
+            assert_close(ub, eub, "ub")
