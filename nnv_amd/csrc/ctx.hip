@@ -134,6 +134,19 @@ int nnvhip_ctx::alloc(size_t bytes, BufRef* out) {
   return NNVHIP_OK;
 }
 
+int nnvhip_ctx::check_room(size_t bytes) {
+  const size_t cls = size_class(bytes ? bytes : 1);
+  if (cls <= (size_t)bytes_cached) return NNVHIP_OK;  // (no question to the driver, 5 us, in a loop of reaches)
+  size_t avail = 0, total = 0;
+  NNV_HIP_TRY(hipMemGetInfo(&avail, &total));
+  if (cls <= avail + (size_t)bytes_cached) return NNVHIP_OK;
+  drop_unreferenced_weights();
+  trim();
+  NNV_HIP_TRY(hipMemGetInfo(&avail, &total));
+  if (cls > avail) NNV_FAIL(NNVHIP_ERR_OOM, "out of device memory allocating %zu bytes", cls);
+  return NNVHIP_OK;
+}
+
 void nnvhip_ctx::release_block(void* p, size_t bytes) {
   // Blocks are recycled without waiting: every consumer runs on the context's single stream, so
   // a later user of the block is ordered after the earlier one.

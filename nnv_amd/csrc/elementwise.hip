@@ -542,6 +542,9 @@ static int rowmap_windows(nnvhip_ctx* c, const RowmapArgs& a, int64_t N, int64_t
 static int rowmap_boxes(nnvhip_ctx* c, const RowmapArgs& a, bool may_flip, int64_t N, int64_t count, nnvhip_star* const* in,
                         nnvhip_star** out) {
   const int64_t ld = a.ld;
+  double whole = 0.0;  // (mapped boxes whose matrices no reader could be given are refused here, as where they are made)
+  for (int64_t i = 0; i < count; ++i) whole += 8.0 * (double)ld * (double)(in[i]->n + 1);
+  NNV_TRY(c->check_room((size_t)whole));
   NNV_TRY(c->begin_op());
   std::map<const double*, int64_t> scale_at;
   for (int64_t i = 0; i < count; ++i) scale_at.emplace(in[i]->oh_scale, (int64_t)scale_at.size());

@@ -412,6 +412,8 @@ struct nnvhip_ctx {
   int kernel_timer_end(bool on, int which, double flop);
 
   int alloc(size_t bytes, nnvhip::BufRef* out);
+  // NNVHIP_ERR_OOM if alloc(bytes) would fail now; allocates nothing (what is cached is given up only where alloc would).
+  int check_room(size_t bytes);
   void release_block(void* p, size_t bytes);
   int trim();
   // Returns host-pinned scratch of `bytes`; waits for the stream when the ring wraps.

@@ -223,10 +223,11 @@ int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* 
     ints += round_up(std::max<int64_t>(sh.n, 1), kLdAlign);
     if (sh.n == N) full = (int64_t)k;
   }
-  // (sets whose whole matrices no reader could ever be given are refused here, as they were when they were written)
+  // (sets whose whole matrices no reader could be given are refused here, as they were when they were written)
   double whole = 0.0;
   for (int64_t s = 0; s < count; ++s) whole += 8.0 * (double)ld * (double)(shapes[(size_t)shape_of[(size_t)s]].n + 1);
   if (whole > (double)c->device_bytes) NNV_FAIL(NNVHIP_ERR_OOM, "out of device memory allocating %.0f bytes", whole);
+  NNV_TRY(c->check_room((size_t)whole));
   const size_t bytes = sizeof(double) * (size_t)doubles + sizeof(int32_t) * (size_t)ints;
   void* st = nullptr;
   NNV_TRY(c->stage(bytes, &st));
