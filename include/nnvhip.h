@@ -144,6 +144,9 @@ NNVHIP_API int nnvhip_pool_stats(nnvhip_ctx* ctx, int64_t* bytes_in_use, int64_t
  * be NULL.  A benchmark reads them around a step that took unusually long. */
 NNVHIP_API int nnvhip_debug_counters(nnvhip_ctx* ctx, int64_t* device_mallocs, int64_t* staging_waits, int64_t* deferred_handles,
                           int64_t* live_handles);
+/* Bytes of pinned host memory the context stages its copies in: the ring in use, and rings it has outgrown (kept until
+ * the context goes).  Either pointer may be NULL. */
+NNVHIP_API int nnvhip_debug_staging(nnvhip_ctx* ctx, int64_t* ring_bytes, int64_t* outgrown_bytes);
 /* Test hook (no counterpart in the reference): how many sets, since the context was created, went through a ReLU
  * step that wrote the bounds of its new predicates behind the input's in the arrays the input already had, and how
  * many through one that copied the input's bounds into arrays of its own (new_pred_lb = [predicate_lb; zeros(m,1)],

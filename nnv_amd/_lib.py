@@ -29,7 +29,7 @@ SYMBOLS = [
     "nnvhip_star_fetch_rows", "nnvhip_relu_apply_lists", "nnvhip_probe_mfma_peak",
     "nnvhip_estimate_ranges_static", "nnvhip_debug_mailbox_pack", "nnvhip_debug_mailbox_unpack",
     "nnvhip_debug_set_relu_call_number", "nnvhip_reach_layers", "nnvhip_reach_is_one_launch", "nnvhip_relu_reduce_mem",
-    "nnvhip_set_switch", "nnvhip_hint_next_fc", "nnvhip_debug_counters", "nnvhip_debug_relu_bounds", "nnvhip_debug_routes", "nnvhip_weight_cache_stats", "nnvhip_weight_cache_release", "nnvhip_debug_weak_weight_hash",
+    "nnvhip_set_switch", "nnvhip_hint_next_fc", "nnvhip_debug_counters", "nnvhip_debug_relu_bounds", "nnvhip_debug_routes", "nnvhip_debug_staging", "nnvhip_weight_cache_stats", "nnvhip_weight_cache_release", "nnvhip_debug_weak_weight_hash",
 ]
 
 
@@ -128,6 +128,7 @@ def load():
         "nnvhip_debug_counters": [p, pi64, pi64, pi64, pi64],
         "nnvhip_debug_relu_bounds": [p, pi64, pi64],
         "nnvhip_debug_routes": [p, C.POINTER(i64)],
+        "nnvhip_debug_staging": [p, pi64, pi64],
         "nnvhip_weight_cache_stats": [p, pi64, pi64, pi64],
         "nnvhip_weight_cache_release": [p, pi64],
         "nnvhip_debug_weak_weight_hash": [C.c_int],
@@ -268,6 +269,12 @@ class Context:
         """(sets whose ReLU step appended its predicate bounds in place, sets whose step copied the old ones)."""
         a, b = C.c_int64(), C.c_int64()
         check(self.lib.nnvhip_debug_relu_bounds(self.handle, C.byref(a), C.byref(b)))
+        return a.value, b.value
+
+    def staging_bytes(self):
+        """(pinned bytes of the staging ring in use, bytes of rings it has outgrown)."""
+        a, b = C.c_int64(), C.c_int64()
+        check(self.lib.nnvhip_debug_staging(self.handle, C.byref(a), C.byref(b)))
         return a.value, b.value
 
     def routes(self):

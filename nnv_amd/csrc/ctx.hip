@@ -171,7 +171,10 @@ int nnvhip_ctx::stage(size_t bytes, void** host) {
     NNV_HIP_TRY(hipStreamSynchronize(stream));
     // a table handed out from the old ring may still be named by a launch that is about to be issued:
     // the old ring stays allocated until the context goes (rings only ever grow, by doubling)
-    if (pinned) retired_rings.push_back(pinned);
+    if (pinned) {
+      retired_rings.push_back(pinned);
+      retired_bytes += pinned_bytes;
+    }
     pinned = nullptr;
     pinned_bytes = std::max(bytes * 2, size_t(4) << 20);
     NNV_HIP_TRY(hipHostMalloc((void**)&pinned, pinned_bytes, hipHostMallocDefault));
@@ -503,6 +506,13 @@ int nnvhip_debug_relu_bounds(nnvhip_ctx* c, int64_t* appended_in_place, int64_t*
   if (!c) NNV_FAIL(NNVHIP_ERR_ARG, "null context");
   if (appended_in_place) *appended_in_place = c->n_bounds_in_place;
   if (copied) *copied = c->n_bounds_copied;
+  return NNVHIP_OK;
+}
+
+int nnvhip_debug_staging(nnvhip_ctx* c, int64_t* ring_bytes, int64_t* outgrown_bytes) {
+  if (!c) NNV_FAIL(NNVHIP_ERR_ARG, "null context");
+  if (ring_bytes) *ring_bytes = (int64_t)c->pinned_bytes;
+  if (outgrown_bytes) *outgrown_bytes = (int64_t)c->retired_bytes;
   return NNVHIP_OK;
 }
 

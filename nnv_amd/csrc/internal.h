@@ -337,7 +337,7 @@ struct nnvhip_ctx {
   // pinned staging ring for descriptor tables and small read-backs
   char* pinned = nullptr;
   std::vector<char*> retired_rings;
-  size_t pinned_bytes = 0;
+  size_t pinned_bytes = 0, retired_bytes = 0;
   size_t pinned_off = 0;
   // mailbox in pinned host memory: a kernel posts {m, inactive, call number} there and the host spins
   // on it (after having stored kMailboxEmpty there), which is quicker than a device-to-host copy plus

@@ -153,9 +153,10 @@ int nnvhip_star_create(nnvhip_ctx* c, int64_t N, int64_t n, const double* V, con
 // Star(lb, ub) for every column of two N x count matrices.  A box's generators are scaled unit vectors, and the handle
 // says which (oh_idx, oh_scale): only the centres go to memory (vcols = 1), back to back, and whoever reads the whole
 // matrix has the columns written then (ensure_dense).  Everything the call puts on the device - centres, half-widths,
-// predicate bounds, index lists - is laid out in pinned memory and travels in one copy; no kernel runs.  (Writing the
-// matrices took 133 us for 100 boxes of 784 dimensions, 1.54 ms for 1024 of them, 6.4 GB nobody read; seven small
+// predicate bounds, index lists - is laid out in pinned memory and travels in one copy (pieces of kBoxPiece entries,
+// so that the staging ring stays at 16 MB whatever the array's size); no kernel runs.  (Writing the matrices took 133 us for 100 boxes of 784 dimensions, 1.54 ms for 1024 of them, 6.4 GB nobody read; seven small
 // copies and kernels took 60 us of a single set's reach.)
+constexpr int64_t kBoxPiece = int64_t(1) << 20;
 int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* lb, const double* ub,
                          nnvhip_star** out) {
   CHECK_CTX(c);
@@ -228,35 +229,50 @@ int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* 
   for (int64_t s = 0; s < count; ++s) whole += 8.0 * (double)ld * (double)(shapes[(size_t)shape_of[(size_t)s]].n + 1);
   if (whole > (double)c->device_bytes) NNV_FAIL(NNVHIP_ERR_OOM, "out of device memory allocating %.0f bytes", whole);
   NNV_TRY(c->check_room((size_t)whole));
-  const size_t bytes = sizeof(double) * (size_t)doubles + sizeof(int32_t) * (size_t)ints;
-  void* st = nullptr;
-  NNV_TRY(c->stage(bytes, &st));
-  BufRef buf;
-  NNV_TRY(c->alloc(bytes, &buf));
-  double* h = static_cast<double*>(st);
-  int32_t* hi = reinterpret_cast<int32_t*>(h + doubles);
-  for (int64_t s = 0; s < count; ++s) {
-    const double *l = lb + s * N, *u = ub + s * N;
-    double* col = h + s * ld;
-    for (int64_t i = 0; i < N; ++i) col[i] = 0.5 * (l[i] + u[i]);  // set/Box.m:35
-    for (int64_t i = N; i < ld; ++i) col[i] = 0.0;
-  }
-  memcpy(h + vec_off, vecs.data(), sizeof(double) * vecs.size());
+  // bounds and lists (what follows the half-widths), as they go to the device
+  const int64_t tail_off = vec_off + ld * (int64_t)shapes.size();
+  std::vector<double> tail((size_t)(doubles - tail_off + (ints + 1) / 2));
   for (const auto& pb : pb_at) {
     const int64_t npad = round_up(std::max<int64_t>(pb.first, 1), kLdAlign);
-    std::fill(h + pb.second, h + pb.second + npad, -1.0);
-    std::fill(h + pb.second + npad, h + pb.second + 2 * npad, 1.0);
+    double* at = tail.data() + (pb.second - tail_off);
+    std::fill(at, at + npad, -1.0);
+    std::fill(at + npad, at + 2 * npad, 1.0);
   }
   for (size_t k = 0; k < shapes.size(); ++k) {
     const Shape& sh = shapes[k];
     if (sh.idx_of != (int64_t)k) continue;
-    int32_t* list = hi + sh.idx_off;
+    int32_t* list = reinterpret_cast<int32_t*>(tail.data() + (doubles - tail_off)) + sh.idx_off;
     int64_t t = 0;
     for (int64_t i = 0; i < N; ++i)
       if (N == 1 || vecs[k * ld + i] != 0.0) list[t++] = (int32_t)i;
     for (const int64_t end = round_up(std::max<int64_t>(sh.n, 1), kLdAlign); t < end; ++t) list[t] = 0;
   }
-  NNV_HIP_TRY(hipMemcpyAsync(buf->ptr, st, bytes, hipMemcpyHostToDevice, c->stream));
+  const int64_t total = tail_off + (int64_t)tail.size();
+  const size_t bytes = sizeof(double) * (size_t)total;
+  BufRef buf;
+  NNV_TRY(c->alloc(bytes, &buf));
+  for (int64_t e0 = 0; e0 < total; e0 += kBoxPiece) {
+    const int64_t e1 = std::min(total, e0 + kBoxPiece);
+    void* st = nullptr;
+    NNV_TRY(c->stage(sizeof(double) * (size_t)(e1 - e0), &st));
+    double* h = static_cast<double*>(st);  // the block's entries [e0, e1)
+    int64_t e = e0;
+    while (e < std::min(e1, vec_off)) {  // centres
+      const int64_t s = e / ld, i0 = e - s * ld, i1 = std::min(ld, i0 + e1 - e);
+      const double *l = lb + s * N, *u = ub + s * N;
+      double* col = h + (e - e0);
+      for (int64_t i = i0; i < std::min(i1, N); ++i) col[i - i0] = 0.5 * (l[i] + u[i]);  // set/Box.m:35
+      for (int64_t i = std::max(i0, N); i < i1; ++i) col[i - i0] = 0.0;
+      e += i1 - i0;
+    }
+    if (e < std::min(e1, tail_off)) {
+      const int64_t end = std::min(e1, tail_off);
+      memcpy(h + (e - e0), vecs.data() + (e - vec_off), sizeof(double) * (size_t)(end - e));
+      e = end;
+    }
+    if (e < e1) memcpy(h + (e - e0), tail.data() + (e - tail_off), sizeof(double) * (size_t)(e1 - e));
+    NNV_HIP_TRY(hipMemcpyAsync(buf->as<double>() + e0, st, sizeof(double) * (size_t)(e1 - e0), hipMemcpyHostToDevice, c->stream));
+  }
   c->h2d_bytes += (int64_t)bytes;
   double* d = buf->as<double>();
   const int32_t* di = reinterpret_cast<const int32_t*>(d + doubles);

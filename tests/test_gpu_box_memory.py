@@ -1,6 +1,7 @@
 """What boxes and released arrays hold on to: a box array that could never be written whole is refused where it is made,
 staging memory stays bounded whatever the array's size, and the queue of released arrays stays bounded in a loop."""
 import ctypes as C
+import gc
 
 import numpy as np
 import pytest
@@ -37,3 +38,31 @@ def test_a_box_that_fits_the_device_but_not_what_is_free_is_refused(nnv):
         nnv.Star(lb, lb + 1.0)
     s = nnv.Star(lb[:1000], lb[:1000] + 1.0)         # the context goes on
     assert np.array_equal(s.estimateRanges()[1], np.ones(1000))
+
+
+@pytest.mark.parametrize("N,count", [(1500, 1100), (70001, 31), (1100000, 2)])
+@pytest.mark.parametrize("shared", [True, False])
+def test_large_box_arrays_travel_in_pieces(nnv, N, count, shared):
+    """More bounds than one piece of the staging ring holds: centres, half-widths and index lists arrive whole, with sets
+    that share their half-widths and sets that all have their own."""
+    from nnv_amd import _lib
+    rs = np.random.RandomState(N + count)
+    ctx = _lib.Context(0)                             # (a context of its own: other tests may have grown the shared one's ring)
+    x = rs.rand(N, count)
+    w = np.where(rs.rand(N, 1 if shared else count) < 3.0 / N, rs.rand(N, 1 if shared else count), 0.0) * np.ones((1, count))
+    lbs, ubs = x - w, x + w
+    sets = nnv.Star.from_boxes(lbs, ubs, ctx=ctx)
+    ring, outgrown = ctx.staging_bytes()
+    assert ring <= 16 << 20 and outgrown <= ring
+    lb, ub = nnv.Star.estimateRanges_array(sets)
+    c, v = 0.5 * (lbs + ubs), 0.5 * (ubs - lbs)
+    assert np.array_equal(lb, c - v) and np.array_equal(ub, c + v)
+    for i in (0, count // 2, count - 1):
+        nz = np.flatnonzero(v[:, i])
+        assert sets[i].nVar == nz.size
+        V = sets[i].V
+        assert np.array_equal(V[:, 0], c[:, i]) and np.array_equal(V[nz, 1 + np.arange(nz.size)], v[nz, i])
+        assert np.count_nonzero(V[:, 1:]) == nz.size
+    del sets
+    gc.collect()
+    _lib.check(ctx.lib.nnvhip_destroy(ctx.handle))
