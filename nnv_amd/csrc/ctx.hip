@@ -57,6 +57,12 @@ int enter_ctx(nnvhip_ctx* ctx) {
   return NNVHIP_OK;
 }
 
+// Brings an object's memory into the cache: thousands of handles and constraint nodes lie scattered, and a miss on each of
+// their lines is most of what making or letting go of them costs (4096 sets through 12 layers: 23 -> 16-17 ms a pass).
+static void prefetch(const void* p, size_t bytes) {
+  for (size_t at = 0; at < bytes; at += 64) __builtin_prefetch(static_cast<const char*>(p) + at, 1);
+}
+
 // Handles come from (and go back to) a list of released ones kept by the context: an array of a thousand sets makes
 // and lets go of a thousand handles per layer, on the host's critical path.
 nnvhip_star* new_star(nnvhip_ctx* ctx) {
@@ -64,6 +70,7 @@ nnvhip_star* new_star(nnvhip_ctx* ctx) {
   if (!ctx->free_stars.empty()) {
     void* mem = ctx->free_stars.back();
     ctx->free_stars.pop_back();
+    if (ctx->free_stars.size() >= 4) prefetch(ctx->free_stars[ctx->free_stars.size() - 4], sizeof(nnvhip_star));
     s = new (mem) nnvhip_star();
   } else {
     s = new (::operator new(sizeof(nnvhip_star))) nnvhip_star();
@@ -91,6 +98,9 @@ void nnvhip_ctx::drain_deferred(size_t at_most) {
   while (!deferred.empty() && at_most-- > 0) {
     nnvhip_star* s = deferred.back();
     deferred.pop_back();
+    const size_t left = deferred.size();
+    if (left >= 8) prefetch(deferred[left - 8], sizeof(nnvhip_star));
+    if (left >= 4 && deferred[left - 4]->cons) prefetch(deferred[left - 4]->cons.get(), sizeof(ConsNode));
     nnvhip_star_release(s);
   }
 }
@@ -99,13 +109,17 @@ int nnvhip_ctx::alloc(size_t bytes, BufRef* out) {
   size_t cls = size_class(bytes ? bytes : 1);
   void* p = nullptr;
   auto it = free_blocks.find(cls);
-  // A released array that has not been let go yet may hold such a block.  While the pool is small next to the
-  // device's memory it grows instead (a loop of reaches then alternates between two generations of blocks and
-  // never waits for the handles of the previous one); past that share the array is let go now.
-  if (it == free_blocks.end() && !deferred.empty() &&
-      (double)(bytes_in_use + bytes_cached) + (double)cls > 0.4 * (double)device_bytes) {
-    drain_deferred();
-    it = free_blocks.find(cls);
+  // A released array that has not been let go yet may hold such a block.  While few handles are queued and the pool is
+  // small next to the device's memory it grows instead (a loop of reaches then alternates between two generations of
+  // blocks and never waits for the handles of the previous one); past that arrays are let go now.  Without the bound on
+  // the queue, a loop whose host waits too little to let go of what it releases grew it pass by pass, up to 40 % of the
+  // memory, with a hipMalloc for every block: 300 boxes through 8-100x5-5, 1.4 ms a pass, now 0.7.
+  if (it == free_blocks.end() && !deferred.empty()) {
+    const bool full = (double)(bytes_in_use + bytes_cached) + (double)cls > 0.4 * (double)device_bytes;
+    if (full || deferred.size() > kMaxDeferred) {
+      drain_deferred(full ? ~size_t(0) : deferred.size() - kMaxDeferred);
+      it = free_blocks.find(cls);
+    }
   }
   if (it != free_blocks.end()) {
     p = it->second;

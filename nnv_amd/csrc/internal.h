@@ -320,8 +320,10 @@ struct nnvhip_ctx {
   // Handles of large arrays that the caller has released but that have not been let go yet: destroying
   // thousands of handles costs hundreds of microseconds of host time, which is spent where the host waits
   // for the device anyway (the ReLU step's wait for its counts, a synchronisation) or when the pool runs
-  // short of a block; pool_stats, trim and destroy let them go first.
+  // short of a block; pool_stats, trim and destroy let them go first.  When the pool runs short, what
+  // is queued beyond kMaxDeferred goes first (alloc).
   std::vector<nnvhip_star*> deferred;
+  static constexpr size_t kMaxDeferred = 4096;
   void drain_deferred(size_t at_most = ~size_t(0));
   // counters for diagnosing a slow step: hipMalloc calls of the pool, waits for the stream because the pinned
   // staging ring wrapped or grew, mailbox waits that went through the slow path
@@ -331,7 +333,7 @@ struct nnvhip_ctx {
   // nnvhip_hint_next_fc: the FC layer the caller will apply to the output of its next ReLU step (consumed by that step)
   const nnvhip_fc* next_fc = nullptr;
   // memory of released handles, reused by new_star (at most kMaxFreeStars of them are kept)
-  static constexpr size_t kMaxFreeStars = 32768;
+  static constexpr size_t kMaxFreeStars = 65536;
   std::vector<void*> free_stars;
   int64_t device_bytes = 0;  // memory of the device (the pool grows past a released array only below a share of it)
   // pinned staging ring for descriptor tables and small read-backs

@@ -66,3 +66,28 @@ def test_large_box_arrays_travel_in_pieces(nnv, N, count, shared):
     del sets
     gc.collect()
     _lib.check(ctx.lib.nnvhip_destroy(ctx.handle))
+
+
+def test_the_queue_of_released_arrays_stays_bounded(nnv):
+    """A loop of reaches over an array of 300 sets: the handles of the passes before are let go, device memory is not asked
+    for once per pass."""
+    rs = np.random.RandomState(1)
+    dims = [8, 100, 100, 100, 100, 100, 5]
+    layers = []
+    for a, b in zip(dims[:-1], dims[1:]):
+        layers += [{"type": "fc", "W": rs.randn(b, a) * np.sqrt(2.0 / a), "b": rs.randn(b) * 0.1}, {"type": "relu"}]
+    net = nnv.NN.from_config(layers[:-1])
+    ctx = nnv.default_context()
+    ctx.synchronize()
+    x = rs.rand(8, 300)
+    queued, mallocs = [], []
+    for _ in range(40):
+        out = net.reach(nnv.Star.from_boxes(x - 0.05, x + 0.05), {"reachMethod": "relax-star-area", "relaxFactor": 1})
+        nnv.Star.estimateRanges_array(out)
+        now = ctx.debug_counters()
+        queued.append(now["deferred_handles"])
+        mallocs.append(now["device_mallocs"])
+    assert max(queued) <= 4096 + 3 * 12 * 300, queued
+    # (which blocks are free when depends on how long the host waits; a queue that only grows asks for one or more per layer,
+    # a hundred in nine passes)
+    assert mallocs[-1] - mallocs[-10] < 9, mallocs
