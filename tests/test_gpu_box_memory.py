@@ -91,3 +91,21 @@ def test_the_queue_of_released_arrays_stays_bounded(nnv):
     # (which blocks are free when depends on how long the host waits; a queue that only grows asks for one or more per layer,
     # a hundred in nine passes)
     assert mallocs[-1] - mallocs[-10] < 9, mallocs
+
+
+@pytest.mark.parametrize("N,count", [(1, 1), (7, 3), (130, 2), (784, 1)])
+def test_a_box_matrix_is_read_without_being_written(nnv, N, count):
+    """V of a box whose matrix nobody has needed on the device: read twice, in memory afterwards as little as before."""
+    rs = np.random.RandomState(N)
+    lbs = rs.randn(N, count)
+    ubs = lbs + rs.rand(N, count) * (rs.rand(N, count) < 0.7)
+    sets = nnv.Star.from_boxes(lbs, ubs)
+    ctx = nnv.default_context()
+    before = ctx.pool_stats()[0]
+    from oracle import nnv_oracle as o
+    for i in range(count):
+        exp = o.star_from_box(lbs[:, i], ubs[:, i]).V
+        assert np.array_equal(sets[i].V, exp)
+        rows = rs.randint(0, N, size=min(N, 9))
+        assert np.array_equal(sets[i]._h.fetch_rows(rows), exp[rows])
+    assert ctx.pool_stats()[0] == before
