@@ -229,25 +229,31 @@ int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* 
   for (int64_t s = 0; s < count; ++s) whole += 8.0 * (double)ld * (double)(shapes[(size_t)shape_of[(size_t)s]].n + 1);
   if (whole > (double)c->device_bytes) NNV_FAIL(NNVHIP_ERR_OOM, "out of device memory allocating %.0f bytes", whole);
   NNV_TRY(c->check_room((size_t)whole));
-  // bounds and lists (what follows the half-widths), as they go to the device
-  const int64_t tail_off = vec_off + ld * (int64_t)shapes.size();
-  std::vector<double> tail((size_t)(doubles - tail_off + (ints + 1) / 2));
-  for (const auto& pb : pb_at) {
-    const int64_t npad = round_up(std::max<int64_t>(pb.first, 1), kLdAlign);
-    double* at = tail.data() + (pb.second - tail_off);
-    std::fill(at, at + npad, -1.0);
-    std::fill(at + npad, at + 2 * npad, 1.0);
+  // bounds and lists (what follows the half-widths)
+  const int64_t tail_off = vec_off + ld * (int64_t)shapes.size(), total = doubles + (ints + 1) / 2;
+  auto write_tail = [&](double* tail) {
+    for (const auto& pb : pb_at) {
+      const int64_t npad = round_up(std::max<int64_t>(pb.first, 1), kLdAlign);
+      double* at = tail + (pb.second - tail_off);
+      std::fill(at, at + npad, -1.0);
+      std::fill(at + npad, at + 2 * npad, 1.0);
+    }
+    int32_t* lists = reinterpret_cast<int32_t*>(tail + (doubles - tail_off));
+    for (size_t k = 0; k < shapes.size(); ++k) {
+      const Shape& sh = shapes[k];
+      if (sh.idx_of != (int64_t)k) continue;
+      int32_t* list = lists + sh.idx_off;
+      int64_t t = 0;
+      for (int64_t i = 0; i < N; ++i)
+        if (N == 1 || vecs[k * ld + i] != 0.0) list[t++] = (int32_t)i;
+      for (const int64_t end = round_up(std::max<int64_t>(sh.n, 1), kLdAlign); t < end; ++t) list[t] = 0;
+    }
+  };
+  std::vector<double> tail;  // (in one piece they are written in their place)
+  if (total > kBoxPiece) {
+    tail.resize((size_t)(total - tail_off));
+    write_tail(tail.data());
   }
-  for (size_t k = 0; k < shapes.size(); ++k) {
-    const Shape& sh = shapes[k];
-    if (sh.idx_of != (int64_t)k) continue;
-    int32_t* list = reinterpret_cast<int32_t*>(tail.data() + (doubles - tail_off)) + sh.idx_off;
-    int64_t t = 0;
-    for (int64_t i = 0; i < N; ++i)
-      if (N == 1 || vecs[k * ld + i] != 0.0) list[t++] = (int32_t)i;
-    for (const int64_t end = round_up(std::max<int64_t>(sh.n, 1), kLdAlign); t < end; ++t) list[t] = 0;
-  }
-  const int64_t total = tail_off + (int64_t)tail.size();
   const size_t bytes = sizeof(double) * (size_t)total;
   BufRef buf;
   NNV_TRY(c->alloc(bytes, &buf));
@@ -270,7 +276,8 @@ int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* 
       memcpy(h + (e - e0), vecs.data() + (e - vec_off), sizeof(double) * (size_t)(end - e));
       e = end;
     }
-    if (e < e1) memcpy(h + (e - e0), tail.data() + (e - tail_off), sizeof(double) * (size_t)(e1 - e));
+    if (e < e1 && tail.empty()) write_tail(h + tail_off);
+    else if (e < e1) memcpy(h + (e - e0), tail.data() + (e - tail_off), sizeof(double) * (size_t)(e1 - e));
     NNV_HIP_TRY(hipMemcpyAsync(buf->as<double>() + e0, st, sizeof(double) * (size_t)(e1 - e0), hipMemcpyHostToDevice, c->stream));
   }
   c->h2d_bytes += (int64_t)bytes;
