@@ -1,5 +1,6 @@
 // Context: device memory pool, pinned staging ring, switches, timers and the measurement probes.
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 
@@ -128,6 +129,7 @@ int nnvhip_ctx::alloc(size_t bytes, BufRef* out) {
   } else {
     hipError_t e = hipMalloc(&p, cls);
     n_device_mallocs++;
+    room_seen -= (int64_t)cls;
     if (e != hipSuccess) {
       (void)hipGetLastError();
       drop_unreferenced_weights();  // layers that only the weight cache still holds
@@ -150,9 +152,15 @@ int nnvhip_ctx::alloc(size_t bytes, BufRef* out) {
 
 int nnvhip_ctx::check_room(size_t bytes) {
   const size_t cls = size_class(bytes ? bytes : 1);
-  if (cls <= (size_t)bytes_cached) return NNVHIP_OK;  // (no question to the driver, 5 us, in a loop of reaches)
+  if (cls <= (size_t)bytes_cached) return NNVHIP_OK;
+  // The driver takes 15 us to answer behind queued work, so its answer serves for a tenth of a second, less what the pool has
+  // asked for since, for anything up to half of it (others may have taken some).
+  const auto now = std::chrono::steady_clock::now();
+  if (room_seen > 0 && (int64_t)cls <= room_seen / 2 && now - room_at < std::chrono::milliseconds(100)) return NNVHIP_OK;
   size_t avail = 0, total = 0;
   NNV_HIP_TRY(hipMemGetInfo(&avail, &total));
+  room_seen = (int64_t)avail;
+  room_at = now;
   if (cls <= avail + (size_t)bytes_cached) return NNVHIP_OK;
   drop_unreferenced_weights();
   trim();

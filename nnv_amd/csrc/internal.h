@@ -5,6 +5,7 @@
 #include <hip/hip_ext.h>
 
 #include <atomic>
+#include <chrono>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -416,6 +417,8 @@ struct nnvhip_ctx {
   int alloc(size_t bytes, nnvhip::BufRef* out);
   // NNVHIP_ERR_OOM if alloc(bytes) would fail now; allocates nothing (what is cached is given up only where alloc would).
   int check_room(size_t bytes);
+  int64_t room_seen = 0;  // what the driver last said was free, less the pool's own requests since ...
+  std::chrono::steady_clock::time_point room_at;  // ... and when
   void release_block(void* p, size_t bytes);
   int trim();
   // Returns host-pinned scratch of `bytes`; waits for the stream when the ring wraps.
