@@ -50,6 +50,8 @@ GROUP_KERNELS = {
     "gemm_f64_kernel": ("gemm_f64_kernel",),
     "gemm_seg_kernel": ("gemm_seg_kernel",),
     "conv2d_fast_kernel": ("conv2d_fast_kernel", "conv2d_fast_stamps_kernel", "conv2d_f64_kernel"),
+    "conv_window_kernel": ("conv_window_kernel",),
+    "fc_window_kernel": ("fc_window_kernel",),
     "gather_columns_kernel": ("gather_columns_kernel", "gather_skinny_kernel", "fc_rowsum_kernel", "conv_stamp_kernel", "conv_stamp_rows_kernel"),
     "ranges_partial_kernel": ("ranges_partial_kernel", "ranges_window_kernel"),
     "relu_classify_kernel": ("relu_classify_kernel", "relu_count_kernel", "relu_compact_kernel"),
@@ -248,14 +250,14 @@ def measure(k, args, ctx, exact_steps, extras):
         return acc / reps
 
     # a small FC / ReLU network is reached by ONE launch (nnvhip_reach_layers): time that kernel on the step's own path
-    for grp in range(11):
+    for grp in range(13):
         ctx.kernel_time(grp)
     ctx.set_timing(2)
     for _ in range(reps):
         step()
     ctx.set_timing(0)
     chain_ms, chain_launches, chain_bytes = ctx.kernel_time(8)
-    for grp in range(11):
+    for grp in range(13):
         ctx.kernel_time(grp)
 
     per_layer = timed_pass(1)          # NN.reachTime-style device time per layer (layer-by-layer calls)
@@ -270,6 +272,8 @@ def measure(k, args, ctx, exact_steps, extras):
     fin_ms, fin_launches, fin_bytes = ctx.kernel_time(7)
     seg_ms, seg_launches, seg_work = ctx.kernel_time(9)
     dlt_ms, dlt_launches, dlt_bytes = ctx.kernel_time(10)
+    fcw_ms, fcw_launches, fcw_work = ctx.kernel_time(11)
+    cvw_ms, cvw_launches, cvw_work = ctx.kernel_time(12)
 
     # algorithmic (unpadded, dense) flop of the launches the kernel timers cover
     gemm_flop = conv_flop = 0.0
@@ -341,19 +345,22 @@ def measure(k, args, ctx, exact_steps, extras):
                 "avg_launch_ms": round(ms_ / n_, 5), "bytes_per_launch": b_ / n_, "ms_per_step": round(ms_ / reps, 5)}
 
     groups = []
-    # (the dense count of the FC layers is quoted with the one of the two FC kernel groups that takes longer)
-    if seg_launches:
-        groups.append((seg_ms, mfma_roofline("gemm_seg_kernel", seg_work, gemm_flop if seg_ms >= gemm_ms else 0.0, seg_ms, seg_launches)))
-    if gemm_launches:
-        groups.append((gemm_ms, mfma_roofline("gemm_f64_kernel", gemm_work, gemm_flop if gemm_ms > seg_ms or not seg_launches else 0.0,
-                                              gemm_ms, gemm_launches)))
-    if conv_launches:
-        g = mfma_roofline("conv2d_fast_kernel", conv_work, conv_flop, conv_ms, conv_launches)
+    # (the dense count of the FC layers is quoted with the one of the FC kernel groups that takes longest, that of the
+    # convolutions likewise)
+    fc_longest = max(seg_ms, gemm_ms, fcw_ms)
+    for name, ms_, n_, work in (("gemm_seg_kernel", seg_ms, seg_launches, seg_work), ("gemm_f64_kernel", gemm_ms, gemm_launches, gemm_work),
+                                ("fc_window_kernel", fcw_ms, fcw_launches, fcw_work)):
+        if n_:
+            groups.append((ms_, mfma_roofline(name, work, gemm_flop if ms_ == fc_longest else 0.0, ms_, n_)))
+    for name, ms_, n_, work in (("conv2d_fast_kernel", conv_ms, conv_launches, conv_work), ("conv_window_kernel", cvw_ms, cvw_launches, cvw_work)):
+        if not n_:
+            continue
+        g = mfma_roofline(name, work, conv_flop if ms_ == max(conv_ms, cvw_ms) else 0.0, ms_, n_)
         if not ctx.switch_is_on("eager_cols", "dense_affine"):
-            # conv2d_fast_stamps_kernel: a layer's launch also writes the filter stamps of its unit-vector columns (blocks
-            # dealt in between the tile blocks); the flop count is that of the tiles, the duration that of the whole launch
+            # conv2d_fast_stamps_kernel, conv_window_kernel: a layer's launch also writes the filter stamps of its unit-vector
+            # columns; the flop count is that of the products, the duration that of the whole launch
             g["stamp_blocks_in_the_same_launch"] = True
-        groups.append((conv_ms, g))
+        groups.append((ms_, g))
     if rng_launches:
         groups.append((rng_ms, hbm_roofline("ranges_partial_kernel", rng_ms, rng_launches, rng_bytes)))
     if app_launches:

@@ -227,7 +227,7 @@ class Context:
     def kernel_time(self, which, reset=True):
         """(total ms, launches, work) of a kernel group accumulated while timing was enabled:
         0 = FC GEMM, 1 = convolution (work = dense flop); 2 = estimateRanges pass, 3 = ReLU apply pass
-        (work = algorithmic bytes)."""
+        (work = algorithmic bytes); the others as listed at nnvhip_kernel_time in nnvhip.h."""
         ms, n, fl = C.c_double(), C.c_int64(), C.c_double()
         check(self.lib.nnvhip_kernel_time(self.handle, int(which), C.byref(ms), C.byref(n), C.byref(fl), 1 if reset else 0))
         return ms.value, n.value, fl.value

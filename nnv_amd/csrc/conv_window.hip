@@ -420,8 +420,9 @@ int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
     max_parts = std::max<int64_t>(max_parts, s.parts);
     ++ctx->routes[NNVHIP_ROUTE_CONV_WINDOW];
     if (s.parts > 1) ++ctx->routes[NNVHIP_ROUTE_CONV_WINDOW_PARTS];
-    // (as the implicit GEMM over the windows counts them; the rows a block leaves out are known on the device only)
-    flop += 2.0 * ((double)(s.dense - 1) * s.eh * s.ew + (double)a.g.P) * (double)cv->Cout * (double)cv->K;
+    // (rows a ReLU step has reset are not multiplied; their share under a filter is taken to be that of the image)
+    const double kept = s.in->rows_pending && s.in->n_kept >= 0 ? (double)s.in->n_kept / (double)s.in->N : 1.0;
+    flop += 2.0 * ((double)(s.dense - 1) * s.eh * s.ew + (double)a.g.P) * (double)cv->Cout * (double)cv->K * kept;
   }
   const ConvWinSet* table = nullptr;
   BufRef dev;
@@ -451,7 +452,7 @@ int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
   else
     NNV_CONV_WINDOW(64, 2, 2);
 #undef NNV_CONV_WINDOW
-  NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 1, flop));
+  NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 12, flop));
   NNV_HIP_TRY(hipGetLastError());
   return NNVHIP_OK;
 }

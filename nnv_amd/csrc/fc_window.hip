@@ -407,6 +407,7 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
   NNV_TRY(ctx->alloc(sizeof(int32_t) * orders, &order));
   NNV_TRY(ctx->alloc(sizeof(double) * fc->Mp * std::max<int64_t>(parts, 1), &cpart));
   int64_t o = 0, p = 0;
+  double flop = 0.0;
   for (int64_t i = 0; i < count; ++i) {
     FcWinSet& d = tab[(size_t)i];
     const nnvhip_star* s = sets[i].in;
@@ -423,6 +424,7 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
     d.plb = sets[i].out->plb;
     d.pub = sets[i].out->pub;
     d.rpart = sets[i].rpart;
+    flop += 2.0 * (double)fc->Mp * (double)(d.ncols - 1) * s->box_eh * s->box_ew * a.C * ((double)d.nk / (double)fc->K);
     o += sets[i].dense;
     p += d.cchunks;
   }
@@ -435,13 +437,14 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
                      tab[0], a);
   const dim3 grid((unsigned)(round_up(max_tiles + 1, 8) * a.tiles_m), (unsigned)count);
 #define NNV_FC_WINDOW(TM, TN, WR, WC, KT) \
-  hipLaunchKernelGGL((fc_window_kernel<TM, TN, WR, WC, KT>), grid, dim3(64 * WR * WC), 0, ctx->stream, table, tab[0], a)
+  NNV_LAUNCH(ctx, ctx->kernel_timing, (fc_window_kernel<TM, TN, WR, WC, KT>), grid, dim3(64 * WR * WC), 0, table, tab[0], a)
   // (one small set: a block or none per CU, nothing to hide a stage's loads behind - stages of 32 rows, half as many)
   if (tm == 32 && tn == 32) NNV_FC_WINDOW(32, 32, 2, 2, 16);
   else if (tm == 32) NNV_FC_WINDOW(32, 64, 2, 4, 16);
   else if (tn == 32) NNV_FC_WINDOW(64, 32, 4, 2, 32);
   else NNV_FC_WINDOW(64, 64, 2, 4, 16);
 #undef NNV_FC_WINDOW
+  NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 11, flop));
   NNV_HIP_TRY(hipGetLastError());
   ctx->routes[NNVHIP_ROUTE_FC_WINDOW] += count;
   return NNVHIP_OK;

@@ -407,7 +407,9 @@ struct nnvhip_ctx {
   // [6] ReLU classification, [7] range reduction, [8] whole-reach kernel of small networks (chain.hip)
   // [9] tile kernel of gemm_seg.hip (work = flop), [10] outputs that start from a product shared by many sets and
   // add only the rows in which a set differs from it (delta_tiles_kernel; work = bytes written)
-  static constexpr int kKernelGroups = 11;
+  // [11] FC contraction inside the images' windows (fc_window_kernel), [12] convolution by output position
+  // (conv_window_kernel); work = flop of the kept rows' products inside the bounds on the columns' windows
+  static constexpr int kKernelGroups = 13;
   double kern_ms[kKernelGroups] = {};
   int64_t kern_launches[kKernelGroups] = {};
   double kern_flop[kKernelGroups] = {};
