@@ -81,6 +81,29 @@ nnvhip_star* new_star(nnvhip_ctx* ctx) {
   return s;
 }
 
+constexpr size_t kNodeHead = 16;  // in front of a node: its context
+
+void* ConsNode::operator new(size_t bytes, nnvhip_ctx* ctx) {
+  if (!ctx->free_nodes.empty()) {
+    void* p = ctx->free_nodes.back();
+    ctx->free_nodes.pop_back();
+    return p;
+  }
+  char* at = static_cast<char*>(::operator new(kNodeHead + bytes));
+  memcpy(at, &ctx, sizeof ctx);
+  return at + kNodeHead;
+}
+
+void ConsNode::operator delete(void* p) {
+  char* at = static_cast<char*>(p) - kNodeHead;
+  nnvhip_ctx* ctx;
+  memcpy(&ctx, at, sizeof ctx);
+  if (ctx->free_nodes.size() < nnvhip_ctx::kMaxFreeNodes)
+    ctx->free_nodes.push_back(p);
+  else
+    ::operator delete(static_cast<void*>(at));
+}
+
 void delete_star(nnvhip_star* s) {
   nnvhip_ctx* c = s->ctx;
   s->~nnvhip_star();
@@ -315,6 +338,8 @@ int nnvhip_destroy(nnvhip_ctx* c) {
   c->trim();
   for (void* mem : c->free_stars) ::operator delete(mem);
   c->free_stars.clear();
+  for (void* mem : c->free_nodes) ::operator delete(static_cast<void*>(static_cast<char*>(mem) - kNodeHead));
+  c->free_nodes.clear();
   if (c->pinned) (void)hipHostFree(c->pinned);
   if (c->mailbox) (void)hipHostFree((void*)c->mailbox);
   for (char* r : c->retired_rings) (void)hipHostFree(r);

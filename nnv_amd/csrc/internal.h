@@ -272,8 +272,15 @@ struct ConsNode {
   int64_t ld_lbub = 0;
   BufRef index;                  // crossing neuron indices in new-predicate order: int32[m] at index_off
   int64_t index_off = 0;
+  // Nodes live in memory of released ones that the context keeps, the one released last first (as handles do, new_star):
+  // the allocator hands such chunks out oldest first, each one cold.  (Made by make_cons; the context's address stands in
+  // front of the object.)
+  static void* operator new(size_t bytes, nnvhip_ctx* ctx);
+  static void operator delete(void* p);
+  static void operator delete(void* p, nnvhip_ctx*) { operator delete(p); }
 };
 using ConsRef = Ref<ConsNode>;
+inline ConsRef make_cons(nnvhip_ctx* ctx) { return ConsRef(new (ctx) ConsNode()); }
 
 // start of every entry point that touches device data: selects the context's device
 int enter_ctx(nnvhip_ctx* ctx);
@@ -336,6 +343,9 @@ struct nnvhip_ctx {
   // memory of released handles, reused by new_star (at most kMaxFreeStars of them are kept)
   static constexpr size_t kMaxFreeStars = 65536;
   std::vector<void*> free_stars;
+  // ... and of constraint nodes (ConsNode::operator new)
+  static constexpr size_t kMaxFreeNodes = 65536;
+  std::vector<void*> free_nodes;
   int64_t device_bytes = 0;  // memory of the device (the pool grows past a released array only below a share of it)
   // pinned staging ring for descriptor tables and small read-backs
   char* pinned = nullptr;

@@ -925,7 +925,7 @@ int relu_relax(nnvhip_ctx* ctx, int order, int64_t count, nnvhip_star* const* in
     nodes.resize(count);
     for (int64_t i = 0; i < count; ++i) {
       pre.v.push_back(new_star(ctx));
-      nodes[i] = make_ref<ConsNode>();
+      nodes[i] = make_cons(ctx);
       init_static(pre.v[i], nodes[i].get(), i);
     }
   }
@@ -1047,7 +1047,7 @@ int relu_relax(nnvhip_ctx* ctx, int order, int64_t count, nnvhip_star* const* in
   for (int64_t i = 0; i < count; ++i) {
     const ReluDesc& d = descs[i];
     nnvhip_star* o = precreate ? pre.v[i] : new_star(ctx);
-    ConsRef node = precreate ? std::move(nodes[i]) : make_ref<ConsNode>();
+    ConsRef node = precreate ? std::move(nodes[i]) : make_cons(ctx);
     if (!precreate) init_static(o, node.get(), i);
     o->n = in[i]->n + d.m;
     if (!lazy_rows) {
