@@ -850,7 +850,7 @@ static int launch_conv_fast(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, const Conv
     for (size_t i = i0; i < i0 + cnt; ++i) grid_x = std::max<int64_t>(grid_x, sets[i].blocks + stamp_blocks);
     const ConvSet* table = nullptr;
     BufRef tab;
-    if (cnt > 1) {  // (a device copy: every block reads its record)
+    if (cnt > 1) {  // (a device copy, as good as the staging ring here: see upload_table)
       NNV_TRY(ctx->upload(sets.data() + i0, sizeof(ConvSet) * cnt, &tab));
       table = tab->as<ConvSet>();
     }

@@ -38,7 +38,8 @@ struct StampSet {
 // non-zero candidates, i.e. the rows inside every column's window - and adds up the row's four range sums tap
 // by tap.  Everything else in the columns is zero and is written by the caller (or left for later).
 // S lanes share a row, lane s taking the taps k = s, s + S, ...; their sums are combined by a butterfly (a fixed
-// order).  S = 1 for filters with few taps, 16 otherwise (a row's taps are then walked by 16 lanes at once).
+// order).  S is the caller's choice: 1 for at most 32 taps; for more, 8 beside the products of another kernel's blocks and
+// 16 in the launch that does nothing else.
 // A block first decodes the taps once into LDS (filter position and the tap's offset from the pixel under the
 // filter's corner), so that the walk has no division in it, and looks up four taps' pixels before it handles them.
 constexpr int kStampTapTable = kMaxTaps;  // taps per output (FH * FW * Cin): no layer has more

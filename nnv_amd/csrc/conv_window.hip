@@ -375,7 +375,8 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
 
 // By position from about 2000 taps x channels on: below that a block's lists cost more than its product (72 taps into 16
 // channels of 16 x 16, 3072 images: 42 us here, 36 us for the implicit GEMM over the windows with the scan behind it; 144 into
-// 32, 25 sets of 784 images: 138 us here, 270 there).
+// 32, 25 sets of 784 images: 138 us here, 270 there).  The other limits are the tables': one thread of the sort per window start
+// (1024 output positions, 32 x 32), the row list (1024 taps), the starts of a window (256 positions), 16-bit column numbers.
 bool conv_window_takes(const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t dense, int eh, int ew) {
   // (and finite weights: an infinite one times the zero of a reset row is NaN, and the rows left out count then)
   return cv->finite && cv->Wk != nullptr && cv->K * cv->Cout >= 2048 && Ho * Wo <= kSortBuckets && H * W * cv->Cin < (int64_t(1) << 31) && H < 32768 && W < 32768 &&
