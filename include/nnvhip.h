@@ -97,7 +97,7 @@ NNVHIP_API int nnvhip_set_eager_columns(nnvhip_ctx* ctx, int enabled);
 NNVHIP_API int nnvhip_set_eager_relu(nnvhip_ctx* ctx, int enabled);
 /* Measurement hook (no counterpart in the reference): while timing level 2 is set, every launch of a
  * kernel group is bracketed by its own pair of HIP events on the context's stream.  which = 0:
- * dense GEMM kernel of the FC layers (tiles of at least 64 rows); 1: implicit-GEMM convolution
+ * dense GEMM kernel of the FC layers (outputs of more than 32 rows); 1: implicit-GEMM convolution
  * kernel; 2: estimateRanges column pass; 3: ReLU apply pass; 4: row-wise affine layers (row map,
  * average pooling, row permutation); 5: column gather of an FC layer (its one-hot generator columns);
  * 6: classification of the ReLU step (incl. the sort of the crossing list and, for small sets,

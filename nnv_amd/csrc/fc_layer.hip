@@ -937,6 +937,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
             sg.kp = (int32_t)kps[i];
             sg.valid = (int32_t)std::min<int64_t>(tn, dense[i] - j);
             segs.push_back(sg);
+            rows.gathered = rows.gathered || (sg.kmap != nullptr && sg.Bk == nullptr);
           }
           if (!filled[i]) {
             rows.flop += 2.0 * (double)fc->Mp * (double)kps[i] * (double)dense[i];

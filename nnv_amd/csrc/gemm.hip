@@ -9,30 +9,380 @@
 #include <string>
 
 #include "internal.h"
+#include "lds_dma.h"
 #include "mfma_tile.h"
 
 namespace nnvhip {
 
-// TM x TN output tile per block of WR x WC waves, each wave owning
-// (TM/WR) x (TN/WC) = (16*FM) x (16*FN).
-// MAPPED = false: the plain product.  MAPPED = true additionally honours a row list (kmap), a per-tile
-// segment table (segs) and a column map (colmap); kept apart so that the plain kernel pays nothing.
-// WPE: waves per SIMD the register allocation is held to (1: whatever the code needs).
-template <int TM, int TN, int WR, int WC, int KT, bool MAPPED, int WPE = 1>
-__global__ __launch_bounds__(64 * WR * WC, WPE) void gemm_f64_kernel(const double* __restrict__ A, int64_t lda,
-                                                        const double* __restrict__ B, int64_t ldb,
-                                                        double* __restrict__ C, int64_t ldc, int Mp, int64_t ncols,
-                                                        int Kp, const double* __restrict__ bias, int tiles_m,
-                                                        int tiles_n, int xr, int local_m, int ksplit,
-                                                        double* __restrict__ part,
-                                                        const double* __restrict__ plb,
-                                                        const double* __restrict__ pub,
-                                                        double* __restrict__ rpart,
-                                                        const int32_t* __restrict__ kmap,
-                                                        const GemmSeg* __restrict__ segs,
-                                                        const int32_t* __restrict__ colmap,
-                                                        const int32_t* __restrict__ bmap,
-                                                        const double* __restrict__ Bk, int64_t ldbk) {
+// Where a block's tile lies and what it reads (both kernels below).
+struct GemmTile {
+  int m0;
+  int64_t nt, n0;
+  const int32_t* kmap;  // rows of B (= columns of A) the product goes over, -1 padded to whole stages; null: all
+  const double* Bk;     // those rows of B packed (row t = row kmap[t]), or null
+  int64_t ldbk, bk_col0;
+  int64_t col_base;     // column of B and C behind the tile's first column
+  int64_t col_end;      // first column past the valid ones, in the same numbering
+  int64_t b_col_base;   // column of B behind the tile's first column
+  // fused range sums: the tile's first column and the end of the valid ones in the numbering of plb / pub (the set's own
+  // columns), and the chunk of partial sums the tile fills
+  const double *plb, *pub;
+  double* rpart;
+  int64_t rcol0, rcol_end, rchunk;
+  int Kp;
+};
+struct GemmArgs {
+  const double* A;
+  const double* B;
+  double* C;
+  const double* bias;
+  double* part;  // split-K workspace
+  const double *plb, *pub;
+  double* rpart;
+  const int32_t* kmap;
+  const GemmSeg* segs;
+  const int32_t* colmap;
+  const int32_t* bmap;
+  const double* Bk;
+  int64_t lda, ldb, ldc, ldbk, ncols;
+  int32_t Mp, Kp, tiles_m, tiles_n, xr, local_m, ksplit;
+};
+
+// XCD-aware tile mapping.  Workgroups are dealt round-robin to the 8 XCDs (each with its own 4 MiB L2) by linear id, so
+// blockIdx.x % 8 names the XCD.  The XCDs form an xr x (8/xr) grid over the tile matrix: XCD (i, j) owns the row tiles
+// congruent to i mod xr and the column tiles congruent to j mod 8/xr, i.e. it touches 1/xr of W and xr/8 of V instead of
+// all of V.  Inside an XCD consecutive blocks walk down the row tiles of one column tile, keeping its V tile hot.
+template <int TM, int TN, bool MAPPED>
+__device__ __forceinline__ bool gemm_tile_of(const GemmArgs& g, GemmTile* t) {
+  const int xcd = blockIdx.x & 7;
+  const int slot = blockIdx.x >> 3;
+  const int xc = 8 / g.xr;
+  const int mt = (slot % g.local_m) * g.xr + (xcd % g.xr);
+  const int64_t nt = (int64_t)(slot / g.local_m) * xc + (xcd / g.xr);
+  if (mt >= g.tiles_m || nt >= g.tiles_n) return false;
+  t->m0 = mt * TM;
+  t->nt = nt;
+  t->n0 = nt * TN;
+  t->kmap = g.kmap;
+  t->Bk = g.Bk;
+  t->ldbk = g.ldbk;
+  t->bk_col0 = t->n0;
+  t->col_base = t->n0;
+  t->col_end = g.ncols;
+  t->b_col_base = t->n0;
+  t->plb = g.plb;
+  t->pub = g.pub;
+  t->rpart = g.rpart;
+  t->rcol0 = t->n0;
+  t->rcol_end = g.ncols;
+  t->rchunk = nt;
+  t->Kp = g.Kp;
+  if (MAPPED && g.segs != nullptr) {
+    const GemmSeg sg = g.segs[nt];
+    t->rpart = sg.rpart;
+    t->plb = sg.plb;
+    t->pub = sg.pub;
+    t->rcol0 = sg.col_local0;
+    t->rcol_end = sg.col_local0 + sg.valid;
+    t->rchunk = 0;
+    t->kmap = sg.kmap;
+    t->Kp = sg.kp;
+    t->col_base = sg.col_base;
+    t->col_end = sg.col_base + sg.valid;
+    t->b_col_base = sg.b_col_base;
+    t->Bk = sg.Bk;
+    t->ldbk = sg.ldbk;
+    t->bk_col0 = sg.col_local0;
+  }
+  return true;
+}
+
+// What both kernels do with a finished tile: the fused range sums, then the bias on column 0 and the stores.
+// pbs: LDS, the predicate bounds of the tile's columns ([2][TN], zero where there is none); red: WC * TM * 4 doubles of LDS
+// that nobody reads any more.
+template <int TM, int TN, int WR, int WC, bool MAPPED>
+__device__ __forceinline__ void gemm_finish(const GemmArgs& g, const GemmTile& t, double* red, const double (*pbs)[TN],
+                                            double4_t (&acc)[TM / WR / 16][TN / WC / 16]) {
+  constexpr int NT = 64 * WR * WC, FM = TM / WR / 16, FN = TN / WC / 16;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wr = wave % WR, wc = wave / WR;
+  const int lrow = lane & 15, lcol = lane >> 4;
+  double* C = g.C;
+  int64_t ldc = g.ldc;
+  const double* bias = g.bias;
+  if (g.ksplit > 1) {  // partial sums go to the workspace (ld = Mp); bias is added by the reduction
+    C = g.part + (int64_t)blockIdx.y * g.Mp * g.ncols;
+    ldc = g.Mp;
+    bias = nullptr;
+  }
+  // ---- fused estimateRanges: partial sums of this column tile ----------------------------------
+  // xmin1 = sum max(v,0)*plb, xmin2 = sum min(v,0)*pub, xmax1 = sum max(v,0)*pub, xmax2 = sum min(v,0)*plb
+  // over the tile's generator columns (column 0, the centre, is skipped), per output row.
+  if (t.rpart != nullptr) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int ct = wc * (TN / WC) + j * 16 + lcol + 4 * r;
+          const int64_t col = t.rcol0 + ct;
+          if (col >= 1 && col < t.rcol_end) {
+            const double v = acc[i][j][r];
+            const double pl = pbs[0][ct], pu = pbs[1][ct];
+            const double p = fmax(v, 0.0), q = fmin(v, 0.0);
+            s0 = fma(p, pl, s0);
+            s1 = fma(q, pu, s1);
+            s2 = fma(p, pu, s2);
+            s3 = fma(q, pl, s3);
+          }
+        }
+      }
+      // the four lane groups (lcol) hold different columns of the same rows
+      s0 += __shfl_xor(s0, 16);
+      s1 += __shfl_xor(s1, 16);
+      s2 += __shfl_xor(s2, 16);
+      s3 += __shfl_xor(s3, 16);
+      s0 += __shfl_xor(s0, 32);
+      s1 += __shfl_xor(s1, 32);
+      s2 += __shfl_xor(s2, 32);
+      s3 += __shfl_xor(s3, 32);
+      if (lcol == 0) {
+        double* dst = red + ((wc * TM) + wr * (TM / WR) + i * 16 + lrow) * 4;
+        dst[0] = s0;
+        dst[1] = s1;
+        dst[2] = s2;
+        dst[3] = s3;
+      }
+    }
+    __syncthreads();
+    for (int e = tid; e < TM * 4; e += NT) {  // waves along the columns are combined in order
+      const int row = e >> 2, q = e & 3;
+      double s = 0.0;
+#pragma unroll
+      for (int w = 0; w < WC; ++w) s += red[(w * TM + row) * 4 + q];
+      if (t.m0 + row < g.Mp) t.rpart[(t.rchunk * 4 + q) * ldc + t.m0 + row] = s;
+    }
+  }
+  // ---- epilogue: bias on column 0, 128-byte line stores --------------------------------------
+#pragma unroll
+  for (int i = 0; i < FM; ++i) {
+    const int row = t.m0 + wr * (TM / WR) + i * 16 + lrow;
+    if (row >= g.Mp) continue;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t ccol = t.col_base + wc * (TN / WC) + j * 16 + lcol + 4 * r;
+        if (ccol < t.col_end) {
+          double v = acc[i][j][r];
+          if (bias != nullptr && ccol == 0) v = v + bias[row];
+          // (partial products of a split go to the workspace column by column; the reduction maps them)
+          C[row + ((MAPPED && g.colmap != nullptr && g.ksplit == 1) ? (int64_t)g.colmap[ccol] : ccol) * ldc] = v;
+        }
+      }
+    }
+  }
+}
+
+// This thread's entry of the predicate bounds of the tile's columns (the lower ones of all columns, then the upper ones).
+template <int TN>
+__device__ __forceinline__ double gemm_pred_bound(const GemmTile& t, int tid) {
+  double v = 0.0;
+  if (t.rpart != nullptr && tid < 2 * TN) {
+    const int64_t col = t.rcol0 + tid % TN;
+    if (col >= 1 && col < t.rcol_end) v = (tid < TN ? t.plb : t.pub)[col - 1];
+  }
+  return v;
+}
+
+constexpr int kMapLds = 2048;  // entries of a row list that are copied into LDS
+__device__ double g_zero_rows[128];  // what a padding entry of a row list reads in place of a column of A (never written)
+
+// TM x TN output tile per block of WR x WC waves, each wave owning (TM/WR) x (TN/WC) = (16*FM) x (16*FN).
+//
+// What bounds it: fp64 MFMA, and where a CU has one tile or two the gaps between the products - every wave of a block
+// waits for the same stage, and what a wave does between its last product of one stage and its first of the next (the wait,
+// the barrier, the next transfers, address arithmetic, the first LDS reads) leaves the matrix cores idle.  So:
+//  - Both operands travel global -> LDS directly (global_load_lds_dwordx4, no staging registers), KT rows of B a stage, S
+//    stages in a ring; S - 1 of them are in flight while one is multiplied.
+//  - Every wave brings the same number of transfers of each operand (UA, UB), so the loop has no branch on who brings what,
+//    and a transfer's address is a scalar that advances plus a lane offset that does not.
+//  - The loop is unrolled over the ring: LDS addresses are lane constants plus immediate offsets.
+//  - Operands are read from LDS four rows ahead of the product they are for, over the end of a stage as well.
+// 1024 x 784 over 480 and 1920 rows: 30 and 91 us with the operands staged through registers one stage ahead, 18 and 59 us
+// now (32 x 64 tiles); 704 x 1501 over 1008 rows 74 -> 47 us; 2048 x 1024 over 1024 rows (64 x 64 tiles) 104 -> 64 us, 70 TFLOP/s at
+// 1920 rows, which is what the largest library product reaches here.
+//
+// A transfer (1 KB, a wave's 64 lanes x 16 bytes) of A holds whole rows k of the stage, lanes along the rows of W.  One of B
+// holds the KT rows of 128 / KT columns; LDS takes its pieces in lane order, so lanes fetch the 16-byte pieces of a column in
+// an order turned by the column's number, and the 16 lanes that read one row of 16 columns meet two to a bank pair instead
+// of 16 to one.  The ring stays inside the first 64 KB of LDS.
+//
+// MAPPED = false: the plain product.  MAPPED = true additionally honours a row list (kmap) with packed rows of B (Bk), a
+// per-tile segment table (segs) and a column map for C; kept apart so that the plain kernel pays nothing.
+constexpr int kMaxLdaDma = 1 << 24, kMaxLdbDma = 1 << 22;  // leading dimensions whose lane offsets fit 32 bits
+template <int TM, int TN, int WR, int WC, int KT, bool MAPPED>
+__global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
+  constexpr int NT = 64 * WR * WC, NW = WR * WC;
+  constexpr int FM = TM / WR / 16, FN = TN / WC / 16;
+  constexpr int kStage = KT * (TM + TN);
+  constexpr int S = 65536 / (8 * kStage) > 4 ? 4 : 65536 / (8 * kStage);
+  constexpr int UA = TM * KT / 128 / NW, UB = TN * KT / 128 / NW, U = UA + UB;
+  static_assert(KT == 16 || KT == 32, "stages of one or two groups of 16 rows");
+  static_assert(S >= 2 && UA >= 1 && UB >= 1 && UA * NW * 128 == TM * KT && UB * NW * 128 == TN * KT, "every wave brings the same share of a stage");
+  static_assert(WC * TM * 4 <= S * kStage && 2 * TN <= NT, "sums and bounds of the epilogue");
+  struct Lds {
+    double ring[S * kStage];
+    double pbs[2][TN];
+    int kmap[MAPPED ? kMapLds : 1];
+  };
+  __shared__ __attribute__((aligned(1024))) Lds sm;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  GemmTile t;
+  if (!gemm_tile_of<TM, TN, MAPPED>(g, &t)) return;
+  const double pb_reg = gemm_pred_bound<TN>(t, tid);
+  const bool mapped = MAPPED && t.kmap != nullptr;          // uniform over the block, like ...
+  const bool map_lds = mapped && t.Kp <= kMapLds;
+  if (map_lds) {
+    for (int k = tid; k < t.Kp; k += NT) sm.kmap[k] = t.kmap[k];
+    __syncthreads();
+  }
+  // split-K: block row blockIdx.y owns the rows [k0, k0 + 16 * n16) and writes a partial product
+  const int nk16 = t.Kp / 16;
+  const int k16 = (int)((int64_t)nk16 * blockIdx.y / g.ksplit);
+  const int n16 = (int)((int64_t)nk16 * (blockIdx.y + 1) / g.ksplit) - k16;
+  const int k0 = k16 * 16;
+  const bool half = KT == 32 && (n16 & 1);  // the last stage has 16 rows
+  const int nk = KT == 32 ? (n16 + 1) / 2 : n16;
+
+  // This wave's transfers of a stage: rows ka + u * kAStep of A, columns cb + u * kBStep of B.  Rows of W past the last and
+  // columns past the tile's end are read from its last rows and first column (such results are neither stored nor summed).
+  constexpr int kAStep = NW * 128 / TM, kBStep = NW * 128 / KT;
+  const int ka = wave * 128 / TM + lane / (TM / 2);
+  const int ra = min(t.m0 + 2 * (lane % (TM / 2)), g.Mp - 2);
+  const int cb = wave * 128 / KT + lane / (KT / 2);
+  const int piece = (lane & (KT / 2 - 1)) ^ (KT == 16 ? (cb >> 1) & 7 : cb & 7);  // (kBStep is a multiple of 16)
+  const bool packed = MAPPED && t.Bk != nullptr;
+  const int64_t ldb = packed ? t.ldbk : g.ldb;
+  const double* a_base = g.A + (mapped ? 0 : (int64_t)k0 * g.lda);
+  const double* b_base = (packed ? t.Bk + t.bk_col0 * ldb : g.B + t.b_col_base * ldb) + k0;
+  const unsigned a_off = (unsigned)((ra + (mapped ? 0 : (int64_t)ka * g.lda)) * 8);
+  unsigned b_col[UB];
+#pragma unroll
+  for (int u = 0; u < UB; ++u) b_col[u] = (unsigned)((t.col_base + cb + u * kBStep < t.col_end ? cb + u * kBStep : 0) * ldb * 8);
+  const unsigned lds0 = lds_addr_of(sm.ring) + wave * 1024;
+  // Stage st into place `slot` of the ring; stages are issued in order.  The rows a half stage does not have are read from
+  // its last one and not multiplied.
+  auto issue = [&](int st, int slot) {
+    const unsigned at = lds0 + slot * (kStage * 8);
+    const int rows = (KT == 32 && half && st == nk - 1) ? 16 : KT;
+    if (mapped) {
+#pragma unroll
+      for (int u = 0; u < UA; ++u) {
+        const int k = k0 + st * KT + min(ka + u * kAStep, rows - 1);
+        const int kk = map_lds ? sm.kmap[k] : t.kmap[k];
+        lds_dma16_at(kk >= 0 ? g.A + ra + (int64_t)kk * g.lda : g_zero_rows + 2 * lane, at + u * (NW * 1024));
+      }
+    } else if (rows == KT) {
+#pragma unroll
+      for (int u = 0; u < UA; ++u) lds_dma16(a_base + (int64_t)u * kAStep * g.lda, a_off, at + u * (NW * 1024));
+      a_base += KT * g.lda;
+    } else {
+#pragma unroll
+      for (int u = 0; u < UA; ++u)
+        lds_dma16(a_base, (unsigned)((ra + (int64_t)min(ka + u * kAStep, rows - 1) * g.lda) * 8), at + u * (NW * 1024));
+    }
+    const unsigned b_row = (unsigned)(rows == KT ? piece : min(piece, rows / 2 - 1)) * 16;
+#pragma unroll
+    for (int u = 0; u < UB; ++u) lds_dma16(b_base, b_col[u] + b_row, at + KT * TM * 8 + u * (NW * 1024));
+    b_base += KT;
+  };
+  double4_t acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int st = 0; st < S; ++st)
+    if (st < nk) issue(st, st);
+
+  const int wr = wave % WR, wc = wave / WR, l16 = lane & 15, q = lane >> 4;
+  const int px = (q >> 1) ^ (KT == 16 ? l16 >> 1 : l16 & 7);  // turns the piece that holds row q of a column
+  // this wave's transfers of a stage have landed (those of `ahead` later ones may be in flight) and its LDS reads are done
+  auto arrived = [&](int ahead) {
+    if (S > 3 && ahead == 3) wait_vm_lds<3 * U>();
+    else if (S > 2 && ahead == 2) wait_vm_lds<2 * U>();
+    else if (ahead == 1) wait_vm_lds<U>();
+    else wait_vm_lds<0>();
+  };
+  struct Frag {
+    double b[FM], a[FN];
+  };
+  const double* as = sm.ring + wr * (TM / WR) + l16 + q * TM;
+  const double* bs[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) bs[s] = sm.ring + KT * TM + (wc * (TN / WC) + l16) * KT + (q & 1) + 2 * ((2 * s) ^ px);
+  auto read = [&](int slot, int s, Frag& f) {  // rows 4 s .. 4 s + 3 of a stage
+#pragma unroll
+    for (int i = 0; i < FM; ++i) f.b[i] = as[slot * kStage + s * 4 * TM + i * 16];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) f.a[j] = bs[s & 3][slot * kStage + j * 16 * KT + (s >> 2) * 16];
+  };
+  auto multiply = [&](const Frag& f) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(f.a[j], f.b[i], acc[i][j], 0, 0, 0);
+  };
+  Frag f0, f1;
+  arrived(min(nk, S) - 1);
+  block_barrier();
+  read(0, 0, f0);
+  for (int st0 = 0; st0 < nk; st0 += S) {
+#pragma unroll
+    for (int slot = 0; slot < S; ++slot) {
+      const int st = st0 + slot;
+      if (st >= nk) break;
+      const bool last = st == nk - 1;
+#pragma unroll
+      for (int s = 0; s < KT / 4; s += 2) {  // (the reads stay in front of the products they overlap)
+        read(slot, s + 1, f1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(f0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (s + 2 == KT / 4 || (KT == 32 && s == 2 && half && last)) break;
+        read(slot, s + 2, f0);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(f1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (!last) {
+        arrived(min(nk - 2 - st, S - 2));
+        block_barrier();  // stage st + 1 is there, and nobody reads stage st any more: its place takes the next transfers
+        read((slot + 1) % S, 0, f0);
+        if (st + S < nk) issue(st + S, slot);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      multiply(f1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if (t.rpart != nullptr) {
+    if (tid < 2 * TN) sm.pbs[tid / TN][tid % TN] = pb_reg;
+    __syncthreads();  // everybody is done with the last stage; the bounds are in place
+  }
+  gemm_finish<TM, TN, WR, WC, MAPPED>(g, t, sm.ring, sm.pbs, acc);
+}
+
+// The same product where the rows of B are read through the row list (nobody packed them: products bound by their launch,
+// and outputs of few rows, where packing would cost more than it saves), where the columns of B are picked by a map, and for
+// matrices whose lane offsets do not fit 32 bits: 8-byte pieces and 64-bit addresses, through registers one stage ahead.
+// Arrays (segs) may mix such tiles with packed ones.
+template <int TM, int TN, int WR, int WC>
+__global__ __launch_bounds__(64 * WR * WC) void gemm_gather_kernel(GemmArgs g) {
+  constexpr int KT = 16;
   constexpr int NT = 64 * WR * WC;  // threads per block
   constexpr int FM = TM / WR / 16;
   constexpr int FN = TN / WC / 16;
@@ -46,55 +396,17 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void gemm_f64_kernel(const doubl
   const int wave = tid >> 6;
   const int wr = wave % WR;
   const int wc = wave / WR;
-  // XCD-aware tile mapping.  Workgroups are dealt round-robin to the 8 XCDs (each with its own
-  // 4 MiB L2) by linear id, so blockIdx.x % 8 names the XCD.  The XCDs form an xr x (8/xr) grid over
-  // the tile matrix: XCD (i, j) owns the row tiles congruent to i mod xr and the column tiles
-  // congruent to j mod 8/xr, i.e. it touches 1/xr of W and xr/8 of V instead of all of V.  Inside
-  // an XCD consecutive blocks walk down the row tiles of one column tile, keeping its V tile hot.
-  const int xcd = blockIdx.x & 7;
-  const int slot = blockIdx.x >> 3;
-  const int xc = 8 / xr;
-  const int mt = (slot % local_m) * xr + (xcd % xr);
-  const int64_t nt = (int64_t)(slot / local_m) * xc + (xcd / xr);
-  if (mt >= tiles_m || nt >= tiles_n) return;
-  const int m0 = mt * TM;
-  const int64_t n0 = nt * TN;
-  // Row-compacted contraction: kmap lists the rows of B (= columns of A) that can be non-zero, padded
-  // to whole K-tiles with -1; with a segment table every column tile has its own list (one per set).
-  int64_t col_base = n0;       // column of B and C behind the tile's first column
-  int64_t col_end = ncols;     // first column past the valid ones, in the same numbering as col_base
-  int64_t bk_col0 = n0;        // column of Bk behind the tile's first column
-  int64_t b_col_base = n0;     // column of B behind the tile's first column
-  // fused range sums: the tile's first column and the end of the valid ones in the numbering of plb / pub
-  // (the set's own columns), and the chunk of partial sums the tile fills
-  int64_t rcol0 = n0, rcol_end = ncols, rchunk = nt;
-  if (MAPPED && segs != nullptr) {
-    const GemmSeg sg = segs[nt];
-    rpart = sg.rpart;
-    plb = sg.plb;
-    pub = sg.pub;
-    rcol0 = sg.col_local0;
-    rcol_end = sg.col_local0 + sg.valid;
-    rchunk = 0;
-    kmap = sg.kmap;
-    Kp = sg.kp;
-    col_base = sg.col_base;
-    col_end = sg.col_base + sg.valid;
-    b_col_base = sg.b_col_base;
-    Bk = sg.Bk;
-    ldbk = sg.ldbk;
-    bk_col0 = sg.col_local0;
-  }
-  // Bk: the listed rows of B already packed into a matrix of their own (row t of Bk = row kmap[t] of B);
-  // only A is gathered then
-  const bool b_packed = MAPPED && Bk != nullptr;
+  GemmTile t;
+  if (!gemm_tile_of<TM, TN, true>(g, &t)) return;
+  const double pb_reg = gemm_pred_bound<TN>(t, tid);
+  const bool b_packed = t.Bk != nullptr;
   // The row list of this tile is copied into LDS first: the staging loads then take their row numbers
   // from there instead of through a dependent global load ahead of every operand load.
-  constexpr int kMapLds = 2048;
-  __shared__ int kmap_s[MAPPED ? kMapLds : 1];
-  const bool map_lds = MAPPED && kmap != nullptr && Kp <= kMapLds;  // uniform over the block
+  __shared__ int kmap_s[kMapLds];
+  __shared__ double pbs[2][TN];
+  const bool map_lds = t.kmap != nullptr && t.Kp <= kMapLds;  // uniform over the block
   if (map_lds) {
-    for (int k = tid; k < Kp; k += NT) kmap_s[k] = kmap[k];
+    for (int k = tid; k < t.Kp; k += NT) kmap_s[k] = t.kmap[k];
     __syncthreads();
   }
 
@@ -109,8 +421,8 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void gemm_f64_kernel(const doubl
 #pragma unroll
   for (int p = 0; p < B_PASS; ++p) {
     const int64_t jl = (tid + p * NT) / (KT / 2);
-    const int64_t col = col_base + jl;
-    bcol[p] = col < col_end ? ((MAPPED && bmap != nullptr) ? (int64_t)bmap[col] : b_col_base + jl) : -1;
+    const int64_t col = t.col_base + jl;
+    bcol[p] = col < t.col_end ? (g.bmap != nullptr ? (int64_t)g.bmap[col] : t.b_col_base + jl) : -1;
   }
 
   auto load_tiles = [&](int k0) {
@@ -119,11 +431,11 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void gemm_f64_kernel(const doubl
       int idx = tid + p * NT;
       int i2 = idx % (TM / 2);
       int k = idx / (TM / 2);
-      int row = m0 + 2 * i2;
+      int row = t.m0 + 2 * i2;
       double2 v = make_double2(0.0, 0.0);
-      if (idx < A_VEC && row < Mp) {
-        const int kk = (MAPPED && kmap != nullptr) ? (map_lds ? kmap_s[k0 + k] : kmap[k0 + k]) : k0 + k;
-        if (kk >= 0) v = *reinterpret_cast<const double2*>(A + row + (int64_t)kk * lda);
+      if (idx < A_VEC && row < g.Mp) {
+        const int kk = t.kmap != nullptr ? (map_lds ? kmap_s[k0 + k] : t.kmap[k0 + k]) : k0 + k;
+        if (kk >= 0) v = *reinterpret_cast<const double2*>(g.A + row + (int64_t)kk * g.lda);
       }
       ra[p] = v;
     }
@@ -135,14 +447,14 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void gemm_f64_kernel(const doubl
       double2 v = make_double2(0.0, 0.0);
       if (idx < B_VEC && bcol[p] >= 0) {
         if (b_packed) {
-          v = *reinterpret_cast<const double2*>(Bk + (k0 + 2 * k2) + (bk_col0 + j) * ldbk);
-        } else if (MAPPED && kmap != nullptr) {
-          const int ka = map_lds ? kmap_s[k0 + 2 * k2] : kmap[k0 + 2 * k2];
-          const int kb = map_lds ? kmap_s[k0 + 2 * k2 + 1] : kmap[k0 + 2 * k2 + 1];
-          if (ka >= 0) v.x = B[ka + bcol[p] * ldb];
-          if (kb >= 0) v.y = B[kb + bcol[p] * ldb];
+          v = *reinterpret_cast<const double2*>(t.Bk + (k0 + 2 * k2) + (t.bk_col0 + j) * t.ldbk);
+        } else if (t.kmap != nullptr) {
+          const int ka = map_lds ? kmap_s[k0 + 2 * k2] : t.kmap[k0 + 2 * k2];
+          const int kb = map_lds ? kmap_s[k0 + 2 * k2 + 1] : t.kmap[k0 + 2 * k2 + 1];
+          if (ka >= 0) v.x = g.B[ka + bcol[p] * g.ldb];
+          if (kb >= 0) v.y = g.B[kb + bcol[p] * g.ldb];
         } else {
-          v = *reinterpret_cast<const double2*>(B + (k0 + 2 * k2) + bcol[p] * ldb);
+          v = *reinterpret_cast<const double2*>(g.B + (k0 + 2 * k2) + bcol[p] * g.ldb);
         }
       }
       rb[p] = v;
@@ -175,102 +487,27 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void gemm_f64_kernel(const doubl
     for (int j = 0; j < FN; ++j) acc[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
 
   // split-K: block row blockIdx.y owns the K-tiles [kt0, kt1) and writes a partial product
-  const int nk_all = Kp / KT;
-  const int kt0 = (int)((int64_t)nk_all * blockIdx.y / ksplit);
-  const int kt1 = (int)((int64_t)nk_all * (blockIdx.y + 1) / ksplit);
+  const int nk_all = t.Kp / KT;
+  const int kt0 = (int)((int64_t)nk_all * blockIdx.y / g.ksplit);
+  const int kt1 = (int)((int64_t)nk_all * (blockIdx.y + 1) / g.ksplit);
   // two LDS stages: tile t+1 travels global -> registers while tile t is multiplied, then goes to the
-  // other stage; one barrier per K-tile.  (A three-stage variant with the barrier hidden behind the
-  // first MFMA step measured no faster: the limit is the per-wave MFMA issue cadence, not the barrier.)
+  // other stage; one barrier per K-tile
   const int nk = kt1 - kt0;
   load_tiles(kt0 * KT);
   store_tiles(0);
   __syncthreads();
-  for (int t = 0; t < nk; ++t) {
-    const int cur = t & 1;
-    if (t + 1 < nk) load_tiles((kt0 + t + 1) * KT);
+  for (int st = 0; st < nk; ++st) {
+    const int cur = st & 1;
+    if (st + 1 < nk) load_tiles((kt0 + st + 1) * KT);
     mfma_tile_k16<FM, FN, KT>(&Ws[cur][wr * (TM / WR)], LDA_S, &Vs[cur][(wc * (TN / WC)) * LDB_S], LDB_S, lane, acc);
-    if (t + 1 < nk) store_tiles(cur ^ 1);
+    if (st + 1 < nk) store_tiles(cur ^ 1);
     __syncthreads();
   }
-  if (ksplit > 1) {  // partial sums go to the workspace (ld = Mp); bias is added by the reduction
-    C = part + (int64_t)blockIdx.y * Mp * ncols;
-    ldc = Mp;
-    bias = nullptr;
-  }
-
-  const int lrow = lane & 15;
-  const int lcol = lane >> 4;
-  // ---- fused estimateRanges: partial sums of this column tile ----------------------------------
-  // xmin1 = sum max(v,0)*plb, xmin2 = sum min(v,0)*pub, xmax1 = sum max(v,0)*pub, xmax2 = sum min(v,0)*plb
-  // over the tile's generator columns (column 0, the centre, is skipped), per output row.
-  if (rpart != nullptr) {
-    double* red = &Ws[0][0];  // the K loop is over (last barrier passed): reuse the W stage
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int64_t col = rcol0 + wc * (TN / WC) + j * 16 + lcol + 4 * r;
-          if (col >= 1 && col < rcol_end) {
-            const double v = acc[i][j][r];
-            const double pl = plb[col - 1], pu = pub[col - 1];
-            const double p = fmax(v, 0.0), q = fmin(v, 0.0);
-            s0 = fma(p, pl, s0);
-            s1 = fma(q, pu, s1);
-            s2 = fma(p, pu, s2);
-            s3 = fma(q, pl, s3);
-          }
-        }
-      }
-      // the four lane groups (lcol) hold different columns of the same rows
-      s0 += __shfl_xor(s0, 16);
-      s1 += __shfl_xor(s1, 16);
-      s2 += __shfl_xor(s2, 16);
-      s3 += __shfl_xor(s3, 16);
-      s0 += __shfl_xor(s0, 32);
-      s1 += __shfl_xor(s1, 32);
-      s2 += __shfl_xor(s2, 32);
-      s3 += __shfl_xor(s3, 32);
-      if (lcol == 0) {
-        double* dst = red + ((wc * TM) + wr * (TM / WR) + i * 16 + lrow) * 4;
-        dst[0] = s0;
-        dst[1] = s1;
-        dst[2] = s2;
-        dst[3] = s3;
-      }
-    }
+  if (t.rpart != nullptr) {
+    if (tid < 2 * TN) pbs[tid / TN][tid % TN] = pb_reg;
     __syncthreads();
-    for (int t = tid; t < TM * 4; t += NT) {  // waves along the columns are combined in order
-      const int row = t >> 2, q = t & 3;
-      double s = 0.0;
-#pragma unroll
-      for (int w = 0; w < WC; ++w) s += red[(w * TM + row) * 4 + q];
-      if (m0 + row < Mp) rpart[(rchunk * 4 + q) * ldc + m0 + row] = s;
-    }
   }
-
-  // ---- epilogue: bias on column 0, 128-byte line stores --------------------------------------
-#pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    int row = m0 + wr * (TM / WR) + i * 16 + lrow;
-    if (row >= Mp) continue;
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        int64_t col = n0 + wc * (TN / WC) + j * 16 + lcol + 4 * r;
-        const int64_t ccol = col_base + (col - n0);
-        if (ccol < col_end) {
-          double v = acc[i][j][r];
-          if (bias != nullptr && ccol == 0) v = v + bias[row];
-          // (partial products of a split go to the workspace column by column; the reduction maps them)
-          C[row + ((MAPPED && colmap != nullptr && ksplit == 1) ? (int64_t)colmap[ccol] : ccol) * ldc] = v;
-        }
-      }
-    }
-  }
+  gemm_finish<TM, TN, WR, WC, true>(g, t, &Ws[0][0], pbs, acc);
 }
 
 // colmap (or null): column t of the partial products belongs at column colmap[t] of C.
@@ -296,7 +533,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const double* __rest
   C[row + (colmap != nullptr ? (int64_t)colmap[col] : col) * ldc] = s;
 }
 
-template <int TM, int TN, int WR, int WC, int KT>
+template <int TM, int TN, int WR, int WC, int KT, bool GATHER = false>
 static int launch_cfg(nnvhip_ctx* ctx, const double* A, int64_t lda, const double* B, int64_t ldb, double* C,
                       int64_t ldc, int64_t Mp, int64_t ncols, int64_t Kp, const double* bias, RangeFuse* fuse,
                       const GemmRows* rows, SplitKDefer* defer) {
@@ -328,7 +565,7 @@ static int launch_cfg(nnvhip_ctx* ctx, const double* A, int64_t lda, const doubl
   const int64_t grid_x = 8 * best_slots;
   // Split-K when the output has too few tiles to occupy the chip: partial products into a workspace,
   // summed in split order by a second kernel (deterministic, no floating-point atomics).
-  const int64_t nk = Kp / KT;
+  const int64_t nk = Kp / 16;
   int64_t ksplit = 1;
   if (blocks < 128 && nk >= 8) ksplit = std::min<int64_t>(std::min<int64_t>(16, nk / 4), ceil_div(512, blocks));
   if (const int v = tune_knobs().gemm_ksplit) ksplit = std::max<int64_t>(1, std::min<int64_t>(v, nk));
@@ -346,26 +583,43 @@ static int launch_cfg(nnvhip_ctx* ctx, const double* A, int64_t lda, const doubl
     fuse->chunks = tiles_n;
     rpart = fuse->part->as<double>();
   }
-  const bool timed = ctx->kernel_timing && TM >= 64;
+  const bool timed = ctx->kernel_timing && Mp > 32;
   NNV_TRY(ctx->kernel_timer_begin(timed));
+  GemmArgs g{};
+  g.A = A;
+  g.B = B;
+  g.C = C;
+  g.bias = bias;
+  g.part = ws ? ws->as<double>() : nullptr;
+  g.plb = fuse ? fuse->plb : nullptr;
+  g.pub = fuse ? fuse->pub : nullptr;
+  g.rpart = rpart;
+  g.lda = lda;
+  g.ldb = ldb;
+  g.ldc = ldc;
+  g.ncols = ncols;
+  g.Mp = (int32_t)Mp;
+  g.Kp = (int32_t)Kp;
+  g.tiles_m = (int32_t)tiles_m;
+  g.tiles_n = (int32_t)tiles_n;
+  g.xr = (int32_t)best_xr;
+  g.local_m = (int32_t)local_m;
+  g.ksplit = (int32_t)ksplit;
+  const dim3 grid((unsigned)grid_x, (unsigned)ksplit), block(64 * WR * WC);
   if (rows != nullptr) {
-    // The mapped 128 x 128 tile needs a few registers more than let two blocks share a CU.  With a short
-    // contraction (few kept rows) the start and the end of a tile weigh as much as its K loop, and a
-    // second resident block hides them: for launches of many such tiles the allocation is held to 128
-    // registers (at the price of a few reloads per K-tile; measured: 12% quicker at K = 240 over
-    // 57344 tiles, 8% slower over 460 tiles, where two rounds of one block per CU do as well).
-    auto kern = gemm_f64_kernel<TM, TN, WR, WC, KT, true>;
-    if (TM == 128 && TN == 128 && Kp <= 512 && blocks >= 2048) kern = gemm_f64_kernel<TM, TN, WR, WC, KT, true, (TM == 128 && TN == 128 ? 4 : 1)>;
-    NNV_LAUNCH(ctx, timed, kern, dim3((unsigned)grid_x, (unsigned)ksplit),
-                       dim3(64 * WR * WC), 0, A, lda, B, ldb, C, ldc, (int)Mp, ncols, (int)Kp, bias, (int)tiles_m,
-                       (int)tiles_n, (int)best_xr, (int)local_m, (int)ksplit, ws ? ws->as<double>() : nullptr,
-                       fuse ? fuse->plb : nullptr, fuse ? fuse->pub : nullptr, rpart, rows->kmap, rows->segs, rows->colmap,
-                       rows->b_plain ? nullptr : rows->colmap, rows->Bk, rows->ldbk);
-  } else
-    NNV_LAUNCH(ctx, timed, (gemm_f64_kernel<TM, TN, WR, WC, KT, false>), dim3((unsigned)grid_x, (unsigned)ksplit),
-                       dim3(64 * WR * WC), 0, A, lda, B, ldb, C, ldc, (int)Mp, ncols, (int)Kp, bias, (int)tiles_m,
-                       (int)tiles_n, (int)best_xr, (int)local_m, (int)ksplit, ws ? ws->as<double>() : nullptr,
-                       fuse ? fuse->plb : nullptr, fuse ? fuse->pub : nullptr, rpart, nullptr, nullptr, nullptr, nullptr, nullptr, 0);
+    g.kmap = rows->kmap;
+    g.segs = rows->segs;
+    g.colmap = rows->colmap;
+    g.bmap = rows->b_plain ? nullptr : rows->colmap;
+    g.Bk = rows->Bk;
+    g.ldbk = rows->ldbk;
+  }
+  if constexpr (GATHER)
+    NNV_LAUNCH(ctx, timed, (gemm_gather_kernel<TM, TN, WR, WC>), grid, block, 0, g);
+  else if (rows != nullptr)
+    NNV_LAUNCH(ctx, timed, (gemm_f64_kernel<TM, TN, WR, WC, KT, true>), grid, block, 0, g);
+  else
+    NNV_LAUNCH(ctx, timed, (gemm_f64_kernel<TM, TN, WR, WC, KT, false>), grid, block, 0, g);
   NNV_TRY(ctx->kernel_timer_end(timed, 0, rows && rows->flop > 0.0 ? rows->flop : 2.0 * (double)Mp * (double)Kp * (double)ncols));
   if (defer != nullptr) {
     defer->ws = ws;
@@ -379,11 +633,10 @@ static int launch_cfg(nnvhip_ctx* ctx, const double* A, int64_t lda, const doubl
   return NNVHIP_OK;
 }
 
-// Tile width of a segmented launch: 128 x 128 tiles when there are enough of them to cover the chip,
-// 64 x 64 for small arrays (and the 16-row tile for skinny outputs).
+// Tile width of a segmented launch: 128 columns when there are enough tiles to cover the chip, 64 for small arrays and
+// outputs of few rows.
 int gemm_seg_cols(int64_t Mp, int64_t count, const int64_t* cols) {
-  if (Mp <= 16) return 64;   // the 16 x 64 tile
-  if (Mp <= 32) return 128;  // the 32 x 128 tile
+  if (Mp <= 32) return 64;
   int64_t tiles = 0;
   for (int64_t i = 0; i < count; ++i) tiles += ceil_div(cols[i], 128);
   return tiles * ceil_div(Mp, 128) < 256 ? 64 : 128;
@@ -396,52 +649,54 @@ int launch_gemm(nnvhip_ctx* ctx, const double* A, int64_t lda, const double* B, 
     NNV_FAIL(NNVHIP_ERR_SHAPE, "internal: GEMM operands violate the padding contract");
   if (Mp >= (int64_t(1) << 31) || Kp >= (int64_t(1) << 31)) NNV_FAIL(NNVHIP_ERR_SHAPE, "matrix too large");
   if (ncols == 0) return NNVHIP_OK;
-  // Tile choice: the largest tile that still yields a few blocks per CU; skinny outputs (the last
-  // layer has 10 rows) get a 16-row tile.  K must be a multiple of the K-tile (16 or 32).
-#define NNV_GEMM(TM, TN, WR, WC, KT) \
-  launch_cfg<TM, TN, WR, WC, KT>(ctx, A, lda, B, ldb, C, ldc, Mp, ncols, Kp, bias, fuse, rows, defer)
+#define NNV_GEMM(TM, TN, WR, WC, KT) launch_cfg<TM, TN, WR, WC, KT>(ctx, A, lda, B, ldb, C, ldc, Mp, ncols, Kp, bias, fuse, rows, defer)
+#define NNV_GEMM_GATHER(TM, TN, WR, WC) \
+  launch_cfg<TM, TN, WR, WC, 16, true>(ctx, A, lda, B, ldb, C, ldc, Mp, ncols, Kp, bias, fuse, rows, defer)
   const int64_t kCUs = 256;
-  if (Mp <= 16) return NNV_GEMM(16, 64, 1, 4, 16);
-  if (Mp <= 32) return NNV_GEMM(32, 128, 1, 4, 16);
-  // Eight-wave tiles (two waves per SIMD issue MFMAs even with one block per CU).  The shape is
-  // fitted to the problem: all tiles of a launch are resident at once and share the MFMA pipes, so
-  // the time goes with ceil(tiles / CUs) * tile area / (measured rate of the shape).  Small outputs
-  // thus get the shape that covers the chip in one round (e.g. 128x80 for 1024 x 2376: 240 tiles).
+  const bool wide_seg = rows != nullptr && rows->segs != nullptr && rows->seg_cols != 64;
+  bool gather = lda >= kMaxLdaDma || ldb >= kMaxLdbDma;
+  if (rows != nullptr)
+    gather = gather || rows->gathered || (rows->segs == nullptr && rows->kmap != nullptr && rows->Bk == nullptr) ||
+             (rows->colmap != nullptr && !rows->b_plain);
+  if (gather) {
+    if (Mp <= 16) return NNV_GEMM_GATHER(16, 64, 1, 4);
+    if (wide_seg || (Mp > 32 && (rows == nullptr || rows->segs == nullptr) && ceil_div(Mp, 64) * ceil_div(ncols, 64) > 4 * kCUs))
+      return NNV_GEMM_GATHER(128, 128, 2, 4);
+    return NNV_GEMM_GATHER(64, 64, 2, 4);
+  }
+  if (Mp <= 16) return NNV_GEMM(16, 64, 1, 4, 32);
+  if (wide_seg) return NNV_GEMM(64, 128, 2, 4, 16);
+  if (rows != nullptr && rows->segs != nullptr) return Mp <= 32 ? NNV_GEMM(32, 64, 2, 4, 32) : NNV_GEMM(64, 64, 4, 2, 32);
+  // The tiles of a launch are dealt evenly to the CUs and those of a CU share its matrix cores, so the time goes with
+  // ceil(tiles / CUs) * tile area / rate.  The rates are those of a 2048 x 1024 x 1920 product; a CU with a single 64 x 64
+  // tile has nothing to fill the gaps between its stages with.  Measured (1920 rows, in this order): 1024 x 784 63.6, 59.1,
+  // 69.0 us; 704 x 1501 113, 85.5, 84.6; 512 x 500 60, 32.5, 21.9; 1024 x 3000 169.5, 168.3, 197.9.  (With operands that are
+  // not in the caches yet the smallest tile, which reads them most often, falls behind: its rate is set for that.)
   struct Shape {
     int tm, tn;
-    double rate;  // TFLOP/s measured on a 1024 x 1024 x 16384 product
+    double rate, rate_alone;  // TFLOP/s
   };
-  static const Shape shapes[] = {{64, 64, 47.0},  {64, 96, 47.8},   {64, 128, 49.6},  {128, 48, 46.8},
-                                 {128, 64, 49.9}, {128, 80, 48.0},  {128, 96, 47.3},  {128, 112, 47.6},
-                                 {128, 128, 54.0}};
+  static const Shape shapes[] = {{64, 64, 70.0, 64.0}, {32, 64, 67.0, 64.0}, {32, 32, 52.0, 45.0}};
   int best = 0;
   double best_cost = 0.0;
   for (int i = 0; i < (int)(sizeof(shapes) / sizeof(shapes[0])); ++i) {
     const int64_t tiles = ceil_div(Mp, shapes[i].tm) * ceil_div(ncols, shapes[i].tn);
-    const double cost = (double)ceil_div(tiles, kCUs) * shapes[i].tm * shapes[i].tn / shapes[i].rate;
+    const double cost = (double)ceil_div(tiles, kCUs) * shapes[i].tm * shapes[i].tn / (tiles <= kCUs ? shapes[i].rate_alone : shapes[i].rate);
     if (i == 0 || cost < best_cost * 0.999) {
       best = i;
       best_cost = cost;
     }
   }
-  if (rows != nullptr && rows->segs != nullptr)  // the table was cut for this width: see gemm_seg_cols
-    return rows->seg_cols == 64 ? NNV_GEMM(64, 64, 2, 4, 16) : NNV_GEMM(128, 128, 2, 4, 16);
-  if (rows != nullptr && rows->tile_hint == 64 && tune_knobs().gemm_tile.empty()) return NNV_GEMM(64, 64, 2, 4, 16);
   if (!tune_knobs().gemm_tile.empty()) {  // tuning knob: "TMxTN" of one of the shapes above
     for (int i = 0; i < (int)(sizeof(shapes) / sizeof(shapes[0])); ++i)
       if (std::to_string(shapes[i].tm) + "x" + std::to_string(shapes[i].tn) == tune_knobs().gemm_tile) best = i;
   }
-  switch (shapes[best].tm * 1000 + shapes[best].tn) {
-    case 64064: return NNV_GEMM(64, 64, 2, 4, 16);
-    case 64096: return NNV_GEMM(64, 96, 4, 2, 16);
-    case 64128: return NNV_GEMM(64, 128, 4, 2, 16);
-    case 128048: return NNV_GEMM(128, 48, 8, 1, 16);
-    case 128064: return NNV_GEMM(128, 64, 4, 2, 16);
-    case 128080: return NNV_GEMM(128, 80, 8, 1, 16);
-    case 128096: return NNV_GEMM(128, 96, 8, 1, 16);
-    case 128112: return NNV_GEMM(128, 112, 8, 1, 16);
-    default: return NNV_GEMM(128, 128, 2, 4, 16);
+  switch (best) {
+    case 0: return NNV_GEMM(64, 64, 4, 2, 32);
+    case 1: return NNV_GEMM(32, 64, 2, 4, 32);
+    default: return NNV_GEMM(32, 32, 2, 2, 32);
   }
+#undef NNV_GEMM_GATHER
 #undef NNV_GEMM
 }
 

@@ -410,7 +410,7 @@ struct nnvhip_ctx {
   // timing of the dominant kernel alone (events directly around its launch), per instantiation group
   hipEvent_t kev0 = nullptr, kev1 = nullptr;
   hipEvent_t read_ev = nullptr;  // marks a read-back in the stream whose arrival the host waits for while later work runs
-  // [0] dense MFMA GEMM (tiles of at least 64 rows), [1] implicit-GEMM convolution (work = flop),
+  // [0] dense MFMA GEMM (outputs of more than 32 rows), [1] implicit-GEMM convolution (work = flop),
   // [2] estimateRanges column pass, [3] ReLU apply pass, [4] row-wise affine layers (batch
   // normalisation, input normalisation, average pooling, flatten), [5] gather of W's columns for the
   // one-hot generator columns of an FC layer (work = algorithmic bytes)
@@ -663,11 +663,8 @@ struct GemmRows {
   const int32_t* colmap = nullptr;
   bool b_plain = false;
   int32_t seg_cols = 128;
+  bool gathered = false;  // some tile of segs has a row list and no packed rows
   double flop = 0.0;  // flop actually executed (for the kernel timers)
-  // 64: take the 64 x 64 tile whatever the shape model says (short products of a few hundred tiles, whose blocks
-  // then sit two or more to a CU and cover each other's start and end: 2048 x 1024 x 1024 runs in 105 us on it,
-  // 141 us on the 128 x 64 tile the model picks)
-  int32_t tile_hint = 0;
 };
 int gemm_seg_cols(int64_t Mp, int64_t count, const int64_t* cols);
 // Vk(t, j) = V(kept[t], j) for t < kp (a multiple of 16; zero where kept[t] < 0), j < ncols; Vk has

@@ -14,6 +14,10 @@ __device__ __forceinline__ void lds_dma16(const double* gbase, unsigned voff, un
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(voff), "s"(gbase)
                : "memory", "m0");
 }
+// The same with every lane's own 64-bit address.
+__device__ __forceinline__ void lds_dma16_at(const double* src, unsigned lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr), "v"(src) : "memory", "m0");
+}
 __device__ __forceinline__ unsigned lds_addr_of(const void* p) {
   return (unsigned)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
@@ -26,6 +30,12 @@ template <int N>
 __device__ __forceinline__ void wait_vm() {
   // vmcnt <= N and nothing else (gfx9 encoding: vmcnt in bits [3:0] and [15:14], expcnt [6:4], lgkmcnt [11:8])
   __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | (0x7 << 4) | (0xf << 8));
+}
+
+// vmcnt <= N and no LDS access of this wave outstanding.
+template <int N>
+__device__ __forceinline__ void wait_vm_lds() {
+  __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | (0x7 << 4));
 }
 
 }  // namespace nnvhip

@@ -1044,8 +1044,8 @@ static int range_sums_upper_half(nnvhip_ctx* ctx, const nnvhip_fc* fc, int64_t n
   NNV_TRY(ctx->upload_table(odd.data(), sizeof(int32_t) * odd.size(), &cmap));
   GemmRows rows;
   rows.colmap = cmap->as<int32_t>();
-  if (Kp <= 2048) rows.tile_hint = 64;
-  return launch_gemm(ctx, fc->Wpn->as<double>(), 2 * Mp, X->as<double>(), Kp, (*out)->as<double>(), 2 * Mp, 2 * Mp, nu, Kp, nullptr,
+  rows.b_plain = true;  // (the odd columns of X are a matrix of leading dimension 2 * Kp)
+  return launch_gemm(ctx, fc->Wpn->as<double>(), 2 * Mp, X->as<double>() + Kp, 2 * Kp, (*out)->as<double>(), 2 * Mp, 2 * Mp, nu, Kp, nullptr,
                      nullptr, &rows);
 }
 
