@@ -180,6 +180,136 @@ __global__ __launch_bounds__(1024) void relu_classify_kernel(const ReluDesc* __r
   }
 }
 
+// The same step for a few sets of at most kClassifyRankN neurons each, by several blocks per set that need nothing from one
+// another: every block classifies the whole set and lists the crossing neurons' keys in its LDS - the loads are in flight
+// together, so that costs what one block's share would - and writes its share of the rows' outputs; then it finds the places
+// of kRankI crossing neurons at a time by counting the entries in front of them.  Bound by latency: a launch, the ranges'
+// trip from memory, three barriers.  The sorting network of the one-block kernel is a chain of 55 exchanges, ten of them
+// through LDS behind barriers.  1024 neurons, nearly all of them crossing: 11.2 -> 6.4 us; 700 neurons 7.6 -> 5.6.
+// Keys are compared through their bit patterns, as the network does.  Grid: (blocks of a set, sets).
+constexpr int kClassifyRankN = 2048;
+constexpr int kRankI = 16;
+// Blocks of a launch: one to a CU.  A set that gets fewer than eight of them (or than it has use for) goes to the one-block
+// kernel: 100 sets of 1024 neurons take 12 - 15 us there, 25 - 60 us here with ten blocks each.
+constexpr int kClassifyRankBlocks = 256;
+__global__ __launch_bounds__(1024) void relu_classify_rank_kernel(const ReluDesc* __restrict__ table, ReluDesc one) {
+  const ReluDesc d = table ? table[blockIdx.y] : one;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  __shared__ long long skey[kClassifyRankN];
+  __shared__ double slb[kClassifyRankN], sub[kClassifyRankN];
+  __shared__ int sidx[kClassifyRankN];
+  __shared__ int4 wcnt[8];  // per 64 rows: crossing | inactive << 16
+  __shared__ int part[16][kRankI];
+  double l[2], u[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = h * 1024 + tid;
+    l[h] = r < d.N ? d.lb[r] : 0.0;
+    u[h] = r < d.N ? d.ub[r] : 1.0;
+  }
+  const int n_in = d.ncols_in - 1;
+  if (d.write_bounds && d.plb_out != d.plb_in) {  // new_pred_lb = [plb; ...], new_pred_ub = [pub; ...]
+    for (int j = blockIdx.x * 1024 + tid; j < n_in; j += gridDim.x * 1024) {
+      d.plb_out[j] = d.plb_in[j];
+      d.pub_out[j] = d.pub_in[j];
+    }
+  }
+  unsigned long long bc[2], bi[2];
+  bool crossing[2], inactive[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const bool valid = h * 1024 + tid < d.N;
+    inactive[h] = valid && (u[h] <= 0.0);                 // map1 = find(ub <= 0)
+    crossing[h] = valid && (l[h] < 0.0) && (u[h] > 0.0);  // map2 = find(lb < 0 & ub > 0)
+    bc[h] = __ballot(crossing[h]);
+    bi[h] = __ballot(inactive[h]);
+    if (lane == 0) reinterpret_cast<int*>(wcnt)[16 * h + wave] = __popcll(bc[h]) | (__popcll(bi[h]) << 16);
+  }
+  __syncthreads();
+  int before[2] = {0, 0}, all = 0;  // both counts stay packed: no sum passes 2^15
+#pragma unroll
+  for (int g = 0; g < 8; ++g) {
+    const int4 c4 = wcnt[g];
+    const int c[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) before[h] += 4 * g + v < 16 * h + wave ? c[v] : 0;
+      all += c[v];
+    }
+  }
+  const int m = all & 0xffff, inact = all >> 16;
+  if (blockIdx.x == 0 && tid == 0) {
+    d.counts[0] = m;
+    d.counts[1] = inact;
+    post_counts(d.mailbox, m, inact, d.mailbox_seq);  // the host can size the output while we sort
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = h * 1024 + tid, group = 16 * h + wave;
+    const bool valid = r < d.N;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    const int pos = (before[h] & 0xffff) + __popcll(bc[h] & below);
+    if (crossing[h]) {
+      // areas = 0.5*(abs(ub).*abs(lb))  |  ub - lb
+      const double key = d.order == NNVHIP_ORDER_AREA ? 0.5 * (fabs(u[h]) * fabs(l[h]))
+                         : d.order == NNVHIP_ORDER_RANGE ? u[h] - l[h] : d.given_key[r];
+      skey[pos] = __double_as_longlong(key);
+      sidx[pos] = r;
+      slb[pos] = l[h];
+      sub[pos] = u[h];
+    }
+    if (group % (int)gridDim.x != (int)blockIdx.x) continue;  // another block writes these rows' outputs
+    const unsigned long long bv = __ballot(valid);
+    const unsigned long long bk = bv & ~bc[h] & ~bi[h];
+    if (d.keep_bits != nullptr && lane == 0 && h * 1024 < d.N)
+      *reinterpret_cast<uint2*>(d.keep_bits + 2 * group) = make_uint2((uint32_t)bk, (uint32_t)(bk >> 32));
+    if (r < d.ld) d.cls[r] = crossing[h] ? pos : inactive[h] ? kZero : kKeep;  // (padding rows stay zero)
+    if (valid && !crossing[h] && d.col_of != nullptr) d.col_of[r] = -1;
+    // rows in front of the group that are kept: those that are neither crossing nor inactive
+    if (bk >> lane & 1) d.keep_idx[64 * group - (before[h] & 0xffff) - (before[h] >> 16) + __popcll(bk & below)] = r;
+  }
+  if (blockIdx.x == 0)
+    for (int64_t r = kClassifyRankN + tid; r < d.ld; r += 1024) d.cls[r] = kKeep;
+  if (blockIdx.x == 0 && tid < 2 * (int)kLdAlign) {  // -1 up to the next multiple of 16 past the list (at least 16 entries in all)
+    const int nk = d.N - m - inact;
+    const int end = max((nk + (int)kLdAlign - 1) / (int)kLdAlign * (int)kLdAlign, (int)kLdAlign);
+    if (nk + tid < end) d.keep_idx[nk + tid] = -1;
+  }
+  const int il = tid & (kRankI - 1), slice = tid / kRankI;
+  for (int i0 = blockIdx.x * kRankI; i0 < m; i0 += gridDim.x * kRankI) {
+    __syncthreads();  // the list is complete; nobody reads the last round's counts any more
+    const int i = i0 + il;
+    const long long ki = i < m ? skey[i] : 0;
+    int cnt = 0;
+#pragma unroll 4
+    for (int j = slice; j < m; j += 1024 / kRankI) {
+      const long long kj = skey[j];
+      cnt += (kj > ki || (kj == ki && j < i)) ? 1 : 0;
+    }
+    cnt += __shfl_xor(cnt, 16);
+    cnt += __shfl_xor(cnt, 32);
+    if (lane < kRankI) part[wave][il] = cnt;
+    __syncthreads();
+    if (tid < kRankI && i < m) {
+      int r = 0;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) r += part[q][il];
+      const int neuron = sidx[i];
+      d.cross_idx[r] = neuron;
+      if (d.col_of != nullptr) d.col_of[neuron] = r;
+      if (d.write_bounds) {  // new_pred_lb = [plb; zeros(m,1)], new_pred_ub = [pub; ub(index)]
+        d.plb_out[n_in + r] = 0.0;
+        d.pub_out[n_in + r] = sub[i];
+        d.lbub[r] = slb[i];
+        d.lbub[d.ld_lbub + r] = sub[i];
+      }
+    }
+  }
+}
+
 // What the kernels that settle the order of a crossing list write besides the list: kRankNewBounds: the bounds
 // of the new predicates (new_pred_lb = [plb; zeros(m,1)], new_pred_ub = [pub; ub(index)]) and the crossing
 // neurons' (lb, ub); kRankOldBounds: also the copy of the bounds of the predicates the set already has.
@@ -335,51 +465,93 @@ __global__ __launch_bounds__(1024) void relu_compact_kernel(const ReluDesc* __re
 
 // Stable descending sort by counting: rank(i) = #{j : key_j > key_i or (key_j == key_i and j < i)}.
 // j < i in the ascending list is "smaller neuron index", which is what MATLAB's stable sort keeps.
-// A block owns kRankI entries of the list and compares them with the whole list, staged through LDS in pieces of
-// kRankStage keys: thread (entry, slice) counts over every 16th key, the 16 slices of an entry are then added.
+// A block owns kRankEntries entries of the list and compares them with the whole list, staged through LDS in pieces.  A thread
+// holds four entries and reads the keys two at a time, so that an LDS read serves eight comparisons of two instructions each:
+// entries in front of the block's own count where they are larger or equal, those behind where they are larger, and only the
+// step that holds the block's own entries looks at their order.  One network's layers of 32 768, 7 200, 14 400 and 3 136 neurons:
+// 9.2, 6.2, 17.6 and 14.6 us with one entry to a thread and a read to a comparison, 6.4, 4.8, 7.5 and 6.3 us now.
 // No block needs anything from another one (the XCDs of this chip share no cache, so counters and atomics
 // between blocks are the expensive part of a tiled count), and a block knows the final places of its entries:
 // it puts their neurons there and, with kRankNewBounds, writes what the new predicates need (new_pred_lb =
 // [plb; zeros(m,1)], new_pred_ub = [pub; ub(index)], and the crossing neurons' (lb, ub)).  kRankOldBounds: the
 // blocks also share out the copy of the bounds of the predicates the set already has.
-constexpr int kRankI = 16;
-constexpr int kRankStage = 2048;
-__global__ __launch_bounds__(256) void relu_rank_kernel(const ReluDesc* __restrict__ table, ReluDesc one, int flags) {
+constexpr int kRankEntries = 32;
+constexpr int kRankThreads = 512;
+constexpr int kRankStep = 2 * kRankThreads / 8;  // keys the block's threads read at a time (eight threads share a pair)
+constexpr int kRankStage = 4096;
+__global__ __launch_bounds__(kRankThreads) void relu_rank_kernel(const ReluDesc* __restrict__ table, ReluDesc one, int flags) {
   const ReluDesc d = table ? table[blockIdx.z] : one;
   const int m = (flags & kRankCountOnDevice) ? d.counts[0] : d.m;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n_in = d.ncols_in - 1;
   if ((flags & kRankOldBounds) && d.plb_out != d.plb_in) {
-    for (int j = blockIdx.x * 256 + tid; j < n_in; j += gridDim.x * 256) {
+    for (int j = blockIdx.x * kRankThreads + tid; j < n_in; j += gridDim.x * kRankThreads) {
       d.plb_out[j] = d.plb_in[j];
       d.pub_out[j] = d.pub_in[j];
     }
   }
-  const int il = tid & (kRankI - 1), slice = tid / kRankI;  // 256 / kRankI = 16 slices
-  __shared__ double keys[kRankStage];
-  __shared__ int part[16][kRankI];
-  for (int i0 = blockIdx.x * kRankI; i0 < m; i0 += gridDim.x * kRankI) {
-    const int i = i0 + il;
-    const double ki = i < m ? d.key[i] : 0.0;
-    int cnt = 0;
+  const int il = tid & 7, pair = 2 * (tid >> 3);
+  __shared__ __attribute__((aligned(16))) double keys[kRankStage];
+  __shared__ int part[kRankThreads / 64][kRankEntries];
+  static_assert(kRankStep % kRankEntries == 0 && kRankStage % kRankStep == 0, "a block's entries lie in one step");
+  for (int i0 = blockIdx.x * kRankEntries; i0 < m; i0 += gridDim.x * kRankEntries) {
+    double ki[4];
+    int cnt[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ki[e] = i0 + il + 8 * e < m ? d.key[i0 + il + 8 * e] : 0.0;
+    const int neuron = tid < kRankEntries && i0 + tid < m ? d.asc_idx[i0 + tid] : 0;
     for (int base = 0; base < m; base += kRankStage) {
-      const int n = min(kRankStage, m - base);
+      const int n = min(kRankStage, m - base), steps = (n + kRankStep - 1) / kRankStep;
       __syncthreads();  // everybody is done with the previous piece
-      for (int t = tid; t < n; t += 256) keys[t] = d.key[base + t];
+      for (int t = tid; t < steps * kRankStep; t += kRankThreads)
+        keys[t] = t < n ? d.key[base + t] : __builtin_nan("");  // (behind the list: comes before nothing)
       __syncthreads();
-#pragma unroll 8
-      for (int t = slice; t < n; t += 16) {
-        const double kj = keys[t];
-        cnt += (kj > ki || (kj == ki && (base + t) < i)) ? 1 : 0;
+      const int own = i0 - base >= 0 ? (i0 - base) / kRankStep : -1;  // the step with the block's own entries (not always in this piece)
+      const double* k = keys + pair;
+      const int before = i0 >= base ? min(own, steps) : 0;
+      int t = 0;
+#pragma unroll 4
+      for (; t < before; ++t) {
+        const double2 kj = *reinterpret_cast<const double2*>(k + t * kRankStep);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          cnt[e] += kj.x >= ki[e] ? 1 : 0;
+          cnt[e] += kj.y >= ki[e] ? 1 : 0;
+        }
+      }
+      if (t == own && t < steps) {
+        const double2 kj = *reinterpret_cast<const double2*>(k + t * kRankStep);
+        const int j = base + t * kRankStep + pair;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = i0 + il + 8 * e;
+          cnt[e] += kj.x > ki[e] || (kj.x == ki[e] && j < i) ? 1 : 0;
+          cnt[e] += kj.y > ki[e] || (kj.y == ki[e] && j + 1 < i) ? 1 : 0;
+        }
+        ++t;
+      }
+#pragma unroll 4
+      for (; t < steps; ++t) {
+        const double2 kj = *reinterpret_cast<const double2*>(k + t * kRankStep);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          cnt[e] += kj.x > ki[e] ? 1 : 0;
+          cnt[e] += kj.y > ki[e] ? 1 : 0;
+        }
       }
     }
-    part[slice][il] = cnt;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      cnt[e] += __shfl_xor(cnt[e], 8);
+      cnt[e] += __shfl_xor(cnt[e], 16);
+      cnt[e] += __shfl_xor(cnt[e], 32);
+      if (lane < 8) part[wave][il + 8 * e] = cnt[e];
+    }
     __syncthreads();
-    if (slice != 0 || i >= m) continue;
+    if (tid >= kRankEntries || i0 + tid >= m) continue;
     int r = 0;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) r += part[q][il];
-    const int neuron = d.asc_idx[i];
+    for (int q = 0; q < kRankThreads / 64; ++q) r += part[q][tid];
     d.cross_idx[r] = neuron;
     if (d.col_of != nullptr) d.col_of[neuron] = r;
     if (flags & kRankNewBounds) {
@@ -830,10 +1002,12 @@ int relu_relax(nnvhip_ctx* ctx, int order, int64_t count, nnvhip_star* const* in
     NNV_TRY(ctx->upload_table(descs.data(), sizeof(ReluDesc) * count, &tab));
     table = tab->as<ReluDesc>();
   }
-  // Up to 8192 neurons: one block per set classifies, compacts and sorts crossing lists of up to 1024
-  // entries (sorting network).  Larger sets: two multi-block passes.  Whatever is still unsorted after
-  // the read-back of the counts goes to the multi-block rank kernels.
-  const int sort_cap = !sorted ? 0 : N <= kOneBlockN ? kSortInBlock : 0;
+  // Up to 2048 neurons: a few sets at once have several blocks each, which also place the crossing neurons; of more, one block
+  // per set classifies, compacts and sorts crossing lists of up to 1024 entries (sorting network).  Larger sets: two
+  // multi-block passes.  Whatever is still unsorted after the read-back of the counts goes to the multi-block rank kernel.
+  const int64_t rank_blocks = std::min<int64_t>(ceil_div(N, kRankI), kClassifyRankBlocks / count);
+  const bool classify_rank = sorted && N <= kOneBlockN && N <= kClassifyRankN && rank_blocks >= std::min<int64_t>(ceil_div(N, kRankI), 8);
+  const int sort_cap = !sorted ? 0 : classify_rank ? kClassifyRankN : N <= kOneBlockN ? kSortInBlock : 0;
   // algorithmic bytes of the classification: lb and ub read, the per-row class and the two index lists
   // written (plus, when it also writes the predicate bounds, the copy of the input's)
   double cls_bytes = 0.0;
@@ -842,6 +1016,8 @@ int relu_relax(nnvhip_ctx* ctx, int order, int64_t count, nnvhip_star* const* in
   if (N <= kOneBlockN) {
     if (!sorted)
       NNV_LAUNCH(ctx, tk, relu_classify_kernel<0>, dim3((unsigned)count), dim3(1024), 0, table, descs[0]);
+    else if (classify_rank)
+      NNV_LAUNCH(ctx, tk, relu_classify_rank_kernel, dim3((unsigned)rank_blocks, (unsigned)count), dim3(1024), 0, table, descs[0]);
     else if (N <= 1024)
       NNV_LAUNCH(ctx, tk, relu_classify_kernel<1024>, dim3((unsigned)count), dim3(1024), 0, table, descs[0]);
     else
@@ -856,10 +1032,10 @@ int relu_relax(nnvhip_ctx* ctx, int order, int64_t count, nnvhip_star* const* in
     NNV_LAUNCH(ctx, tk, relu_compact_kernel, grid, dim3(1024), 0, table, descs[0]);
     NNV_TRY(ctx->kernel_timer_end(tk, 6, 0.5 * cls_bytes));
     if (early_rank)
-      // (the host does not know m yet: enough blocks to fill the chip once, which walk the list; a block for every 16 neurons
-      // that might cross were 19 600 for 25 sets of 12 544 neurons, most of them idle: 39 us, now 11)
-      hipLaunchKernelGGL(relu_rank_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(N, kRankI), std::max<int64_t>(64, 1024 / count)), 1, (unsigned)count),
-                         dim3(256), 0, ctx->stream, table, descs[0], kRankNewBounds | kRankOldBounds | kRankCountOnDevice);
+      // (the host does not know m yet: enough blocks to fill the chip, which walk the list; a block for every 32 neurons that
+      // might cross would be 9 800 for 25 sets of 12 544 neurons, most of them idle)
+      hipLaunchKernelGGL(relu_rank_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(N, kRankEntries), std::max<int64_t>(32, 1024 / count)), 1, (unsigned)count),
+                         dim3(kRankThreads), 0, ctx->stream, table, descs[0], kRankNewBounds | kRankOldBounds | kRankCountOnDevice);
   }
   NNV_HIP_TRY(hipGetLastError());
 
@@ -1023,7 +1199,7 @@ int relu_relax(nnvhip_ctx* ctx, int order, int64_t count, nnvhip_star* const* in
     // one-block classification where that ran with the output buffers in place)
     ranked_with_bounds = lazy_rows;
     const int flags = lazy_rows ? (kRankNewBounds | (fold_bounds ? 0 : kRankOldBounds)) : 0;
-    hipLaunchKernelGGL(relu_rank_kernel, dim3((unsigned)ceil_div(max_m, kRankI), 1, (unsigned)count), dim3(256), 0, ctx->stream, table,
+    hipLaunchKernelGGL(relu_rank_kernel, dim3((unsigned)ceil_div(max_m, kRankEntries), 1, (unsigned)count), dim3(kRankThreads), 0, ctx->stream, table,
                        descs[0], flags);
   }
   if ((fold_bounds && !need_rank) || ranked_with_bounds) {
