@@ -480,6 +480,43 @@ __global__ __launch_bounds__(320) void ranges_final_kernel(const RangeDesc* __re
 }
 
 
+// The same for few rows and many chunks (the last layer of a network): 16 rows per block, its sixteen waves take every
+// sixteenth chunk each and are added in order.  With a row to a lane and the chunks one behind the other the loads were ten trips to
+// memory in a row: 16 rows, 299 and 75 chunks 18.5 and 7.2 us, 5.2 and 2.9 now.  Plain chunk sums only.
+__global__ __launch_bounds__(1024) void ranges_final_rows_kernel(const RangeDesc* __restrict__ table, RangeDesc one) {
+  const RangeDesc d = table ? table[blockIdx.z] : one;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = lane & 15, q = lane >> 4;
+  const int64_t r = (int64_t)blockIdx.x * 16 + row;  // (leading dimensions are multiples of 16)
+  __shared__ double red[16][64];
+  const double* p = d.part + (int64_t)q * d.ld + r;
+  const double c0 = d.V[r];
+  double s = 0.0;
+  for (int c = wave; c < d.chunks; c += 8 * 16) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = c + 16 * u < d.chunks ? p[(int64_t)(c + 16 * u) * 4 * d.ld] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (c + 16 * u < d.chunks) s += v[u];
+  }
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave != 0) return;
+  s = 0.0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) s += red[w][lane];
+  const double s1 = __shfl(s, (lane + 16) & 63);  // lanes 0..15: xmin2, lanes 32..47: xmax2
+  if (q == 0) d.lb[r] = (c0 + s) + s1;
+  if (q == 2) d.ub[r] = (c0 + s) + s1;
+}
+
+// A launch of the combining kernel takes that route from kManyChunks chunks on, where its rows are few.
+constexpr int kManyChunks = 17;
+static bool final_by_rows(const RangeDesc& d) {
+  return d.ld <= 64 && d.chunks >= kManyChunks && d.chunks2 == 0 && d.part3 == nullptr && d.cchunks == 0 && d.blk3 == nullptr;
+}
+
 // ---- W * (block of scaled unit vectors) -------------------------------------------------------
 // Column j of the block is scale * e_r, so the product column is W(:, r) * scale: a gather of W's
 // columns.  0 + w*scale reproduces what the dense accumulation (starting from +0) leaves, bit for bit.
@@ -848,27 +885,41 @@ struct RowSumArgs {
   double* ub;
 };
 
+// Bound by the latency of the trips to memory a block makes one behind the other, so the sums the GEMM's tiles left are asked
+// for first, a number to a thread, and added from LDS in tile order: 1024 x 1024 behind a GEMM 6.5 -> 5.9 us, 704 x 704
+// 6.6 -> 5.4.  (Fewer rows to a block, for a block on every CU, cost more
+// than they bring: a load then touches twice as many lines.  1024 x 1024: 12.9 us with 4 rows, 6.5 with 8, 8.2 with 16.)
 constexpr int kRowSumRows = 8;  // output rows per block
-
 __global__ __launch_bounds__(1024) void fc_rowsum_kernel(RowSumArgs a) {
-  __shared__ double red[16][3][kRowSumRows];
-  __shared__ double skey[4 * kRowSumRows];
+  constexpr int R = kRowSumRows;
+  constexpr int kGroups = 64 / R;      // input rows a wave takes at a time, R lanes each
+  constexpr int kStep = 16 * kGroups;  // ... and the block
+  constexpr int kEarly = 1024 / (4 * R);
+  __shared__ double red[16][3][R];
+  __shared__ double skey[4 * R];
+  __shared__ double early[1024];
+  const int rb = blockIdx.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rl = lane & 7, cs = lane >> 3;
-  const int row = blockIdx.x * kRowSumRows + rl;
+  const int rl = lane % R, cs = lane / R;
+  const int row = rb * R + rl;
   const double* wrow = a.W + row;
   const bool with_centre = a.centre_mode == 1;
+  double pv = 0.0, c_in = 0.0, c_bias = 0.0;
+  if (a.part != nullptr && tid / (4 * R) < a.chunks) pv = a.part[(int64_t)(tid / R) * a.ld + rb * R + tid % R];  // (chunk * 4 + sum)
+  if (tid < R) {
+    if (a.centre_mode == 0) c_in = a.centre[row];
+    else if (a.bias != nullptr) c_bias = a.bias[row];
+  }
   double sp = 0.0, sn = 0.0, cacc = 0.0;
-  // 128 input rows per step (16 waves x 8 lane groups, 8 lanes = 64 contiguous bytes of a column of W);
   // eight steps' loads -- none depends on another -- are issued before any is used
-  for (int r0 = wave * 8 + cs; r0 < a.K; r0 += 8 * 128) {
+  for (int r0 = wave * kGroups + cs; r0 < a.K; r0 += 8 * kStep) {
     double w[8], b[8], cj[8];
     int cl[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int r = r0 + u * 128;
+      const int r = r0 + u * kStep;
       w[u] = 0.0;
       b[u] = 0.0;
       cj[u] = 0.0;
@@ -893,9 +944,9 @@ __global__ __launch_bounds__(1024) void fc_rowsum_kernel(RowSumArgs a) {
       cacc = fma(w[u], cj[u], cacc);
     }
   }
-  // the eight lane groups, then the sixteen waves, in a fixed order
+  // the lane groups, then the sixteen waves, in a fixed order
 #pragma unroll
-  for (int off = 8; off < 64; off <<= 1) {
+  for (int off = R; off < 64; off <<= 1) {
     sp += __shfl_xor(sp, off);
     sn += __shfl_xor(sn, off);
     cacc += __shfl_xor(cacc, off);
@@ -905,22 +956,20 @@ __global__ __launch_bounds__(1024) void fc_rowsum_kernel(RowSumArgs a) {
     red[wave][1][rl] = sn;
     red[wave][2][rl] = cacc;
   }
+  early[tid] = pv;
   __syncthreads();
-  if (tid < 3 * kRowSumRows) {
-    const int which = tid / kRowSumRows, r8 = tid % kRowSumRows;
-    double t = 0.0;
+  if (tid < 4 * R) {  // sum q of a row: the GEMM tiles' chunks in order, then the gathered columns' term
+    const int q = tid / R, r8 = tid % R;
+    const int orow = rb * R + r8;
+    const int which = a.mode == 0 ? (q == 0 || q == 2 ? 0 : 1) : (q == 2 ? 0 : 1);
+    double S = 0.0, x = 0.0;
 #pragma unroll
-    for (int w2 = 0; w2 < 16; ++w2) t += red[w2][which][r8];
-    red[0][which][r8] = t;  // (the thread's own slot: read before it is written)
-  }
-  __syncthreads();
-  if (tid < 4 * kRowSumRows) {  // sum q of a row: the GEMM tiles' chunks in order, then the gathered columns' term
-    const int q = tid / kRowSumRows, r8 = tid % kRowSumRows;
-    const int orow = blockIdx.x * kRowSumRows + r8;
-    double x = 0.0;
+    for (int w2 = 0; w2 < 16; ++w2) S += red[w2][which][r8];
     if (a.part != nullptr) {
+      const int n = min(a.chunks, kEarly);
+      for (int c = 0; c < n; ++c) x += early[c * 4 * R + tid];
       // (sixteen loads in flight at a time, added in chunk order: one at a time they cost a trip to memory each)
-      for (int c = 0; c < a.chunks; c += 16) {
+      for (int c = kEarly; c < a.chunks; c += 16) {
         double v[16];
 #pragma unroll
         for (int u = 0; u < 16; ++u) v[u] = c + u < a.chunks ? a.part[((int64_t)(c + u) * 4 + q) * a.ld + orow] : 0.0;
@@ -929,27 +978,24 @@ __global__ __launch_bounds__(1024) void fc_rowsum_kernel(RowSumArgs a) {
           if (c + u < a.chunks) x += v[u];
       }
     }
-    const double Sp = red[0][0][r8], Sn = red[0][1][r8];
-    double term;
-    if (a.mode == 0) term = q == 0 ? -Sp : q == 1 ? Sn : q == 2 ? Sp : -Sn;
-    else term = q == 1 ? Sn : q == 2 ? Sp : 0.0;
-    x += term;
+    // [W+ s, W- s] meet the bounds -1, 1 of a box's predicates or 0, ub of a ReLU step's
+    x += a.mode == 0 ? (q == 0 || q == 3 ? -S : S) : (q == 1 || q == 2 ? S : 0.0);
     skey[tid] = x;
   }
   __syncthreads();
-  if (tid < kRowSumRows) {
-    const int orow = blockIdx.x * kRowSumRows + tid;
-    double c0;
-    if (a.centre_mode == 0) {
-      c0 = a.centre[orow];
-    } else {
-      c0 = a.centre_mode == 1 ? red[0][2][tid] : 0.0;
-      if (a.bias != nullptr) c0 = c0 + a.bias[orow];
-      a.centre[orow] = c0;
+  if (tid < R) {
+    double c0 = c_in;
+    if (a.centre_mode != 0) {
+      if (a.centre_mode == 1) {
+#pragma unroll
+        for (int w2 = 0; w2 < 16; ++w2) c0 += red[w2][2][tid];
+      }
+      if (a.bias != nullptr) c0 = c0 + c_bias;
+      a.centre[row] = c0;
     }
     // lb = (c + xmin1) + xmin2, the reference's left-to-right order (set/Star.m:1098-1104)
-    a.lb[orow] = (c0 + skey[tid]) + skey[kRowSumRows + tid];
-    a.ub[orow] = (c0 + skey[2 * kRowSumRows + tid]) + skey[3 * kRowSumRows + tid];
+    a.lb[row] = (c0 + skey[tid]) + skey[R + tid];
+    a.ub[row] = (c0 + skey[2 * R + tid]) + skey[3 * R + tid];
   }
 }
 
@@ -975,10 +1021,10 @@ int launch_fc_rowsum(nnvhip_ctx* ctx, const nnvhip_fc* fc, nnvhip_star* out, int
   a.ld = out->ld;
   a.lb = rb->as<double>();
   a.ub = a.lb + out->ld;
-  const int64_t row_blocks = fc->Mp / kRowSumRows;
+  const unsigned blocks = (unsigned)(fc->Mp / kRowSumRows);
   // algorithmic bytes: W once, the finished ranges (timed with the gather passes it stands in for)
   const double bytes = 8.0 * (double)fc->Mp * (double)fc->K + 16.0 * (double)fc->Mp;
-  NNV_LAUNCH(ctx, ctx->kernel_timing, fc_rowsum_kernel, dim3((unsigned)row_blocks), dim3(1024), 0, a);
+  NNV_LAUNCH(ctx, ctx->kernel_timing, fc_rowsum_kernel, dim3(blocks), dim3(1024), 0, a);
   NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 5, bytes));
   NNV_HIP_TRY(hipGetLastError());
   out->rbuf = rb;
@@ -1450,7 +1496,11 @@ int compute_ranges(nnvhip_ctx* ctx, int64_t count, nnvhip_star* const* s, RangeC
   if (chunks > 1 || any_pending) {
     double fbytes = 0.0;  // every chunk's four sums read, lb and ub written
     for (int64_t i = 0; i < nset; ++i) fbytes += 8.0 * (double)ld * (4.0 * (double)(descs[i].chunks + descs[i].chunks2) + 3.0);
-    if (wide_final)
+    bool by_rows = true;
+    for (int64_t i = 0; i < nset && by_rows; ++i) by_rows = final_by_rows(descs[i]);
+    if (by_rows)
+      NNV_LAUNCH(ctx, ctx->kernel_timing, ranges_final_rows_kernel, dim3((unsigned)(ld / 16), 1, (unsigned)nset), dim3(1024), 0, table, descs[0]);
+    else if (wide_final)
       NNV_LAUNCH(ctx, ctx->kernel_timing, ranges_final_kernel<2>, dim3((unsigned)ceil_div(ld, 128), 1, (unsigned)nset), dim3(256), 0,
                  table, descs[0]);
     else
@@ -1499,8 +1549,11 @@ int finalize_fused_ranges(nnvhip_ctx* ctx, nnvhip_star* s, const BufRef& part, i
   d.cpart = cpart;
   d.cbias = cbias;
   d.cout = s->V;
-  NNV_LAUNCH(ctx, ctx->kernel_timing, ranges_final_kernel<1>, dim3((unsigned)ceil_div(s->ld, 64), 1, 1),
-             dim3(cchunks > 0 ? 320 : 256), 0, nullptr, d);
+  if (final_by_rows(d))
+    NNV_LAUNCH(ctx, ctx->kernel_timing, ranges_final_rows_kernel, dim3((unsigned)(d.ld / 16), 1, 1), dim3(1024), 0, nullptr, d);
+  else
+    NNV_LAUNCH(ctx, ctx->kernel_timing, ranges_final_kernel<1>, dim3((unsigned)ceil_div(s->ld, 64), 1, 1),
+               dim3(cchunks > 0 ? 320 : 256), 0, nullptr, d);
   NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 7, 8.0 * (double)s->ld * (4.0 * (double)chunks + 3.0)));
   NNV_HIP_TRY(hipGetLastError());
   s->rbuf = rb;
