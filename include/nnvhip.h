@@ -163,6 +163,7 @@ enum {
   NNVHIP_ROUTE_ROWMAP_WINDOW,      /* row map inside windows */
   NNVHIP_ROUTE_ROWMAP_BOX,         /* row map of a box of which only the centre is in memory */
   NNVHIP_ROUTE_POOL_WINDOW,        /* average pooling inside windows */
+  NNVHIP_ROUTE_CONV_PIXELS,        /* convolution whose output images are kept pixel by pixel */
   NNVHIP_ROUTES
 };
 NNVHIP_API int nnvhip_debug_routes(nnvhip_ctx* ctx, int64_t* sets);

@@ -318,6 +318,10 @@ __device__ __forceinline__ ConvSet conv_set_of_block(const ConvSet* __restrict__
   s.d.m = t->d.m;
   s.d.win_only = t->d.win_only;
   s.d.pixel_col = t->d.pixel_col;
+  s.d.pix = t->d.pix;
+  s.d.pix_ld = t->d.pix_ld;
+  s.d.pix_eh = t->d.pix_eh;
+  s.d.pix_ew = t->d.pix_ew;
   return s;
 }
 
@@ -700,10 +704,13 @@ __global__ __launch_bounds__(256) void keep_bits_kernel(const KeepBits* __restri
 }
 
 template <int S>
-__global__ __launch_bounds__(256) void conv_stamp_rows_kernel(StampSet d, ConvGeom g, const double* __restrict__ Wt,
-                                                              const int32_t* __restrict__ pixel_col, int64_t ldout) {
+__global__ __launch_bounds__(256) void conv_stamp_rows_kernel(StampSet d, ConvGeom g, const double* __restrict__ Wt, const double* __restrict__ Wk,
+                                                              int coutp, const int32_t* __restrict__ pixel_col, int64_t ldout) {
   __shared__ int2 taps[kStampTapTable];
-  conv_stamp_rows_block<S, 256>(blockIdx.x, taps, d, g, Wt, pixel_col, ldout);
+  if (d.pix != nullptr)
+    conv_stamp_pixels_block<S, 256>(blockIdx.x, taps, d, g, Wk, coutp, pixel_col, ldout);
+  else
+    conv_stamp_rows_block<S, 256>(blockIdx.x, taps, d, g, Wt, pixel_col, ldout);
 }
 
 // The dense images' convolution and the stamps of the unit-vector columns of the same layer in one launch: the two
@@ -720,7 +727,10 @@ __global__ __launch_bounds__(512) void conv2d_fast_stamps_kernel(ConvFastArgs a,
   const int p = blockIdx.x;
   const int k = (p + 1) / set.stride;
   if ((p + 1) % set.stride == 0 && k <= a.stamp_blocks) {
-    conv_stamp_rows_block<S, 512>(k - 1, reinterpret_cast<int2*>(lds), set.d, a.g, Wt, set.d.pixel_col, a.ldout);
+    if (set.d.pix != nullptr)
+      conv_stamp_pixels_block<S, 512>(k - 1, reinterpret_cast<int2*>(lds), set.d, a.g, a.Wk, a.coutp, set.d.pixel_col, a.ldout);
+    else
+      conv_stamp_rows_block<S, 512>(k - 1, reinterpret_cast<int2*>(lds), set.d, a.g, Wt, set.d.pixel_col, a.ldout);
     return;
   }
   const int bid = p - min(a.stamp_blocks, p / set.stride);
@@ -1120,10 +1130,10 @@ int launch_conv_stamps(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
         NNV_HIP_TRY(hipMemsetAsync(one.out, 0, sizeof(double) * (size_t)ldout * (size_t)one.m, ctx->stream));
       if (g.K <= 32)
         NNV_LAUNCH(ctx, ctx->kernel_timing && i == 0, conv_stamp_rows_kernel<1>, dim3((unsigned)ceil_div(ldout, 256)), dim3(256), 0, one, g,
-                   cv->W->as<double>(), pc, ldout);
+                   cv->W->as<double>(), cv->Wk ? cv->Wk->as<double>() : nullptr, (int)cv->coutp, pc, ldout);
       else
         NNV_LAUNCH(ctx, ctx->kernel_timing && i == 0, conv_stamp_rows_kernel<16>, dim3((unsigned)ceil_div(ldout * 16, 256)), dim3(256), 0,
-                   one, g, cv->W->as<double>(), pc, ldout);
+                   one, g, cv->W->as<double>(), cv->Wk ? cv->Wk->as<double>() : nullptr, (int)cv->coutp, pc, ldout);
     }
     NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 5, bytes));
     NNV_HIP_TRY(hipGetLastError());

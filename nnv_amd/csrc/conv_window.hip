@@ -45,6 +45,11 @@ struct ConvWinSet {
   double* part;               // [parts][4][ldo] range sums
   int32_t parts;
   int32_t eh, ew;             // bound on the output windows
+  // images kept pixel by pixel (ColSource::pix), or null: those of the input, those of the output
+  const double* in_pix;
+  double* out_pix;
+  int64_t in_pix_ld, out_pix_ld;
+  int32_t in_eh, in_ew, out_eh, out_ew;
   StampSet stamps;            // unit-vector columns whose stamps go into the same launch (m: 0: none)
 };
 struct ConvWinArgs {
@@ -80,7 +85,8 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
   extern __shared__ __attribute__((aligned(16))) int s_rows[];  // kept input rows under the filter, by tap, -1 padded to whole pairs of stages ...
   int* const s_row = s_rows;
   int* const s_tap = s_rows + a.list;      // ... their taps ...
-  int* const s_pos = s_rows + 2 * a.list;  // ... and their positions in the image: h | w << 16
+  int* const s_pos = s_rows + 2 * a.list;  // ... their positions in the image: h | w << 16 (-1: none) ...
+  int* const s_off = s_rows + 3 * a.list;  // ... and, with images kept pixel by pixel, where they lie in one
   __shared__ int s_col[kConvWinCols];
   __shared__ double s_pl[kConvWinCols], s_pu[kConvWinCols];
   __shared__ int s_from[kConvWinStarts], s_end[kConvWinStarts];
@@ -97,6 +103,9 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
   S.plb = in_global(S.plb);
   S.pub = in_global(S.pub);
   S.part = in_global(S.part);
+  S.in_pix = in_global(S.in_pix);
+  S.out_pix = in_global(S.out_pix);
+  S.stamps.pix = in_global(S.stamps.pix);
   S.stamps.idx = in_global(S.stamps.idx);
   S.stamps.scale = in_global(S.stamps.scale);
   S.stamps.out = in_global(S.stamps.out);
@@ -106,8 +115,12 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
   S.stamps.pixel_col = in_global(S.stamps.pixel_col);
   const int blk = (int)blockIdx.x - a.stamp_blocks;
   if (blk < 0) {
-    if (S.stamps.m > 0 && blockIdx.z == 0)
-      conv_stamp_rows_block<S_LANES, NT>(blockIdx.x, reinterpret_cast<int2*>(s_rows), S.stamps, a.g, a.Wt, S.stamps.pixel_col, a.ldo);
+    if (S.stamps.m > 0 && blockIdx.z == 0) {
+      if (S.stamps.pix != nullptr)
+        conv_stamp_pixels_block<S_LANES, NT>(blockIdx.x, reinterpret_cast<int2*>(s_rows), S.stamps, a.g, a.Wk, a.coutp, S.stamps.pixel_col, a.ldo);
+      else
+        conv_stamp_rows_block<S_LANES, NT>(blockIdx.x, reinterpret_cast<int2*>(s_rows), S.stamps, a.g, a.Wt, S.stamps.pixel_col, a.ldo);
+    }
     return;
   }
   const int item = (blk & 7) * a.per + (blk >> 3);  // (stamp_blocks is a multiple of eight)
@@ -128,17 +141,30 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
     s_from[t] = h0 >= 0 ? S.first[s] : 0;
     s_end[t] = h0 >= 0 ? S.first[s + 1] - s_from[t] : 0;
   }
-  // kept rows under the filter, in tap order
+  // kept rows under the filter, in tap order; of images kept pixel by pixel pixel by pixel, so that a stage's rows lie together
+  const bool pixels = S.in_pix != nullptr;
   int nrow = 0;
   const int hb = ph * a.g.sh - a.g.pt, wb = pw * a.g.sw - a.g.pl;
   for (int k0 = 0; k0 < a.g.K; k0 += NT) {
-    const int k = k0 + tid;
+    int k = k0 + tid;
     bool keep = k < a.g.K;
-    int r = 0, h = 0, w = 0;
+    int r = 0, h = 0, w = 0, ci = 0;
     if (keep) {
-      const int t = k / a.g.FH, ci = t / a.g.FW;
-      h = hb + (k - t * a.g.FH) * a.g.dh;
-      w = wb + (t - ci * a.g.FW) * a.g.dw;
+      int fh, fw;
+      if (pixels) {
+        const int t = k / a.g.Cin;
+        ci = k - t * a.g.Cin;
+        fw = t / a.g.FH;
+        fh = t - fw * a.g.FH;
+        k = (ci * a.g.FW + fw) * a.g.FH + fh;
+      } else {
+        const int t = k / a.g.FH;
+        ci = t / a.g.FW;
+        fh = k - t * a.g.FH;
+        fw = t - ci * a.g.FW;
+      }
+      h = hb + fh * a.g.dh;
+      w = wb + fw * a.g.dw;
       keep = (unsigned)h < (unsigned)a.g.H && (unsigned)w < (unsigned)a.g.W;
       if (keep) {
         r = ci * a.g.HW + w * a.g.H + h;
@@ -161,6 +187,7 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
       s_row[at] = r;
       s_tap[at] = k;
       s_pos[at] = h | (w << 16);
+      if (pixels) s_off[at] = pix_slot(h, w, S.in_eh, S.in_ew) * a.g.Cin + ci;
     }
     __syncthreads();
   }
@@ -168,7 +195,8 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
   if (tid < nk * KT - nrow) {
     s_row[nrow + tid] = -1;
     s_tap[nrow + tid] = 0;
-    s_pos[nrow + tid] = 0;
+    s_pos[nrow + tid] = -1;
+    if (pixels) s_off[nrow + tid] = 0;
   }
   int total = 0;
   for (int g = 0; g < runs; ++g) total += s_end[g];
@@ -187,6 +215,7 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
     const int co = m0 + wr * (TM / WR) + i * 16 + lrow;
     bias[i] = a.bias != nullptr && co < a.g.Cout ? a.bias[co] : 0.0;
   }
+  const int out_slot = S.out_pix != nullptr ? pix_slot(ph, pw, S.out_eh, S.out_ew) * a.g.Cout : 0;
   double x[FM][4];  // xmin1, xmin2, xmax1, xmax2 of the lane's rows over the columns it has held
 #pragma unroll
   for (int i = 0; i < FM; ++i)
@@ -244,15 +273,19 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
       // the images this thread stages: rows 2 * (tid % 8) and the next of every stage
       const int bk = 2 * (tid % (KT / 2));
       const double* img[B_PASS];
+      const int* at[B_PASS];  // where the listed rows lie in it
       ColBox bb[B_PASS];
 #pragma unroll
       for (int u = 0; u < B_PASS; ++u) {
         const int j = c0 + (tid + u * NT) / (KT / 2);
         bb[u] = ColBox{1, 0, 1, 0};
         img[u] = S.V;
+        at[u] = s_row;
         if (j < n) {
-          bb[u] = s_col[j] == 0 ? ColBox{0, (int16_t)(a.g.H - 1), 0, (int16_t)(a.g.W - 1)} : S.in_box[s_col[j]];
-          img[u] = S.V + (int64_t)s_col[j] * S.ld;
+          const int col = s_col[j];
+          bb[u] = col == 0 ? ColBox{0, (int16_t)(a.g.H - 1), 0, (int16_t)(a.g.W - 1)} : S.in_box[col];
+          img[u] = pixels && col > 0 ? S.in_pix + (int64_t)col * S.in_pix_ld : S.V + (int64_t)col * S.ld;
+          at[u] = pixels && col > 0 ? s_off : s_row;
         }
       }
       // A stage's operands travel through registers while the two stages before it are multiplied.  Every load is issued
@@ -274,9 +307,9 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
 #pragma unroll
         for (int u = 0; u < B_PASS; ++u) {
           auto pixel = [&](int k, unsigned bit) {
-            const int r = s_row[k], pos = s_pos[k];
-            const int h = pos & 0xffff, w = pos >> 16;
-            const bool in = r >= 0 && h >= bb[u].h0 && h <= bb[u].h1 && w >= bb[u].w0 && w <= bb[u].w1;
+            const int r = at[u][k], pos = s_pos[k];
+            const int h = pos & 0xffff, w = pos >> 16;  // (h past any window where there is no row)
+            const bool in = h >= bb[u].h0 && h <= bb[u].h1 && w >= bb[u].w0 && w <= bb[u].w1;
             g.use |= in ? bit : 0u;
             return in_global(in ? img[u] + r : S.V)[0];
           };
@@ -339,7 +372,10 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
             x[i][2] = fma(vp, pu, x[i][2]);
             x[i][3] = fma(vn, pl, x[i][3]);
             if (co < a.g.Cout) {
-              S.out[(int64_t)col * a.ldo + (int64_t)co * a.g.P + p] = col == 0 && a.bias != nullptr ? v + bias[i] : v;
+              if (col > 0 && S.out_pix != nullptr)
+                S.out_pix[(int64_t)col * S.out_pix_ld + out_slot + co] = v;
+              else
+                S.out[(int64_t)col * a.ldo + (int64_t)co * a.g.P + p] = col == 0 && a.bias != nullptr ? v + bias[i] : v;
             }
           }
       }
@@ -412,7 +448,20 @@ int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
     const ConvWindowSet& s = sets[i];
     tab[(size_t)i] = ConvWinSet{s.in->V, s.in->ld, s.in->box, s.out->box, s.in->rows_pending ? s.in->keep_bits : nullptr,
                                 s.in->rows_pending ? s.in->cls : nullptr, s.order, s.first, s.out->V, s.out->plb, s.out->pub, s.part,
-                                (int32_t)s.parts, s.eh, s.ew, StampSet{}};
+                                (int32_t)s.parts, s.eh, s.ew, nullptr, nullptr, 0, 0, 1, 1, 1, 1, StampSet{}};
+    ConvWinSet& t = tab[(size_t)i];
+    if (s.in->cs.in_pixels()) {
+      t.in_pix = s.in->cs.pix;
+      t.in_pix_ld = s.in->cs.pix_ld;
+      t.in_eh = s.in->cs.pix_eh;
+      t.in_ew = s.in->cs.pix_ew;
+    }
+    if (s.out->cs.in_pixels()) {
+      t.out_pix = const_cast<double*>(s.out->cs.pix);
+      t.out_pix_ld = s.out->cs.pix_ld;
+      t.out_eh = s.out->cs.pix_eh;
+      t.out_ew = s.out->cs.pix_ew;
+    }
     if (s.stamp != nullptr) {
       static_assert(sizeof(ConvStampSet) == sizeof(StampSet), "same layout");
       memcpy(&tab[(size_t)i].stamps, s.stamp, sizeof(StampSet));
@@ -437,7 +486,7 @@ int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
   const bool wide_stamps = a.g.K > 32;  // lanes per output row as in the launch that shares the implicit GEMM's
   a.stamp_blocks = any_stamps ? (int32_t)round_up(ceil_div(ldout * (wide_stamps ? 8 : 1), nt), 8) : 0;
   const dim3 grid((unsigned)(a.stamp_blocks + 8 * a.per), (unsigned)count, (unsigned)ceil_div(cv->Cout, tm));
-  const size_t dyn = 3 * sizeof(int32_t) * (size_t)a.list;  // (also holds the stamps' tap table, 8 bytes a tap)
+  const size_t dyn = 4 * sizeof(int32_t) * (size_t)a.list;  // (also holds the stamps' tap table, 8 bytes a tap)
   NNV_TRY(ctx->kernel_timer_begin(ctx->kernel_timing));
 #define NNV_CONV_WINDOW(TM, WR, WC)                                                                                                    \
   do {                                                                                                                                \

@@ -489,7 +489,7 @@ static bool rowmap_in_windows(const nnvhip_ctx* c, const nnvhip_rowmap* m, const
   if (s->box == nullptr || s->box_cols < s->n + 1 || s->box_H <= 0 || s->box_W <= 0) return false;
   const int64_t P = (int64_t)s->box_H * s->box_W;
   return s->N % P == 0 && small_windows(s->box_eh, s->box_ew, P) && !s->cs.pending && s->cs.zero_to <= 1 && !s->cs.delta_pending() &&
-         s->n < 1000000;
+         !s->cs.in_pixels() && s->n < 1000000;
 }
 
 // One launch for all sets of a call, here and in pool_windows.  (With a launch or three per image, 100 images of 12 x 12
@@ -601,7 +601,7 @@ static bool pool_in_windows(const nnvhip_ctx* c, const nnvhip_avgpool2d* p, cons
   pl->dense = (s->oh_from > 0 && s->oh_from < nc) ? s->oh_from : nc;
   pl->m = nc - pl->dense;
   if (pl->dense > s->stored_cols() || (pl->m > 0 && s->oh_idx == nullptr)) return false;
-  if (s->cs.pending || s->cs.zero_to > 1 || s->cs.delta_pending() || (s->rows_pending && s->cls == nullptr)) return false;
+  if (s->cs.pending || s->cs.zero_to > 1 || s->cs.delta_pending() || s->cs.in_pixels() || (s->rows_pending && s->cls == nullptr)) return false;
   if (pl->dense > 1 && !(s->box != nullptr && s->box_H == H && s->box_W == W && s->box_cols >= pl->dense)) return false;
   auto extent = [&](int d, int64_t e, int64_t size) { return std::min<int64_t>(size, (e - 1 + p->pool[d] - 1) / p->stride[d] + 1); };
   pl->eh = pl->ew = 0;

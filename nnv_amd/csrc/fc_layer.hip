@@ -261,7 +261,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
         int64_t kp = 0;
         bool pack = false;
         const bool compact = rows_of(i, &r, &kp, &pack);
-        if (!(compact && (nothing_kept(i, r) || (pack && r.kmap != nullptr)))) cols.push_back(in[i]);
+        if (!(compact && (nothing_kept(i, r) || (pack && r.kmap != nullptr && !in[i]->cs.in_pixels())))) cols.push_back(in[i]);
       }
       if (!cols.empty()) st = write_pending_columns(c, (int64_t)cols.size(), cols.data());
     }

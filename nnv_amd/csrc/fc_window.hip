@@ -39,6 +39,10 @@ struct FcWinSet {
   const double* pub;
   double* rpart;              // [tiles][4][ldo] range sums
   int32_t ncols, tiles, nk, kper, cchunks;
+  // images kept pixel by pixel (ColSource::pix), or null
+  const double* pix;
+  int64_t pix_ld;
+  int32_t pix_eh, pix_ew;
 };
 struct FcWinArgs {
   const double* W;
@@ -65,6 +69,7 @@ __device__ __forceinline__ FcWinSet win_set(const FcWinSet* __restrict__ table, 
   s.plb = in_global(s.plb);
   s.pub = in_global(s.pub);
   s.rpart = in_global(s.rpart);
+  s.pix = in_global(s.pix);
   return s;
 }
 
@@ -121,7 +126,7 @@ __global__ __launch_bounds__(kSortThreads) void fc_window_setup_kernel(const FcW
 
 // TM x TN output tile per block of WR x WC waves.  Column tiles are dealt to the XCDs (blockIdx.x % 8) with all their row
 // tiles, which read the same images.  The last column tile of a set is its centre: the sum of the partial products.
-constexpr int kWinRows = 2048;  // rows a stage list holds; a union with more kept rows is walked in several lists
+constexpr int kWinRows = 1024;  // rows a stage list holds; a union with more kept rows is walked in several lists
 template <int TM, int TN, int WR, int WC, int KT>
 __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet* __restrict__ table, FcWinSet one, FcWinArgs a) {
   constexpr int NT = 64 * WR * WC, NW = WR * WC;
@@ -130,8 +135,10 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
   static_assert(NT == TN * KT / 2, "one pair of rows of the image tile per thread");
   __shared__ double Ws[2][KT * LDA_S];
   __shared__ double Vs[2][TN * LDB_S];
-  __shared__ int s_row[kWinRows + KT];  // rows of the union's windows, ascending, -1 padded to whole stages
-  __shared__ int s_pos[kWinRows + KT];  // their positions: h | w << 16
+  // rows of the union's windows, -1 padded to whole stages: ascending; of images kept pixel by pixel pixel by pixel
+  __shared__ int s_row[kWinRows + KT];
+  __shared__ int s_pos[kWinRows + KT];  // their positions: h | w << 16 (-1: none) ...
+  __shared__ int s_off[kWinRows + KT];  // ... and where they lie in an image
   __shared__ int s_col[TN];
   __shared__ double s_pl[TN], s_pu[TN];
   __shared__ int s_u[4];
@@ -189,7 +196,8 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
   // the image this thread stages: rows 2 * (tid % 8) and the next of every stage, of column tid / 8
   const int bj = tid / (KT / 2), bk = 2 * (tid % (KT / 2));
   const int bcol = s_col[bj];
-  const double* img = S.V + (int64_t)max(bcol, 0) * S.ld;
+  const bool pixels = S.pix != nullptr;
+  const double* img = pixels ? S.pix + (int64_t)max(bcol, 0) * S.pix_ld : S.V + (int64_t)max(bcol, 0) * S.ld;
   ColBox bb = {1, 0, 1, 0};
   if (bcol >= 0) bb = S.box[bcol];
 
@@ -213,9 +221,9 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
       }
     }
     auto pixel = [&](int k) {
-      const int r = s_row[k], pos = s_pos[k];
-      const int h = pos & 0xffff, w = pos >> 16;
-      return r >= 0 && h >= bb.h0 && h <= bb.h1 && w >= bb.w0 && w <= bb.w1 ? img[r] : 0.0;
+      const int at = s_off[k], pos = s_pos[k];
+      const int h = pos & 0xffff, w = pos >> 16;  // (h past any window where there is no row)
+      return h >= bb.h0 && h <= bb.h1 && w >= bb.w0 && w <= bb.w1 ? img[at] : 0.0;
     };
     rb.x = pixel(k0 + bk);
     rb.y = pixel(k0 + bk + 1);
@@ -236,9 +244,16 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
     while (cand < total && nrow + NT <= kWinRows) {  // kept rows among the next NT of the union, ascending
       const int e = cand + tid;
       bool keep = e < total;
-      int r = 0, h = 0, w = 0;
+      int r = 0, h = 0, w = 0, ch = 0;
       if (keep) {
-        const int ch = e / P, q = e - ch * P;
+        int q;
+        if (pixels) {
+          q = e / a.C;
+          ch = e - q * a.C;
+        } else {
+          ch = e / P;
+          q = e - ch * P;
+        }
         w = q / uh;
         h = uh0 + q - w * uh;
         w += uw0;
@@ -260,6 +275,7 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
         const int at = before + __popcll(m & ((1ull << lane) - 1ull));
         s_row[at] = r;
         s_pos[at] = h | (w << 16);
+        s_off[at] = pixels ? pix_slot(h, w, S.pix_eh, S.pix_ew) * a.C + ch : r;
       }
       __syncthreads();
       cand += NT;
@@ -267,7 +283,8 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
     const int nk = (nrow + KT - 1) / KT;
     if (tid < nk * KT - nrow) {
       s_row[nrow + tid] = -1;
-      s_pos[nrow + tid] = 0;
+      s_pos[nrow + tid] = -1;
+      s_off[nrow + tid] = 0;
     }
     __syncthreads();
     if (nk > 0) {
@@ -352,6 +369,10 @@ int fc_window_tile(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in, c
     if (s->rows_pending && s->kept_idx == nullptr) return 0;
     cols += dense[i] - 1;
   }
+  return fc_window_tile_of(fc, count, cols, H, W, f->box_eh, f->box_ew);
+}
+
+int fc_window_tile_of(const nnvhip_fc* fc, int64_t count, int64_t cols, int64_t H, int64_t W, int64_t eh, int64_t ew) {
   // The positions a tile walks: its columns' windows plus what the columns' starts spread over two strips.  The contraction
   // over all kept rows multiplies at about twice the rate (its stages need no position tests and its tiles are larger), so
   // the line is half of the image: windows of 16 of 49 positions take 65 us here and 174 us there, and from windows as
@@ -359,7 +380,7 @@ int fc_window_tile(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in, c
   const int64_t tiles_m = ceil_div(fc->Mp, 64);
   const int tn = ceil_div(cols, 64) * tiles_m >= 512 ? 64 : 32;
   const double starts = (double)tn * (double)(H * W) * (double)count / (double)cols;  // distinct starts of a tile's columns
-  const double uh = std::min((double)H, (double)f->box_eh + 0.5 * starts), uw = std::min((double)W, (double)f->box_ew + std::min(1.0, starts));
+  const double uh = std::min((double)H, (double)eh + 0.5 * starts), uw = std::min((double)W, (double)ew + std::min(1.0, starts));
   return 2.0 * uh * uw <= (double)(H * W) ? tn : 0;
 }
 
@@ -414,6 +435,12 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
     d.V = s->V;
     d.ld = s->ld;
     d.box = s->box;
+    if (s->cs.in_pixels()) {
+      d.pix = s->cs.pix;
+      d.pix_ld = s->cs.pix_ld;
+      d.pix_eh = s->cs.pix_eh;
+      d.pix_ew = s->cs.pix_ew;
+    }
     if (s->rows_pending) {
       d.keep_bits = s->keep_bits;
       d.cls = s->cls;

@@ -213,6 +213,9 @@ struct DeltaCall {
 // next layers reads them then, and whoever does (a host read, a layer that needs the whole matrix) has
 // them written first.  Writing them is idempotent, so every handle that shares the matrix keeps a copy
 // of this description with its own flags.  W == null: no such knowledge.
+// Place of a pixel among those of a window of at most eh x ew positions (ColSource::pix).
+__host__ __device__ inline int pix_slot(int h, int w, int eh, int ew) { return (w % ew) * eh + h % eh; }
+
 struct ColSource {
   BufRef W_buf, idx_buf, scale_buf, Wt_buf;
   const double* Wt = nullptr;  // the same matrix row-major (row r at Wt + r * ldwt), or null
@@ -240,6 +243,15 @@ struct ColSource {
   int64_t win_rows = 0;  // rows of the image (H * W * channels)
   int32_t win_H = 0, win_W = 0;
   bool win_pending() const { return win_to > win_from; }
+  // Such columns may be in a buffer of their own instead, pixel by pixel (pix != null while win_pending): element (h, w,
+  // channel) of column j, inside its window, is pix[j * pix_ld + pix_slot(h, w) * channels + channel], the channels of a pixel
+  // side by side; the matrix then holds nothing of them.  A place depends on the pixel only, not on where the column's window
+  // lies, and is the column's own because no window spans more than pix_eh x pix_ew positions.
+  BufRef pix_buf;
+  const double* pix = nullptr;
+  int64_t pix_ld = 0;
+  int32_t pix_eh = 0, pix_ew = 0;
+  bool in_pixels() const { return pix != nullptr && win_pending(); }
   // The leading (contracted) columns 1 .. of the matrix are the output of a shared-product call that has not written
   // them yet (column 0, the centre, is in memory).
   Ref<DeltaCall> delta;
@@ -340,6 +352,10 @@ struct nnvhip_ctx {
   uint64_t next_layer_uid = 0;
   // nnvhip_hint_next_fc: the FC layer the caller will apply to the output of its next ReLU step (consumed by that step)
   const nnvhip_fc* next_fc = nullptr;
+  // The layer behind the ReLU step that follows the convolution about to run, as the layer loop of nnvhip_reach_layers knows
+  // it (both null: not known)
+  const nnvhip_conv2d* behind_conv = nullptr;
+  const nnvhip_fc* behind_fc = nullptr;
   // memory of released handles, reused by new_star (at most kMaxFreeStars of them are kept)
   static constexpr size_t kMaxFreeStars = 65536;
   std::vector<void*> free_stars;
@@ -802,6 +818,9 @@ struct ConvStampSet {
   int32_t m;
   int32_t win_only;     // 1: write the rows inside each column's window only
   const int32_t* pixel_col;  // input row -> its one-hot column (index into idx), -1: none (ConvSetup::inv); undilated filters only
+  double* pix;          // not null: the stamps go here, pixel by pixel (ColSource::pix, shifted to the first of these columns) ...
+  int64_t pix_ld;
+  int32_t pix_eh, pix_ew;
 };
 // The dense images of one set of a call.
 struct ConvJob {
@@ -959,6 +978,8 @@ int finalize_fused_ranges(nnvhip_ctx* ctx, nnvhip_star* s, const BufRef& part, i
 // (nnvhip_star::box), tile by tile over the windows' union only.
 // Columns per tile where the sets of a call (all of them) take it, 0: they do not.  dense: leading columns to contract.
 int fc_window_tile(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in, const int64_t* dense);
+// ... by the sizes alone: `cols` images of H x W positions in windows of at most eh x ew, in `count` sets
+int fc_window_tile_of(const nnvhip_fc* fc, int64_t count, int64_t cols, int64_t H, int64_t W, int64_t eh, int64_t ew);
 struct FcWindowSet {
   const nnvhip_star* in;
   nnvhip_star* out;   // its leading `dense` columns are written, bias included

@@ -9,11 +9,18 @@
 
 using namespace nnvhip;
 
+static const ColBox kAnyBox = {0, 0, 0, 0};  // stands for a window table in a question about sizes
+
 extern "C" {
 
 int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t count,
                          nnvhip_star* const* in, nnvhip_star** out) {
   CHECK_CTX(c);
+  // (what the caller knows about the layers behind is for this call, whatever becomes of it)
+  const nnvhip_conv2d* const behind_conv = c->behind_conv;
+  const nnvhip_fc* const behind_fc = c->behind_fc;
+  c->behind_conv = nullptr;
+  c->behind_fc = nullptr;
   if (!cv || cv->ctx != c) NNV_FAIL(NNVHIP_ERR_ARG, "invalid layer handle");
   NNV_TRY(check_set_array(c, count, in, out));
   if (H <= 0 || W <= 0) NNV_FAIL(NNVHIP_ERR_SHAPE, "The input is not an ImageStar object");
@@ -68,12 +75,23 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
       pl.compact = conv2d_in_windows(cv, H, W, Ho, Wo, in[i]->ld, pl.dense, in[i]->box, pl.dense_eh, pl.dense_ew);
     }
   }
+  // Images with windows go by output position (conv_window.hip), which leaves their range sums too; not when the caller
+  // wants every column in memory (the zeros around the windows are then written first).
+  auto by_position = [&](const Plan& pl) {
+    return !c->eager_cols && pl.out_boxes && pl.compact && conv_window_takes(cv, H, W, Ho, Wo, pl.dense, pl.dense_eh, pl.dense_ew);
+  };
   {
     // The implicit GEMM reads whole images: pending row resets are run first, and sets whose unit-vector
     // columns take part in the contraction get those written out.  (A pending reset alone is applied by the
     // kernel as it loads, from one bit per row, where that fits; images that are in memory inside their windows
     // only are fine for the kernel that stays inside the windows.)
-    std::vector<nnvhip_star*> full, prefix;
+    // Images kept pixel by pixel are for the kernel that goes by output position; another one gets their columns first.
+    std::vector<nnvhip_star*> full, prefix, columns;
+    for (int64_t i = 0; i < count; ++i) {
+      const ColSource& cs = in[i]->cs;
+      if (cs.in_pixels() && !by_position(plan[i])) columns.push_back(in[i]);
+    }
+    if (st == NNVHIP_OK && !columns.empty()) st = write_pending_columns(c, (int64_t)columns.size(), columns.data());
     for (int64_t i = 0; i < count; ++i) {
       const ColSource& cs = in[i]->cs;
       if (plan[i].dense > in[i]->stored_cols())
@@ -91,17 +109,63 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
     max_m = std::max<int64_t>(max_m, plan[i].m);
   }
   const int64_t sch = any_stamps && st == NNVHIP_OK ? conv_stamp_chunks(cv, outs[0]->ld, count, max_m) : 0;
-  // Images with windows go by output position (conv_window.hip), which leaves their range sums too; not when the caller
-  // wants every column in memory (the zeros around the windows are then written first).
   std::vector<int64_t> parts((size_t)count, 0), chunk_at((size_t)count + 1, 0);  // parts > 0: by position
   for (int64_t i = 0; i < count; ++i) {
     const Plan& pl = plan[i];
-    if (!c->eager_cols && pl.out_boxes && pl.compact && conv_window_takes(cv, H, W, Ho, Wo, pl.dense, pl.dense_eh, pl.dense_ew))
+    if (by_position(pl))
       parts[(size_t)i] = conv_window_parts(cv, Ho, Wo, pl.dense, pl.dense_eh, pl.dense_ew);
     chunk_at[(size_t)i + 1] = chunk_at[(size_t)i] + parts[(size_t)i] + sch;
   }
   BufRef sums;
   if (chunk_at[(size_t)count] > 0 && st == NNVHIP_OK) st = c->alloc(sizeof(double) * 4 * outs[0]->ld * chunk_at[(size_t)count], &sums);
+  // Bound on the windows of a set's output columns.
+  auto out_extent = [&](const Plan& pl, int64_t* eh, int64_t* ew) {
+    *eh = pl.dense > 1 ? pl.dense_eh : 0;
+    *ew = pl.dense > 1 ? pl.dense_ew : 0;
+    if (pl.m > 0) {
+      *eh = std::max(*eh, conv_box_extent(cv, 0, 1, Ho));
+      *ew = std::max(*ew, conv_box_extent(cv, 1, 1, Wo));
+    }
+  };
+  // The output's images are kept pixel by pixel (ColSource::pix) where every one of them is made by a kernel that can write
+  // them so, and the layer behind the next ReLU step is known and will read them so: another reader would have the columns
+  // written first, which costs what is saved here.
+  auto keep_pixels = [&](int64_t i) {
+    const Plan& pl = plan[(size_t)i];
+    if ((behind_conv == nullptr && behind_fc == nullptr) || c->eager_cols || c->eager_rows || c->eager_tail || c->dense_affine) return false;
+    if (!pl.out_boxes || pl.nc < 2 || (pl.dense > 1 && parts[(size_t)i] == 0) || (pl.m > 0 && !conv_stamps_by_pixel(cv)) || cv->Wk == nullptr)
+      return false;
+    int64_t eh = 0, ew = 0;
+    out_extent(pl, &eh, &ew);
+    if (eh < 1 || ew < 1) return false;
+    const int64_t ldo = round_up(Nout, kLdAlign);
+    if (behind_conv != nullptr) {
+      int64_t H2 = 0, W2 = 0;
+      if (behind_conv->ctx != c || behind_conv->Cin != cv->Cout || c->no_conv_mask || nnvhip_conv2d_output_size(behind_conv, Ho, Wo, &H2, &W2) != NNVHIP_OK)
+        return false;
+      const int eh2 = (int)conv_box_extent(behind_conv, 0, eh, H2), ew2 = (int)conv_box_extent(behind_conv, 1, ew, W2);
+      return conv2d_can_mask(behind_conv, Ho, Wo, H2, W2, ldo) &&
+             conv2d_in_windows(behind_conv, Ho, Wo, H2, W2, ldo, pl.nc, &kAnyBox, eh2, ew2) &&
+             conv_window_takes(behind_conv, Ho, Wo, H2, W2, pl.nc, eh2, ew2);
+    }
+    return behind_fc->ctx == c && behind_fc->K == Nout && pl.nc <= 65535 &&
+           (double)behind_fc->Mp * (double)behind_fc->Kp * (double)pl.nc * (double)count >= 4.0e6 &&
+           fc_window_tile_of(behind_fc, count, (pl.nc - 1) * count, Ho, Wo, eh, ew) > 0;
+  };
+  std::vector<int64_t> pix_at((size_t)count, -1);
+  BufRef pixels;
+  {
+    int64_t total = 0;
+    for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i) {
+      if (!keep_pixels(i)) continue;
+      int64_t eh = 0, ew = 0;
+      out_extent(plan[(size_t)i], &eh, &ew);
+      pix_at[(size_t)i] = total;
+      total += plan[(size_t)i].nc * round_up(eh * ew * cv->Cout, kLdAlign);  // (column 0, the centre, stays in the matrix)
+    }
+    if (total > 0) st = c->alloc(sizeof(double) * total, &pixels);
+    if (total > 0 && st == NNVHIP_OK && c->poison_pending) NNV_HIP_TRY(hipMemsetAsync(pixels->ptr, 0xff, sizeof(double) * total, c->stream));
+  }
   // windows of the output's columns and the pixel tables of the unit-vector columns: one buffer each, one launch
   std::vector<ConvSetup> setup((size_t)count);
   BufRef boxes, invs, orders;
@@ -155,11 +219,8 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
     nnvhip_star* o = outs[i];
     const ColBox* ob = nullptr;
     if (pl.out_boxes) {
-      int64_t eh = pl.dense > 1 ? pl.dense_eh : 0, ew = pl.dense > 1 ? pl.dense_ew : 0;
-      if (pl.m > 0) {
-        eh = std::max(eh, conv_box_extent(cv, 0, 1, Ho));
-        ew = std::max(ew, conv_box_extent(cv, 1, 1, Wo));
-      }
+      int64_t eh = 0, ew = 0;
+      out_extent(pl, &eh, &ew);
       ob = setup[(size_t)i].out_box;
       o->box_buf = boxes;
       o->box = ob;
@@ -194,6 +255,21 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
     stamps[i].m = (int32_t)pl.m;
     stamps[i].pixel_col = in[i]->oh_inv;
     stamps[i].win_only = (lazy && pl.m > 0) ? 1 : 0;
+    stamps[i].pix = nullptr;
+    if (pix_at[(size_t)i] >= 0) {
+      o->cs.pix_buf = pixels;
+      o->cs.pix = pixels->as<double>() + pix_at[(size_t)i];
+      o->cs.pix_ld = round_up((int64_t)o->box_eh * o->box_ew * cv->Cout, kLdAlign);
+      o->cs.pix_eh = o->box_eh;
+      o->cs.pix_ew = o->box_ew;
+      ++c->routes[NNVHIP_ROUTE_CONV_PIXELS];
+      if (pl.m > 0) {
+        stamps[i].pix = pixels->as<double>() + pix_at[(size_t)i] + pl.dense * o->cs.pix_ld;
+        stamps[i].pix_ld = o->cs.pix_ld;
+        stamps[i].pix_eh = o->box_eh;
+        stamps[i].pix_ew = o->box_ew;
+      }
+    }
     if (parts[(size_t)i] > 0) {
       const bool stamp = sch == 1 && pl.m > 0 && in[i]->oh_inv != nullptr && conv_stamps_by_pixel(cv);
       windows.push_back(ConvWindowSet{in[i], o, pl.dense, pl.dense_eh, pl.dense_ew, setup[(size_t)i].order, setup[(size_t)i].first, parts[(size_t)i],
@@ -297,6 +373,9 @@ int nnvhip_reach_layers(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, co
     // the set that is handed back is written in full by the layer that produces it
     const bool eager = l == n_layers - 1 && !c->eager_cols;
     if (eager) c->eager_cols = true;
+    const bool known = kind[l] == NNVHIP_LAYER_CONV2D && l + 2 < n_layers && kind[l + 1] == NNVHIP_LAYER_RELU;
+    c->behind_conv = known && kind[l + 2] == NNVHIP_LAYER_CONV2D ? static_cast<const nnvhip_conv2d*>(layer[l + 2]) : nullptr;
+    c->behind_fc = known && kind[l + 2] == NNVHIP_LAYER_FC ? static_cast<const nnvhip_fc*>(layer[l + 2]) : nullptr;
     switch (kind[l]) {
       case NNVHIP_LAYER_FC:
         st = nnvhip_affine_fc(c, static_cast<const nnvhip_fc*>(layer[l]), count, cur, dst);
@@ -317,6 +396,8 @@ int nnvhip_reach_layers(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, co
         st = NNVHIP_ERR_ARG;
     }
     if (eager) c->eager_cols = false;
+    c->behind_conv = nullptr;
+    c->behind_fc = nullptr;
     if (st == NNVHIP_OK) {
       cur = dst;
       done = l + 1;

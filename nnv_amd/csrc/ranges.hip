@@ -1161,7 +1161,7 @@ int launch_range_sums_mm(nnvhip_ctx* ctx, const nnvhip_fc* fc, int64_t count, co
 // Whether the range scan of a set reads its generator images inside their windows only: the windows must cover
 // every column the scan reads (all stored ones), describe this set's image, and be small next to it.
 static bool scan_in_windows(const nnvhip_star* t) {
-  if (t->box == nullptr || t->rows_pending || t->box_H <= 0 || t->box_W <= 0) return false;
+  if (t->box == nullptr || t->rows_pending || t->cs.in_pixels() || t->box_H <= 0 || t->box_W <= 0) return false;
   const int64_t P = (int64_t)t->box_H * t->box_W;
   if (t->N % P != 0 || t->box_cols < t->stored_cols()) return false;
   return 2 * (int64_t)t->box_eh * t->box_ew <= P;
@@ -1713,6 +1713,26 @@ __global__ __launch_bounds__(512) void zero_outside_windows_kernel(double* __res
   }
 }
 
+// Writes the columns [j0, j1) of images that are kept pixel by pixel (ColSource::pix) into the matrix, zeros around their
+// windows included.  Lane = one row, the waves of a block interleave columns.
+__global__ __launch_bounds__(512) void write_pixel_columns_kernel(double* __restrict__ V, int64_t ld, int64_t N, const ColBox* __restrict__ box,
+                                                                  int64_t j0, int64_t j1, int H, int W, int cols_per_chunk,
+                                                                  const double* __restrict__ pix, int64_t pix_ld, int eh, int ew, int C) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t r = (int64_t)blockIdx.x * 64 + lane;
+  if (r >= N) return;
+  const int c = (int)(r / ((int64_t)H * W)), p = (int)(r - (int64_t)c * H * W);
+  const int w = p / H, h = p - w * H;
+  const int64_t at = (int64_t)pix_slot(h, w, eh, ew) * C + c;
+  const int64_t ja = j0 + (int64_t)blockIdx.y * cols_per_chunk;
+  const int64_t jb = min(j1, ja + cols_per_chunk);
+  for (int64_t j = ja + wave; j < jb; j += 8) {
+    const ColBox b = box[j];
+    V[r + j * ld] = h >= b.h0 && h <= b.h1 && w >= b.w0 && w <= b.w1 ? pix[j * pix_ld + at] : 0.0;
+  }
+}
+
 static int write_window_zeros(nnvhip_ctx* ctx, double* V, int64_t ld, ColSource* cs) {
   const int64_t ncols = cs->win_to - cs->win_from;
   if (ncols > 0) {
@@ -1721,11 +1741,18 @@ static int write_window_zeros(nnvhip_ctx* ctx, double* V, int64_t ld, ColSource*
     int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(ceil_div(8192, row_blocks), ceil_div(ncols, 32)));
     const int64_t cpc = ceil_div(ncols, chunks);
     chunks = ceil_div(ncols, cpc);
-    hipLaunchKernelGGL(zero_outside_windows_kernel, dim3((unsigned)row_blocks, (unsigned)chunks), dim3(512), 0, ctx->stream, V, ld, rows,
-                       cs->win_box, cs->win_from, cs->win_to, (int)cs->win_H, (int)cs->win_W, (int)cpc);
+    if (cs->in_pixels())
+      hipLaunchKernelGGL(write_pixel_columns_kernel, dim3((unsigned)row_blocks, (unsigned)chunks), dim3(512), 0, ctx->stream, V, ld, rows,
+                         cs->win_box, cs->win_from, cs->win_to, (int)cs->win_H, (int)cs->win_W, (int)cpc, cs->pix, cs->pix_ld, (int)cs->pix_eh,
+                         (int)cs->pix_ew, (int)(rows / ((int64_t)cs->win_H * cs->win_W)));
+    else
+      hipLaunchKernelGGL(zero_outside_windows_kernel, dim3((unsigned)row_blocks, (unsigned)chunks), dim3(512), 0, ctx->stream, V, ld, rows,
+                         cs->win_box, cs->win_from, cs->win_to, (int)cs->win_H, (int)cs->win_W, (int)cpc);
     NNV_HIP_TRY(hipGetLastError());
   }
   cs->win_from = cs->win_to = 0;
+  cs->pix_buf.reset();
+  cs->pix = nullptr;
   return NNVHIP_OK;
 }
 

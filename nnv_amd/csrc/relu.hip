@@ -842,6 +842,8 @@ int ensure_dense_batch(nnvhip_ctx* ctx, int64_t count, nnvhip_star* const* sets,
       s->cs.pending = false;
       s->cs.zero_to = 0;
       s->cs.win_from = s->cs.win_to = 0;
+      s->cs.pix_buf.reset();
+      s->cs.pix = nullptr;
       s->cs.rows_reset = true;
       if (need_tail) s->vcols = -1;
     }
@@ -1235,6 +1237,8 @@ int relu_relax(nnvhip_ctx* ctx, int order, int64_t count, nnvhip_star* const* in
       o->cs.pending = false;
       o->cs.zero_to = 0;
       o->cs.win_from = o->cs.win_to = 0;
+      o->cs.pix_buf.reset();
+      o->cs.pix = nullptr;
       o->cs.rows_reset = true;
     }
     (fold_bounds && in_place[i] ? ctx->n_bounds_in_place : ctx->n_bounds_copied)++;

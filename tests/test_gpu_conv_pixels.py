@@ -1,0 +1,124 @@
+"""Convolution outputs kept pixel by pixel between two layers of one reach call: against the oracle and against the same layers called
+one by one (which write columns), with what is left unwritten poisoned; at the edges of channel tiles, windows that wrap around their
+bound, borders, strides, empty windows, one set and arrays.  And every other reader of such a set: its columns, a pooling, a row
+map, an FC layer without windows, a convolution that does not go by position.  Every case asserts which layers kept pixels.
+Tolerance: the products are the same, their sums of up to K = 1100 terms are added in another order, |difference| <= 2 K eps of the
+largest sum of magnitudes, which for these nets stays below 50 times the largest value: 2.5e-11."""
+import numpy as np
+import pytest
+
+from oracle import nnv_oracle as o
+from tests.gpu_util import assert_close, compare_sets
+
+pytestmark = pytest.mark.gpu
+TOL = 2.5e-11
+
+
+@pytest.fixture(scope="module")
+def nnv():
+    import nnv_amd
+    return nnv_amd
+
+
+def _layers(rs, hw, cin, convs, fc):
+    out, c, (h, w) = [], cin, hw
+    for k, s, p, co in convs:
+        out.append({"type": "conv", "W": rs.randn(k, k, c, co) / k, "b": rs.randn(co) * 0.1, "padding": [p] * 4, "stride": [s] * 2, "dilation": [1, 1]})
+        out.append({"type": "relu"})
+        h, w, c = (h + 2 * p - k) // s + 1, (w + 2 * p - k) // s + 1, co
+    if fc:
+        out.append({"type": "fc", "W": rs.randn(fc, h * w * c) / np.sqrt(h * w * c), "b": rs.randn(fc)})
+    return out
+
+
+# image, channels, (filter, stride, padding, channels) per layer, rows of an FC layer at the end (0: none), layers that keep pixels
+NETS = [
+    ((12, 11), 1, [(3, 1, 1, 16), (3, 1, 1, 16)], 0, 1),
+    ((13, 9), 2, [(3, 1, 0, 15), (3, 2, 1, 17), (3, 1, 1, 33)], 0, 1),
+    ((20, 22), 1, [(3, 1, 1, 17), (3, 1, 1, 40), (3, 2, 0, 64)], 70, 3),
+    ((24, 20), 3, [(5, 2, 2, 16), (3, 1, 1, 65)], 24, 2),
+    ((11, 11), 1, [(1, 2, 0, 40), (1, 1, 0, 60)], 100, 2),
+    ((17, 16), 1, [(3, 1, 1, 8), (3, 1, 1, 16)], 90, 0),         # the second convolution is too small to go by position
+]
+
+
+def _boxes(rs, hw, cin, count):
+    out = []
+    for i in range(count):
+        x = rs.rand(*hw, cin)
+        eps = 0.01 * (rs.rand(*hw, cin) < (2.0, 0.7, 0.05)[i % 3])
+        out.append((x - eps, x + eps))
+    return out
+
+
+def _one_by_one(nnv, net, sets):
+    out = []
+    for L in net.Layers:
+        sets = L.reach(sets, "relax-star-area", [], 1, None, "linprog")
+        out.append(sets)
+    return out
+
+
+@pytest.mark.parametrize("hw,cin,convs,fc,kept", NETS)
+@pytest.mark.parametrize("count", [1, 3])
+def test_pixels_between_layers(nnv, hw, cin, convs, fc, kept, count):
+    rs = np.random.RandomState(hw[0] + 31 * cin + len(convs))
+    layers = _layers(rs, hw, cin, convs, fc)
+    boxes = _boxes(rs, hw, cin, count)
+    ctx = nnv.default_context()
+    was = ctx.switch_is_on("poison_pending")
+    ctx.set_switch("poison_pending", True)
+    try:
+        net = nnv.NN.from_config(layers)
+        sets = [nnv.ImageStar(*b) for b in boxes]
+        before = ctx.routes()
+        net.reach(sets if count > 1 else sets[0], {"reachMethod": "relax-star-area", "relaxFactor": 1})
+        took = ctx.routes()["conv_pixels"] - before["conv_pixels"]
+        assert took <= kept * count and (took > 0) == (kept > 0), took
+        plain = _one_by_one(nnv, net, [nnv.ImageStar(*b) for b in boxes] if count > 1 else nnv.ImageStar(*boxes[0]))
+        assert ctx.routes()["conv_pixels"] - before["conv_pixels"] == took       # (nothing was known about the layers behind)
+        for i in range(count):
+            _, exp = o.nn_reach(layers, o.image_star_from_bounds(*boxes[i]), "relax-star-area", 1.0, keep=True)
+            for li, es in enumerate(exp):
+                ds, ps = (net.reachSet[li][i], plain[li][i]) if count > 1 else (net.reachSet[li], plain[li])
+                tag = "layer %d set %d" % (li + 1, i)
+                lb, ub = ds.estimateRanges()
+                plb, pub = ps.estimateRanges()
+                assert_close(lb, plb, tag + " lb", TOL)
+                assert_close(ub, pub, tag + " ub", TOL)
+                assert_close(np.array(ds.V), np.array(ps.V), tag + " V", TOL)
+                compare_sets(ds, es, tag, check_constraints=layers[li]["type"] == "relu")
+    finally:
+        ctx.set_switch("poison_pending", was)
+
+
+def test_other_readers_of_kept_pixels(nnv):
+    rs = np.random.RandomState(5)
+    hw, cin = (18, 16), 1
+    layers = _layers(rs, hw, cin, [(3, 1, 1, 16), (3, 1, 1, 32)], 40)
+    net = nnv.NN.from_config(layers)
+    (lb, ub), = _boxes(rs, hw, cin, 1)
+    readers = [nnv.layers.Conv2DLayer(rs.randn(3, 3, 16, 4), rs.randn(4), [1] * 4, [2, 2], [1, 1]),
+               nnv.layers_affine.AveragePooling2DLayer([2, 2], [2, 2], [0] * 4),
+               nnv.layers_affine.BatchNormalizationLayer(NumChannels=16, TrainedMean=rs.rand(16), TrainedVariance=rs.rand(16) + 0.5, Epsilon=1e-5,
+                                                         Scale=rs.rand(16), Offset=rs.randn(16)),
+               nnv.layers.FullyConnectedLayer(rs.randn(3, 16 * hw[0] * hw[1]), rs.randn(3)), nnv.layers.ReluLayer()]
+    ctx = nnv.default_context()
+    was = ctx.switch_is_on("poison_pending")
+    ctx.set_switch("poison_pending", True)
+    try:
+        plain = _one_by_one(nnv, net, nnv.ImageStar(lb, ub))
+        for at in (0, 1):                                    # the convolution's output, the ReLU step's (its rows not yet reset)
+            for L in readers:
+                before = ctx.routes()["conv_pixels"]
+                net.reach(nnv.ImageStar(lb, ub), {"reachMethod": "relax-star-area", "relaxFactor": 1})
+                assert ctx.routes()["conv_pixels"] > before
+                got = L.reach(net.reachSet[at], "relax-star-area", [], 1, None, "linprog")
+                exp = L.reach(plain[at], "relax-star-area", [], 1, None, "linprog")
+                tag = "%s on layer %d" % (type(L).__name__, at + 1)
+                assert_close(np.array(got.V), np.array(exp.V), tag, TOL)
+                for a, b in zip(got.estimateRanges(), exp.estimateRanges()):
+                    assert_close(a, b, tag, TOL)
+                assert_close(np.array(net.reachSet[at].V), np.array(plain[at].V), tag + ": its input", TOL)
+    finally:
+        ctx.set_switch("poison_pending", was)
