@@ -18,6 +18,7 @@
 #include <cstring>
 
 #include "internal.h"
+#include "lds_dma.h"
 #include "mfma_tile.h"
 #include "relu_sort.h"
 
@@ -497,13 +498,458 @@ __global__ __launch_bounds__(kChainThreads) void reach_chain_kernel(const ChainS
   if (tid < 2 * a.n_layers) counts[tid] = s_counts[tid];
 }
 
+// The same launch for networks no layer of which is wider than 64 neurons, every ReLU layer behind an FC layer: the set stays on the
+// compute unit.  What the kernel above spends its time on are trips to the cache: a layer's matrix goes out, is read back for
+// the row reset, and its kept rows, the weights and the bounds are read again by the next layer.  Here
+//  - eight waves: what every wave does for itself (the classification, addresses) costs the block half of what sixteen make of it;
+//  - the next FC layer's weights are on their way (in registers) while this one is multiplied;
+//  - the columns of a layer stay in the accumulators until its neurons are classified, and then leave for the output
+//    matrices and, only the kept rows and without gaps, for the LDS the next layer multiplies from; nothing that went out is
+//    read back, so no barrier waits for a store;
+//  - a neuron is a lane: every wave classifies all of them by itself, and they meet for the ranking only.
+// One box through 5 - 50 x 6 - 5: 48 us there, 38 here (43 with sixteen waves, 60 with four); 128 boxes 70 -> 51.
+constexpr int kLdsChainN = 64;     // widest layer
+constexpr int kLdsChainThreads = 512;
+constexpr int kLdsChainTiles = 8;  // column tiles of a wave
+// x summed over the four rows of 16 lanes, in every one of them
+__device__ __forceinline__ double sum_of_rows(double x) {
+  union {
+    double d;
+    unsigned w[2];
+  } a, b;
+  a.d = x;
+  {
+    const auto lo = __builtin_amdgcn_permlane32_swap(a.w[0], a.w[0], false, false), hi = __builtin_amdgcn_permlane32_swap(a.w[1], a.w[1], false, false);
+    a.w[0] = lo[0], b.w[0] = lo[1], a.w[1] = hi[0], b.w[1] = hi[1];
+    a.d = a.d + b.d;
+  }
+  const auto lo = __builtin_amdgcn_permlane16_swap(a.w[0], a.w[0], false, false), hi = __builtin_amdgcn_permlane16_swap(a.w[1], a.w[1], false, false);
+  a.w[0] = lo[0], b.w[0] = lo[1], a.w[1] = hi[0], b.w[1] = hi[1];
+  return a.d + b.d;
+}
+constexpr int kLdsChainStatic = 16 * 1024;  // bytes of LDS beside the dynamic part, at most
+struct ChainLds {
+  int32_t pred;    // doubles: where the predicate bounds lie in the dynamic LDS (the kept rows first), lower, then upper ones ...
+  int32_t ncap;    // ... room for so many of either
+  int32_t weights; // where the weights lie
+};
+
+__global__ __launch_bounds__(kLdsChainThreads) void reach_chain_lds_kernel(const ChainSet* __restrict__ sets, ChainSet one, ChainArgs a, ChainLds p) {
+  constexpr int NT = kLdsChainThreads, NW = NT / 64, kParts = NW * 16;
+  constexpr int kUnits = kLdsChainN / NW;  // columns of the appended unit vectors, to a wave
+  extern __shared__ __attribute__((aligned(16))) double lds[];
+  double* const sV = lds;             // kept row k of column j at j * ldv + k
+  double* const s_pl = lds + p.pred;
+  double* const s_pu = s_pl + p.ncap;
+  double* const sW = lds + p.weights;
+  __shared__ double part[4][kParts];  // [sum][column group * ld + row]: range sums of the contracted columns
+  __shared__ double gat[NW][2][kLdsChainN];  // ... of the columns that are columns of the weights, S+ / S-, by wave
+  __shared__ double cen[kLdsChainN], s_lb[kLdsChainN], s_ub[kLdsChainN];
+  __shared__ int s_keep[kLdsChainN], s_cross[kLdsChainN], s_rank[kLdsChainN];
+  __shared__ int s_counts[2 * kChainMaxLayers];
+  const ChainSet S = sets ? sets[blockIdx.x] : one;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, kq = lane >> 4;
+  double* const A = a.arena + (int64_t)blockIdx.x * a.set_stride;
+  int32_t* const IA = a.iarena + (int64_t)blockIdx.x * a.iset_stride;
+
+  // weights of a layer: pieces of 16 bytes (64 x 64 at most)
+  constexpr int kPieces = kLdsChainN * kLdsChainN / 2 / NT;
+  double2 wreg[kPieces];
+  auto load_weights = [&](const ChainLayer& L) {
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) {
+      const int e = 2 * (tid + u * NT);
+      wreg[u] = e < L.ldw * L.K ? *reinterpret_cast<const double2*>(L.W + e) : make_double2(0.0, 0.0);
+    }
+  };
+  auto store_weights = [&]() {  // (the LDS has room for 64 x 64, or for what the layers need)
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) {
+      const int e = 2 * (tid + u * NT);
+      if (e < p.pred - p.weights) *reinterpret_cast<double2*>(sW + e) = wreg[u];
+    }
+  };
+  load_weights(a.layers[0]);
+  // the input set: everything of it is asked for at once
+  const int N = S.N;
+  int n = S.n;                   // predicates of the current set
+  int nk = N, ldv = N | 1;       // its rows in the LDS (an odd stride: 16 columns meet 16 bank pairs)
+  int nd = n + 1, mg = 0;        // columns there; unit vectors of s_cross behind them
+  const int order = a.order, n_layers = a.n_layers;
+  const bool box = S.idx != nullptr;  // column 1 + t is scale[idx[t]] at row idx[t], the centre is in memory
+  double in[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int j = wave + NW * u;
+    in[u] = lane < N && j <= (box ? 0 : n) ? S.V[lane + (int64_t)j * S.ld] : 0.0;
+  }
+  const double scale = box && tid < N ? S.scale[tid] : 0.0;
+  const int hot = box && tid < n ? S.idx[tid] : 0;  // (a box has no more columns than rows)
+  const double pl0 = tid < n ? S.plb[tid] : 0.0, pu0 = tid < n ? S.pub[tid] : 0.0;
+  // The layer list is read through the scalar cache, a line or two a layer: all of it is brought in now, and so is a line of the
+  // later layers' weights per thread and step.
+  {
+    int touched = 0;
+#pragma unroll
+    for (int l = 0; l < kChainMaxLayers; ++l) touched ^= a.layers[l].kind ^ (int)a.layers[l].idx_off;
+    asm volatile("" ::"s"(touched));
+  }
+  int first = 0;  // lines in front of a layer's
+  for (int l = 1; l < n_layers; ++l) {
+    const ChainLayer& L = a.layers[l];
+    if (L.kind != NNVHIP_LAYER_FC) continue;
+    const int lines = L.ldw * L.K / 16, e = (tid - first) & (NT - 1);  // (at most 256)
+    if (e < lines) lds_dma16_at(L.W + (int64_t)e * 16, lds_addr_of(&gat[wave][0][0]));  // (nobody reads it there)
+    first += lines;
+  }
+  if (tid < n) {
+    s_pl[tid] = pl0;
+    s_pu[tid] = pu0;
+  }
+  for (int j = tid + NT; j < n; j += NT) {
+    s_pl[j] = S.plb[j];
+    s_pu[j] = S.pub[j];
+  }
+  if (tid < kLdsChainN) {
+    s_keep[tid] = tid;
+    cen[tid] = scale;
+  }
+  if (tid < 2 * n_layers) s_counts[tid] = 0;
+  if (box) {
+    for (int j = wave; j <= n; j += NW)
+      if (lane < N) sV[j * ldv + lane] = j == 0 ? in[0] : 0.0;
+    lds_barrier();
+    if (tid < n) sV[(1 + tid) * ldv + hot] = cen[hot];
+  } else {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (wave + NW * u <= n && lane < N) sV[(wave + NW * u) * ldv + lane] = in[u];
+    for (int j = wave + 4 * NW; j <= n; j += NW)
+      if (lane < N) sV[j * ldv + lane] = S.V[lane + (int64_t)j * S.ld];
+  }
+  store_weights();
+  wait_vm_lds<0>();  // (the touched weights have landed: their place is about to be used)
+  lds_barrier();
+
+  int relu_ord = 0;
+  for (int l = 0; l < n_layers;) {
+    const ChainLayer& L = a.layers[l];
+    const bool relu = l + 1 < n_layers && a.layers[l + 1].kind == NNVHIP_LAYER_RELU;
+    const int next = l + (relu ? 2 : 1);
+    const int M = L.M, ldo = L.ld, ldw = L.ldw, R = ldo / 16;
+    const int RW = R > 2 ? 4 : R, WC = NW / RW;
+    const int wr = wave % RW, wc = wave / RW;
+    const int row = wr * 16 + l16;  // of the tiles this lane has columns of
+    const bool tiles = wr < R;
+    const int CT = (nd + 15) / 16;
+    if (next < n_layers) load_weights(a.layers[next]);
+    const double bias = tiles && wc == 0 && kq == 0 && L.bias != nullptr ? L.bias[row] : 0.0;
+    if (tid < kLdsChainN) s_rank[tid] = 0;
+
+    // ---- Star.affineMap of the columns in the LDS (operand layout as above)
+    double4_t acc[kLdsChainTiles];
+#pragma unroll
+    for (int t = 0; t < kLdsChainTiles; ++t) acc[t] = double4_t{0.0, 0.0, 0.0, 0.0};
+    if (tiles) {
+      for (int k0 = 0; k0 < nk; k0 += 32) {  // eight products a round, their operands asked for together
+        int kk[8];
+        double bv[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) kk[u] = s_keep[min(k0 + 4 * u + kq, kLdsChainN - 1)];  // (past the list: some row's number)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) bv[u] = sW[(kk[u] & (kLdsChainN - 1)) * ldw + row];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) bv[u] = k0 + 4 * u + kq < nk ? bv[u] : 0.0;
+#pragma unroll
+        for (int t = 0; t < kLdsChainTiles; ++t) {
+          const int tc = wc + t * WC;
+          if (tc >= CT) break;
+          const double* col = sV + min(tc * 16 + l16, nd - 1) * ldv;  // (columns past the last one: computed and dropped)
+#pragma unroll
+          for (int u0 = 0; u0 < 8; u0 += 4) {
+            if (k0 + 4 * u0 >= nk) break;
+            double av[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) av[u] = col[min(k0 + 4 * (u0 + u) + kq, nk - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) av[u] = k0 + 4 * (u0 + u) + kq < nk ? av[u] : 0.0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[u], bv[u0 + u], acc[t], 0, 0, 0);
+          }
+        }
+      }
+      if (wc == 0 && kq == 0) {
+        acc[0][0] = acc[0][0] + bias;  // newV(:,1) = newV(:,1) + b
+        cen[row] = acc[0][0];
+      }
+      double x[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int t = 0; t < kLdsChainTiles; ++t) {
+        const int tc = wc + t * WC;
+        if (tc >= CT) break;
+        double pl[4], pu[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {  // (the centre and columns past the last one take no part)
+          const int col = tc * 16 + kq + 4 * r, j = min(max(col, 1), max(nd - 1, 1)) - 1;
+          pl[r] = s_pl[j];
+          pu[r] = s_pu[j];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int col = tc * 16 + kq + 4 * r;
+          const bool in = col >= 1 && col < nd;
+          const double vp = in ? fmax(acc[t][r], 0.0) : 0.0, vn = in ? fmin(acc[t][r], 0.0) : 0.0;
+          const double l0 = in ? pl[r] : 0.0, u0 = in ? pu[r] : 0.0;
+          x[0] = fma(vp, l0, x[0]);  // xmin1
+          x[1] = fma(vn, u0, x[1]);  // xmin2
+          x[2] = fma(vp, u0, x[2]);  // xmax1
+          x[3] = fma(vn, l0, x[3]);  // xmax2
+        }
+      }
+      // the four lane groups hold different columns of the same rows
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[q] = sum_of_rows(x[q]);
+      if (kq == 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) part[q][wc * ldo + row] = x[q];
+      }
+    }
+    // the appended unit vectors: W * e_r = W(:, r), and their range sums (bounds 0 / ub_r); a column to a wave, a row to a lane
+    double unit[kUnits];
+#pragma unroll
+    for (int s = 0; s < kUnits; ++s) unit[s] = 0.0;
+    if (mg > 0) {
+      double sp = 0.0, sn = 0.0;
+      int at[kUnits];
+      double u[kUnits];
+#pragma unroll
+      for (int s = 0; s < kUnits; ++s) {
+        const int t = min(wave + NW * s, mg - 1);
+        at[s] = s_cross[t];
+        u[s] = s_pu[nd - 1 + t];
+      }
+#pragma unroll
+      for (int s = 0; s < kUnits; ++s) {
+        if (wave + NW * s >= mg) break;
+        unit[s] = 0.0 + sW[at[s] * ldw + min(lane, ldo - 1)];
+      }
+#pragma unroll
+      for (int s = 0; s < kUnits; ++s) {
+        if (wave + NW * s >= mg) break;
+        sp = fma(fmax(unit[s], 0.0), u[s], sp);
+        sn = fma(fmin(unit[s], 0.0), u[s], sn);
+      }
+      gat[wave][0][lane] = sp;
+      gat[wave][1][lane] = sn;
+    }
+    lds_barrier();  // the sums are there; nobody reads this layer's weights, rows or lists any more
+    if (tid < 256) {  // the column groups in order, then the gathered columns; lb = (c + xmin1) + xmin2
+      const int i = wave * 16 + l16;  // kq: which sum
+      const int np = min(WC, CT), ng = kq == 1 || kq == 2 ? min(NW, mg) : 0;
+      const double c = cen[i];
+      double s = 0.0, t = 0.0;
+#pragma unroll
+      for (int w0 = 0; w0 < NW; w0 += 4) {  // four reads at a time
+        if (w0 >= np) break;
+        double v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = part[kq][min(min(w0 + u, np - 1) * ldo + i, kParts - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s += w0 + u < np ? v[u] : 0.0;
+      }
+      if (mg > 0) {
+        double g[NW];
+#pragma unroll
+        for (int u = 0; u < NW; ++u) g[u] = gat[min(u, min(NW, mg) - 1)][kq == 1][i];
+#pragma unroll
+        for (int u = 0; u < NW; ++u) t += u < ng ? g[u] : 0.0;
+      }
+      if (ng > 0) s += t;
+      const double s1 = __shfl(s, (lane + 16) & 63);
+      if (i < M && kq == 0) s_lb[i] = (c + s) + s1;
+      if (i < M && kq == 2) s_ub[i] = (c + s) + s1;
+    }
+    lds_barrier();
+    // ---- the ReLU layer: classification, a neuron to a lane, by every wave; the waves share the comparisons of the ranking
+    const double lo = lane < M ? s_lb[lane] : 0.0, up = lane < M ? s_ub[lane] : 1.0;
+    bool crossing = false, kept = lane < M;
+    int m = 0, inact = 0, nk_out = M, kpos = lane, rank = 0;
+    if (relu) {
+      const bool inactive = lane < M && (up <= 0.0);      // map1 = find(ub <= 0)
+      crossing = lane < M && (lo < 0.0) && (up > 0.0);    // map2 = find(lb < 0 & ub > 0)
+      kept = lane < M && !inactive && !crossing;
+      const unsigned long long bc = __ballot(crossing), bk = __ballot(kept), below = (1ull << lane) - 1ull;
+      m = __popcll(bc);
+      inact = __popcll(__ballot(inactive));
+      nk_out = __popcll(bk);
+      kpos = __popcll(bk & below);
+      rank = __popcll(bc & below);
+      if (order != NNVHIP_ORDER_INDEX && m > 1) {
+        // stable descending key sort by counting: areas = 0.5*(abs(ub).*abs(lb))  |  ub - lb  (nn/funcs/PosLin.m:1049-1052, 934-936)
+        const double key = order == NNVHIP_ORDER_AREA ? 0.5 * (fabs(up) * fabs(lo)) : up - lo;
+        const long long bits = __double_as_longlong(key);
+        int cnt = 0;
+        for (unsigned mine = (unsigned)(bc >> (kLdsChainN / NW * wave)) & ((1u << (kLdsChainN / NW)) - 1u); mine != 0; mine &= mine - 1) {
+          const int j = kLdsChainN / NW * wave + __builtin_ctz(mine);
+          const int jl = __builtin_amdgcn_readlane((int)(unsigned)(bits & 0xffffffffll), j), jh = __builtin_amdgcn_readlane((int)(bits >> 32), j);
+          const double kj = __longlong_as_double(((long long)jh << 32) | (unsigned)jl);
+          cnt += (kj > key || (kj == key && j < lane)) ? 1 : 0;
+        }
+        if (crossing && cnt) atomicAdd(&s_rank[lane], cnt);
+        lds_barrier();
+        rank = s_rank[lane];
+      }
+    }
+    // ---- what the next layer reads (everybody is past the last reader of what is overwritten)
+    const int ldv_out = nk_out | 1;
+    const bool more = next < n_layers;
+    if (more) store_weights();
+    const int kp = __shfl(kept ? kpos : -1, row & 63);  // place of this lane's tile row among the kept ones
+    if (tiles && more && kp >= 0) {
+#pragma unroll
+      for (int t = 0; t < kLdsChainTiles; ++t) {
+        const int tc = wc + t * WC;
+        if (tc >= CT) break;
+        double* const v = sV + (tc * 16 + kq) * ldv_out + kp;
+        const int left = nd - tc * 16 - kq;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (4 * r < left) v[4 * r * ldv_out] = acc[t][r];
+      }
+    }
+    if (more && mg > 0 && kept) {
+#pragma unroll
+      for (int s = 0; s < kUnits; ++s)
+        if (wave + NW * s < mg) sV[(nd + wave + NW * s) * ldv_out + kpos] = unit[s];
+    }
+    if (wave == 0) {
+      if (kept) s_keep[kpos] = lane;
+      if (crossing) {
+        s_cross[rank] = lane;
+        s_pl[n + rank] = 0.0;
+        s_pu[n + rank] = up;
+      }
+    }
+    // ---- the output sets, which nothing in this launch reads
+    double* const O = A + L.v_off;
+    double* const g = A + L.rng_off;
+    if (tid < M) {
+      g[tid] = lo;
+      g[ldo + tid] = up;
+    }
+    double* const O2 = relu ? A + a.layers[l + 1].v_off : nullptr;  // V' = [V with the inactive and crossing rows reset, unit vectors]
+    if (tiles) {
+      const bool stays = kp >= 0 || row >= M;  // rows [M, ld): zeros, W's padding rows
+#pragma unroll
+      for (int t = 0; t < kLdsChainTiles; ++t) {
+        const int tc = wc + t * WC;
+        if (tc >= CT) break;
+        double* const o = O + row + (int64_t)(tc * 16 + kq) * ldo;
+        double* const o2 = O2 + row + (int64_t)(tc * 16 + kq) * ldo;
+        const int left = nd - tc * 16 - kq;  // columns from this lane's first on
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (4 * r < left) o[4 * r * ldo] = acc[t][r];
+        if (relu) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (4 * r < left) o2[4 * r * ldo] = stays ? acc[t][r] : 0.0;
+        }
+      }
+    }
+    if (lane < ldo) {
+      if (mg > 0) {
+#pragma unroll
+        for (int s = 0; s < kUnits; ++s) {
+          const int t = wave + NW * s;
+          if (t >= mg) break;
+          O[lane + (int64_t)(nd + t) * ldo] = unit[s];
+          if (relu) O2[lane + (int64_t)(nd + t) * ldo] = kept || lane >= M ? unit[s] : 0.0;
+        }
+      }
+      for (int t = wave; t < m; t += NW) O2[lane + (int64_t)(n + 1 + t) * ldo] = crossing && rank == t ? 1.0 : 0.0;
+    }
+    if (relu) {
+      const ChainLayer& Q = a.layers[l + 1];
+      double* const P = A + Q.pred_off;    // new_pred_lb = [plb; 0], new_pred_ub = [pub; ub(index)]  (nn/funcs/PosLin.m:737-738)
+      double* const LU = A + Q.lbub_off;
+      int32_t* const cross_g = IA + Q.idx_off;
+      int32_t* const keep_g = cross_g + ldo;
+      for (int j = tid; j < n; j += NT) {
+        P[j] = s_pl[j];
+        P[Q.npad + j] = s_pu[j];
+      }
+      if (wave == 0) {
+        if (crossing) {
+          P[n + rank] = 0.0;
+          P[Q.npad + n + rank] = up;
+          LU[rank] = lo;
+          LU[ldo + rank] = up;
+          cross_g[rank] = lane;
+        }
+        if (kept) keep_g[kpos] = lane;
+      }
+      if (tid < 2 * (int)kLdAlign) {  // the kept-row list ends with -1 up to a whole group of 16 (at least one group)
+        const int end = max((nk_out + (int)kLdAlign - 1) / (int)kLdAlign * (int)kLdAlign, (int)kLdAlign);
+        if (nk_out + tid < end) keep_g[nk_out + tid] = -1;
+      }
+      if (tid == 0) {
+        s_counts[2 * (l + 1)] = m;
+        s_counts[2 * (l + 1) + 1] = inact;
+        if (a.mailbox != nullptr)
+          post_counts(a.mailbox + 2 * ((int64_t)relu_ord * a.n_sets + blockIdx.x), m, inact, a.mailbox_seq);
+      }
+      ++relu_ord;
+    }
+    nd = n + 1;
+    n += m;
+    mg = m;
+    nk = nk_out;
+    ldv = ldv_out;
+    l = next;
+    lds_barrier();
+  }
+  if (tid < 2 * a.n_layers) a.counts[(int64_t)blockIdx.x * a.n_layers * 2 + tid] = s_counts[tid];
+}
+
 // Worst-case layout of one set's slice of the arenas for the given layer list.
 struct ChainPlan {
   ChainArgs args{};
   std::vector<int64_t> ncap;  // worst-case predicate count of every layer's output
   int64_t doubles = 0, ints = 0;
   int n_relu = 0;
+  bool in_lds = false;  // reach_chain_lds_kernel takes it
+  ChainLds lds{};
+  int64_t lds_doubles = 0;
 };
+
+// Whether a set of at most n0_max predicates stays in the LDS through the planned layers, whatever crosses.
+static void plan_chain_lds(int64_t N0, int64_t n0_max, ChainPlan* plan) {
+  const ChainArgs& a = plan->args;
+  int64_t rows = 0, weights = 0, before = n0_max, dense = n0_max;  // predicates in front of the layer, and those that are not its ReLU layer's
+  if (N0 > kLdsChainN || a.layers[0].kind != NNVHIP_LAYER_FC) return;
+  rows = (n0_max + 1) * (N0 | 1);
+  for (int l = 0; l < a.n_layers; ++l) {
+    const ChainLayer& L = a.layers[l];
+    if (L.ld > kLdsChainN) return;
+    if (L.kind == NNVHIP_LAYER_FC) {
+      const int64_t groups = kLdsChainThreads / 64 / (L.ld > 32 ? 4 : L.ld / 16);  // of waves along the columns
+      if (ceil_div(dense + 1, 16) > groups * kLdsChainTiles) return;  // (the columns a ReLU layer appends are columns of the weights)
+      weights = std::max(weights, (int64_t)L.ldw * L.K);
+    } else if (a.layers[l - 1].kind != NNVHIP_LAYER_FC) {
+      return;
+    }
+    // (the columns a ReLU layer appends do not lie there; the last layer leaves nothing)
+    if (l + 1 < a.n_layers) rows = std::max(rows, (before + 1) * (L.M | 1));
+    dense = before;
+    before = plan->ncap[(size_t)l];
+  }
+  rows = round_up(rows, 2);
+  plan->lds = ChainLds{(int32_t)(rows + weights), (int32_t)std::max<int64_t>(before, 1), (int32_t)rows};
+  plan->lds_doubles = rows + weights + 2 * std::max<int64_t>(before, 1);
+  plan->in_lds = 8 * plan->lds_doubles + kLdsChainStatic <= 160 * 1024;
+}
 
 static bool plan_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, int64_t N0, int64_t n0_max,
                        ChainPlan* plan) {
@@ -556,6 +1002,7 @@ static bool plan_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, con
   plan->doubles = off;
   plan->ints = std::max<int64_t>(ioff, kLdAlign);
   plan->args.n_layers = (int32_t)n_layers;
+  plan_chain_lds(N0, n0_max, plan);
   return true;
 }
 
@@ -630,7 +1077,11 @@ int reach_small_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, cons
     NNV_TRY(c->upload(sets.data(), sizeof(ChainSet) * count, &tab));
     table = tab->as<ChainSet>();
   }
-  NNV_LAUNCH(c, c->kernel_timing, reach_chain_kernel, dim3((unsigned)count), dim3(kChainThreads), 0, table, sets[0], a);
+  if (plan.in_lds)
+    NNV_LAUNCH(c, c->kernel_timing, reach_chain_lds_kernel, dim3((unsigned)count), dim3(kLdsChainThreads), (unsigned)(8 * plan.lds_doubles), table,
+               sets[0], a, plan.lds);
+  else
+    NNV_LAUNCH(c, c->kernel_timing, reach_chain_kernel, dim3((unsigned)count), dim3(kChainThreads), 0, table, sets[0], a);
   NNV_HIP_TRY(hipGetLastError());
   // Handles of earlier arrays that were released but not let go yet go now, all of them, while the kernel runs: their
   // arenas are what the next call of this size takes (a thousand sets come to a gigabyte, and a queue that grows from
