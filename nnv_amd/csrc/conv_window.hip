@@ -64,6 +64,9 @@ struct ConvWinArgs {
   int32_t stamp_blocks;
 };
 
+// PIXELS: places in an image and positions of a filter that fit one word
+constexpr int kPosBits = 26, kNoPosition = 31;
+__device__ double g_zero[1];  // (never written)
 constexpr int kConvWinTaps = 1024;  // taps of a filter (FH * FW * Cin) at most
 constexpr int kConvWinStarts = 256;  // positions of an output window at most
 constexpr int kConvWinCols = 128;   // columns of a position listed at a time
@@ -71,7 +74,13 @@ constexpr int kConvWinCols = 128;   // columns of a position listed at a time
 // neighbouring positions, whose elements share lines of every image, meet in its L2.  Grid: (items, sets, channel tiles).
 // The first stamp_blocks blocks of a set write the stamps of its unit-vector columns (S lanes per output row): bound by
 // scattered stores, they share the compute units with the products.
-template <int TM, int TN, int WR, int WC, int S_LANES>
+//
+// PIXELS: every set's images are kept pixel by pixel (ColSource::pix).  A stage's operands are then half of the vector and LDS
+// instructions they are for columns: where a listed row lies in an image and which of the filter's positions it belongs to are
+// one word, a column's window is one bit per position, made once a tile, and an element that is not wanted is read from a zero
+// instead of being dropped later (a row of padding meets zeros, so its weights need not be).  32 x 32 x 3 network, second to
+// fourth layer: 38, 129 and 151 us with columns, 26, 97 and 108 with pixels through the same instructions, 22, 85 and 91 now.
+template <int TM, int TN, int WR, int WC, int S_LANES, bool PIXELS>
 __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_kernel(const ConvWinSet* __restrict__ table, ConvWinSet one, ConvWinArgs a) {
   constexpr int NT = 64 * WR * WC, NW = WR * WC;
   constexpr int KT = 16;
@@ -85,8 +94,9 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
   extern __shared__ __attribute__((aligned(16))) int s_rows[];  // kept input rows under the filter, by tap, -1 padded to whole pairs of stages ...
   int* const s_row = s_rows;
   int* const s_tap = s_rows + a.list;      // ... their taps ...
-  int* const s_pos = s_rows + 2 * a.list;  // ... their positions in the image: h | w << 16 (-1: none) ...
-  int* const s_off = s_rows + 3 * a.list;  // ... and, with images kept pixel by pixel, where they lie in one
+  int* const s_pos = s_rows + 2 * a.list;  // ... and their positions in the image: h | w << 16
+  // PIXELS: s_row and s_pos hold where a row lies in the centre and in the other images, | the filter's position << kPosBits
+  // (kNoPosition behind the list); s_tap where its weights lie
   __shared__ int s_col[kConvWinCols];
   __shared__ double s_pl[kConvWinCols], s_pu[kConvWinCols];
   __shared__ int s_from[kConvWinStarts], s_end[kConvWinStarts];
@@ -142,16 +152,14 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
     s_end[t] = h0 >= 0 ? S.first[s + 1] - s_from[t] : 0;
   }
   // kept rows under the filter, in tap order; of images kept pixel by pixel pixel by pixel, so that a stage's rows lie together
-  const bool pixels = S.in_pix != nullptr;
   int nrow = 0;
   const int hb = ph * a.g.sh - a.g.pt, wb = pw * a.g.sw - a.g.pl;
   for (int k0 = 0; k0 < a.g.K; k0 += NT) {
     int k = k0 + tid;
     bool keep = k < a.g.K;
-    int r = 0, h = 0, w = 0, ci = 0;
+    int r = 0, h = 0, w = 0, ci = 0, fh = 0, fw = 0;
     if (keep) {
-      int fh, fw;
-      if (pixels) {
+      if (PIXELS) {
         const int t = k / a.g.Cin;
         ci = k - t * a.g.Cin;
         fw = t / a.g.FH;
@@ -184,19 +192,24 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
     }
     if (keep) {
       const int at = before + __popcll(m & ((1ull << lane) - 1ull));
-      s_row[at] = r;
-      s_tap[at] = k;
-      s_pos[at] = h | (w << 16);
-      if (pixels) s_off[at] = pix_slot(h, w, S.in_eh, S.in_ew) * a.g.Cin + ci;
+      if (PIXELS) {
+        const int position = (fw * a.g.FH + fh) << kPosBits;
+        s_row[at] = r | position;
+        s_tap[at] = k * a.coutp;
+        s_pos[at] = (pix_slot(h, w, S.in_eh, S.in_ew) * a.g.Cin + ci) | position;
+      } else {
+        s_row[at] = r;
+        s_tap[at] = k;
+        s_pos[at] = h | (w << 16);
+      }
     }
     __syncthreads();
   }
   const int nk = max(2, (nrow + 2 * KT - 1) / (2 * KT) * 2);  // stages: an even number, so that the loop over them has no branch
   if (tid < nk * KT - nrow) {
-    s_row[nrow + tid] = -1;
+    s_row[nrow + tid] = PIXELS ? kNoPosition << kPosBits : -1;
     s_tap[nrow + tid] = 0;
-    s_pos[nrow + tid] = -1;
-    if (pixels) s_off[nrow + tid] = 0;
+    s_pos[nrow + tid] = PIXELS ? kNoPosition << kPosBits : 0;
   }
   int total = 0;
   for (int g = 0; g < runs; ++g) total += s_end[g];
@@ -273,19 +286,31 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
       // the images this thread stages: rows 2 * (tid % 8) and the next of every stage
       const int bk = 2 * (tid % (KT / 2));
       const double* img[B_PASS];
-      const int* at[B_PASS];  // where the listed rows lie in it
       ColBox bb[B_PASS];
+      const int* at[B_PASS];       // PIXELS: the list of where the rows lie in it ...
+      unsigned inside[B_PASS];     // ... and the filter's positions inside its window
 #pragma unroll
       for (int u = 0; u < B_PASS; ++u) {
         const int j = c0 + (tid + u * NT) / (KT / 2);
         bb[u] = ColBox{1, 0, 1, 0};
         img[u] = S.V;
-        at[u] = s_row;
+        at[u] = s_pos;
+        inside[u] = 0;
         if (j < n) {
           const int col = s_col[j];
           bb[u] = col == 0 ? ColBox{0, (int16_t)(a.g.H - 1), 0, (int16_t)(a.g.W - 1)} : S.in_box[col];
-          img[u] = pixels && col > 0 ? S.in_pix + (int64_t)col * S.in_pix_ld : S.V + (int64_t)col * S.ld;
-          at[u] = pixels && col > 0 ? s_off : s_row;
+          img[u] = PIXELS && col > 0 ? S.in_pix + (int64_t)col * S.in_pix_ld : S.V + (int64_t)col * S.ld;
+          if (PIXELS) {
+            if (col == 0) at[u] = s_row;
+            for (int fw = 0; fw < a.g.FW; ++fw) {
+              const int w = wb + fw * a.g.dw;
+              if (w < bb[u].w0 || w > bb[u].w1) continue;
+              for (int fh = 0; fh < a.g.FH; ++fh) {
+                const int h = hb + fh * a.g.dh;
+                inside[u] |= (h >= bb[u].h0 && h <= bb[u].h1 ? 1u : 0u) << (fw * a.g.FH + fh);
+              }
+            }
+          }
         }
       }
       // A stage's operands travel through registers while the two stages before it are multiplied.  Every load is issued
@@ -301,35 +326,42 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
         for (int u = 0; u < A_PASS; ++u) {
           const int idx = tid + u * NT;
           const int row = m0 + 2 * (idx % (TM / 2)), k = k0 + idx / (TM / 2);
-          g.a[u] = *reinterpret_cast<const double2*>(a.Wk + row + (int64_t)s_tap[k] * a.coutp);
-          g.use |= s_row[k] >= 0 ? 1u << u : 0u;
+          g.a[u] = *reinterpret_cast<const double2*>(a.Wk + row + (PIXELS ? s_tap[k] : (int64_t)s_tap[k] * a.coutp));
+          if (!PIXELS) g.use |= s_row[k] >= 0 ? 1u << u : 0u;
         }
 #pragma unroll
         for (int u = 0; u < B_PASS; ++u) {
-          auto pixel = [&](int k, unsigned bit) {
-            const int r = at[u][k], pos = s_pos[k];
-            const int h = pos & 0xffff, w = pos >> 16;  // (h past any window where there is no row)
-            const bool in = h >= bb[u].h0 && h <= bb[u].h1 && w >= bb[u].w0 && w <= bb[u].w1;
-            g.use |= in ? bit : 0u;
-            return in_global(in ? img[u] + r : S.V)[0];
-          };
-          g.b[u].x = pixel(k0 + bk, 1u << (16 + 2 * u));
-          g.b[u].y = pixel(k0 + bk + 1, 1u << (17 + 2 * u));
+          if (PIXELS) {
+            const int2 word = *reinterpret_cast<const int2*>(at[u] + k0 + bk);
+            auto element = [&](int x) { return in_global(inside[u] >> (x >> kPosBits) & 1u ? img[u] + (x & ((1 << kPosBits) - 1)) : g_zero)[0]; };
+            g.b[u].x = element(word.x);
+            g.b[u].y = element(word.y);
+          } else {
+            auto pixel = [&](int k, unsigned bit) {
+              const int r = s_row[k], pos = s_pos[k];
+              const int h = pos & 0xffff, w = pos >> 16;
+              const bool in = r >= 0 && h >= bb[u].h0 && h <= bb[u].h1 && w >= bb[u].w0 && w <= bb[u].w1;
+              g.use |= in ? bit : 0u;
+              return in_global(in ? img[u] + r : S.V)[0];
+            };
+            g.b[u].x = pixel(k0 + bk, 1u << (16 + 2 * u));
+            g.b[u].y = pixel(k0 + bk + 1, 1u << (17 + 2 * u));
+          }
         }
       };
       auto store_tiles = [&](int buf, const Regs& g) {
 #pragma unroll
         for (int u = 0; u < A_PASS; ++u) {
           const int idx = tid + u * NT;
-          const bool on = g.use >> u & 1;
+          const bool on = PIXELS || (g.use >> u & 1);
           *reinterpret_cast<double2*>(&Ws[buf][(idx / (TM / 2)) * LDA_S + 2 * (idx % (TM / 2))]) =
               make_double2(on ? g.a[u].x : 0.0, on ? g.a[u].y : 0.0);
         }
 #pragma unroll
         for (int u = 0; u < B_PASS; ++u) {
           const int j = (tid + u * NT) / (KT / 2);
-          Vs[buf][j * LDB_S + bk] = g.use >> (16 + 2 * u) & 1 ? g.b[u].x : 0.0;  // odd column stride: two 64-bit stores
-          Vs[buf][j * LDB_S + bk + 1] = g.use >> (17 + 2 * u) & 1 ? g.b[u].y : 0.0;
+          Vs[buf][j * LDB_S + bk] = PIXELS || (g.use >> (16 + 2 * u) & 1) ? g.b[u].x : 0.0;  // odd column stride: two 64-bit stores
+          Vs[buf][j * LDB_S + bk + 1] = PIXELS || (g.use >> (17 + 2 * u) & 1) ? g.b[u].y : 0.0;
         }
       };
       double4_t acc[FM][FN];
@@ -428,8 +460,14 @@ int conv_window_parts(const nnvhip_conv2d* cv, int64_t Ho, int64_t Wo, int64_t d
   return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, 32), (int64_t)(cols / 32.0)));
 }
 
-int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldout, int64_t count,
-                       const ConvWindowSet* sets) {
+bool conv_window_takes_pixels(const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t eh, int64_t ew) {
+  return cv->FH * cv->FW <= kNoPosition && H * W * cv->Cin < (int64_t(1) << kPosBits) && eh * ew * cv->Cin < (int64_t(1) << kPosBits) &&
+         cv->K * cv->coutp < (int64_t(1) << 31);
+}
+
+template <bool PIXELS>
+static int launch_windows(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldout, int64_t count,
+                          const ConvWindowSet* sets) {
   if (count < 1) return NNVHIP_OK;
   if (count > 65535) NNV_FAIL(NNVHIP_ERR_SHAPE, "at most 65535 sets per call");
   ConvWinArgs a{};
@@ -450,7 +488,7 @@ int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
                                 s.in->rows_pending ? s.in->cls : nullptr, s.order, s.first, s.out->V, s.out->plb, s.out->pub, s.part,
                                 (int32_t)s.parts, s.eh, s.ew, nullptr, nullptr, 0, 0, 1, 1, 1, 1, StampSet{}};
     ConvWinSet& t = tab[(size_t)i];
-    if (s.in->cs.in_pixels()) {
+    if (PIXELS) {
       t.in_pix = s.in->cs.pix;
       t.in_pix_ld = s.in->cs.pix_ld;
       t.in_eh = s.in->cs.pix_eh;
@@ -486,14 +524,14 @@ int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
   const bool wide_stamps = a.g.K > 32;  // lanes per output row as in the launch that shares the implicit GEMM's
   a.stamp_blocks = any_stamps ? (int32_t)round_up(ceil_div(ldout * (wide_stamps ? 8 : 1), nt), 8) : 0;
   const dim3 grid((unsigned)(a.stamp_blocks + 8 * a.per), (unsigned)count, (unsigned)ceil_div(cv->Cout, tm));
-  const size_t dyn = 4 * sizeof(int32_t) * (size_t)a.list;  // (also holds the stamps' tap table, 8 bytes a tap)
+  const size_t dyn = 3 * sizeof(int32_t) * (size_t)a.list;  // (also holds the stamps' tap table, 8 bytes a tap)
   NNV_TRY(ctx->kernel_timer_begin(ctx->kernel_timing));
 #define NNV_CONV_WINDOW(TM, WR, WC)                                                                                                    \
   do {                                                                                                                                \
     if (wide_stamps)                                                                                                                  \
-      NNV_LAUNCH(ctx, ctx->kernel_timing, (conv_window_kernel<TM, 32, WR, WC, 8>), grid, dim3(64 * WR * WC), dyn, table, tab[0], a);  \
+      NNV_LAUNCH(ctx, ctx->kernel_timing, (conv_window_kernel<TM, 32, WR, WC, 8, PIXELS>), grid, dim3(64 * WR * WC), dyn, table, tab[0], a);  \
     else                                                                                                                              \
-      NNV_LAUNCH(ctx, ctx->kernel_timing, (conv_window_kernel<TM, 32, WR, WC, 1>), grid, dim3(64 * WR * WC), dyn, table, tab[0], a);  \
+      NNV_LAUNCH(ctx, ctx->kernel_timing, (conv_window_kernel<TM, 32, WR, WC, 1, PIXELS>), grid, dim3(64 * WR * WC), dyn, table, tab[0], a);  \
   } while (0)
   if (tm == 16)
     NNV_CONV_WINDOW(16, 1, 2);
@@ -505,6 +543,14 @@ int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
   NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 12, flop));
   NNV_HIP_TRY(hipGetLastError());
   return NNVHIP_OK;
+}
+
+int launch_conv_window(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t ldout, int64_t count,
+                       const ConvWindowSet* sets) {
+  std::vector<ConvWindowSet> columns, pixels;
+  for (int64_t i = 0; i < count; ++i) (sets[i].in->cs.in_pixels() ? pixels : columns).push_back(sets[i]);
+  NNV_TRY(launch_windows<false>(ctx, cv, H, W, Ho, Wo, ldout, (int64_t)columns.size(), columns.data()));
+  return launch_windows<true>(ctx, cv, H, W, Ho, Wo, ldout, (int64_t)pixels.size(), pixels.data());
 }
 
 }  // namespace nnvhip

@@ -874,6 +874,8 @@ int conv2d_prepare_weights(nnvhip_ctx* ctx, nnvhip_conv2d* conv);  // builds con
 // conv_window.hip: the dense images 0 .. dense - 1 of sets with windows (ConvJob::in_box / out_box), by output position, with
 // their range sums.  The elements inside the output windows are written, nothing else.
 bool conv_window_takes(const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t dense, int eh, int ew);
+// ... and takes images that are kept pixel by pixel, in windows of at most eh x ew
+bool conv_window_takes_pixels(const nnvhip_conv2d* conv, int64_t H, int64_t W, int64_t eh, int64_t ew);
 int conv_window_parts(const nnvhip_conv2d* conv, int64_t Ho, int64_t Wo, int64_t dense, int eh, int ew);  // chunks of range sums of such a set
 struct ConvWindowSet {
   const nnvhip_star* in;

@@ -89,7 +89,7 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
     std::vector<nnvhip_star*> full, prefix, columns;
     for (int64_t i = 0; i < count; ++i) {
       const ColSource& cs = in[i]->cs;
-      if (cs.in_pixels() && !by_position(plan[i])) columns.push_back(in[i]);
+      if (cs.in_pixels() && !(by_position(plan[i]) && conv_window_takes_pixels(cv, H, W, cs.pix_eh, cs.pix_ew))) columns.push_back(in[i]);
     }
     if (st == NNVHIP_OK && !columns.empty()) st = write_pending_columns(c, (int64_t)columns.size(), columns.data());
     for (int64_t i = 0; i < count; ++i) {
@@ -146,7 +146,7 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
       const int eh2 = (int)conv_box_extent(behind_conv, 0, eh, H2), ew2 = (int)conv_box_extent(behind_conv, 1, ew, W2);
       return conv2d_can_mask(behind_conv, Ho, Wo, H2, W2, ldo) &&
              conv2d_in_windows(behind_conv, Ho, Wo, H2, W2, ldo, pl.nc, &kAnyBox, eh2, ew2) &&
-             conv_window_takes(behind_conv, Ho, Wo, H2, W2, pl.nc, eh2, ew2);
+             conv_window_takes(behind_conv, Ho, Wo, H2, W2, pl.nc, eh2, ew2) && conv_window_takes_pixels(behind_conv, Ho, Wo, eh, ew);
     }
     return behind_fc->ctx == c && behind_fc->K == Nout && pl.nc <= 65535 &&
            (double)behind_fc->Mp * (double)behind_fc->Kp * (double)pl.nc * (double)count >= 4.0e6 &&
