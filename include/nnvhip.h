@@ -193,6 +193,8 @@ NNVHIP_API int nnvhip_debug_weak_weight_hash(int on);
 NNVHIP_API int nnvhip_star_create(nnvhip_ctx* ctx, int64_t N, int64_t n, const double* V, const double* pred_lb,
                        const double* pred_ub, const double* C, const double* d, int64_t p,
                        nnvhip_star** out);
+/* dst[0 .. n) = src[0 .. n), host arrays that do not overlap; a large one is shared out to a few threads of the context. */
+NNVHIP_API int nnvhip_copy_host(nnvhip_ctx* ctx, int64_t n, const double* src, double* dst);
 /* Star(lb, ub), set/Star.m:220-237 with Box (set/Box.m:16-58): centre 0.5*(lb+ub), one
  * generator 0.5*(ub-lb)(i)*e_i per dimension with non-zero half-width, C = zeros(1,n), d = 0,
  * predicate bounds -1/+1.  Built on the device from the two N-vectors.  `count` boxes are given

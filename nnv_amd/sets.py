@@ -320,7 +320,11 @@ class Star:
         out = (C.c_void_p * count)()
         check(ctx.lib.nnvhip_star_from_box(ctx.handle, N, count, ptr(lbs), ptr(ubs), out))
         # state_lb / state_ub of the elements (set/Star.m:232-233) are columns of private copies
-        return SetArray(ctx, out, state=(lbs.copy(order="F"), ubs.copy(order="F")))
+        state = []
+        for a in (lbs, ubs):
+            state.append(np.empty((N, count), order="F"))
+            check(ctx.lib.nnvhip_copy_host(ctx.handle, a.size, ptr(a), ptr(state[-1])))
+        return SetArray(ctx, out, state=tuple(state))
 
     # ---- NNV properties ------------------------------------------------------------------
     @property
