@@ -706,9 +706,11 @@ __global__ __launch_bounds__(256) void keep_bits_kernel(const KeepBits* __restri
 template <int S>
 __global__ __launch_bounds__(256) void conv_stamp_rows_kernel(StampSet d, ConvGeom g, const double* __restrict__ Wt, const double* __restrict__ Wk,
                                                               int coutp, const int32_t* __restrict__ pixel_col, int64_t ldout) {
-  __shared__ int2 taps[kStampTapTable];
+  __shared__ __attribute__((aligned(16))) int2 taps[kStampTapTable];
+  __shared__ int cnt[4];
+  static_assert(sizeof(int2) * kStampTapTable >= 8192 + sizeof(int2) * kStampPixelTaps, "sums and list of the pass by position");
   if (d.pix != nullptr)
-    conv_stamp_pixels_block<S, 256>(blockIdx.x, taps, d, g, Wk, coutp, pixel_col, ldout);
+    conv_stamp_pixels_block<256>(blockIdx.x, reinterpret_cast<double*>(taps), cnt, taps + 1024, d, g, Wk, coutp, pixel_col, ldout);
   else
     conv_stamp_rows_block<S, 256>(blockIdx.x, taps, d, g, Wt, pixel_col, ldout);
 }
@@ -721,6 +723,7 @@ template <int TC, int WR, int WC, bool MASK, bool COMPACT, int S>
 __global__ __launch_bounds__(512) void conv2d_fast_stamps_kernel(ConvFastArgs a, const double* __restrict__ Wt,
                                                                  const ConvSet* __restrict__ table, ConvSet one) {
   static_assert(sizeof(int2) * kStampTapTable <= conv_fast_lds_bytes(TC), "the stamp blocks' tap table fits the tiles' LDS");
+  static_assert(8 * 2064 + sizeof(int2) * kStampPixelTaps <= conv_fast_lds_bytes(TC), "... and so do sums and list by position");
   __shared__ __attribute__((aligned(1024))) double lds[2 * kKt * (128 + TC)];
   extern __shared__ uint32_t keep_s[];  // row mask (MASK only)
   const ConvSet set = conv_set_of_block(table, one);
@@ -728,7 +731,8 @@ __global__ __launch_bounds__(512) void conv2d_fast_stamps_kernel(ConvFastArgs a,
   const int k = (p + 1) / set.stride;
   if ((p + 1) % set.stride == 0 && k <= a.stamp_blocks) {
     if (set.d.pix != nullptr)
-      conv_stamp_pixels_block<S, 512>(k - 1, reinterpret_cast<int2*>(lds), set.d, a.g, a.Wk, a.coutp, set.d.pixel_col, a.ldout);
+      conv_stamp_pixels_block<512>(k - 1, lds, reinterpret_cast<int*>(lds + 2048), reinterpret_cast<int2*>(lds + 2064), set.d, a.g, a.Wk, a.coutp,
+                                   set.d.pixel_col, a.ldout);
     else
       conv_stamp_rows_block<S, 512>(k - 1, reinterpret_cast<int2*>(lds), set.d, a.g, Wt, set.d.pixel_col, a.ldout);
     return;
@@ -841,7 +845,9 @@ static int launch_conv_fast(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, const Conv
   // lanes per output row of the stamp blocks: 8 for filters with many taps (beside the tile blocks that measured best:
   // CNN 32x32x3 0.747 ms against 0.752 with 16 lanes, 0.756 with 4, 0.782 with 32), else 1
   const bool wide_stamps = g.K > 32;
-  const int64_t stamp_blocks = stamps ? ceil_div(ldout * (wide_stamps ? 8 : 1), 512) : 0;
+  int64_t stamp_blocks = stamps ? ceil_div(ldout * (wide_stamps ? 8 : 1), 512) : 0;
+  for (const ConvSet& s : jobs)
+    if (stamps && s.d.pix != nullptr) stamp_blocks = std::max<int64_t>(stamp_blocks, conv_stamp_pixel_blocks(g.P, g.K, 512));
   a.stamp_blocks = (int)stamp_blocks;
   std::vector<ConvSet> sets = jobs;
   double rows = 0.0;
@@ -1128,11 +1134,12 @@ int launch_conv_stamps(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, int6
       if (pc == nullptr) NNV_FAIL(NNVHIP_ERR_ARG, "internal: stamps without their pixel table");
       if (!one.win_only)  // whole columns: the zeros first
         NNV_HIP_TRY(hipMemsetAsync(one.out, 0, sizeof(double) * (size_t)ldout * (size_t)one.m, ctx->stream));
+      const int64_t blocks = one.pix != nullptr ? conv_stamp_pixel_blocks(g.P, g.K, 256) : ceil_div(ldout * (g.K <= 32 ? 1 : 16), 256);
       if (g.K <= 32)
-        NNV_LAUNCH(ctx, ctx->kernel_timing && i == 0, conv_stamp_rows_kernel<1>, dim3((unsigned)ceil_div(ldout, 256)), dim3(256), 0, one, g,
+        NNV_LAUNCH(ctx, ctx->kernel_timing && i == 0, conv_stamp_rows_kernel<1>, dim3((unsigned)blocks), dim3(256), 0, one, g,
                    cv->W->as<double>(), cv->Wk ? cv->Wk->as<double>() : nullptr, (int)cv->coutp, pc, ldout);
       else
-        NNV_LAUNCH(ctx, ctx->kernel_timing && i == 0, conv_stamp_rows_kernel<16>, dim3((unsigned)ceil_div(ldout * 16, 256)), dim3(256), 0,
+        NNV_LAUNCH(ctx, ctx->kernel_timing && i == 0, conv_stamp_rows_kernel<16>, dim3((unsigned)blocks), dim3(256), 0,
                    one, g, cv->W->as<double>(), cv->Wk ? cv->Wk->as<double>() : nullptr, (int)cv->coutp, pc, ldout);
     }
     NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 5, bytes));

@@ -88,6 +88,7 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
   constexpr int LDA_S = TM + kPadRow, LDB_S = KT + kPadK;
   constexpr int A_VEC = TM * KT / 2, A_PASS = (A_VEC + NT - 1) / NT;
   constexpr int B_PASS = TN * KT / 2 / NT;
+  static_assert(NW * 256 <= 2 * TN * LDB_S, "the stamp blocks' sums fit the image stages");
   static_assert(A_PASS * NT == A_VEC && B_PASS * NT == TN * KT / 2 && kConvWinCols % TN == 0, "whole passes, whole tiles");
   __shared__ double Ws[2][KT * LDA_S];
   __shared__ double Vs[2][TN * LDB_S];
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
   if (blk < 0) {
     if (S.stamps.m > 0 && blockIdx.z == 0) {
       if (S.stamps.pix != nullptr)
-        conv_stamp_pixels_block<S_LANES, NT>(blockIdx.x, reinterpret_cast<int2*>(s_rows), S.stamps, a.g, a.Wk, a.coutp, S.stamps.pixel_col, a.ldo);
+        conv_stamp_pixels_block<NT>(blockIdx.x, &Vs[0][0], s_cnt, reinterpret_cast<int2*>(s_rows), S.stamps, a.g, a.Wk, a.coutp, S.stamps.pixel_col, a.ldo);
       else
         conv_stamp_rows_block<S_LANES, NT>(blockIdx.x, reinterpret_cast<int2*>(s_rows), S.stamps, a.g, a.Wt, S.stamps.pixel_col, a.ldo);
     }
@@ -481,7 +482,6 @@ static int launch_windows(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, i
   int64_t max_parts = 1;
   std::vector<ConvWinSet> tab((size_t)count);
   double flop = 0.0;
-  bool any_stamps = false;
   for (int64_t i = 0; i < count; ++i) {
     const ConvWindowSet& s = sets[i];
     tab[(size_t)i] = ConvWinSet{s.in->V, s.in->ld, s.in->box, s.out->box, s.in->rows_pending ? s.in->keep_bits : nullptr,
@@ -503,7 +503,6 @@ static int launch_windows(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, i
     if (s.stamp != nullptr) {
       static_assert(sizeof(ConvStampSet) == sizeof(StampSet), "same layout");
       memcpy(&tab[(size_t)i].stamps, s.stamp, sizeof(StampSet));
-      any_stamps = true;
     }
     max_parts = std::max<int64_t>(max_parts, s.parts);
     ++ctx->routes[NNVHIP_ROUTE_CONV_WINDOW];
@@ -522,9 +521,15 @@ static int launch_windows(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, int64_t H, i
   const int tm = conv_window_tile(cv);
   const int nt = tm == 16 ? 128 : 256;
   const bool wide_stamps = a.g.K > 32;  // lanes per output row as in the launch that shares the implicit GEMM's
-  a.stamp_blocks = any_stamps ? (int32_t)round_up(ceil_div(ldout * (wide_stamps ? 8 : 1), nt), 8) : 0;
+  int64_t stamp_blocks = 0;
+  for (int64_t i = 0; i < count; ++i)
+    if (sets[i].stamp != nullptr)
+      stamp_blocks = std::max<int64_t>(stamp_blocks, sets[i].stamp->pix != nullptr ? conv_stamp_pixel_blocks(a.g.P, a.g.K, nt)
+                                                                                     : ceil_div(ldout * (wide_stamps ? 8 : 1), nt));
+  a.stamp_blocks = (int32_t)round_up(stamp_blocks, 8);
   const dim3 grid((unsigned)(a.stamp_blocks + 8 * a.per), (unsigned)count, (unsigned)ceil_div(cv->Cout, tm));
-  const size_t dyn = 3 * sizeof(int32_t) * (size_t)a.list;  // (also holds the stamps' tap table, 8 bytes a tap)
+  // (also holds the stamps' tap table, 8 bytes a tap, or a wave's 64 columns each)
+  const size_t dyn = std::max(3 * sizeof(int32_t) * (size_t)a.list, sizeof(int2) * (size_t)nt);
   NNV_TRY(ctx->kernel_timer_begin(ctx->kernel_timing));
 #define NNV_CONV_WINDOW(TM, WR, WC)                                                                                                    \
   do {                                                                                                                                \

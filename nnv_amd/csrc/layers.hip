@@ -133,7 +133,7 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
   auto keep_pixels = [&](int64_t i) {
     const Plan& pl = plan[(size_t)i];
     if ((behind_conv == nullptr && behind_fc == nullptr) || c->eager_cols || c->eager_rows || c->eager_tail || c->dense_affine) return false;
-    if (!pl.out_boxes || pl.nc < 2 || (pl.dense > 1 && parts[(size_t)i] == 0) || (pl.m > 0 && !conv_stamps_by_pixel(cv)) || cv->Wk == nullptr)
+    if (!pl.out_boxes || pl.nc < 2 || (pl.dense > 1 && parts[(size_t)i] == 0) || (pl.m > 0 && !(conv_stamps_by_pixel(cv) && cv->K <= 1024)) || cv->Wk == nullptr)
       return false;
     int64_t eh = 0, ew = 0;
     out_extent(pl, &eh, &ew);
