@@ -47,14 +47,15 @@ MIN_WARM_SECONDS = 0.3
 
 # kernels whose launches a timed group of the library covers (nnvhip_kernel_time), by the group's label below
 GROUP_KERNELS = {
-    "gemm_f64_kernel": ("gemm_f64_kernel",),
+    "gemm_f64_kernel": ("gemm_f64_kernel", "gemm_gather_kernel"),
     "gemm_seg_kernel": ("gemm_seg_kernel",),
     "conv2d_fast_kernel": ("conv2d_fast_kernel", "conv2d_fast_stamps_kernel", "conv2d_f64_kernel"),
     "conv_window_kernel": ("conv_window_kernel",),
     "fc_window_kernel": ("fc_window_kernel",),
     "gather_columns_kernel": ("gather_columns_kernel", "gather_skinny_kernel", "fc_rowsum_kernel", "conv_stamp_kernel", "conv_stamp_rows_kernel"),
     "ranges_partial_kernel": ("ranges_partial_kernel", "ranges_window_kernel"),
-    "relu_classify_kernel": ("relu_classify_kernel", "relu_count_kernel", "relu_compact_kernel"),
+    "relu_classify_kernel": ("relu_classify_kernel", "relu_classify_rank_kernel", "relu_count_kernel", "relu_compact_kernel"),
+    "reach_chain_kernel": ("reach_chain_kernel", "reach_chain_lds_kernel"),
 }
 
 
@@ -408,10 +409,10 @@ def measure(k, args, ctx, exact_steps, extras):
         groups.append((dlt_ms, g))
     if cls_launches:
         # classification, sort of the crossing list and the new predicate bounds: one block per set of up
-        # to 8192 neurons - with a single input set a dependent chain on one CU, bound by latency, which
-        # the fraction of the HBM peak then shows
+        # to 8192 neurons, several where there are few sets - with a single input set a dependent chain on a few
+        # CUs, bound by latency, which the fraction of the HBM peak then shows
         c = hbm_roofline("relu_classify_kernel", cls_ms, cls_launches, cls_bytes)
-        c["blocks_per_launch"] = n_sets
+        c["sets_per_launch"] = n_sets
         if n_sets < 256:
             c["latency_bound"] = True
         groups.append((cls_ms, c))

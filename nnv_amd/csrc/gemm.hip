@@ -1,6 +1,6 @@
 // affineMap of a fully connected layer: C = W * [c V] on fp64 MFMA (v_mfma_f64_16x16x4_f64).
 //
-// Both operands are staged through LDS in K-tiles of 16.  The MFMA operand roles are chosen for
+// Both operands are staged through LDS.  The MFMA operand roles are chosen for
 // column-major stores: the instruction's "b" operand carries 16 consecutive ROWS of W (the
 // memory-contiguous direction of C), its "a" operand 16 columns of V, so lane l, register r of
 // an accumulator holds C[row0 + l%16][col0 + l/16 + 4r] and lanes 0..15 store one 128-byte line.
@@ -212,8 +212,8 @@ __device__ double g_zero_rows[128];  // what a padding entry of a row list reads
 //  - The loop is unrolled over the ring: LDS addresses are lane constants plus immediate offsets.
 //  - Operands are read from LDS four rows ahead of the product they are for, over the end of a stage as well.
 // 1024 x 784 over 480 and 1920 rows: 30 and 91 us with the operands staged through registers one stage ahead, 18 and 59 us
-// now (32 x 64 tiles); 704 x 1501 over 1008 rows 74 -> 47 us; 2048 x 1024 over 1024 rows (64 x 64 tiles) 104 -> 64 us, 70 TFLOP/s at
-// 1920 rows, which is what the largest library product reaches here.
+// now (32 x 64 tiles); 704 x 1501 over 1008 rows 74 -> 47 us; 2048 x 1024 over 1024 rows (64 x 64 tiles) 104 -> 77 us inside a reach;
+// 70 TFLOP/s over 1920 rows, which is what the largest library product reaches here.
 //
 // A transfer (1 KB, a wave's 64 lanes x 16 bytes) of A holds whole rows k of the stage, lanes along the rows of W.  One of B
 // holds the KT rows of 128 / KT columns; LDS takes its pieces in lane order, so lanes fetch the 16-byte pieces of a column in
