@@ -1,9 +1,10 @@
 // A few threads of a context for work on host arrays that one thread's share of the memory bandwidth bounds.
 #pragma once
+#include <unistd.h>
+
 #include <condition_variable>
 #include <functional>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -12,6 +13,10 @@ namespace nnvhip {
 // run(parts, f) calls f(0) .. f(parts - 1), each once, on the calling thread and the workers, and returns when all are done.
 // f must not throw.  Workers start with the first call (a host that gives none: the caller does all of it) and sleep in
 // between.  One caller at a time, like the context it belongs to.
+//
+// A process that was forked off has no workers, only this object's memory, in whatever state the threads it does not have left
+// it: it starts workers of its own where it needs them, and never touches the old ones' lock, conditions (destroying one waits
+// for its waiters) and thread handles, which stay behind.
 class HostPool {
  public:
   static constexpr int kWorkers = 3;
@@ -19,67 +24,76 @@ class HostPool {
   HostPool(const HostPool&) = delete;
   HostPool& operator=(const HostPool&) = delete;
   ~HostPool() {
+    if (own_ == nullptr || pid_ != getpid()) return;
     {
-      std::lock_guard<std::mutex> lock(mu_);
-      stop_ = true;
+      std::lock_guard<std::mutex> lock(own_->mu);
+      own_->stop = true;
     }
-    wake_.notify_all();
-    for (auto& t : threads_) t.join();
+    own_->wake.notify_all();
+    for (auto& t : own_->threads) t.join();
+    delete own_;
   }
   void run(int parts, const std::function<void(int)>& f) {
-    if (parts > 1 && !started_) start();
-    if (parts < 2 || threads_.empty()) {
+    if (parts > 1 && (own_ == nullptr || pid_ != getpid())) start();
+    if (parts < 2 || own_ == nullptr || own_->threads.empty()) {
       for (int i = 0; i < parts; ++i) f(i);
       return;
     }
+    State& s = *own_;
     {
-      std::lock_guard<std::mutex> lock(mu_);
-      f_ = &f;
-      parts_ = parts;
-      next_ = 0;
-      left_ = parts;
+      std::lock_guard<std::mutex> lock(s.mu);
+      s.f = &f;
+      s.parts = parts;
+      s.next = 0;
+      s.left = parts;
     }
-    wake_.notify_all();
-    std::unique_lock<std::mutex> lock(mu_);
-    work(lock);
-    done_.wait(lock, [&] { return left_ == 0; });
-    f_ = nullptr;
+    s.wake.notify_all();
+    std::unique_lock<std::mutex> lock(s.mu);
+    s.work(lock);
+    s.done.wait(lock, [&] { return s.left == 0; });
+    s.f = nullptr;
   }
 
  private:
+  struct State {
+    std::mutex mu;
+    std::condition_variable wake, done;
+    std::vector<std::thread> threads;
+    const std::function<void(int)>* f = nullptr;
+    int parts = 0, next = 0, left = 0;
+    bool stop = false;
+    // Parts that nobody has taken yet; `lock` is held on entry and on return.
+    void work(std::unique_lock<std::mutex>& lock) {
+      while (next < parts) {
+        const int i = next++;
+        const std::function<void(int)>* g = f;
+        lock.unlock();
+        (*g)(i);
+        lock.lock();
+        if (--left == 0) done.notify_all();
+      }
+    }
+  };
   void start() {
-    started_ = true;
+    own_ = nullptr;  // (a forked process: its parent's)
+    pid_ = getpid();
     try {
-      threads_.reserve(kWorkers);
+      State* s = own_ = new State();
+      s->threads.reserve(kWorkers);
       for (int i = 0; i < kWorkers; ++i)
-        threads_.emplace_back([this] {
-          std::unique_lock<std::mutex> lock(mu_);
+        s->threads.emplace_back([s] {
+          std::unique_lock<std::mutex> lock(s->mu);
           for (;;) {
-            wake_.wait(lock, [&] { return stop_ || next_ < parts_; });
-            if (stop_) return;
-            work(lock);
+            s->wake.wait(lock, [&] { return s->stop || s->next < s->parts; });
+            if (s->stop) return;
+            s->work(lock);
           }
         });
     } catch (const std::exception&) {  // (those that did start are enough)
     }
   }
-  // Parts that nobody has taken yet; `lock` is held on entry and on return.
-  void work(std::unique_lock<std::mutex>& lock) {
-    while (next_ < parts_) {
-      const int i = next_++;
-      const std::function<void(int)>* f = f_;
-      lock.unlock();
-      (*f)(i);
-      lock.lock();
-      if (--left_ == 0) done_.notify_all();
-    }
-  }
-  std::mutex mu_;
-  std::condition_variable wake_, done_;
-  std::vector<std::thread> threads_;
-  const std::function<void(int)>* f_ = nullptr;
-  int parts_ = 0, next_ = 0, left_ = 0;
-  bool stop_ = false, started_ = false;
+  State* own_ = nullptr;
+  pid_t pid_ = 0;  // the process that started them
 };
 
 }  // namespace nnvhip
