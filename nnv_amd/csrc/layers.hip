@@ -373,7 +373,9 @@ int nnvhip_reach_layers(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, co
     // the set that is handed back is written in full by the layer that produces it
     const bool eager = l == n_layers - 1 && !c->eager_cols;
     if (eager) c->eager_cols = true;
-    const bool known = kind[l] == NNVHIP_LAYER_CONV2D && l + 2 < n_layers && kind[l + 1] == NNVHIP_LAYER_RELU;
+    // (a convolution at the end writes every column and does not go by position: it reads columns)
+    const bool known = kind[l] == NNVHIP_LAYER_CONV2D && l + 2 < n_layers && kind[l + 1] == NNVHIP_LAYER_RELU &&
+                       !(kind[l + 2] == NNVHIP_LAYER_CONV2D && l + 2 == n_layers - 1);
     c->behind_conv = known && kind[l + 2] == NNVHIP_LAYER_CONV2D ? static_cast<const nnvhip_conv2d*>(layer[l + 2]) : nullptr;
     c->behind_fc = known && kind[l + 2] == NNVHIP_LAYER_FC ? static_cast<const nnvhip_fc*>(layer[l + 2]) : nullptr;
     switch (kind[l]) {

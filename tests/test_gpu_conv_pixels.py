@@ -122,3 +122,22 @@ def test_other_readers_of_kept_pixels(nnv):
                 assert_close(np.array(net.reachSet[at].V), np.array(plain[at].V), tag + ": its input", TOL)
     finally:
         ctx.set_switch("poison_pending", was)
+
+
+@pytest.mark.parametrize("count", [1, 3])
+@pytest.mark.parametrize("convs,kept", [([(3, 1, 1, 16), (3, 1, 1, 40)], 0), ([(3, 1, 1, 17), (3, 1, 1, 40), (3, 2, 0, 64)], 1)])
+def test_a_convolution_at_the_end_reads_columns(nnv, convs, kept, count):
+    """The layer that hands the result back writes every column, which the kernel that reads pixels does not do."""
+    rs = np.random.RandomState(len(convs))
+    hw, cin = (20, 22), 1
+    layers = _layers(rs, hw, cin, convs, 0)[:-1]
+    boxes = _boxes(rs, hw, cin, count)
+    ctx = nnv.default_context()
+    net = nnv.NN.from_config(layers)
+    sets = [nnv.ImageStar(*b) for b in boxes]
+    before = ctx.routes()
+    out = net.reach(sets if count > 1 else sets[0], {"reachMethod": "relax-star-area", "relaxFactor": 1})
+    assert ctx.routes()["conv_pixels"] - before["conv_pixels"] == kept * count
+    for i in range(count):
+        exp = o.nn_reach(layers, o.image_star_from_bounds(*boxes[i]), "relax-star-area", 1.0)
+        compare_sets(out[i] if count > 1 else out, exp, "set %d" % i)
