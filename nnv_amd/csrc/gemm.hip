@@ -197,7 +197,7 @@ __device__ __forceinline__ double gemm_pred_bound(const GemmTile& t, int tid) {
   return v;
 }
 
-constexpr int kMapLds = 2048;  // entries of a row list that are copied into LDS
+constexpr int kMapLds = 2048;  // entries of a row list in LDS at a time
 __device__ double g_zero_rows[128];  // what a padding entry of a row list reads in place of a column of A (never written)
 
 // TM x TN output tile per block of WR x WC waves, each wave owning (TM/WR) x (TN/WC) = (16*FM) x (16*FN).
@@ -238,22 +238,42 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
     double pbs[2][TN];
     int kmap[MAPPED ? kMapLds : 1];
   };
+  static_assert(kMapLds / 2 % NT == 0 && kMapLds / 2 % KT == 0, "halves of whole stages, whole passes of the block");
   __shared__ __attribute__((aligned(1024))) Lds sm;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   GemmTile t;
   if (!gemm_tile_of<TM, TN, MAPPED>(g, &t)) return;
   const double pb_reg = gemm_pred_bound<TN>(t, tid);
-  const bool mapped = MAPPED && t.kmap != nullptr;          // uniform over the block, like ...
-  const bool map_lds = mapped && t.Kp <= kMapLds;
-  if (map_lds) {
-    for (int k = tid; k < t.Kp; k += NT) sm.kmap[k] = t.kmap[k];
-    __syncthreads();
-  }
+  const bool mapped = MAPPED && t.kmap != nullptr;  // uniform over the block
   // split-K: block row blockIdx.y owns the rows [k0, k0 + 16 * n16) and writes a partial product
   const int nk16 = t.Kp / 16;
   const int k16 = (int)((int64_t)nk16 * blockIdx.y / g.ksplit);
   const int n16 = (int)((int64_t)nk16 * (blockIdx.y + 1) / g.ksplit) - k16;
   const int k0 = k16 * 16;
+  // The transfers' row numbers come from LDS: a load from the list in memory would have to be waited for, and with it all
+  // transfers in flight.  (So would a choice between the two: it becomes one load that may go to either.)  Entry k of the
+  // block's rows lies at k % kMapLds; a longer list goes through there half by half, the next half when nobody needs the place of
+  // the last but one any more, which is the one such wait in kMapLds / 2 rows.  A lane reads its row numbers of a stage while
+  // it issues the one before.  100 x 1900 rows over 1200 columns, 512 x 4275 over 300, 512 x 8550 over 1200: with the choice 53,
+  // 135 and 536 us, from LDS alone 42, 89 and 387, read a stage ahead 36, 74 and 339.
+  auto copy_list = [&](int from, int to) {  // entries of the block's rows; at most half of kMapLds
+    constexpr int E = kMapLds / 2 / NT;
+    const int32_t* const list = in_global(t.kmap) + k0;
+    int v[E];
+#pragma unroll
+    for (int u = 0; u < E; ++u) v[u] = from + u * NT + tid < to ? list[from + u * NT + tid] : 0;
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+      if (from + u * NT + tid < to) sm.kmap[(from + u * NT + tid) % kMapLds] = v[u];
+  };
+  if (mapped) {
+    copy_list(0, min(16 * n16, kMapLds / 2));
+    copy_list(kMapLds / 2, min(16 * n16, kMapLds));
+    __syncthreads();
+  }
+  auto next_half = [&](int k) {  // in front of the transfers of rows k ..., behind a barrier behind those of the rows before
+    if (mapped && k != 0 && k % (kMapLds / 2) == 0) copy_list(k + kMapLds / 2, min(16 * n16, k + kMapLds));
+  };
   const bool half = KT == 32 && (n16 & 1);  // the last stage has 16 rows
   const int nk = KT == 32 ? (n16 + 1) / 2 : n16;
 
@@ -273,6 +293,15 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
 #pragma unroll
   for (int u = 0; u < UB; ++u) b_col[u] = (unsigned)((t.col_base + cb + u * kBStep < t.col_end ? cb + u * kBStep : 0) * ldb * 8);
   const unsigned lds0 = lds_addr_of(sm.ring) + wave * 1024;
+  const char* const a_row0 = reinterpret_cast<const char*>(g.A + ra);
+  const uint32_t lda8 = (uint32_t)g.lda * 8;
+  int a_row[UA];  // the listed rows that this lane's transfers of the stage to be issued next bring
+  auto rows_of_stage = [&](int st) {
+    const int rows = (KT == 32 && half && st == nk - 1) ? 16 : KT;
+#pragma unroll
+    for (int u = 0; u < UA; ++u) a_row[u] = sm.kmap[(st * KT + min(ka + u * kAStep, rows - 1)) % kMapLds];
+  };
+  if (mapped) rows_of_stage(0);
   // Stage st into place `slot` of the ring; stages are issued in order.  The rows a half stage does not have are read from
   // its last one and not multiplied.
   auto issue = [&](int st, int slot) {
@@ -281,10 +310,10 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
     if (mapped) {
 #pragma unroll
       for (int u = 0; u < UA; ++u) {
-        const int k = k0 + st * KT + min(ka + u * kAStep, rows - 1);
-        const int kk = map_lds ? sm.kmap[k] : t.kmap[k];
-        lds_dma16_at(kk >= 0 ? g.A + ra + (int64_t)kk * g.lda : g_zero_rows + 2 * lane, at + u * (NW * 1024));
+        const char* const row = a_row0 + (uint64_t)(uint32_t)a_row[u] * lda8;
+        lds_dma16_at(a_row[u] >= 0 ? reinterpret_cast<const double*>(row) : g_zero_rows + 2 * lane, at + u * (NW * 1024));
       }
+      if (st + 1 < nk) rows_of_stage(st + 1);
     } else if (rows == KT) {
 #pragma unroll
       for (int u = 0; u < UA; ++u) lds_dma16(a_base + (int64_t)u * kAStep * g.lda, a_off, at + u * (NW * 1024));
@@ -362,7 +391,10 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
         arrived(min(nk - 2 - st, S - 2));
         block_barrier();  // stage st + 1 is there, and nobody reads stage st any more: its place takes the next transfers
         read((slot + 1) % S, 0, f0);
-        if (st + S < nk) issue(st + S, slot);
+        if (st + S < nk) {
+          next_half((st + S) * KT);
+          issue(st + S, slot);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
       multiply(f1);

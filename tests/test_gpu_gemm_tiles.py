@@ -78,6 +78,25 @@ def test_product_over_kept_rows(nnv, count, M, K, n):
         assert np.all(np.abs(lb - elb) <= tol) and np.all(np.abs(ub - eub) <= tol), "ranges of set %d" % i
 
 
+@pytest.mark.parametrize("kept", [1023, 1024, 2016, 2048, 2049, 3072, 3088, 5000])
+@pytest.mark.parametrize("M,n", [(20, 30), (150, 70), (520, 300)])
+def test_long_lists_of_kept_rows(nnv, kept, M, n):
+    """The numbers of the kept rows go through LDS 2048 at a time, half by half; few output rows and columns split the contraction."""
+    rs = np.random.RandomState(kept + M)
+    K = kept + kept // 3
+    V = rs.randn(K, n + 1) * 0.01
+    V[:, 0] = -2.0 * n
+    V[np.sort(rs.permutation(K)[:kept]), 0] *= -1.0
+    S = nnv.Star(V, np.zeros((1, n)), np.zeros(1), -np.ones(n), np.ones(n))
+    W, b = rs.randn(M, K), rs.randn(M)
+    mid = nnv.layers.ReluLayer().reach(S, "relax-star-area", [], 1, None, "linprog")
+    out = nnv.layers.FullyConnectedLayer(W, b).reach(mid, "relax-star-area", [], 1, None, "linprog")
+    got = np.array(out.V)
+    keep = V[:, 0] > 0
+    assert mid.nVar == n and keep.sum() == kept
+    _check(got, W[:, keep], b, V[keep], "kept %d" % kept)
+
+
 def test_infinite_weight_meets_no_padding(nnv):
     """Rows a list is padded with are no rows of the set: an infinite weight in column 0 does not reach them."""
     rs = np.random.RandomState(3)
