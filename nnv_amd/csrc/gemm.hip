@@ -599,7 +599,15 @@ static int launch_cfg(nnvhip_ctx* ctx, const double* A, int64_t lda, const doubl
   // summed in split order by a second kernel (deterministic, no floating-point atomics).
   const int64_t nk = Kp / 16;
   int64_t ksplit = 1;
-  if (blocks < 128 && nk >= 8) ksplit = std::min<int64_t>(std::min<int64_t>(16, nk / 4), ceil_div(512, blocks));
+  // From 128 tiles on, one to a CU, that is worth its second kernel and the range sums that are no longer formed along the way only
+  // where the rows are listed (a stage then takes half as long again) and many for a tile's size.  Product and ReLU step behind it,
+  // in one part and in three: 100 x 950 rows over 1200 columns 56 us, 56; 100 x 1615 67, 60; 512 x 1900 over 300 68, 61; 512 x 4275
+  // 109, 82; 512 x 8550 180, 118; 1024 x 1900 over 300 (32 x 64 tiles) 81, 85; 1024 x 4275 136, 132; all rows of 200 x 2100 over 700
+  // 56, 61.
+  if (blocks < 128 && nk >= 8)
+    ksplit = std::min<int64_t>(std::min<int64_t>(16, nk / 4), ceil_div(512, blocks));
+  else if (rows != nullptr && rows->kmap != nullptr && blocks < 256 && 2 * Kp >= 3 * TM * TN)
+    ksplit = 512 / blocks;
   if (const int v = tune_knobs().gemm_ksplit) ksplit = std::max<int64_t>(1, std::min<int64_t>(v, nk));
   // the split-K workspace is laid out for one plain column range: no segment tables (a column map is
   // applied by the reduction)
