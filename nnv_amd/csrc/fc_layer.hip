@@ -249,6 +249,11 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
         work = !(in[i]->n_kept == 0 && in[i]->kept_idx != nullptr) &&
                (double)fc->Mp * (double)fc->Kp * (double)dense[i] * (double)count >= 4.0e6;
       if (work) win_tile = fc_window_tile(fc, count, in, dense.data());
+      // (the kernel takes images kept pixel by pixel of all sets or of none)
+      std::vector<nnvhip_star*> pixels;
+      for (int64_t i = 0; i < count; ++i)
+        if (in[i]->cs.in_pixels()) pixels.push_back(in[i]);
+      if (win_tile > 0 && !pixels.empty() && (int64_t)pixels.size() < count) st = write_pending_columns(c, (int64_t)pixels.size(), pixels.data());
     }
     // Inputs with columns that are described but not in memory yet: the contraction reads them from
     // memory unless it goes over no row at all or through the packing pass (which takes such columns

@@ -39,7 +39,7 @@ struct FcWinSet {
   const double* pub;
   double* rpart;              // [tiles][4][ldo] range sums
   int32_t ncols, tiles, nk, kper, cchunks;
-  // images kept pixel by pixel (ColSource::pix), or null
+  // images kept pixel by pixel (ColSource::pix), those of all sets or of none
   const double* pix;
   int64_t pix_ld;
   int32_t pix_eh, pix_ew;
@@ -126,9 +126,13 @@ __global__ __launch_bounds__(kSortThreads) void fc_window_setup_kernel(const FcW
 
 // TM x TN output tile per block of WR x WC waves.  Column tiles are dealt to the XCDs (blockIdx.x % 8) with all their row
 // tiles, which read the same images.  The last column tile of a set is its centre: the sum of the partial products.
-constexpr int kWinRows = 1024;  // rows a stage list holds; a union with more kept rows is walked in several lists
-template <int TM, int TN, int WR, int WC, int KT>
-__global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet* __restrict__ table, FcWinSet one, FcWinArgs a) {
+// PIXELS: every set's images are kept pixel by pixel (ColSource::pix).  A listed row then has a place in the image beside its number
+// and its position.  As one kernel for both ways, with lists of half the length and eight registers more, a CU held one block of
+// 64 x 64 less and unions of windows went through several lists: 25 images of 28 x 28 x 1 and of 40 x 40 x 1, column by column, 119 and
+// 245 us, 101 and 213 apart (101 and 206 before there were pixels); pixel by pixel 115 and 232, 101 and 204 now.
+constexpr int kWinRows = 2048, kWinPixelRows = 1536;  // rows a stage list holds; a union with more kept rows is walked in several lists
+template <int TM, int TN, int WR, int WC, int KT, bool PIXELS>
+__global__ __launch_bounds__(64 * WR * WC, TN == 64 ? 6 : 4) void fc_window_kernel(const FcWinSet* __restrict__ table, FcWinSet one, FcWinArgs a) {
   constexpr int NT = 64 * WR * WC, NW = WR * WC;
   constexpr int FM = TM / WR / 16, FN = TN / WC / 16;
   constexpr int LDA_S = TM + kPadRow, LDB_S = KT + kPadK;
@@ -136,9 +140,10 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
   __shared__ double Ws[2][KT * LDA_S];
   __shared__ double Vs[2][TN * LDB_S];
   // rows of the union's windows, -1 padded to whole stages: ascending; of images kept pixel by pixel pixel by pixel
-  __shared__ int s_row[kWinRows + KT];
-  __shared__ int s_pos[kWinRows + KT];  // their positions: h | w << 16 (-1: none) ...
-  __shared__ int s_off[kWinRows + KT];  // ... and where they lie in an image
+  constexpr int kRows = PIXELS ? kWinPixelRows : kWinRows;
+  __shared__ int s_row[kRows + KT];
+  __shared__ int s_pos[kRows + KT];  // their positions: h | w << 16 (-1: none) ...
+  __shared__ int s_pix[PIXELS ? kRows + KT : 1];  // ... and where they lie in an image kept pixel by pixel
   __shared__ int s_col[TN];
   __shared__ double s_pl[TN], s_pu[TN];
   __shared__ int s_u[4];
@@ -196,8 +201,7 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
   // the image this thread stages: rows 2 * (tid % 8) and the next of every stage, of column tid / 8
   const int bj = tid / (KT / 2), bk = 2 * (tid % (KT / 2));
   const int bcol = s_col[bj];
-  const bool pixels = S.pix != nullptr;
-  const double* img = pixels ? S.pix + (int64_t)max(bcol, 0) * S.pix_ld : S.V + (int64_t)max(bcol, 0) * S.ld;
+  const double* img = PIXELS ? S.pix + (int64_t)max(bcol, 0) * S.pix_ld : S.V + (int64_t)max(bcol, 0) * S.ld;
   ColBox bb = {1, 0, 1, 0};
   if (bcol >= 0) bb = S.box[bcol];
 
@@ -221,7 +225,7 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
       }
     }
     auto pixel = [&](int k) {
-      const int at = s_off[k], pos = s_pos[k];
+      const int at = PIXELS ? s_pix[k] : s_row[k], pos = s_pos[k];
       const int h = pos & 0xffff, w = pos >> 16;  // (h past any window where there is no row)
       return h >= bb.h0 && h <= bb.h1 && w >= bb.w0 && w <= bb.w1 ? img[at] : 0.0;
     };
@@ -241,13 +245,13 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
   const int wr = wave % WR, wc = wave / WR;
   for (int cand = 0; cand < total;) {
     int nrow = 0;
-    while (cand < total && nrow + NT <= kWinRows) {  // kept rows among the next NT of the union, ascending
+    while (cand < total && nrow + NT <= kRows) {  // kept rows among the next NT of the union, ascending
       const int e = cand + tid;
       bool keep = e < total;
       int r = 0, h = 0, w = 0, ch = 0;
       if (keep) {
         int q;
-        if (pixels) {
+        if (PIXELS) {
           q = e / a.C;
           ch = e - q * a.C;
         } else {
@@ -275,7 +279,7 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
         const int at = before + __popcll(m & ((1ull << lane) - 1ull));
         s_row[at] = r;
         s_pos[at] = h | (w << 16);
-        s_off[at] = pixels ? pix_slot(h, w, S.pix_eh, S.pix_ew) * a.C + ch : r;
+        if (PIXELS) s_pix[at] = pix_slot(h, w, S.pix_eh, S.pix_ew) * a.C + ch;
       }
       __syncthreads();
       cand += NT;
@@ -284,7 +288,7 @@ __global__ __launch_bounds__(64 * WR * WC) void fc_window_kernel(const FcWinSet*
     if (tid < nk * KT - nrow) {
       s_row[nrow + tid] = -1;
       s_pos[nrow + tid] = -1;
-      s_off[nrow + tid] = 0;
+      if (PIXELS) s_pix[nrow + tid] = 0;
     }
     __syncthreads();
     if (nk > 0) {
@@ -435,6 +439,7 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
     d.V = s->V;
     d.ld = s->ld;
     d.box = s->box;
+    if (s->cs.in_pixels() != f->cs.in_pixels()) NNV_FAIL(NNVHIP_ERR_ARG, "internal: images kept in different ways");
     if (s->cs.in_pixels()) {
       d.pix = s->cs.pix;
       d.pix_ld = s->cs.pix_ld;
@@ -463,8 +468,13 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
   hipLaunchKernelGGL(fc_window_setup_kernel, dim3((unsigned)(a.sort_blocks + max_chunks), (unsigned)count), dim3(kSortThreads), 0, ctx->stream, table,
                      tab[0], a);
   const dim3 grid((unsigned)(round_up(max_tiles + 1, 8) * a.tiles_m), (unsigned)count);
-#define NNV_FC_WINDOW(TM, TN, WR, WC, KT) \
-  NNV_LAUNCH(ctx, ctx->kernel_timing, (fc_window_kernel<TM, TN, WR, WC, KT>), grid, dim3(64 * WR * WC), 0, table, tab[0], a)
+#define NNV_FC_WINDOW(TM, TN, WR, WC, KT)                                                                                                      \
+  do {                                                                                                                                         \
+    if (f->cs.in_pixels())                                                                                                                     \
+      NNV_LAUNCH(ctx, ctx->kernel_timing, (fc_window_kernel<TM, TN, WR, WC, KT, true>), grid, dim3(64 * WR * WC), 0, table, tab[0], a);  \
+    else                                                                                                                                       \
+      NNV_LAUNCH(ctx, ctx->kernel_timing, (fc_window_kernel<TM, TN, WR, WC, KT, false>), grid, dim3(64 * WR * WC), 0, table, tab[0], a); \
+  } while (0)
   // (one small set: a block or none per CU, nothing to hide a stage's loads behind - stages of 32 rows, half as many)
   if (tm == 32 && tn == 32) NNV_FC_WINDOW(32, 32, 2, 2, 16);
   else if (tm == 32) NNV_FC_WINDOW(32, 64, 2, 4, 16);
