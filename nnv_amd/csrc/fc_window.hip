@@ -356,17 +356,24 @@ __global__ __launch_bounds__(64 * WR * WC, TN == 64 ? 6 : 4) void fc_window_kern
   }
 }
 
+static_assert(kFcWindowColumns == kSortColumns, "the columns' windows are sorted");
+
+bool fc_window_takes(const nnvhip_fc* fc, int64_t H, int64_t W) {
+  // (0 * Inf is NaN: the rows the union leaves out count then)
+  return fc->finite && H >= 1 && W >= 1 && H <= 8192 && W <= 8192 && fc->K % (H * W) == 0 && fc->K < (int64_t(1) << 31) && fc->Mp < (int64_t(1) << 20);
+}
+
 int fc_window_tile(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in, const int64_t* dense) {
   const nnvhip_star* f = in[0];
-  if (!fc->finite || f->box == nullptr || f->box_H < 1 || f->box_W < 1) return 0;  // (0 * Inf is NaN: the rows the union leaves out count then)
+  if (f->box == nullptr) return 0;
   const int64_t H = f->box_H, W = f->box_W;
-  if (H > 8192 || W > 8192 || fc->K % (H * W) != 0 || fc->K >= (int64_t(1) << 31) || fc->Mp >= (int64_t(1) << 20)) return 0;
+  if (!fc_window_takes(fc, H, W)) return 0;
   int64_t cols = 0;
   for (int64_t i = 0; i < count; ++i) {
     const nnvhip_star* s = in[i];
     const ColSource& cs = s->cs;
     if (s->box == nullptr || s->box_H != H || s->box_W != W || s->box_eh != f->box_eh || s->box_ew != f->box_ew) return 0;
-    if (dense[i] < 2 || dense[i] > kSortColumns || dense[i] > s->box_cols || dense[i] > s->stored_cols()) return 0;
+    if (dense[i] < 2 || dense[i] > kFcWindowColumns || dense[i] > s->box_cols || dense[i] > s->stored_cols()) return 0;
     // (unit-vector columns carry their one in a row the step has reset: they are the gather pass's)
     if (s->oh_from > 0 && dense[i] > s->oh_from) return 0;
     if (cs.pending || cs.zero_to > 1 || cs.delta_pending()) return 0;

@@ -980,6 +980,9 @@ int finalize_fused_ranges(nnvhip_ctx* ctx, nnvhip_star* s, const BufRef& part, i
 
 // fc_window.hip: the contraction of a fully connected layer over sets whose generator images are zero outside known windows
 // (nnvhip_star::box), tile by tile over the windows' union only.
+// Whether the layer may at all, over images of H x W positions ...
+bool fc_window_takes(const nnvhip_fc* fc, int64_t H, int64_t W);
+constexpr int64_t kFcWindowColumns = 65535;  // ... and columns of a set, at most
 // Columns per tile where the sets of a call (all of them) take it, 0: they do not.  dense: leading columns to contract.
 int fc_window_tile(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in, const int64_t* dense);
 // ... by the sizes alone: `cols` images of H x W positions in windows of at most eh x ew, in `count` sets

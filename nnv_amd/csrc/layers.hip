@@ -130,28 +130,43 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
   // The output's images are kept pixel by pixel (ColSource::pix) where every one of them is made by a kernel that can write
   // them so, and the layer behind the next ReLU step is known and will read them so: another reader would have the columns
   // written first, which costs what is saved here.
-  auto keep_pixels = [&](int64_t i) {
+  auto can_write_pixels = [&](int64_t i) {
     const Plan& pl = plan[(size_t)i];
     if ((behind_conv == nullptr && behind_fc == nullptr) || c->eager_cols || c->eager_rows || c->eager_tail || c->dense_affine) return false;
     if (!pl.out_boxes || pl.nc < 2 || (pl.dense > 1 && parts[(size_t)i] == 0) || (pl.m > 0 && !(conv_stamps_by_pixel(cv) && cv->K <= 1024)) || cv->Wk == nullptr)
       return false;
     int64_t eh = 0, ew = 0;
     out_extent(pl, &eh, &ew);
-    if (eh < 1 || ew < 1) return false;
-    const int64_t ldo = round_up(Nout, kLdAlign);
-    if (behind_conv != nullptr) {
-      int64_t H2 = 0, W2 = 0;
-      if (behind_conv->ctx != c || behind_conv->Cin != cv->Cout || c->no_conv_mask || nnvhip_conv2d_output_size(behind_conv, Ho, Wo, &H2, &W2) != NNVHIP_OK)
-        return false;
-      const int eh2 = (int)conv_box_extent(behind_conv, 0, eh, H2), ew2 = (int)conv_box_extent(behind_conv, 1, ew, W2);
-      return conv2d_can_mask(behind_conv, Ho, Wo, H2, W2, ldo) &&
-             conv2d_in_windows(behind_conv, Ho, Wo, H2, W2, ldo, pl.nc, &kAnyBox, eh2, ew2) &&
-             conv_window_takes(behind_conv, Ho, Wo, H2, W2, pl.nc, eh2, ew2) && conv_window_takes_pixels(behind_conv, Ho, Wo, eh, ew);
-    }
-    return behind_fc->ctx == c && behind_fc->K == Nout && pl.nc <= 65535 &&
-           (double)behind_fc->Mp * (double)behind_fc->Kp * (double)pl.nc * (double)count >= 4.0e6 &&
-           fc_window_tile_of(behind_fc, count, (pl.nc - 1) * count, Ho, Wo, eh, ew) > 0;
+    return eh >= 1 && ew >= 1;
   };
+  auto conv_reads_pixels = [&](int64_t i) {  // (which goes set by set)
+    const Plan& pl = plan[(size_t)i];
+    int64_t eh = 0, ew = 0, H2 = 0, W2 = 0;
+    out_extent(pl, &eh, &ew);
+    const int64_t ldo = round_up(Nout, kLdAlign);
+    if (behind_conv->ctx != c || behind_conv->Cin != cv->Cout || c->no_conv_mask || nnvhip_conv2d_output_size(behind_conv, Ho, Wo, &H2, &W2) != NNVHIP_OK)
+      return false;
+    const int eh2 = (int)conv_box_extent(behind_conv, 0, eh, H2), ew2 = (int)conv_box_extent(behind_conv, 1, ew, W2);
+    return conv2d_can_mask(behind_conv, Ho, Wo, H2, W2, ldo) &&
+           conv2d_in_windows(behind_conv, Ho, Wo, H2, W2, ldo, pl.nc, &kAnyBox, eh2, ew2) &&
+           conv_window_takes(behind_conv, Ho, Wo, H2, W2, pl.nc, eh2, ew2) && conv_window_takes_pixels(behind_conv, Ho, Wo, eh, ew);
+  };
+  auto fc_reads_pixels = [&] {  // (which takes all sets of an array that way or none)
+    if (behind_fc->ctx != c || behind_fc->K != Nout || !fc_window_takes(behind_fc, Ho, Wo)) return false;
+    int64_t eh0 = 0, ew0 = 0, images = 0;
+    for (int64_t i = 0; i < count; ++i) {
+      if (!can_write_pixels(i)) return false;
+      int64_t eh = 0, ew = 0;
+      out_extent(plan[(size_t)i], &eh, &ew);
+      if (i == 0) eh0 = eh, ew0 = ew;
+      const int64_t nc = plan[(size_t)i].nc;
+      if (eh != eh0 || ew != ew0 || nc > kFcWindowColumns || (double)behind_fc->Mp * (double)behind_fc->Kp * (double)nc * (double)count < 4.0e6) return false;
+      images += nc - 1;
+    }
+    return fc_window_tile_of(behind_fc, count, images, Ho, Wo, eh0, ew0) > 0;
+  };
+  const bool for_fc = behind_fc != nullptr && st == NNVHIP_OK && fc_reads_pixels();
+  auto keep_pixels = [&](int64_t i) { return behind_conv != nullptr ? can_write_pixels(i) && conv_reads_pixels(i) : for_fc; };
   std::vector<int64_t> pix_at((size_t)count, -1);
   BufRef pixels;
   {

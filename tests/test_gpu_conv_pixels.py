@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 
 from oracle import nnv_oracle as o
-from tests.gpu_util import assert_close, compare_sets
+from tests.gpu_util import assert_close, compare_sets, flat_V
 
 pytestmark = pytest.mark.gpu
 TOL = 2.5e-11
@@ -141,3 +141,28 @@ def test_a_convolution_at_the_end_reads_columns(nnv, convs, kept, count):
     for i in range(count):
         exp = o.nn_reach(layers, o.image_star_from_bounds(*boxes[i]), "relax-star-area", 1.0)
         compare_sets(out[i] if count > 1 else out, exp, "set %d" % i)
+
+
+def test_an_fc_layer_that_reads_columns(nnv):
+    """An FC layer stays inside the windows of all sets of an array, or of none: not where a weight is infinite (0 * Inf is NaN), and not
+    where the windows of one set are others, as those of an image without generators."""
+    rs = np.random.RandomState(3)
+    hw, cin = (20, 22), 1
+    layers = _layers(rs, hw, cin, [(3, 1, 1, 16)], 70)
+    (box, _, _), point = _boxes(rs, hw, cin, 3), rs.rand(*hw, cin)
+    wild = [dict(L) for L in layers]
+    wild[-1]["W"] = layers[-1]["W"].copy()
+    wild[-1]["W"][3, 5] = np.inf
+    ctx = nnv.default_context()
+    for net, bounds, kept in ((layers, [box], 1), (layers, [box, box], 2), (layers, [box, (point, point)], 0), (wild, [box], 0)):
+        sets = [nnv.ImageStar(*b) for b in bounds]
+        before = ctx.routes()["conv_pixels"]
+        n = nnv.NN.from_config(net)
+        out = n.reach(sets if len(sets) > 1 else sets[0], {"reachMethod": "relax-star-area", "relaxFactor": 1})
+        assert ctx.routes()["conv_pixels"] - before == kept
+        plain = _one_by_one(nnv, n, [nnv.ImageStar(*b) for b in bounds] if len(sets) > 1 else nnv.ImageStar(*bounds[0]))[-1]
+        for i in range(len(sets)):
+            got, exp = (flat_V(x[i] if len(sets) > 1 else x) for x in (out, plain))
+            rows = np.arange(70) != 3 if net is wild else slice(None)
+            assert_close(got[rows], exp[rows], "set %d" % i, TOL)
+            assert np.array_equal(np.isfinite(got), np.isfinite(exp))
