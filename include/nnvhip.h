@@ -350,7 +350,8 @@ NNVHIP_API int nnvhip_set_small_chain(nnvhip_ctx* ctx, int enabled);
  * the product over the rows most sets keep once and contracting each set over its differences from that list),
  * "no_sum_shortcuts" (NNVHIP_NO_SUM_SHORTCUTS: where that layer sums its sets' pieces without storing them, every
  * set is summed in full and with both bounds of every predicate - not once per run of sets that agree in list and
- * bounds, and not with one bound where the bounds mirror each other; the sums are the same to the bit).
+ * bounds, and not with one bound where the bounds mirror each other; the sums are the same to the bit), "no_host_pool"
+ * (NNVHIP_NO_HOST_POOL: passes over large host arrays stay on the caller's thread, and the context starts none).
  * A switch applies to the layer calls made
  * after it; sets produced before keep what they recorded.  Unknown name: NNVHIP_ERR_ARG. */
 NNVHIP_API int nnvhip_set_switch(nnvhip_ctx* ctx, const char* name, int enabled);

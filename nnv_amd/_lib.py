@@ -38,7 +38,7 @@ SWITCH_ENV = {"dense_affine": "NNVHIP_DENSE_AFFINE", "eager_rows": "NNVHIP_EAGER
               "eager_cols": "NNVHIP_EAGER_COLS", "poison_pending": "NNVHIP_POISON_PENDING",
               "no_small_chain": "NNVHIP_NO_SMALL_CHAIN", "no_conv_mask": "NNVHIP_NO_CONV_MASK",
               "no_conv_boxes": "NNVHIP_NO_CONV_BOXES", "no_row_deltas": "NNVHIP_NO_ROW_DELTAS",
-              "no_sum_shortcuts": "NNVHIP_NO_SUM_SHORTCUTS"}
+              "no_sum_shortcuts": "NNVHIP_NO_SUM_SHORTCUTS", "no_host_pool": "NNVHIP_NO_HOST_POOL"}
 
 
 class NNVHipError(RuntimeError):

@@ -1,5 +1,6 @@
 // A few threads of a context for work on host arrays that one thread's share of the memory bandwidth bounds.
 #pragma once
+#include <sched.h>
 #include <unistd.h>
 
 #include <condition_variable>
@@ -11,15 +12,15 @@
 namespace nnvhip {
 
 // run(parts, f) calls f(0) .. f(parts - 1), each once, on the calling thread and the workers, and returns when all are done.
-// f must not throw.  Workers start with the first call (a host that gives none: the caller does all of it) and sleep in
-// between.  One caller at a time, like the context it belongs to.
+// f must not throw.  Workers start with the first call, no more than the process has CPUs beside the caller's (a host that gives
+// none: the caller does all of it), and sleep in between.  One caller at a time, like the context it belongs to.
 //
 // A process that was forked off has no workers, only this object's memory, in whatever state the threads it does not have left
 // it: it starts workers of its own where it needs them, and never touches the old ones' lock, conditions (destroying one waits
 // for its waiters) and thread handles, which stay behind.
 class HostPool {
  public:
-  static constexpr int kWorkers = 3;
+  static constexpr int kWorkers = 3;  // at most
   HostPool() = default;
   HostPool(const HostPool&) = delete;
   HostPool& operator=(const HostPool&) = delete;
@@ -79,8 +80,10 @@ class HostPool {
     pid_ = getpid();
     try {
       State* s = own_ = new State();
+      cpu_set_t cpus;
+      const int others = sched_getaffinity(0, sizeof cpus, &cpus) == 0 ? CPU_COUNT(&cpus) - 1 : kWorkers;
       s->threads.reserve(kWorkers);
-      for (int i = 0; i < kWorkers; ++i)
+      for (int i = 0; i < (others < kWorkers ? others : kWorkers); ++i)
         s->threads.emplace_back([s] {
           std::unique_lock<std::mutex> lock(s->mu);
           for (;;) {

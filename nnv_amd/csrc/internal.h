@@ -346,7 +346,8 @@ struct nnvhip_ctx {
   std::vector<nnvhip_star*> deferred;
   static constexpr size_t kMaxDeferred = 4096;
   void drain_deferred(size_t at_most = ~size_t(0));
-  nnvhip::HostPool host_pool;  // for large host arrays
+  nnvhip::HostPool host_pool;  // for large host arrays ...
+  bool no_host_pool = false;   // ... or the caller's thread does all of it (environment NNVHIP_NO_HOST_POOL)
   // counters for diagnosing a slow step: hipMalloc calls of the pool, waits for the stream because the pinned
   // staging ring wrapped or grew, mailbox waits that went through the slow path
   int64_t n_device_mallocs = 0, n_staging_waits = 0;

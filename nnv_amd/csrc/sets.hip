@@ -174,12 +174,12 @@ constexpr int64_t kBoxPiece = int64_t(1) << 20;
 // Host arrays of 1 MB and more are worth waking the context's workers for (some 20 us); several parts to a thread, so that
 // one that starts late costs little.
 constexpr int64_t kPoolDoubles = int64_t(1) << 17;
-static int host_parts(int64_t doubles) { return doubles >= kPoolDoubles ? 4 * (HostPool::kWorkers + 1) : 1; }
+static int host_parts(const nnvhip_ctx* c, int64_t doubles) { return doubles >= kPoolDoubles && !c->no_host_pool ? 4 * (HostPool::kWorkers + 1) : 1; }
 
 int nnvhip_copy_host(nnvhip_ctx* c, int64_t n, const double* src, double* dst) {
   if (!c) NNV_FAIL(NNVHIP_ERR_ARG, "null context");
   if (n < 0 || (n > 0 && (!src || !dst))) NNV_FAIL(NNVHIP_ERR_ARG, "null argument");
-  const int parts = host_parts(n);
+  const int parts = host_parts(c, n);
   c->host_pool.run(parts, [&](int part) {
     const int64_t a = n * part / parts, b = n * (part + 1) / parts;
     if (b > a) memcpy(dst + a, src + a, sizeof(double) * (size_t)(b - a));
@@ -211,7 +211,7 @@ int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* 
   // First pass: half-widths only (they decide the sizes); the centres are formed below, in their place.  Both passes over the
   // host arrays are bound by one thread's share of the memory bandwidth, so those of a large array are shared out: 1024 boxes of
   // 784 dimensions take 340 + 390 us on one thread (and their private copies 250); a reach of them 3.07 -> 2.05 ms.
-  const int parts = host_parts(count * N);
+  const int parts = host_parts(c, count * N);
   auto half_widths = [&](int64_t s) {
     const double *l = lb + s * N, *u = ub + s * N;
     for (int64_t i = 0; i < N; ++i) vec[(size_t)i] = 0.5 * (u[i] - l[i]);  // Box constructor, set/Box.m:36

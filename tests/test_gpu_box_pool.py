@@ -37,3 +37,13 @@ def test_boxes_of_large_arrays(nnv, N, count, widths):
         one = nnv.Star(klb[:, i], kub[:, i])
         assert sets[i].nVar == one.nVar and np.array_equal(sets[i].V, one.V)
         assert np.array_equal(sets[i].state_lb, klb[:, i]) and np.array_equal(sets[i].state_ub, kub[:, i])
+
+
+def test_without_threads(nnv):
+    ctx = nnv.default_context()
+    was = ctx.switch_is_on("no_host_pool")
+    ctx.set_switch("no_host_pool", True)
+    try:
+        test_boxes_of_large_arrays(nnv, 785, 1400, "few")
+    finally:
+        ctx.set_switch("no_host_pool", was)

@@ -1,6 +1,6 @@
 """The threads a context keeps for large host arrays (csrc/host_pool.h), in a program of their own: every part is done once, calls
-may follow one another, and a process forked off after the workers started has none of them: it must neither wait for them where
-it uses a pool of its parent's nor where it destroys one."""
+may follow one another, a process has no more of them than CPUs beside the caller's, and one forked off after the workers started
+has none of them: it must neither wait for them where it uses a pool of its parent's nor where it destroys one."""
 import os
 import shutil
 import subprocess
@@ -9,6 +9,8 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PROGRAM = r"""
+#include <dirent.h>
+#include <sched.h>
 #include <sys/wait.h>
 #include <unistd.h>
 
@@ -43,6 +45,29 @@ int main() {
     int status = 0;
     if (waitpid(child, &status, 0) != child || status != 0) return 3 + use;
   }
+  const pid_t child = fork();
+  if (child == 0) {  // a process that may use one CPU, or two: the caller and so many workers
+    alarm(20);
+    for (int cpus = 1; cpus <= 2; ++cpus) {
+      cpu_set_t all, some;
+      if (sched_getaffinity(0, sizeof all, &all) != 0 || CPU_COUNT(&all) < cpus) _exit(0);
+      CPU_ZERO(&some);
+      for (int i = 0, n = 0; n < cpus; ++i)
+        if (CPU_ISSET(i, &all)) CPU_SET(i, &some), ++n;
+      if (sched_setaffinity(0, sizeof some, &some) != 0) _exit(0);
+      nnvhip::HostPool pool;
+      if (!each_once(pool, 16)) _exit(6);
+      DIR* tasks = opendir("/proc/self/task");
+      int n = 0;
+      while (const dirent* e = readdir(tasks)) n += e->d_name[0] != '.';
+      closedir(tasks);
+      if (n != cpus) _exit(7);
+      if (sched_setaffinity(0, sizeof all, &all) != 0) _exit(0);
+    }
+    _exit(0);
+  }
+  int status = 0;
+  if (waitpid(child, &status, 0) != child || status != 0) return 8;
   return each_once(*used, 16) && each_once(*fresh, 16) ? 0 : 5;
 }
 """
