@@ -171,9 +171,10 @@ int nnvhip_star_create(nnvhip_ctx* c, int64_t N, int64_t n, const double* V, con
 // so that the staging ring stays at 16 MB whatever the array's size); no kernel runs.  (Writing the matrices took 133 us for 100 boxes of 784 dimensions, 1.54 ms for 1024 of them, 6.4 GB nobody read; seven small
 // copies and kernels took 60 us of a single set's reach.)
 constexpr int64_t kBoxPiece = int64_t(1) << 20;
-// Host arrays of 1 MB and more are worth waking the context's workers for (some 20 us); several parts to a thread, so that
-// one that starts late costs little.
-constexpr int64_t kPoolDoubles = int64_t(1) << 17;
+// Host arrays of 1.5 MB and more are worth waking the context's workers for (some 20 us); several parts to a thread, so that
+// one that starts late costs little.  Boxes on one thread and on four: 1400 of 100 dimensions (1.1 MB) 287 -> 305 us, 2000 of them
+// (1.6 MB) 422 -> 401, 170 of 784 (1.1 MB) 224 -> 203, 512 of 784 (3.2 MB) 733 -> 599, 8000 of 20 (1.3 MB) 777 -> 787, 14 000 1813 -> 1716.
+constexpr int64_t kPoolDoubles = int64_t(3) << 16;
 static int host_parts(const nnvhip_ctx* c, int64_t doubles) { return doubles >= kPoolDoubles && !c->no_host_pool ? 4 * (HostPool::kWorkers + 1) : 1; }
 
 int nnvhip_copy_host(nnvhip_ctx* c, int64_t n, const double* src, double* dst) {
@@ -210,15 +211,18 @@ int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* 
   std::vector<double> vec((size_t)ld, 0.0);
   // First pass: half-widths only (they decide the sizes); the centres are formed below, in their place.  Both passes over the
   // host arrays are bound by one thread's share of the memory bandwidth, so those of a large array are shared out: 1024 boxes of
-  // 784 dimensions take 340 + 390 us on one thread (and their private copies 250); a reach of them 3.07 -> 2.05 ms.
+  // 784 dimensions take 340 + 390 us on one thread (and their private copies 250); a reach of them 3.0 -> 2.5 ms, or 4.0 -> 3.2
+  // on bounds not seen before.  What the workers have read lies in their caches too, and whoever writes it next has those
+  // copies invalidated first: a caller that makes its next bounds in the same memory takes 2.46 ms for it where it took 2.27 (26 MB
+  // written by one thread after it was read by itself 0.77 ms, after four 1.2 - 1.6, after four have written it 0.77).
   const int parts = host_parts(c, count * N);
   auto half_widths = [&](int64_t s) {
     const double *l = lb + s * N, *u = ub + s * N;
     for (int64_t i = 0; i < N; ++i) vec[(size_t)i] = 0.5 * (u[i] - l[i]);  // Box constructor, set/Box.m:36
   };
-  std::vector<char> as_first((size_t)count, 0);  // has the first set's half-widths, bit for bit
-  half_widths(0);
-  c->host_pool.run(parts, [&](int part) {
+  std::vector<char> as_first((size_t)count, 0);  // has the first set's half-widths, bit for bit (known where threads have looked)
+  if (parts > 1) half_widths(0);
+  if (parts > 1) c->host_pool.run(parts, [&](int part) {
     for (int64_t s = std::max<int64_t>(1, count * part / parts); s < count * (part + 1) / parts; ++s) {
       const double *l = lb + s * N, *u = ub + s * N;
       bool same = true;
@@ -233,7 +237,7 @@ int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* 
   });
   for (int64_t s = 0; s < count; ++s) {
     if (as_first[(size_t)s]) continue;  // (shape 0)
-    if (s > 0) half_widths(s);
+    if (s > 0 || parts == 1) half_widths(s);
     int64_t found = -1;
     for (int64_t k = 0; k < kept_shapes && found < 0; ++k)
       if (memcmp(&vecs[(size_t)(k * ld)], vec.data(), sizeof(double) * N) == 0) found = k;
@@ -315,8 +319,8 @@ int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* 
     NNV_TRY(c->stage(sizeof(double) * (size_t)(e1 - e0), &st));
     double* h = static_cast<double*>(st);  // the block's entries [e0, e1)
     int64_t e = std::max(e0, std::min(e1, vec_off));
-    c->host_pool.run(e - e0 >= kPoolDoubles ? parts : 1, [&](int part) {  // centres
-      const int64_t np = e - e0 >= kPoolDoubles ? parts : 1;
+    const int64_t np = host_parts(c, e - e0);
+    c->host_pool.run((int)np, [&](int part) {  // centres
       int64_t q = e0 + (e - e0) * part / np;
       for (const int64_t q1 = e0 + (e - e0) * (part + 1) / np; q < q1;) {
         const int64_t s = q / ld, i0 = q - s * ld, i1 = std::min(ld, i0 + q1 - q);

@@ -322,9 +322,9 @@ class Star:
         # state_lb / state_ub of the elements (set/Star.m:232-233) are columns of private copies
         return SetArray(ctx, out, state=(Star._private_copy(ctx, lbs), Star._private_copy(ctx, ubs)))
 
-    # values from which a copy goes over the context's threads (nnvhip_copy_host shares out 1 MB and more); a small one is
+    # values from which a copy goes over the context's threads (nnvhip_copy_host shares out 1.5 MB and more); a small one is
     # numpy's, which costs less than the call: 256 boxes through a 10-60x3-7 network 206 -> 181 us
-    _THREADED_COPY = 1 << 17
+    _THREADED_COPY = 3 << 16
 
     @staticmethod
     def _private_copy(ctx, a):

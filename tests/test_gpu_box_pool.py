@@ -1,6 +1,6 @@
-"""Boxes whose host arrays are large enough to be shared out to the context's threads (1 MB): the same sets, to the bit, as boxes made
-one by one; half-widths all alike, alike in all but a few sets, all different, zero in some dimensions, parts that end inside a
-set and inside the copied pieces; and the private copies of the bounds."""
+"""Boxes whose host arrays are large enough to be shared out to the context's threads (1.5 MB), or just not: the same sets, to the
+bit, as boxes made one by one; half-widths all alike, alike in all but a few sets, all different, zero in some dimensions, parts
+that end inside a set and inside the copied pieces; and the private copies of the bounds."""
 import numpy as np
 import pytest
 
@@ -13,7 +13,8 @@ def nnv():
     return nnv_amd
 
 
-@pytest.mark.parametrize("N,count", [(131, 1000), (132, 1001), (1031, 129), (785, 1400), (4, 35000), (17, 9000)])
+@pytest.mark.parametrize("N,count", [(131, 1000), (132, 1001), (1031, 129), (785, 1400), (4, 35000), (17, 9000),
+                                     (196, 1003), (197, 1001), (1031, 193), (4, 50000), (22, 9000)])
 @pytest.mark.parametrize("widths", ["alike", "few", "different", "degenerate"])
 def test_boxes_of_large_arrays(nnv, N, count, widths):
     rs = np.random.RandomState(N + count)
