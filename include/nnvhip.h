@@ -154,6 +154,10 @@ NNVHIP_API int nnvhip_debug_staging(nnvhip_ctx* ctx, int64_t* ring_bytes, int64_
  * many through one that copied the input's bounds into arrays of its own (new_pred_lb = [predicate_lb; zeros(m,1)],
  * nn/funcs/PosLin.m:737-738, either way).  Either pointer may be NULL. */
 NNVHIP_API int nnvhip_debug_relu_bounds(nnvhip_ctx* ctx, int64_t* appended_in_place, int64_t* copied);
+/* Test hook (no counterpart in the reference): the pool holds at most `bytes` of device memory and reports
+ * NNVHIP_ERR_OOM past that, as it does where the device has no more; 0: no such limit.  The context also forgets that it
+ * ever ran out of memory. */
+NNVHIP_API int nnvhip_debug_pool_limit(nnvhip_ctx* ctx, int64_t bytes);
 /* Which way the sets of the layer calls went since the context was created, for tests of the dispatch rules: sets[r] =
  * how many took route r (NNVHIP_ROUTES entries).  A set counts where a kernel of the route was launched for it. */
 enum {
@@ -345,7 +349,7 @@ NNVHIP_API int nnvhip_set_small_chain(nnvhip_ctx* ctx, int enabled);
  * same sets, and exist so that a test suite can drive every route in one process): "dense_affine"
  * (NNVHIP_DENSE_AFFINE), "eager_rows", "eager_tail", "eager_cols" (NNVHIP_EAGER_*), "poison_pending"
  * (NNVHIP_POISON_PENDING: whatever a layer leaves unwritten until first read is filled with NaNs),
- * "no_small_chain", "no_conv_mask", "no_conv_boxes" (NNVHIP_NO_*), "no_row_deltas" (NNVHIP_NO_ROW_DELTAS: an FC
+ * "no_small_chain", "no_conv_mask", "no_conv_boxes", "no_conv_pixels" (NNVHIP_NO_*), "no_row_deltas" (NNVHIP_NO_ROW_DELTAS: an FC
  * layer over an array of sets of one shape contracts every set over its whole kept-row list instead of forming
  * the product over the rows most sets keep once and contracting each set over its differences from that list),
  * "no_sum_shortcuts" (NNVHIP_NO_SUM_SHORTCUTS: where that layer sums its sets' pieces without storing them, every

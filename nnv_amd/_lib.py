@@ -29,7 +29,7 @@ SYMBOLS = [
     "nnvhip_star_fetch_rows", "nnvhip_relu_apply_lists", "nnvhip_probe_mfma_peak",
     "nnvhip_estimate_ranges_static", "nnvhip_debug_mailbox_pack", "nnvhip_debug_mailbox_unpack",
     "nnvhip_debug_set_relu_call_number", "nnvhip_reach_layers", "nnvhip_reach_is_one_launch", "nnvhip_relu_reduce_mem",
-    "nnvhip_set_switch", "nnvhip_hint_next_fc", "nnvhip_debug_counters", "nnvhip_debug_relu_bounds", "nnvhip_debug_routes", "nnvhip_debug_staging", "nnvhip_weight_cache_stats", "nnvhip_weight_cache_release", "nnvhip_debug_weak_weight_hash",
+    "nnvhip_set_switch", "nnvhip_hint_next_fc", "nnvhip_debug_counters", "nnvhip_debug_relu_bounds", "nnvhip_debug_routes", "nnvhip_debug_pool_limit", "nnvhip_debug_staging", "nnvhip_weight_cache_stats", "nnvhip_weight_cache_release", "nnvhip_debug_weak_weight_hash",
 ]
 
 
@@ -37,7 +37,8 @@ SYMBOLS = [
 SWITCH_ENV = {"dense_affine": "NNVHIP_DENSE_AFFINE", "eager_rows": "NNVHIP_EAGER_ROWS", "eager_tail": "NNVHIP_EAGER_TAIL",
               "eager_cols": "NNVHIP_EAGER_COLS", "poison_pending": "NNVHIP_POISON_PENDING",
               "no_small_chain": "NNVHIP_NO_SMALL_CHAIN", "no_conv_mask": "NNVHIP_NO_CONV_MASK",
-              "no_conv_boxes": "NNVHIP_NO_CONV_BOXES", "no_row_deltas": "NNVHIP_NO_ROW_DELTAS",
+              "no_conv_boxes": "NNVHIP_NO_CONV_BOXES", "no_conv_pixels": "NNVHIP_NO_CONV_PIXELS",
+              "no_row_deltas": "NNVHIP_NO_ROW_DELTAS",
               "no_sum_shortcuts": "NNVHIP_NO_SUM_SHORTCUTS", "no_host_pool": "NNVHIP_NO_HOST_POOL"}
 
 
@@ -129,6 +130,7 @@ def load():
         "nnvhip_debug_counters": [p, pi64, pi64, pi64, pi64],
         "nnvhip_debug_relu_bounds": [p, pi64, pi64],
         "nnvhip_debug_routes": [p, C.POINTER(i64)],
+        "nnvhip_debug_pool_limit": [p, i64],
         "nnvhip_debug_staging": [p, pi64, pi64],
         "nnvhip_weight_cache_stats": [p, pi64, pi64, pi64],
         "nnvhip_weight_cache_release": [p, pi64],
@@ -277,6 +279,10 @@ class Context:
         a, b = C.c_int64(), C.c_int64()
         check(self.lib.nnvhip_debug_staging(self.handle, C.byref(a), C.byref(b)))
         return a.value, b.value
+
+    def debug_pool_limit(self, nbytes):
+        """At most nbytes of device memory for the pool (0: no limit), see nnvhip_debug_pool_limit."""
+        check(self.lib.nnvhip_debug_pool_limit(self.handle, int(nbytes)))
 
     def routes(self):
         """{route: sets that took it} since the context was created (nnvhip_debug_routes)."""

@@ -19,6 +19,7 @@ void set_error(const char* fmt, ...) {
 }
 
 Buffer::~Buffer() {
+  if (tally) *tally -= (int64_t)bytes;
   if (ctx && ptr) ctx->release_block(ptr, bytes);
 }
 
@@ -129,7 +130,7 @@ void nnvhip_ctx::drain_deferred(size_t at_most) {
   }
 }
 
-int nnvhip_ctx::alloc(size_t bytes, BufRef* out) {
+int nnvhip_ctx::alloc(size_t bytes, BufRef* out, bool spare) {
   size_t cls = size_class(bytes ? bytes : 1);
   void* p = nullptr;
   auto it = free_blocks.find(cls);
@@ -150,14 +151,21 @@ int nnvhip_ctx::alloc(size_t bytes, BufRef* out) {
     free_blocks.erase(it);
     bytes_cached -= (int64_t)cls;
   } else {
-    hipError_t e = hipMalloc(&p, cls);
+    auto from_driver = [&] {
+      return pool_limit > 0 && bytes_in_use + bytes_cached + (int64_t)cls > pool_limit ? hipErrorOutOfMemory : hipMalloc(&p, cls);
+    };
+    hipError_t e = from_driver();
     n_device_mallocs++;
     room_seen -= (int64_t)cls;
+    if (e != hipSuccess && spare) {
+      (void)hipGetLastError();
+      return NNVHIP_ERR_OOM;
+    }
     if (e != hipSuccess) {
       (void)hipGetLastError();
       drop_unreferenced_weights();  // layers that only the weight cache still holds
       trim();                       // let released arrays go, give cached blocks back and retry once
-      e = hipMalloc(&p, cls);
+      e = from_driver();
       if (e != hipSuccess) {
         (void)hipGetLastError();
         NNV_FAIL(NNVHIP_ERR_OOM, "out of device memory allocating %zu bytes", cls);
@@ -312,6 +320,8 @@ int nnvhip_create(int device, nnvhip_ctx** out) {
   c->small_chain = getenv("NNVHIP_NO_SMALL_CHAIN") == nullptr;
   c->no_conv_mask = getenv("NNVHIP_NO_CONV_MASK") != nullptr;
   c->no_conv_boxes = getenv("NNVHIP_NO_CONV_BOXES") != nullptr;
+  c->no_conv_pixels = getenv("NNVHIP_NO_CONV_PIXELS") != nullptr;
+  c->pixel_limit = c->device_bytes / 8;
   c->no_row_deltas = getenv("NNVHIP_NO_ROW_DELTAS") != nullptr;
   c->no_sum_shortcuts = getenv("NNVHIP_NO_SUM_SHORTCUTS") != nullptr;
   c->no_host_pool = getenv("NNVHIP_NO_HOST_POOL") != nullptr;
@@ -408,6 +418,7 @@ int nnvhip_set_switch(nnvhip_ctx* c, const char* name, int enabled) {
       {"eager_tail", &c->eager_tail, false},       {"eager_cols", &c->eager_cols, false},
       {"poison_pending", &c->poison_pending, false}, {"no_small_chain", &c->small_chain, true},
       {"no_conv_mask", &c->no_conv_mask, false},   {"no_conv_boxes", &c->no_conv_boxes, false},
+      {"no_conv_pixels", &c->no_conv_pixels, false},
       {"no_row_deltas", &c->no_row_deltas, false}, {"no_sum_shortcuts", &c->no_sum_shortcuts, false},
       {"no_host_pool", &c->no_host_pool, false},
   };
@@ -562,6 +573,13 @@ int nnvhip_debug_staging(nnvhip_ctx* c, int64_t* ring_bytes, int64_t* outgrown_b
   if (!c) NNV_FAIL(NNVHIP_ERR_ARG, "null context");
   if (ring_bytes) *ring_bytes = (int64_t)c->pinned_bytes;
   if (outgrown_bytes) *outgrown_bytes = (int64_t)c->retired_bytes;
+  return NNVHIP_OK;
+}
+
+int nnvhip_debug_pool_limit(nnvhip_ctx* c, int64_t bytes) {
+  if (!c || bytes < 0) NNV_FAIL(NNVHIP_ERR_ARG, "null context or negative limit");
+  c->pool_limit = bytes;
+  c->pixel_limit = c->device_bytes / 8;
   return NNVHIP_OK;
 }
 

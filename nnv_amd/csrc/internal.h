@@ -128,6 +128,7 @@ struct Buffer {
   nnvhip_ctx* ctx = nullptr;
   void* ptr = nullptr;
   size_t bytes = 0;  // size class the block belongs to
+  int64_t* tally = nullptr;  // (or null) a sum this block's bytes are part of
   ~Buffer();
   template <class T>
   T* as() const { return static_cast<T*>(ptr); }
@@ -410,6 +411,12 @@ struct nnvhip_ctx {
   // a convolution whose input has a pending row reset runs that reset first instead of masking the rows as
   // it loads them (environment NNVHIP_NO_CONV_MASK)
   bool no_conv_mask = false;
+  // convolutions never keep their images pixel by pixel (ColSource::pix; environment NNVHIP_NO_CONV_PIXELS)
+  bool no_conv_pixels = false;
+  // Memory of images kept pixel by pixel, which comes on top of their matrices, and what it may come to: an eighth of the
+  // device's, and nothing any more once a reach has run out of memory with such images about (nnvhip_reach_layers).
+  int64_t pixel_bytes = 0, pixel_limit = 0;
+  int64_t pool_limit = 0;  // > 0: the pool holds no more than so many bytes (nnvhip_debug_pool_limit)
   // convolutions compute every generator image in full instead of inside its window (nnvhip_star::box;
   // environment NNVHIP_NO_CONV_BOXES)
   bool no_conv_boxes = false;
@@ -445,7 +452,8 @@ struct nnvhip_ctx {
   int kernel_timer_begin(bool on);
   int kernel_timer_end(bool on, int which, double flop);
 
-  int alloc(size_t bytes, nnvhip::BufRef* out);
+  // spare: for something that can be done without; nothing is given up for it.
+  int alloc(size_t bytes, nnvhip::BufRef* out, bool spare = false);
   // NNVHIP_ERR_OOM if alloc(bytes) would fail now; allocates nothing (what is cached is given up only where alloc would).
   int check_room(size_t bytes);
   int64_t room_seen = 0;  // what the driver last said was free, less the pool's own requests since ...

@@ -178,8 +178,15 @@ int nnvhip_affine_conv2d(nnvhip_ctx* c, const nnvhip_conv2d* cv, int64_t H, int6
       pix_at[(size_t)i] = total;
       total += plan[(size_t)i].nc * round_up(eh * ew * cv->Cout, kLdAlign);  // (column 0, the centre, stays in the matrix)
     }
-    if (total > 0) st = c->alloc(sizeof(double) * total, &pixels);
-    if (total > 0 && st == NNVHIP_OK && c->poison_pending) NNV_HIP_TRY(hipMemsetAsync(pixels->ptr, 0xff, sizeof(double) * total, c->stream));
+    // (the buffer comes on top of the matrices: without room for it they hold the columns)
+    const bool kept = total > 0 && c->pixel_bytes + 8 * total <= c->pixel_limit && c->alloc(sizeof(double) * total, &pixels, true) == NNVHIP_OK;
+    if (kept) {
+      pixels->tally = &c->pixel_bytes;
+      c->pixel_bytes += (int64_t)pixels->bytes;
+    } else {
+      std::fill(pix_at.begin(), pix_at.end(), -1);
+    }
+    if (kept && c->poison_pending) NNV_HIP_TRY(hipMemsetAsync(pixels->ptr, 0xff, sizeof(double) * total, c->stream));
   }
   // windows of the output's columns and the pixel tables of the unit-vector columns: one buffer each, one launch
   std::vector<ConvSetup> setup((size_t)count);
@@ -361,35 +368,19 @@ int nnvhip_reach_is_one_launch(nnvhip_ctx* c, int64_t n_layers, const int32_t* k
   return NNVHIP_OK;
 }
 
-int nnvhip_reach_layers(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, const int64_t* hw,
-                        int order, double relax_factor, int64_t count, nnvhip_star* const* in, nnvhip_star** out) {
-  if (!c) NNV_FAIL(NNVHIP_ERR_ARG, "null context");
-  if (n_layers < 0 || count <= 0 || !in || (n_layers > 0 && (!kind || !layer || !out))) NNV_FAIL(NNVHIP_ERR_ARG, "null argument");
+// The layer loop of nnvhip_reach_layers.  pixels: a convolution may keep its images pixel by pixel where the layers behind it read them so.
+static int layer_by_layer(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, const int64_t* hw, int order,
+                          double relax_factor, int64_t count, nnvhip_star* const* in, nnvhip_star** out, bool pixels) {
   nnvhip_star* const* cur = in;
   int st = NNVHIP_OK;
   int64_t done = 0;
-  if (n_layers > 0 && relax_factor == 1.0) {
-    // small fully connected networks: the whole loop below as one launch
-    NNV_TRY(nnvhip::enter_ctx(c));
-    bool taken = false;
-    for (int64_t t = 0; t < n_layers * count; ++t) out[t] = nullptr;
-    st = reach_small_chain(c, n_layers, kind, layer, order, count, in, out, &taken);
-    if (taken) {
-      if (st != NNVHIP_OK)
-        for (int64_t t = 0; t < n_layers * count; ++t) {
-          nnvhip_star_release(out[t]);
-          out[t] = nullptr;
-        }
-      return st;
-    }
-  }
   for (int64_t l = 0; l < n_layers && st == NNVHIP_OK; ++l) {
     nnvhip_star** dst = out + l * count;
     // the set that is handed back is written in full by the layer that produces it
     const bool eager = l == n_layers - 1 && !c->eager_cols;
     if (eager) c->eager_cols = true;
     // (a convolution at the end writes every column and does not go by position: it reads columns)
-    const bool known = kind[l] == NNVHIP_LAYER_CONV2D && l + 2 < n_layers && kind[l + 1] == NNVHIP_LAYER_RELU &&
+    const bool known = pixels && kind[l] == NNVHIP_LAYER_CONV2D && l + 2 < n_layers && kind[l + 1] == NNVHIP_LAYER_RELU &&
                        !(kind[l + 2] == NNVHIP_LAYER_CONV2D && l + 2 == n_layers - 1);
     c->behind_conv = known && kind[l + 2] == NNVHIP_LAYER_CONV2D ? static_cast<const nnvhip_conv2d*>(layer[l + 2]) : nullptr;
     c->behind_fc = known && kind[l + 2] == NNVHIP_LAYER_FC ? static_cast<const nnvhip_fc*>(layer[l + 2]) : nullptr;
@@ -425,6 +416,37 @@ int nnvhip_reach_layers(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, co
       nnvhip_star_release(out[t]);
       out[t] = nullptr;
     }
+  }
+  return st;
+}
+
+int nnvhip_reach_layers(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, const void* const* layer, const int64_t* hw,
+                        int order, double relax_factor, int64_t count, nnvhip_star* const* in, nnvhip_star** out) {
+  if (!c) NNV_FAIL(NNVHIP_ERR_ARG, "null context");
+  if (n_layers < 0 || count <= 0 || !in || (n_layers > 0 && (!kind || !layer || !out))) NNV_FAIL(NNVHIP_ERR_ARG, "null argument");
+  int st = NNVHIP_OK;
+  if (n_layers > 0 && relax_factor == 1.0) {
+    // small fully connected networks: the whole loop below as one launch
+    NNV_TRY(nnvhip::enter_ctx(c));
+    bool taken = false;
+    for (int64_t t = 0; t < n_layers * count; ++t) out[t] = nullptr;
+    st = reach_small_chain(c, n_layers, kind, layer, order, count, in, out, &taken);
+    if (taken) {
+      if (st != NNVHIP_OK)
+        for (int64_t t = 0; t < n_layers * count; ++t) {
+          nnvhip_star_release(out[t]);
+          out[t] = nullptr;
+        }
+      return st;
+    }
+  }
+  const int64_t pixels = c->routes[NNVHIP_ROUTE_CONV_PIXELS];
+  st = layer_by_layer(c, n_layers, kind, layer, hw, order, relax_factor, count, in, out, !c->no_conv_pixels);
+  if (st == NNVHIP_ERR_OOM && c->routes[NNVHIP_ROUTE_CONV_PIXELS] > pixels) {
+    // what its own images took on top of their matrices may be what was missing: the reach starts over with columns, and so does
+    // every later one of this context
+    c->pixel_limit = 0;
+    st = layer_by_layer(c, n_layers, kind, layer, hw, order, relax_factor, count, in, out, false);
   }
   return st;
 }

@@ -166,3 +166,49 @@ def test_an_fc_layer_that_reads_columns(nnv):
             rows = np.arange(70) != 3 if net is wild else slice(None)
             assert_close(got[rows], exp[rows], "set %d" % i, TOL)
             assert np.array_equal(np.isfinite(got), np.isfinite(exp))
+
+
+def test_without_room_for_pixels(nnv):
+    """Memory in which a reach fits with columns is enough: pixels come on top of the matrices, and are done without."""
+    rs = np.random.RandomState(8)
+    hw, cin = (20, 22), 1
+    layers = _layers(rs, hw, cin, [(3, 1, 1, 17), (3, 1, 1, 40), (3, 2, 0, 64)], 70)
+    ctx = nnv.default_context()
+    net = nnv.NN.from_config(layers)
+    (lb, ub), = _boxes(rs, hw, cin, 1)
+    options = {"reachMethod": "relax-star-area", "relaxFactor": 1}
+
+    def reach():
+        out = net.reach(nnv.ImageStar(lb, ub), options)
+        return [np.array(x) for x in out.estimateRanges()]
+
+    def nothing_cached():
+        net.reachSet = []
+        ctx.synchronize()
+        ctx.trim_pool()
+
+    was = ctx.switch_is_on("no_conv_pixels")
+    before = ctx.routes()["conv_pixels"]
+    ctx.set_switch("no_conv_pixels", True)
+    try:
+        reach()                                              # (the weights are on the device from here on)
+        nothing_cached()
+        exp = reach()
+        room = sum(ctx.pool_stats())
+        assert ctx.routes()["conv_pixels"] == before
+        ctx.set_switch("no_conv_pixels", False)
+        nothing_cached()
+        reach()
+        took = ctx.routes()["conv_pixels"] - before
+        assert took > 0 and sum(ctx.pool_stats()) > room     # it does come on top
+        for some in (room, room + (sum(ctx.pool_stats()) - room) // 2):
+            ctx.debug_pool_limit(some)
+            for _ in range(2):
+                nothing_cached()
+                for a, b in zip(reach(), exp):
+                    assert_close(a, b, "room for %d bytes" % some, TOL)
+                assert sum(ctx.pool_stats()) <= some
+            ctx.debug_pool_limit(0)
+    finally:
+        ctx.debug_pool_limit(0)
+        ctx.set_switch("no_conv_pixels", was)
