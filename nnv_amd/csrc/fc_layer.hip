@@ -522,13 +522,19 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
       } else if (any_rows || any_onehot) {
         std::vector<GemmSeg> segs;
         GemmRows rows;
-        const int64_t tn = gemm_seg_cols(fc->Mp, count, dense.data());
-        rows.seg_cols = (int32_t)tn;
+        int64_t tn = gemm_seg_cols(fc->Mp, count, dense.data());
         // Large arrays whose sets all come with packed rows take the tile kernel of gemm_seg.hip: rows packed
         // transposed, operands staged straight into LDS, a narrow last tile per set, bias added in the kernel.
         bool seg_tiles = tn == 128 && !dense_only;
         for (int64_t i = 0; i < count; ++i)
           if (!filled[i] && (!pk[i] || kps[i] > 2048 || dense[i] >= (int64_t(1) << 24))) seg_tiles = false;
+        if (!seg_tiles) {
+          // (wide tiles are for that kernel and for the one that reads rows through a list)
+          bool listed = false;
+          for (int64_t i = 0; i < count; ++i) listed = listed || (!filled[i] && !pk[i] && rws[i].kmap != nullptr);
+          if (!listed) tn = 64;
+        }
+        rows.seg_cols = (int32_t)tn;
         if (seg_tiles) {
           const int64_t ldo = outs[0]->ld;
           BufRef packed, shared_rows;

@@ -230,9 +230,13 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
   constexpr int kStage = KT * (TM + TN);
   constexpr int S = 65536 / (8 * kStage) > 4 ? 4 : 65536 / (8 * kStage);
   constexpr int UA = TM * KT / 128 / NW, UB = TN * KT / 128 / NW, U = UA + UB;
-  static_assert(KT == 16 || KT == 32, "stages of one or two groups of 16 rows");
+  static_assert(KT == 32, "stages of two groups of 16 rows");
   static_assert(S >= 2 && UA >= 1 && UB >= 1 && UA * NW * 128 == TM * KT && UB * NW * 128 == TN * KT, "every wave brings the same share of a stage");
   static_assert(WC * TM * 4 <= S * kStage && 2 * TN <= NT, "sums and bounds of the epilogue");
+  // (rows 0 .. KT - 1 of A, less than lda entries into one; columns 0 .. TN - 1 of B, less than KT entries into one; packed rows of B
+  // have no larger leading dimension than B)
+  static_assert((uint64_t)KT * (kMaxLdaDma - 1) * 8 < (uint64_t(1) << 32) && ((uint64_t)(TN - 1) * (kMaxLdbDma - 1) + KT) * 8 < (uint64_t(1) << 32),
+                "lane offsets of a stage");
   struct Lds {
     double ring[S * kStage];
     double pbs[2][TN];
@@ -274,8 +278,8 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
   auto next_half = [&](int k) {  // in front of the transfers of rows k ..., behind a barrier behind those of the rows before
     if (mapped && k != 0 && k % (kMapLds / 2) == 0) copy_list(k + kMapLds / 2, min(16 * n16, k + kMapLds));
   };
-  const bool half = KT == 32 && (n16 & 1);  // the last stage has 16 rows
-  const int nk = KT == 32 ? (n16 + 1) / 2 : n16;
+  const bool half = n16 & 1;  // the last stage has 16 rows
+  const int nk = (n16 + 1) / 2;
 
   // This wave's transfers of a stage: rows ka + u * kAStep of A, columns cb + u * kBStep of B.  Rows of W past the last and
   // columns past the tile's end are read from its last rows and first column (such results are neither stored nor summed).
@@ -283,7 +287,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
   const int ka = wave * 128 / TM + lane / (TM / 2);
   const int ra = min(t.m0 + 2 * (lane % (TM / 2)), g.Mp - 2);
   const int cb = wave * 128 / KT + lane / (KT / 2);
-  const int piece = (lane & (KT / 2 - 1)) ^ (KT == 16 ? (cb >> 1) & 7 : cb & 7);  // (kBStep is a multiple of 16)
+  const int piece = (lane & (KT / 2 - 1)) ^ (cb & 7);  // (kBStep is a multiple of 16)
   const bool packed = MAPPED && t.Bk != nullptr;
   const int64_t ldb = packed ? t.ldbk : g.ldb;
   const double* a_base = g.A + (mapped ? 0 : (int64_t)k0 * g.lda);
@@ -297,7 +301,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
   const uint32_t lda8 = (uint32_t)g.lda * 8;
   int a_row[UA];  // the listed rows that this lane's transfers of the stage to be issued next bring
   auto rows_of_stage = [&](int st) {
-    const int rows = (KT == 32 && half && st == nk - 1) ? 16 : KT;
+    const int rows = (half && st == nk - 1) ? 16 : KT;
 #pragma unroll
     for (int u = 0; u < UA; ++u) a_row[u] = sm.kmap[(st * KT + min(ka + u * kAStep, rows - 1)) % kMapLds];
   };
@@ -306,7 +310,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
   // its last one and not multiplied.
   auto issue = [&](int st, int slot) {
     const unsigned at = lds0 + slot * (kStage * 8);
-    const int rows = (KT == 32 && half && st == nk - 1) ? 16 : KT;
+    const int rows = (half && st == nk - 1) ? 16 : KT;
     if (mapped) {
 #pragma unroll
       for (int u = 0; u < UA; ++u) {
@@ -338,7 +342,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
     if (st < nk) issue(st, st);
 
   const int wr = wave % WR, wc = wave / WR, l16 = lane & 15, q = lane >> 4;
-  const int px = (q >> 1) ^ (KT == 16 ? l16 >> 1 : l16 & 7);  // turns the piece that holds row q of a column
+  const int px = (q >> 1) ^ (l16 & 7);  // turns the piece that holds row q of a column
   // this wave's transfers of a stage have landed (those of `ahead` later ones may be in flight) and its LDS reads are done
   auto arrived = [&](int ahead) {
     if (S > 3 && ahead == 3) wait_vm_lds<3 * U>();
@@ -381,7 +385,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_f64_kernel(GemmArgs g) {
         __builtin_amdgcn_sched_barrier(0);
         multiply(f0);
         __builtin_amdgcn_sched_barrier(0);
-        if (s + 2 == KT / 4 || (KT == 32 && s == 2 && half && last)) break;
+        if (s + 2 == KT / 4 || (s == 2 && half && last)) break;
         read(slot, s + 2, f0);
         __builtin_amdgcn_sched_barrier(0);
         multiply(f1);
@@ -673,8 +677,8 @@ static int launch_cfg(nnvhip_ctx* ctx, const double* A, int64_t lda, const doubl
   return NNVHIP_OK;
 }
 
-// Tile width of a segmented launch: 128 columns when there are enough tiles to cover the chip, 64 for small arrays and
-// outputs of few rows.
+// Tile width of an array's launch by the kernels that take wide tiles (gemm_seg.hip, and products whose rows are read through a list):
+// 128 columns when there are enough tiles to cover the chip, 64 for small arrays and outputs of few rows.
 int gemm_seg_cols(int64_t Mp, int64_t count, const int64_t* cols) {
   if (Mp <= 32) return 64;
   int64_t tiles = 0;
@@ -700,12 +704,13 @@ int launch_gemm(nnvhip_ctx* ctx, const double* A, int64_t lda, const double* B, 
              (rows->colmap != nullptr && !rows->b_plain);
   if (gather) {
     if (Mp <= 16) return NNV_GEMM_GATHER(16, 64, 1, 4);
-    if (wide_seg || (Mp > 32 && (rows == nullptr || rows->segs == nullptr) && ceil_div(Mp, 64) * ceil_div(ncols, 64) > 4 * kCUs))
-      return NNV_GEMM_GATHER(128, 128, 2, 4);
+    if (wide_seg) return NNV_GEMM_GATHER(128, 128, 2, 4);
+    // (2^24 rows of W, 16 and 64 columns of it, over 130 columns: 8.9 and 15.2 ms; on 128 x 128 tiles 13.0 and 22.9)
     return NNV_GEMM_GATHER(64, 64, 2, 4);
   }
   if (Mp <= 16) return NNV_GEMM(16, 64, 1, 4, 32);
-  if (wide_seg) return NNV_GEMM(64, 128, 2, 4, 16);
+  if (wide_seg) NNV_FAIL(NNVHIP_ERR_ARG, "internal: segment table built for another kernel");
+  // (an array's tiles: 20 sets of 601 columns, 300 x 2627 rows each, 397 us; with 64 x 128 tiles 500, 128 x 128 from registers 915)
   if (rows != nullptr && rows->segs != nullptr) return Mp <= 32 ? NNV_GEMM(32, 64, 2, 4, 32) : NNV_GEMM(64, 64, 4, 2, 32);
   // The tiles of a launch are dealt evenly to the CUs and those of a CU share its matrix cores, so the time goes with
   // ceil(tiles / CUs) * tile area / rate.  The rates are those of a 2048 x 1024 x 1920 product; a CU with a single 64 x 64

@@ -97,6 +97,25 @@ def test_long_lists_of_kept_rows(nnv, kept, M, n):
     _check(got, W[:, keep], b, V[keep], "kept %d" % kept)
 
 
+@pytest.mark.parametrize("M", [(1 << 24) - 16, 1 << 24])
+def test_offsets_at_the_end_of_32_bits(nnv, M):
+    """Leading dimensions of W on both sides of the line behind which offsets have 64 bits.  Small whole numbers: exact."""
+    from nnv_amd import _lib
+    K = 3
+    rs = np.random.RandomState(M % 97)
+    n = 4
+    ctx = _lib.Context(0)
+    W = np.asfortranarray(rs.randint(-3, 4, (M, K)).astype(np.float64))
+    b = rs.randint(-3, 4, M).astype(np.float64)
+    V = np.asfortranarray(rs.randint(-3, 4, (K, n + 1)).astype(np.float64))
+    S = nnv.Star(V, np.zeros((1, n)), np.zeros(1), -np.ones(n), np.ones(n), ctx=ctx)
+    out = S.affineMap(W, b)
+    lb, ub = out.estimateRanges()
+    P = W @ V
+    half = np.abs(P[:, 1:]).sum(1)
+    assert np.array_equal(lb, P[:, 0] + b - half) and np.array_equal(ub, P[:, 0] + b + half)
+
+
 def test_infinite_weight_meets_no_padding(nnv):
     """Rows a list is padded with are no rows of the set: an infinite weight in column 0 does not reach them."""
     rs = np.random.RandomState(3)
