@@ -168,6 +168,8 @@ enum {
   NNVHIP_ROUTE_ROWMAP_BOX,         /* row map of a box of which only the centre is in memory */
   NNVHIP_ROUTE_POOL_WINDOW,        /* average pooling inside windows */
   NNVHIP_ROUTE_CONV_PIXELS,        /* convolution whose output images are kept pixel by pixel */
+  NNVHIP_ROUTE_CHAIN,              /* whole reach in one launch, layers' matrices through memory */
+  NNVHIP_ROUTE_CHAIN_LDS,          /* ... sets in the LDS throughout */
   NNVHIP_ROUTES
 };
 NNVHIP_API int nnvhip_debug_routes(nnvhip_ctx* ctx, int64_t* sets);

@@ -507,7 +507,10 @@ __global__ __launch_bounds__(kChainThreads) void reach_chain_kernel(const ChainS
 //    matrices and, only the kept rows and without gaps, for the LDS the next layer multiplies from; nothing that went out is
 //    read back, so no barrier waits for a store;
 //  - a neuron is a lane: every wave classifies all of them by itself, and they meet for the ranking only.
-// One box through 5 - 50 x 6 - 5: 48 us there, 38 here (43 with sixteen waves, 60 with four); 128 boxes 70 -> 51.
+// One box through 5 - 50 x 6 - 5: 48 us there, 38 here (43 with sixteen waves, 60 with four); 128 boxes 70 -> 51.  A set takes up to
+// 160 KB of LDS, so a CU has one block where the kernel above has two, and this one is the quicker all the same, however many sets
+// there are (us, by events): 256 boxes 88 -> 58, 512 173 -> 111, 1024 331 -> 210, 2048 640 -> 401; 256, 1024 and 4096 through
+// 5 - 20 x 3 - 5 (several blocks to a CU either way) 28 -> 23, 102 -> 84, 383 -> 314.
 constexpr int kLdsChainN = 64;     // widest layer
 constexpr int kLdsChainThreads = 512;
 constexpr int kLdsChainTiles = 8;  // column tiles of a wave
@@ -924,7 +927,8 @@ struct ChainPlan {
   int64_t lds_doubles = 0;
 };
 
-// Whether a set of at most n0_max predicates stays in the LDS through the planned layers, whatever crosses.
+// Whether a set of at most n0_max predicates stays in the LDS through the planned layers, whatever crosses.  (How many sets there are
+// does not matter: see the kernel.)
 static void plan_chain_lds(int64_t N0, int64_t n0_max, ChainPlan* plan) {
   const ChainArgs& a = plan->args;
   int64_t rows = 0, weights = 0, before = n0_max, dense = n0_max;  // predicates in front of the layer, and those that are not its ReLU layer's
@@ -1083,6 +1087,7 @@ int reach_small_chain(nnvhip_ctx* c, int64_t n_layers, const int32_t* kind, cons
   else
     NNV_LAUNCH(c, c->kernel_timing, reach_chain_kernel, dim3((unsigned)count), dim3(kChainThreads), 0, table, sets[0], a);
   NNV_HIP_TRY(hipGetLastError());
+  c->routes[plan.in_lds ? NNVHIP_ROUTE_CHAIN_LDS : NNVHIP_ROUTE_CHAIN] += count;
   // Handles of earlier arrays that were released but not let go yet go now, all of them, while the kernel runs: their
   // arenas are what the next call of this size takes (a thousand sets come to a gigabyte, and a queue that grows from
   // call to call would have the pool ask the driver for another one each time).

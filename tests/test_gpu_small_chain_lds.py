@@ -1,11 +1,13 @@
 """The one-launch reach whose sets stay in the LDS (no layer wider than 64 neurons), against the oracle: one to four row tiles, column
 tiles at their edges, every neuron crossing, none, no row kept, FC layers behind one another, a dense input set, the widest and
-deepest networks that fit and the first that do not (those take the other kernel and must give the same)."""
+deepest networks that fit and the first that do not (those take the other kernel and must give the same).  Every case asserts
+which kernel its sets took."""
 import numpy as np
 import pytest
 
 from oracle import nnv_oracle
-from tests.test_gpu_small_chain import _check_against_oracle, _fc, _net
+from tests import test_gpu_small_chain
+from tests.test_gpu_small_chain import _fc, _net
 
 pytestmark = pytest.mark.gpu
 AREA = "relax-star-area"
@@ -18,6 +20,16 @@ def nnv():
     return nnv_amd
 
 
+def _check_against_oracle(nnv, oracle, layers, dev_in, ora_in, method, in_lds=True):
+    ctx = nnv.default_context()
+    before = ctx.routes()
+    test_gpu_small_chain._check_against_oracle(nnv, oracle, layers, dev_in, ora_in, method)
+    if not ctx.switch_is_on("no_small_chain", "dense_affine"):
+        count = len(ora_in) if isinstance(ora_in, list) else 1
+        took = {r: n - before[r] for r, n in ctx.routes().items() if r in ("chain", "chain_lds")}
+        assert took == {"chain_lds": count if in_lds else 0, "chain": 0 if in_lds else count}
+
+
 @pytest.mark.parametrize("widths,eps", [
     ((1, 1, 1), 0.5), ((2, 16, 16, 16), 0.3), ((5, 17, 32, 33, 2), 0.1), ((15, 48, 49, 1), 0.05), ((64, 64, 64, 64), 0.01), ((63, 63, 47, 64), 0.2),
     ((5, 50, 50, 50, 50, 50, 50, 5), 1.0), ((5, 50, 50, 50, 50, 50, 50, 5), 0.02), ((6, 50, 50, 50, 50, 50, 50, 5), 0.05),
@@ -27,6 +39,18 @@ def test_widths(nnv, widths, eps, method):
     rs = np.random.RandomState(sum(widths))
     c = rs.rand(widths[0]) - 0.5
     _check_against_oracle(nnv, nnv_oracle, _net(rs, widths), nnv.Star(c - eps, c + eps), nnv_oracle.star_from_box(c - eps, c + eps), method)
+
+
+# by the memory of the sets in front of the last layers (160 KB of LDS), the width of a layer (64), the columns of a layer (256)
+@pytest.mark.parametrize("widths,n,in_lds", [
+    ((34, 50, 50, 50, 50, 50, 50, 5), 34, True), ((35, 50, 50, 50, 50, 50, 50, 5), 35, False), ((5, 64, 64, 64, 64, 9), 5, True),
+    ((5, 64, 64, 64, 64, 64, 9), 5, False), ((5, 50, 50, 50, 50, 50, 50, 50, 5), 5, False), ((64, 64, 64, 3), 64, True), ((65, 64, 64, 3), 65, False),
+    ((8, 65, 40, 3), 8, False), ((8, 50, 4), 255, True), ((8, 50, 4), 256, False), ((8, 30, 4), 511, True), ((8, 30, 4), 512, False)])
+def test_the_last_that_fit_and_the_first_that_do_not(nnv, widths, n, in_lds):
+    rs = np.random.RandomState(n + len(widths))
+    V = np.concatenate([rs.rand(widths[0], 1) - 0.5, rs.randn(widths[0], n) * (0.2 / n)], axis=1)
+    args = (V, np.zeros((1, n)), np.zeros(1), -np.ones(n), np.ones(n))
+    _check_against_oracle(nnv, nnv_oracle, _net(rs, widths), nnv.Star(*args), nnv_oracle.OStar(*args), AREA, in_lds)
 
 
 @pytest.mark.parametrize("bias", [-30.0, 30.0, 0.0])
