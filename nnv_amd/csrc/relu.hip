@@ -271,8 +271,6 @@ __global__ __launch_bounds__(1024) void relu_classify_rank_kernel(const ReluDesc
     // rows in front of the group that are kept: those that are neither crossing nor inactive
     if (bk >> lane & 1) d.keep_idx[64 * group - (before[h] & 0xffff) - (before[h] >> 16) + __popcll(bk & below)] = r;
   }
-  if (blockIdx.x == 0)
-    for (int64_t r = kClassifyRankN + tid; r < d.ld; r += 1024) d.cls[r] = kKeep;
   if (blockIdx.x == 0 && tid < 2 * (int)kLdAlign) {  // -1 up to the next multiple of 16 past the list (at least 16 entries in all)
     const int nk = d.N - m - inact;
     const int end = max((nk + (int)kLdAlign - 1) / (int)kLdAlign * (int)kLdAlign, (int)kLdAlign);
