@@ -211,8 +211,8 @@ int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* 
   std::vector<double> vec((size_t)ld, 0.0);
   // First pass: half-widths only (they decide the sizes); the centres are formed below, in their place.  Both passes over the
   // host arrays are bound by one thread's share of the memory bandwidth, so those of a large array are shared out: 1024 boxes of
-  // 784 dimensions take 340 + 390 us on one thread (and their private copies 250); a reach of them 3.0 -> 2.5 ms, or 4.0 -> 3.2
-  // on bounds not seen before.  What the workers have read lies in their caches too, and whoever writes it next has those
+  // 784 dimensions take 340 + 390 us on one thread (and their private copies 250); a reach of them 2.95 -> 2.03 - 2.10 ms, on bounds
+  // not seen before 3.6 - 4.4 -> 2.8 - 3.5.  What the workers have read lies in their caches too, and whoever writes it next has those
   // copies invalidated first: a caller that makes its next bounds in the same memory takes 2.46 ms for it where it took 2.27 (26 MB
   // written by one thread after it was read by itself 0.77 ms, after four 1.2 - 1.6, after four have written it 0.77).
   const int parts = host_parts(c, count * N);
