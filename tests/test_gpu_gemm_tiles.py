@@ -97,6 +97,25 @@ def test_long_lists_of_kept_rows(nnv, kept, M, n):
     _check(got, W[:, keep], b, V[keep], "kept %d" % kept)
 
 
+@pytest.mark.parametrize("M,share", [(150, 0.7), (24, 0.7), (150, 0.3)])
+def test_long_lists_in_an_array(nnv, M, share):
+    """The same for the sets of an array, each with a list of its own, longer or shorter than what LDS holds at a time."""
+    rs = np.random.RandomState(M)
+    n, H, count = 30, 4500, 12
+    c = rs.rand(n, count)
+    h = 0.001 * rs.rand(n, count)
+    L1 = nnv.layers.FullyConnectedLayer(rs.randn(H, n) * 0.1, np.where(rs.rand(H) < share, 3.0, -3.0) + 0.2 * rs.randn(H))
+    mid = nnv.layers.ReluLayer().reach(L1.reach(nnv.Star.from_boxes(c - h, c + h), "relax-star-area", [], 1, None, "linprog"), "relax-star-area", [],
+                                       1, None, "linprog")
+    W, b = rs.randn(M, H), rs.randn(M)
+    out = nnv.layers.FullyConnectedLayer(W, b).reach(mid, "relax-star-area", [], 1, None, "linprog")
+    for i in (0, 5, count - 1):
+        Vm = np.array(mid[i].V)
+        keep = np.any(Vm != 0, axis=1)
+        assert (keep.sum() > 2048) == (share > 0.5)
+        _check(np.array(out[i].V), W[:, keep], b, Vm[keep], "set %d" % i)
+
+
 @pytest.mark.parametrize("M", [(1 << 24) - 16, 1 << 24])
 def test_offsets_at_the_end_of_32_bits(nnv, M):
     """Leading dimensions of W on both sides of the line behind which offsets have 64 bits.  Small whole numbers: exact."""
