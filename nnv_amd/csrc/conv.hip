@@ -843,8 +843,10 @@ static int launch_conv_fast(nnvhip_ctx* ctx, const nnvhip_conv2d* cv, const Conv
   a.tiles_c = (int)tiles_c;
   a.keep_words = keep_words;
   // lanes per output row of the stamp blocks: 8 for filters with many taps (beside the tile blocks that measured best:
-  // CNN 32x32x3 0.747 ms against 0.752 with 16 lanes, 0.756 with 4, 0.782 with 32), else 1
-  const bool wide_stamps = g.K > 32;
+  // CNN 32x32x3 0.747 ms against 0.752 with 16 lanes, 0.756 with 4, 0.782 with 32) and where one lane to a row would leave half
+  // of the chip without a block (32 x 32 x 3 into 8 channels, 16 blocks of stamps: 23.8 us, with 8 lanes 128 blocks and 8.0 us),
+  // else 1
+  const bool wide_stamps = g.K > 32 || ceil_div(ldout, 512) * (int64_t)jobs.size() < 128;
   int64_t stamp_blocks = stamps ? ceil_div(ldout * (wide_stamps ? 8 : 1), 512) : 0;
   for (const ConvSet& s : jobs)
     if (stamps && s.d.pix != nullptr) stamp_blocks = std::max<int64_t>(stamp_blocks, conv_stamp_pixel_blocks(g.P, g.K, 512));
