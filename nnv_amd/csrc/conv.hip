@@ -506,7 +506,8 @@ __device__ __forceinline__ ColBox conv_out_box(const ConvSetup& d, const ConvGeo
   if (j == 0) return ColBox{0, (int16_t)(g.Ho - 1), 0, (int16_t)(g.Wo - 1)};
   if (h0 > h1 || w0 > w1) return ColBox{1, 0, 1, 0};
   // output rows whose taps ho*sh - pt + fh*dh (0 <= fh < FH) reach [h0, h1]
-  auto floordiv = [](int a, int s) { return a >= 0 ? a / s : -((-a + s - 1) / s); };
+  // (strides are the layer's: the branch is uniform, and a division takes some thirty instructions)
+  auto floordiv = [](int a, int s) { return (s & (s - 1)) == 0 ? a >> (31 - __builtin_clz(s)) : a >= 0 ? a / s : -((-a + s - 1) / s); };
   const int a0 = h0 + g.pt - (g.FH - 1) * g.dh, a1 = h1 + g.pt;
   const int b0 = w0 + g.pl - (g.FW - 1) * g.dw, b1 = w1 + g.pl;
   const int ho0 = max(0, -floordiv(-a0, g.sh)), ho1 = min(g.Ho - 1, floordiv(a1, g.sh));
@@ -521,12 +522,12 @@ __device__ __forceinline__ ColBox conv_out_box(const ConvSetup& d, const ConvGeo
 // or not a column names it, then out in order.  Latency bound (a few KB).
 constexpr int kInvRows = 4096;
 __global__ __launch_bounds__(kSortThreads) void conv_setup_kernel(const ConvSetup* __restrict__ table, ConvSetup one, int sort_blocks,
-                                                                  int inv_blocks, ConvGeom g) {
+                                                                  int sort_run, int inv_blocks, ConvGeom g) {
   const ConvSetup d = table ? table[blockIdx.y] : one;
   const int blk = (int)blockIdx.x - sort_blocks;
   if (blk < 0) {
     if (d.order == nullptr) return;
-    sort_windows(d.dense - 1, g.P, d.order, d.first, blockIdx.x, sort_blocks, [&](int j) {
+    sort_windows(d.dense - 1, g.P, d.order, d.first, sort_run, blockIdx.x, [&](int j) {
       const ColBox b = conv_out_box(d, g, j);
       return b.h0 > b.h1 ? 0 : b.w0 * g.Ho + b.h0;
     });
@@ -918,12 +919,16 @@ static int launch_setup(nnvhip_ctx* ctx, const ConvGeom& g, int64_t count, const
   for (int64_t i0 = 0; i0 < count; i0 += 65535) {
     const int64_t cnt = std::min<int64_t>(65535, count - i0);
     int64_t inv_rows = 0, cols = 0;
-    int sort_blocks = 0;
+    int64_t sorted = 0, sort_sets = 0;  // columns of a set at most, sets
     for (int64_t i = i0; i < i0 + cnt; ++i) {
-      if (sets[i].order != nullptr) sort_blocks = std::max(sort_blocks, sort_window_blocks(sets[i].dense - 1));
+      if (sets[i].order != nullptr) {
+        sorted = std::max<int64_t>(sorted, sets[i].dense - 1);
+        ++sort_sets;
+      }
       if (sets[i].inv != nullptr) inv_rows = std::max<int64_t>(inv_rows, sets[i].n_inv);
       if (sets[i].out_box != nullptr) cols = std::max<int64_t>(cols, (int64_t)sets[i].dense + sets[i].m);
     }
+    const int sort_run = sort_window_run(sorted, sort_sets), sort_blocks = sort_sets > 0 ? sort_window_blocks(sorted, sort_run) : 0;
     const int64_t inv_blocks = ceil_div(inv_rows, kInvRows), blocks = sort_blocks + inv_blocks + ceil_div(cols, kSortThreads);
     if (blocks == 0) continue;
     const ConvSetup* table = nullptr;
@@ -933,7 +938,7 @@ static int launch_setup(nnvhip_ctx* ctx, const ConvGeom& g, int64_t count, const
       table = tab->as<ConvSetup>();
     }
     hipLaunchKernelGGL(conv_setup_kernel, dim3((unsigned)blocks, (unsigned)cnt), dim3(kSortThreads), 0, ctx->stream, table, sets[i0],
-                       sort_blocks, (int)inv_blocks, g);
+                       sort_blocks, sort_run, (int)inv_blocks, g);
     NNV_HIP_TRY(hipGetLastError());
   }
   return NNVHIP_OK;

@@ -52,7 +52,7 @@ struct FcWinArgs {
   int32_t shift;         // window starts are told apart in steps of 1 << shift positions
   int32_t buckets;
   int32_t tiles_m;
-  int32_t sort_blocks;
+  int32_t sort_blocks, sort_run;
 };
 
 // This block's set.
@@ -121,7 +121,7 @@ __global__ __launch_bounds__(kSortThreads) void fc_window_setup_kernel(const FcW
     }
     return;
   }
-  sort_windows(S.ncols - 1, a.buckets, S.order, nullptr, blockIdx.x, a.sort_blocks, [&](int j) { return window_bucket(S.box[j], a); });
+  sort_windows(S.ncols - 1, a.buckets, S.order, nullptr, a.sort_run, blockIdx.x, [&](int j) { return window_bucket(S.box[j], a); });
 }
 
 // TM x TN output tile per block of WR x WC waves.  Column tiles are dealt to the XCDs (blockIdx.x % 8) with all their row
@@ -417,7 +417,7 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
   const int tm = fc->Mp <= 32 ? 32 : 64;
   a.tiles_m = (int32_t)ceil_div(fc->Mp, tm);
   std::vector<FcWinSet> tab((size_t)count);
-  int64_t orders = 0, parts = 0, max_tiles = 0, max_chunks = 0;
+  int64_t orders = 0, parts = 0, max_cols = 0, max_tiles = 0, max_chunks = 0;
   for (int64_t i = 0; i < count; ++i) {
     FcWinSet& d = tab[(size_t)i];
     const nnvhip_star* s = sets[i].in;
@@ -433,8 +433,10 @@ int launch_fc_window(nnvhip_ctx* ctx, const nnvhip_fc* fc, int tn, int64_t count
     parts += d.cchunks;
     max_tiles = std::max<int64_t>(max_tiles, d.tiles);
     max_chunks = std::max<int64_t>(max_chunks, d.cchunks);
-    a.sort_blocks = std::max(a.sort_blocks, sort_window_blocks(sets[i].dense - 1));
+    max_cols = std::max<int64_t>(max_cols, sets[i].dense - 1);
   }
+  a.sort_run = sort_window_run(max_cols, count);
+  a.sort_blocks = sort_window_blocks(max_cols, a.sort_run);
   BufRef order, cpart, dev;
   NNV_TRY(ctx->alloc(sizeof(int32_t) * orders, &order));
   NNV_TRY(ctx->alloc(sizeof(double) * fc->Mp * std::max<int64_t>(parts, 1), &cpart));
