@@ -10,7 +10,11 @@
 // over all kept rows; only sums over columns (the range sums) and over the whole image (the centre, whose partial
 // products are formed next to the sort) are cut differently.
 //
-// Measured, kernels of the layer alone: 25 sets of 28 x 28 x 1 through two convolutions into 100 rows, 25 zero fills and a
+// Two stages of operands are in flight in front of the one that is multiplied, none of them behind a branch: one stage ahead,
+// loads under their conditions 42.7 us (32 x 32 x 3 through four convolutions), 18.9 (28 x 28 x 1 through two) and 106 (25 of
+// those), now 39.3, 15.4 and 95; the centre's partial products next to the sort likewise (25 sets 24.3 -> 21.1 us).
+//
+// Measured as it came in, kernels of the layer alone: 25 sets of 28 x 28 x 1 through two convolutions into 100 rows, 25 zero fills and a
 // product 875 us -> 142 us; one such set 45 -> 24 us; 32 x 32 x 3 through four convolutions into 512 rows (15 000 columns,
 // windows of 16 of 49 positions) 174 -> 65 us.
 //
@@ -102,10 +106,10 @@ __global__ __launch_bounds__(kSortThreads) void fc_window_setup_kernel(const FcW
           double w[8], v[8];
 #pragma unroll
           for (int u = 0; u < 8; ++u) {
-            const int k = kk + u * groups;
-            const int r = k >= k1 ? -1 : S.kept != nullptr ? S.kept[k] : k;
-            w[u] = r >= 0 ? a.W[row + (int64_t)r * a.lda] : 0.0;
-            v[u] = r >= 0 ? S.V[r] : 0.0;
+            const int k = min(kk + u * groups, k1 - 1);
+            const int r = S.kept != nullptr ? S.kept[k] : k;
+            w[u] = a.W[row + (int64_t)r * a.lda];
+            v[u] = S.V[r];
           }
 #pragma unroll
           for (int u = 0; u < 8; ++u)
@@ -130,6 +134,7 @@ __global__ __launch_bounds__(kSortThreads) void fc_window_setup_kernel(const FcW
 // and its position.  As one kernel for both ways, with lists of half the length and eight registers more, a CU held one block of
 // 64 x 64 less and unions of windows went through several lists: 25 images of 28 x 28 x 1 and of 40 x 40 x 1, column by column, 119 and
 // 245 us, 101 and 213 apart (101 and 206 before there were pixels); pixel by pixel 115 and 232, 101 and 204 now.
+__device__ double g_win_zero[1];  // (never written)
 constexpr int kWinRows = 2048, kWinPixelRows = 1536;  // rows a stage list holds; a union with more kept rows is walked in several lists
 template <int TM, int TN, int WR, int WC, int KT, bool PIXELS>
 __global__ __launch_bounds__(64 * WR * WC, TN == 64 ? 6 : 4) void fc_window_kernel(const FcWinSet* __restrict__ table, FcWinSet one, FcWinArgs a) {
@@ -139,11 +144,11 @@ __global__ __launch_bounds__(64 * WR * WC, TN == 64 ? 6 : 4) void fc_window_kern
   static_assert(NT == TN * KT / 2, "one pair of rows of the image tile per thread");
   __shared__ double Ws[2][KT * LDA_S];
   __shared__ double Vs[2][TN * LDB_S];
-  // rows of the union's windows, -1 padded to whole stages: ascending; of images kept pixel by pixel pixel by pixel
+  // rows of the union's windows, padded to whole stages: ascending; of images kept pixel by pixel pixel by pixel
   constexpr int kRows = PIXELS ? kWinPixelRows : kWinRows;
-  __shared__ int s_row[kRows + KT];
-  __shared__ int s_pos[kRows + KT];  // their positions: h | w << 16 (-1: none) ...
-  __shared__ int s_pix[PIXELS ? kRows + KT : 1];  // ... and where they lie in an image kept pixel by pixel
+  // where they lie in an image (x) and their positions (y): h | w << 16 (-1: none) ...
+  __shared__ __attribute__((aligned(16))) int2 s_at[kRows + KT];
+  __shared__ int s_row[PIXELS ? kRows + KT : 1];  // ... and their numbers where an image is kept pixel by pixel
   __shared__ int s_col[TN];
   __shared__ double s_pl[TN], s_pu[TN];
   __shared__ int s_u[4];
@@ -202,8 +207,13 @@ __global__ __launch_bounds__(64 * WR * WC, TN == 64 ? 6 : 4) void fc_window_kern
   const int bj = tid / (KT / 2), bk = 2 * (tid % (KT / 2));
   const int bcol = s_col[bj];
   const double* img = PIXELS ? S.pix + (int64_t)max(bcol, 0) * S.pix_ld : S.V + (int64_t)max(bcol, 0) * S.ld;
-  ColBox bb = {1, 0, 1, 0};
-  if (bcol >= 0) bb = S.box[bcol];
+  ColBox bb = {0x4000, 0x4000, 0, 0};  // (images have at most 8192 rows and columns)
+  if (bcol >= 0) {
+    const ColBox b = S.box[bcol];
+    if (b.h0 <= b.h1 && b.w0 <= b.w1) bb = b;
+  }
+  const unsigned hspan = bb.h1 - bb.h0, wspan = bb.w1 - bb.w0;
+  const double* const zero = g_win_zero;
 
   double4_t acc[FM][FN];
 #pragma unroll
@@ -212,35 +222,41 @@ __global__ __launch_bounds__(64 * WR * WC, TN == 64 ? 6 : 4) void fc_window_kern
     for (int j = 0; j < FN; ++j) acc[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
 
   constexpr int A_VEC = TM * KT / 2, A_PASS = (A_VEC + NT - 1) / NT;
-  double2 ra[A_PASS], rb;
-  auto load_tiles = [&](int k0) {
+  // A stage's operands travel through registers while the two stages before it are multiplied.  Every load is issued whatever
+  // its row and column are: behind a branch the compiler would wait for all loads in flight.  (An element that is not wanted is
+  // read from a zero; a row behind the list, or a row of the tile behind the weights, meets zeros or is not stored.)
+  typedef double pair_t __attribute__((ext_vector_type(2)));
+  struct Regs {
+    pair_t a[A_PASS], b;
+  };
+  const double* const weights = a.W + min(m0 + 2 * (tid % (TM / 2)), a.Mp - 2);
+  auto load_tiles = [&](int k0, Regs& g) {
 #pragma unroll
     for (int p = 0; p < A_PASS; ++p) {
-      const int idx = tid + p * NT;
-      const int row = m0 + 2 * (idx % (TM / 2));
-      ra[p] = make_double2(0.0, 0.0);
-      if (idx < A_VEC && row < a.Mp) {
-        const int r = s_row[k0 + idx / (TM / 2)];
-        if (r >= 0) ra[p] = *reinterpret_cast<const double2*>(a.W + row + (int64_t)r * a.lda);
-      }
+      const int k = min((tid + p * NT) / (TM / 2), KT - 1);
+      const uint32_t row = PIXELS ? s_row[k0 + k] : s_at[k0 + k].x;
+      g.a[p] = *reinterpret_cast<const pair_t*>(weights + (uint64_t)row * (uint32_t)a.lda);
     }
-    auto pixel = [&](int k) {
-      const int at = PIXELS ? s_pix[k] : s_row[k], pos = s_pos[k];
+    int4 two = *reinterpret_cast<const int4*>(&s_at[k0 + bk]);
+    asm("" : "+v"(two.x), "+v"(two.z));  // (read here, not behind a branch on the window tests)
+    auto pixel = [&](int at, int pos) {
       const int h = pos & 0xffff, w = pos >> 16;  // (h past any window where there is no row)
-      return h >= bb.h0 && h <= bb.h1 && w >= bb.w0 && w <= bb.w1 ? img[at] : 0.0;
+      const bool in = ((unsigned)(h - bb.h0) <= hspan) & ((unsigned)(w - bb.w0) <= wspan);
+      return in_global(in ? img + at : zero)[0];
     };
-    rb.x = pixel(k0 + bk);
-    rb.y = pixel(k0 + bk + 1);
+    g.b.x = pixel(two.x, two.y);
+    g.b.y = pixel(two.z, two.w);
   };
-  auto store_tiles = [&](int buf) {
+  auto store_tiles = [&](int buf, const Regs& g) {
 #pragma unroll
     for (int p = 0; p < A_PASS; ++p) {
       const int idx = tid + p * NT;
-      if (idx < A_VEC) *reinterpret_cast<double2*>(&Ws[buf][(idx / (TM / 2)) * LDA_S + 2 * (idx % (TM / 2))]) = ra[p];
+      if (A_PASS * NT == A_VEC || idx < A_VEC) *reinterpret_cast<pair_t*>(&Ws[buf][(idx / (TM / 2)) * LDA_S + 2 * (idx % (TM / 2))]) = g.a[p];
     }
-    Vs[buf][bj * LDB_S + bk] = rb.x;  // odd column stride: two 64-bit stores
-    Vs[buf][bj * LDB_S + bk + 1] = rb.y;
+    Vs[buf][bj * LDB_S + bk] = g.b.x;  // odd column stride: two 64-bit stores
+    Vs[buf][bj * LDB_S + bk + 1] = g.b.y;
   };
+  static_assert(NT % (TM / 2) == 0, "a thread's weights are of the same rows in every pass");
 
   const int wr = wave % WR, wc = wave / WR;
   for (int cand = 0; cand < total;) {
@@ -277,30 +293,40 @@ __global__ __launch_bounds__(64 * WR * WC, TN == 64 ? 6 : 4) void fc_window_kern
       }
       if (keep) {
         const int at = before + __popcll(m & ((1ull << lane) - 1ull));
-        s_row[at] = r;
-        s_pos[at] = h | (w << 16);
-        if (PIXELS) s_pix[at] = pix_slot(h, w, S.pix_eh, S.pix_ew) * a.C + ch;
+        s_at[at] = make_int2(PIXELS ? pix_slot(h, w, S.pix_eh, S.pix_ew) * a.C + ch : r, h | (w << 16));
+        if (PIXELS) s_row[at] = r;
       }
       __syncthreads();
       cand += NT;
     }
     const int nk = (nrow + KT - 1) / KT;
     if (tid < nk * KT - nrow) {
-      s_row[nrow + tid] = -1;
-      s_pos[nrow + tid] = -1;
-      if (PIXELS) s_pix[nrow + tid] = 0;
+      s_at[nrow + tid] = make_int2(0, -1);
+      if (PIXELS) s_row[nrow + tid] = 0;
     }
     __syncthreads();
-    if (nk > 0) {
-      load_tiles(0);
-      store_tiles(0);
-    }
+    if (nk == 0) continue;
+    Regs g0, g1;
+    load_tiles(0, g0);
+    load_tiles(KT * min(1, nk - 1), g1);
+    store_tiles(0, g0);
     __syncthreads();
-    for (int t = 0; t < nk; ++t) {  // two LDS stages: stage t + 1 travels while stage t is multiplied
-      const int cur = t & 1;
-      if (t + 1 < nk) load_tiles((t + 1) * KT);
+    auto multiply = [&](int cur) {
       mfma_tile_k16<FM, FN, KT>(&Ws[cur][wr * (TM / WR)], LDA_S, &Vs[cur][(wc * (TN / WC)) * LDB_S], LDB_S, lane, acc);
-      if (t + 1 < nk) store_tiles(cur ^ 1);
+    };
+    // stage t from LDS half t & 1; `next` holds stage t + 1, `far` receives stage t + 2 (past the end: the last again)
+    auto step = [&](int t, Regs& next, Regs& far) {
+      load_tiles(KT * min(t + 2, nk - 1), far);
+      multiply(t & 1);
+      store_tiles((t & 1) ^ 1, next);
+      __syncthreads();
+    };
+    for (int t = 0; t + 1 < nk; t += 2) {
+      step(t, g1, g0);
+      step(t + 1, g0, g1);
+    }
+    if (nk & 1) {
+      multiply(0);
       __syncthreads();
     }
   }
