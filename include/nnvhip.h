@@ -170,6 +170,7 @@ enum {
   NNVHIP_ROUTE_CONV_PIXELS,        /* convolution whose output images are kept pixel by pixel */
   NNVHIP_ROUTE_CHAIN,              /* whole reach in one launch, layers' matrices through memory */
   NNVHIP_ROUTE_CHAIN_LDS,          /* ... sets in the LDS throughout */
+  NNVHIP_ROUTE_FC_SKINNY,          /* FC layer of few outputs straight behind a ReLU step */
   NNVHIP_ROUTES
 };
 NNVHIP_API int nnvhip_debug_routes(nnvhip_ctx* ctx, int64_t* sets);

@@ -286,7 +286,7 @@ class Context:
 
     def routes(self):
         """{route: sets that took it} since the context was created (nnvhip_debug_routes)."""
-        names = ("conv_window", "conv_window_parts", "fc_window", "rowmap_window", "rowmap_box", "pool_window", "conv_pixels", "chain", "chain_lds")
+        names = ("conv_window", "conv_window_parts", "fc_window", "rowmap_window", "rowmap_box", "pool_window", "conv_pixels", "chain", "chain_lds", "fc_skinny")
         v = (C.c_int64 * len(names))()
         check(self.lib.nnvhip_debug_routes(self.handle, v))
         return dict(zip(names, v))

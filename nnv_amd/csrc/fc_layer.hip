@@ -176,10 +176,12 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
                          in[0]->rows_pending && in[0]->cls != nullptr && in[0]->pre_ub != nullptr;
     // (skinny layers keep the gather pass: a handful of 16-row blocks would not cover the chip)
     bool rowsum = (box_in || relu_in) && fc->Mp >= 128 && fc->K < (int64_t(1) << 31);
+    // Few outputs straight behind a ReLU step: one launch that takes the step's rows and unit vectors as it recorded them
+    const bool skinny = !dense_only && fc_skinny_takes(fc, count, in);
     // sets whose implicit unit-vector columns take part in the contraction after all get them written out
     // (which also runs a pending row reset)
     std::vector<nnvhip_star*> full;
-    for (int64_t i = 0; i < count; ++i)
+    for (int64_t i = 0; i < count && !skinny; ++i)
       if (dense[i] > in[i]->stored_cols() || (dense_only && (in[i]->rows_pending || in[i]->cs.any_pending()))) full.push_back(in[i]);
     if (!full.empty()) {
       // (boxes of one array move together: the array stays back to back)
@@ -199,7 +201,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
     // that keeps no row reads none.
     {
       std::vector<nnvhip_star*> need;
-      for (int64_t i = 0; i < count; ++i)
+      for (int64_t i = 0; i < count && !skinny; ++i)
         if (in[i]->cs.delta_pending() && !(in[i]->rows_pending && in[i]->n_kept == 0)) need.push_back(in[i]);
       if (!need.empty() && st == NNVHIP_OK) st = write_pending_columns(c, (int64_t)need.size(), need.data());
     }
@@ -243,7 +245,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
     // (fc_window.hip) and reads nothing outside.  Calls that are launch bound take one dense launch as before; a set that
     // keeps no row contracts over nothing.
     int win_tile = 0;
-    if (st == NNVHIP_OK && !dense_only && (count == 1 || contig)) {
+    if (st == NNVHIP_OK && !dense_only && !skinny && (count == 1 || contig)) {
       bool work = true;
       for (int64_t i = 0; i < count && work; ++i)
         work = !(in[i]->n_kept == 0 && in[i]->kept_idx != nullptr) &&
@@ -258,7 +260,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
     // Inputs with columns that are described but not in memory yet: the contraction reads them from
     // memory unless it goes over no row at all or through the packing pass (which takes such columns
     // from the weights they were gathered from).  Everybody else has them written now.
-    if (st == NNVHIP_OK && win_tile == 0) {
+    if (st == NNVHIP_OK && win_tile == 0 && !skinny) {
       std::vector<nnvhip_star*> cols;
       for (int64_t i = 0; i < count; ++i) {
         if (!in[i]->cs.any_pending()) continue;
@@ -274,7 +276,23 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
     // follows works from the sums, and the next FC map either contracts over no row or packs its rows
     // from the weights.  lazy[i] is set where the sums are produced.
     std::vector<char> lazy((size_t)count, 0);
-    if (count == 1 && rowsum && st == NNVHIP_OK) {
+    if (skinny && st == NNVHIP_OK) {
+      const int waves = fc_skinny_waves(fc, count, in);
+      std::vector<int64_t> chunk_off((size_t)count + 1, 0);
+      for (int64_t i = 0; i < count; ++i) chunk_off[(size_t)i + 1] = chunk_off[(size_t)i] + fc_skinny_chunks(in[i], waves);
+      BufRef sums;
+      st = c->alloc(sizeof(double) * 4 * outs[0]->ld * chunk_off[(size_t)count], &sums);
+      std::vector<double*> part((size_t)count);
+      for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i) part[(size_t)i] = sums->as<double>() + 4 * outs[0]->ld * chunk_off[(size_t)i];
+      if (st == NNVHIP_OK) st = launch_fc_skinny(c, fc, count, in, outs.data(), part.data(), waves);
+      if (st == NNVHIP_OK && count == 1) st = finalize_fused_ranges(c, outs[0], sums, chunk_off[1]);
+      for (int64_t i = 0; i < count && count > 1 && st == NNVHIP_OK; ++i) {
+        outs[i]->rng_buf = sums;
+        outs[i]->rng_part = part[(size_t)i];
+        outs[i]->rng_chunks = chunk_off[(size_t)i + 1] - chunk_off[(size_t)i];
+        outs[i]->rng_first_col = 1;
+      }
+    } else if (count == 1 && rowsum && st == NNVHIP_OK) {
       GemmRows rows;
       int64_t kp = fc->Kp;
       bool pack = false;

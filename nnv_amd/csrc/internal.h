@@ -987,6 +987,15 @@ int launch_fc_rowsum(nnvhip_ctx* ctx, const nnvhip_fc* fc, nnvhip_star* out, int
 int finalize_fused_ranges(nnvhip_ctx* ctx, nnvhip_star* s, const BufRef& part, int64_t chunks,
                           const double* cpart = nullptr, int64_t cchunks = 0, const double* cbias = nullptr);
 
+// fc_skinny.hip: a fully connected layer of few outputs over sets a ReLU step has just made, in one launch that needs neither the
+// step's rows reset nor its unit vectors in memory.  Whether all sets of a call take it, how many chunks of range sums it
+// leaves of a set, and the launch (part[i]: room for set i's chunks of [4][Mp]).
+bool fc_skinny_takes(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in);
+int fc_skinny_waves(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in);  // ... of a block, which its chunks depend on
+int64_t fc_skinny_chunks(const nnvhip_star* in, int waves);
+int launch_fc_skinny(nnvhip_ctx* ctx, const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in, nnvhip_star* const* out, double* const* part,
+                     int waves);
+
 // fc_window.hip: the contraction of a fully connected layer over sets whose generator images are zero outside known windows
 // (nnvhip_star::box), tile by tile over the windows' union only.
 // Whether the layer may at all, over images of H x W positions ...
