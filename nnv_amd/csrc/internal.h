@@ -297,7 +297,9 @@ using ConsRef = Ref<ConsNode>;
 inline ConsRef make_cons(nnvhip_ctx* ctx) { return ConsRef(new (ctx) ConsNode()); }
 
 // start of every entry point that touches device data: selects the context's device
-int enter_ctx(nnvhip_ctx* ctx);
+// Every entry point that may put work on the context's stream comes through here first.  makes_sets: copies of staged bounds may go
+// on waiting for more of them (nnvhip_ctx::waiting).
+int enter_ctx(nnvhip_ctx* ctx, bool makes_sets = false);
 
 // Key of the per-context weight cache: a 128-bit hash of the layer's host arrays plus its geometry.  Layers are
 // created from host arrays by value (FullyConnectedLayer(W, b), Star.affineMap(W, b) have no handle to pass
@@ -462,6 +464,21 @@ struct nnvhip_ctx {
   int trim();
   // Returns host-pinned scratch of `bytes`; waits for the stream when the ring wraps.
   int stage(size_t bytes, void** host);
+  // Copies `bytes` of the staging ring to a buffer, `at` bytes from its start (all aligned to 16 bytes; async on the stream).
+  // may_wait: the copy may be put off until the next entry point (enter_ctx) so that several travel together; the buffer
+  // is held until then.
+  static constexpr size_t kStagedByKernel = size_t(256) << 10;  // larger ones go to a copy engine
+  static constexpr size_t kWaitingCopies = 16;
+  struct WaitingCopy {
+    nnvhip::BufRef dev;
+    size_t at;
+    const void* staged;
+    uint32_t words;
+  };
+  std::vector<WaitingCopy> waiting;
+  bool copied_last = false;  // nothing but constructors has come in since a copy was launched at once
+  int copy_staged(const nnvhip::BufRef& dev, size_t at, const void* staged, size_t bytes, bool may_wait = false);
+  int flush_copies();
   // Copies a host table to a fresh device buffer through the pinned ring (async on the stream).
   int upload(const void* host, size_t bytes, nnvhip::BufRef* out);
   // A descriptor table that only the launches of the current call read.  Small ones stay in the pinned

@@ -190,7 +190,8 @@ int nnvhip_copy_host(nnvhip_ctx* c, int64_t n, const double* src, double* dst) {
 
 int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* lb, const double* ub,
                          nnvhip_star** out) {
-  CHECK_CTX(c);
+  if (!c) NNV_FAIL(NNVHIP_ERR_ARG, "null context");
+  NNV_TRY(nnvhip::enter_ctx(c, true));
   if (!lb || !ub || !out) NNV_FAIL(NNVHIP_ERR_ARG, "null argument");
   if (N <= 0 || count <= 0 || count > 65535) NNV_FAIL(NNVHIP_ERR_SHAPE, "Inconsistent dimensions between lb and ub");
   const int64_t ld = round_up(N, kLdAlign);
@@ -338,7 +339,7 @@ int nnvhip_star_from_box(nnvhip_ctx* c, int64_t N, int64_t count, const double* 
     }
     if (e < e1 && tail.empty()) write_tail(h + tail_off);
     else if (e < e1) memcpy(h + (e - e0), tail.data() + (e - tail_off), sizeof(double) * (size_t)(e1 - e));
-    NNV_HIP_TRY(hipMemcpyAsync(buf->as<double>() + e0, st, sizeof(double) * (size_t)(e1 - e0), hipMemcpyHostToDevice, c->stream));
+    NNV_TRY(c->copy_staged(buf, sizeof(double) * (size_t)e0, st, sizeof(double) * (size_t)(e1 - e0), e1 == total && e0 == 0));
   }
   c->h2d_bytes += (int64_t)bytes;
   double* d = buf->as<double>();

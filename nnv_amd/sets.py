@@ -13,7 +13,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
-from ._lib import check, f64, ptr
+from ._lib import check, f64, ptr, ref
 
 
 class _Handle:
@@ -73,7 +73,7 @@ class _Handle:
         N, _, _ = self.dims()
         lb = np.empty(N)
         ub = np.empty(N)
-        check(self.ctx.lib.nnvhip_estimate_ranges(self.ctx.handle, self.h, ptr(lb), ptr(ub)))
+        check(self.ctx.lib.nnvhip_estimate_ranges(self.ctx.handle, self.h, ref(lb), ref(ub)))
         return lb, ub
 
     def relu_info(self):
@@ -108,18 +108,24 @@ def _change_device(obj, deviceTarget):
     raise ValueError("Device target must be 'cpu' or 'gpu'.")
 
 
+def _box_bounds(lb, ub):
+    """The bounds of a box as two vectors of one length (set/Box.m:20-33)."""
+    lb = np.asarray(lb, dtype=np.float64)
+    ub = np.asarray(ub, dtype=np.float64)
+    if (lb.ndim == 2 and lb.shape[1] != 1) or (ub.ndim == 2 and ub.shape[1] != 1):
+        raise ValueError("lb and ub should be a vector")
+    lb = lb.reshape(-1)
+    ub = ub.reshape(-1)
+    if lb.size != ub.size:
+        raise ValueError("Inconsistent dimensions between lb and ub")
+    return lb, ub
+
+
 class Box:
     """set/Box.m: hyper-rectangle with centre/generator form and uniform partitioning."""
 
     def __init__(self, lb, ub):
-        lb = np.asarray(lb, dtype=np.float64)
-        ub = np.asarray(ub, dtype=np.float64)
-        if (lb.ndim == 2 and lb.shape[1] != 1) or (ub.ndim == 2 and ub.shape[1] != 1):
-            raise ValueError("lb and ub should be a vector")
-        lb = lb.reshape(-1)
-        ub = ub.reshape(-1)
-        if lb.size != ub.size:
-            raise ValueError("Inconsistent dimensions between lb and ub")
+        lb, ub = _box_bounds(lb, ub)
         self.lb = lb
         self.ub = ub
         self.dim = lb.size
@@ -259,14 +265,14 @@ class Star:
         ctx = ctx or _lib.default_context()
         lib = ctx.lib
         if len(args) == 2:
-            lb = np.asarray(args[0], dtype=np.float64)
-            ub = np.asarray(args[1], dtype=np.float64)
-            b = Box(lb, ub)  # size checks
-            out = (C.c_void_p * 1)()
-            check(lib.nnvhip_star_from_box(ctx.handle, b.dim, 1, ptr(f64(b.lb)), ptr(f64(b.ub)), out))
-            self._h = _Handle(C.c_void_p(out[0]), ctx)
-            self.state_lb = b.lb.copy()
-            self.state_ub = b.ub.copy()
+            # the set's private copies of its bounds are what the library reads: contiguous whatever was handed in
+            lb, ub = _box_bounds(args[0], args[1])
+            lb, ub = lb.copy(), ub.copy()
+            out = C.c_void_p()
+            check(lib.nnvhip_star_from_box(ctx.handle, lb.size, 1, ref(lb), ref(ub), C.byref(out)))
+            self._h = _Handle(out.value, ctx)
+            self.state_lb = lb
+            self.state_ub = ub
             return
         if len(args) in (3, 5):
             V = f64(args[0])
@@ -508,7 +514,7 @@ class Star:
         lb = np.empty((N, len(sets)), order="F")
         ub = np.empty((N, len(sets)), order="F")
         arr = sets.handles() if isinstance(sets, SetArray) else (C.c_void_p * len(sets))(*[s._h.h for s in sets])
-        check(ctx.lib.nnvhip_estimate_ranges_batch(ctx.handle, len(sets), arr, ptr(lb), ptr(ub)))
+        check(ctx.lib.nnvhip_estimate_ranges_batch(ctx.handle, len(sets), arr, ref(lb.T), ref(ub.T)))
         return lb, ub
 
 

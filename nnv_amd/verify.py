@@ -13,7 +13,7 @@ import ctypes as C
 import numpy as np
 
 from . import _lib
-from ._lib import HS_DISJOINT, HS_INSIDE, HS_UNDECIDED, check, f64, ptr
+from ._lib import HS_DISJOINT, HS_INSIDE, HS_UNDECIDED, check, f64, ptr, ref
 from .sets import ImageStar, SetArray, Star
 
 
@@ -89,8 +89,8 @@ def halfspace_check(sets, halfspaces):
     lo = np.empty((R, count), order="F")
     hi = np.empty((R, count), order="F")
     arr = (C.c_void_p * count)(*[S._h.h for S in sets])
-    check(ctx.lib.nnvhip_halfspace_check(ctx.handle, count, arr, n_hs, ptr(row_ptr), ptr(G), ptr(g), N,
-                                         ptr(verdict), ptr(lo), ptr(hi)))
+    check(ctx.lib.nnvhip_halfspace_check(ctx.handle, count, arr, n_hs, ref(row_ptr), ref(G.T), ref(g), N,
+                                         ref(verdict.T), ref(lo.T), ref(hi.T)))
     return verdict, lo, hi
 
 

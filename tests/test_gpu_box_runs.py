@@ -1,0 +1,68 @@
+"""Sets made one after the other: their bounds are fetched several sets at a time (the first at once, up to sixteen later ones with the
+next call that is not a constructor).  Whatever comes in between - sets that are dropped at once, sizes that differ, a set too
+large for it, a staging ring that wraps - every set has its own centre and generators, to the bit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def nnv():
+    import nnv_amd
+    return nnv_amd
+
+
+def _check(S, lb, ub):
+    V = np.array(S.V)
+    half = 0.5 * (ub - lb)
+    keep = np.flatnonzero(half != 0) if lb.size > 1 else np.arange(1)
+    exp = np.zeros((lb.size, keep.size + 1))
+    exp[:, 0] = 0.5 * (lb + ub)
+    exp[keep, 1 + np.arange(keep.size)] = half[keep]
+    assert np.array_equal(V, exp)
+    assert np.array_equal(S.predicate_lb, -np.ones(keep.size)) and np.array_equal(S.predicate_ub, np.ones(keep.size))
+
+
+@pytest.mark.parametrize("count", [1, 2, 16, 17, 18, 40])
+def test_runs_of_constructors(nnv, count):
+    rs = np.random.RandomState(count)
+    made = []
+    for i in range(count):
+        n = int(rs.choice([1, 2, 15, 16, 17, 300, 784]))
+        lb = rs.randn(n)
+        ub = lb + rs.rand(n) * (rs.rand(n) < 0.8)
+        S = nnv.Star(lb, ub)
+        if i % 3 == 1:
+            del S            # its memory is free for the next one's only behind the copy that still goes there
+            continue
+        made.append((S, lb.copy(), ub.copy()))
+        lb += 1.0            # the caller's arrays are its own again
+        ub -= 7.0
+    for S, lb, ub in made:
+        _check(S, lb, ub)
+
+
+def test_large_and_small_in_turn_past_the_end_of_the_ring(nnv):
+    rs = np.random.RandomState(9)
+    for rep in range(4):
+        made = []
+        for n in [3000, 70000, 5, 120000, 64, 64, 20000]:
+            lb = rs.randn(n)
+            ub = lb.copy()
+            ub[:: max(1, n // 40)] += 0.25     # few generators: the matrices stay small
+            made.append((nnv.Star(lb, ub), lb, ub))
+        for S, lb, ub in made:
+            l, u = S.estimateRanges()
+            tol = 4 * np.finfo(float).eps * (np.abs(lb) + np.abs(ub))
+            assert np.all(np.abs(l - lb) <= tol) and np.all(np.abs(u - ub) <= tol)
+
+
+def test_bounds_in_any_layout(nnv):
+    """Strided, transposed, integer and read-only bounds: the set reads a copy."""
+    a = np.arange(60.0).reshape(6, 10)
+    ro = a[2].copy()
+    ro.setflags(write=False)
+    for lb in (a[:, 3], a.T[2], a[1, ::3], np.arange(5), ro, a[:, :1]):
+        lbf = np.asarray(lb, dtype=np.float64)
+        _check(nnv.Star(lb, lb + 2), lbf.reshape(-1), lbf.reshape(-1) + 2)
