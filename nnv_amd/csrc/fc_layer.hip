@@ -573,25 +573,35 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
           };
           std::vector<RowShape> shapes;
           std::vector<int> shape_of((size_t)count, -1);
-          bool shared = true;
-          for (int64_t i = 0; i < count && shared; ++i) {
-            if (filled[i]) continue;
-            const ColSource& cs = in[i]->cs;
-            shared = cs.W != nullptr && cs.Wt != nullptr && cs.from == 1 && cs.from + cs.cols >= dense[i] && cs.zero_to <= 1 &&
-                     !cs.win_pending() && dense[i] >= 128 && cs.rows < (int64_t(1) << 30);
-            if (!shared) break;
-            for (size_t k = 0; k < shapes.size() && shape_of[i] < 0; ++k) {
-              const RowShape& r = shapes[k];
-              if (r.Wt == cs.Wt && r.ldwt == cs.ldwt && r.rows == cs.rows && r.idx == cs.idx && r.scale == cs.scale && r.dense == dense[i])
-                shape_of[i] = (int)k;
-            }
-            if (shape_of[i] < 0) {
-              if (shapes.size() == 16) {  // too many different shapes for the matrices to pay
-                shared = false;
-                break;
+          // Sets with scales of their own (boxes around different points: half-widths that differ by a rounding) share the
+          // rows of the weights as they are, and the tiles multiply by the set's scales on the way to the matrix cores: for
+          // 100 sets of 785 columns the packing of 100 copies took 109 us and the product 1189, now 16 + 8 and 1233.
+          bool shared = false, scaled = false;
+          for (int own_scales = 0; own_scales < 2 && !shared; ++own_scales) {
+            shapes.clear();
+            std::fill(shape_of.begin(), shape_of.end(), -1);
+            shared = true;
+            scaled = own_scales != 0;
+            for (int64_t i = 0; i < count && shared; ++i) {
+              if (filled[i]) continue;
+              const ColSource& cs = in[i]->cs;
+              shared = cs.W != nullptr && cs.Wt != nullptr && cs.from == 1 && cs.from + cs.cols >= dense[i] && cs.zero_to <= 1 &&
+                       !cs.win_pending() && dense[i] >= 128 && cs.rows < (int64_t(1) << 30);
+              if (!shared) break;
+              const double* scale = scaled ? nullptr : cs.scale;
+              for (size_t k = 0; k < shapes.size() && shape_of[i] < 0; ++k) {
+                const RowShape& r = shapes[k];
+                if (r.Wt == cs.Wt && r.ldwt == cs.ldwt && r.rows == cs.rows && r.idx == cs.idx && r.scale == scale && r.dense == dense[i])
+                  shape_of[i] = (int)k;
               }
-              shape_of[i] = (int)shapes.size();
-              shapes.push_back(RowShape{cs.Wt, cs.ldwt, cs.rows, cs.idx, cs.scale, dense[i], round_up(dense[i], 128), dense[i] / 128, 0});
+              if (shape_of[i] < 0) {
+                if (shapes.size() == 16) {  // too many different shapes for the matrices to pay
+                  shared = false;
+                  break;
+                }
+                shape_of[i] = (int)shapes.size();
+                shapes.push_back(RowShape{cs.Wt, cs.ldwt, cs.rows, cs.idx, scale, dense[i], round_up(dense[i], 128), dense[i] / 128, 0});
+              }
             }
           }
           shared = shared && !shapes.empty();
@@ -600,7 +610,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
           // little - the group's product over the rows most of its sets keep is formed once (by the tile kernel), and a
           // set's output is that product plus the few rows in which the set differs, written by one streaming pass
           // (delta_try / delta_done below).
-          bool delta_try = shared && count >= 32 && !c->no_row_deltas;
+          bool delta_try = shared && !scaled && count >= 32 && !c->no_row_deltas;
           for (size_t k = 1; k < shapes.size() && delta_try; ++k) delta_try = shapes[k].rows == shapes[0].rows;
           delta_try = delta_try && !shapes.empty() && shapes[0].rows == fc->Kp && shapes[0].rows < (int64_t(1) << 20);
           if (shared) {
@@ -897,6 +907,10 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
                 sg.centre = in[i]->V;
                 sg.gather_b = 1;
                 sg.zero_row = (int32_t)r.rows;
+                if (scaled) {
+                  sg.scale = in[i]->cs.scale;
+                  sg.scale_idx = in[i]->cs.idx;
+                }
               } else {
                 sg.Bt = bt[i];
                 sg.ldbt = ldt[i];
@@ -921,7 +935,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
             st = c->upload_table(tiles[w].data(), sizeof(SegTile) * tiles[w].size(), &dt);
             if (st == NNVHIP_OK)
               st = launch_gemm_seg(c, Wd, fc->Mp, outs[0]->V, ldo, fc->Mp, bias, widths[w], dt->as<SegTile>(), (int64_t)tiles[w].size(),
-                                   flop[w], w == 3);
+                                   flop[w], w == 3, scaled);
           }
           bias_in_kernel = true;
           }  // !delta_done

@@ -31,7 +31,7 @@ constexpr int kSegS = 4;     // stages in LDS
 constexpr int kSegNT = 512;  // threads per block
 
 // TN columns per tile; WR x WC waves, each owning (16*FM) rows x (16*FN) columns.
-template <int TN, int WR, int WC, int FM, int FN, bool GATHER = false>
+template <int TN, int WR, int WC, int FM, int FN, bool GATHER = false, bool SCALED = false>
 __global__ __launch_bounds__(kSegNT, 4) void gemm_seg_kernel(const double* __restrict__ A, int64_t lda,
                                                             double* __restrict__ C, int64_t ldc, int Mp,
                                                             const double* __restrict__ bias, int tiles_m, int64_t tiles_n,
@@ -71,6 +71,17 @@ __global__ __launch_bounds__(kSegNT, 4) void gemm_seg_kernel(const double* __res
     const bool ok = t < sg.valid && sc >= 1 && sg.rpart != nullptr;
     const double* src = tid < TN ? sg.plb : sg.pub;
     if (ok) pb_reg = src[sc - 1];
+  }
+  // SCALED: the rows of B are those of the weights as they are, and what a column is multiplied by is the set's own: the factors of
+  // the lane's columns (one multiplication per operand and column ahead of FM matrix instructions).  Asked for before the row list, whose arrival the first transfers wait for:
+  // nothing in the K loop waits for them.
+  static_assert(!SCALED || GATHER, "only gathered rows come without their scales");
+  double fac[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int t = wc * (16 * FN) + l16 * FN + j;
+    fac[j] = 1.0;
+    if (SCALED && sg.scale != nullptr && t < sg.valid && sg.col_local0 + t >= 1) fac[j] = sg.scale[sg.scale_idx[sg.col_local0 + t - 1]];
   }
   // row list: wave w stages row 8 * st + w of stage st; lane j keeps the entries of stages j, j + 64, ...
   static_assert(!GATHER || TN == 128, "rows of B are gathered one per wave");
@@ -166,6 +177,10 @@ __global__ __launch_bounds__(kSegNT, 4) void gemm_seg_kernel(const double* __res
         vv[0] = v01[0], vv[1] = v01[1];
       } else {
         vv[0] = bs[k * TN];
+      }
+      if constexpr (SCALED) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) vv[j] = __dmul_rn(vv[j], fac[j]);
       }
 #pragma unroll
       for (int i = 0; i < FM; ++i)
@@ -370,7 +385,7 @@ __global__ __launch_bounds__(256) void pack_rows_t_direct_kernel(const PackSet* 
   }
 }
 
-template <int TN, int WR, int WC, int FM, int FN, bool GATHER = false>
+template <int TN, int WR, int WC, int FM, int FN, bool GATHER = false, bool SCALED = false>
 int launch_seg_cfg(nnvhip_ctx* ctx, const double* A, int64_t lda, double* C, int64_t ldc, int64_t Mp, const double* bias,
                    const SegTile* segs, int64_t ntiles, double flop) {
   const int64_t tiles_m = ceil_div(Mp, kSegTM);
@@ -380,7 +395,7 @@ int launch_seg_cfg(nnvhip_ctx* ctx, const double* A, int64_t lda, double* C, int
   const int64_t xr = 1, local_m = tiles_m;
   const int64_t slots = local_m * ceil_div(ntiles, 8 / xr);
   const bool timed = ctx->kernel_timing;
-  NNV_LAUNCH(ctx, timed, (gemm_seg_kernel<TN, WR, WC, FM, FN, GATHER>), dim3((unsigned)(8 * slots)), dim3(kSegNT), 0, A, lda, C, ldc, (int)Mp,
+  NNV_LAUNCH(ctx, timed, (gemm_seg_kernel<TN, WR, WC, FM, FN, GATHER, SCALED>), dim3((unsigned)(8 * slots)), dim3(kSegNT), 0, A, lda, C, ldc, (int)Mp,
              bias, (int)tiles_m, ntiles, (int)xr, (int)local_m, segs);
   NNV_TRY(ctx->kernel_timer_end(timed, 9, flop));  // a timing group of its own
   NNV_HIP_TRY(hipGetLastError());
@@ -1136,10 +1151,11 @@ int launch_masked_centres(nnvhip_ctx* ctx, int64_t count, const CentreSet* sets_
 }
 
 int launch_gemm_seg(nnvhip_ctx* ctx, const double* A, int64_t lda, double* C, int64_t ldc, int64_t Mp, const double* bias,
-                    int tn, const SegTile* segs, int64_t ntiles, double flop, bool gather_b) {
+                    int tn, const SegTile* segs, int64_t ntiles, double flop, bool gather_b, bool scaled) {
   if (ntiles == 0) return NNVHIP_OK;
   if (Mp % 16 || lda % 2 || Mp > ldc) NNV_FAIL(NNVHIP_ERR_SHAPE, "internal: GEMM operands violate the padding contract");
   if (gather_b && tn != 128) NNV_FAIL(NNVHIP_ERR_ARG, "internal: rows of B are gathered by the 128-column tile only");
+  if (gather_b && scaled) return launch_seg_cfg<128, 2, 4, 4, 2, true, true>(ctx, A, lda, C, ldc, Mp, bias, segs, ntiles, flop);
   if (gather_b) return launch_seg_cfg<128, 2, 4, 4, 2, true>(ctx, A, lda, C, ldc, Mp, bias, segs, ntiles, flop);
   switch (tn) {
     case 128: return launch_seg_cfg<128, 2, 4, 4, 2>(ctx, A, lda, C, ldc, Mp, bias, segs, ntiles, flop);

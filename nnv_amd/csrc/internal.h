@@ -758,6 +758,9 @@ struct SegTile {
   // gather_b (128-column tiles only): Bt holds one row per input row plus a row of zeros at index zero_row (for
   // the padded entries of kmap); a tile with col_local0 == 0 takes its column 0 from centre[kmap[t]] instead
   const double* centre;
+  // ... launched as scaled: Bt's column j >= 1 is multiplied by scale[scale_idx[j - 1]] on its way (null: by one)
+  const double* scale;
+  const int32_t* scale_idx;
   int32_t gather_b;
   int32_t zero_row;
   int32_t kp;
@@ -770,7 +773,7 @@ struct SegTile {
 constexpr int32_t kSegSubtract = 1 << 30;
 int launch_pack_rows_t(nnvhip_ctx* ctx, int64_t count, const PackSet* sets);
 int launch_gemm_seg(nnvhip_ctx* ctx, const double* A, int64_t lda, double* C, int64_t ldc, int64_t Mp, const double* bias,
-                    int tn, const SegTile* segs, int64_t ntiles, double flop, bool gather_b = false);
+                    int tn, const SegTile* segs, int64_t ntiles, double flop, bool gather_b = false, bool scaled = false);
 // Row lists of the sets of an array, by group (sets whose packed rows agree wherever they keep the same row): the
 // rows a majority of a group keeps (`common`, ascending, padded with -1 to a multiple of 16; its padded length in
 // ncommon[group]) and, per set, the rows in which it differs from its group's list (`delta`: at most cap entries
