@@ -45,6 +45,10 @@ struct SetDesc {
   double* out;
   int32_t ncols;
   int32_t pad_;
+  // columns [box_from, box_to) are zero outside their windows box[j], whatever the memory holds there (images of HW positions, H a
+  // column; permute_rows_lds_kernel only; null: none)
+  const ColBox* box;
+  int32_t box_from, box_to, H, HW;
 };
 
 struct RowmapArgs {
@@ -357,31 +361,57 @@ __global__ __launch_bounds__(64 * kEwWaves) void permute_rows_kernel(const SetDe
 }
 
 // Short columns (N <= kPermLdsRows): a block stages whole columns in LDS with coalesced loads and
-// gathers from there, so global memory sees only contiguous traffic.  Grid: (1, column chunks, sets).
+// gathers from there, so global memory sees only contiguous traffic.  Images that are in memory inside their windows only
+// (SetDesc::box) are read there and zero elsewhere: 3400 images of 8 x 8 x 16 10.4 us of zeros written + 13.7 -> 15.8.
+// Grid: (1, column chunks, sets).
 constexpr int kPermLdsRows = 4096;
-constexpr int kPermCols = 2;  // columns staged per step
+__host__ __device__ constexpr int perm_stride(int n_rows) { return n_rows + n_rows / 32 + 1; }
+// columns staged per step: four where four blocks of them fit a CU, two within 64 KB
+constexpr int perm_columns(int n_rows) { return n_rows <= 1024 ? 4 : n_rows <= 3968 ? 2 : 1; }
 
 __global__ __launch_bounds__(64 * kEwWaves) void permute_rows_lds_kernel(const SetDesc* __restrict__ table, SetDesc one,
-                                                                         PermArgs a, int n_rows) {
+                                                                         PermArgs a, int n_rows, int step) {
   const SetDesc d = table ? table[blockIdx.z] : one;
   const int j0 = blockIdx.y * a.cols_per_chunk;
   if (j0 >= d.ncols) return;
   const int j1 = min(d.ncols, j0 + a.cols_per_chunk);
-  __shared__ double stage[kPermCols][kPermLdsRows];
+  // (a place left free behind every 32: the rows that neighbouring outputs come from are often a multiple of 32 apart, 64 lanes on
+  // one bank)
+  extern __shared__ double stage[];
+  const int stride = perm_stride(n_rows);
   const int tid = threadIdx.x;
-  for (int jb = j0; jb < j1; jb += kPermCols) {
+  for (int jb = j0; jb < j1; jb += step) {
+    const int nc = min(step, j1 - jb);
+    // a row's place in the image serves all columns; four columns' entries are asked for together
+    for (int r = tid; r < n_rows; r += 64 * kEwWaves) {
+      int h = 0, w = 0;
+      if (d.box != nullptr) {
+        const int p = r % d.HW;
+        w = p / d.H, h = p - w * d.H;
+      }
+      for (int u0 = 0; u0 < nc; u0 += 4) {
+        double v[4];
 #pragma unroll
-    for (int u = 0; u < kPermCols; ++u)
-      if (jb + u < j1)
-        for (int r = tid; r < n_rows; r += 64 * kEwWaves) stage[u][r] = d.in[r + (int64_t)(jb + u) * a.ldin];
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < kPermCols; ++u)
-      if (jb + u < j1)
-        for (int64_t r = tid; r < a.ldout; r += 64 * kEwWaves) {
-          const int src = a.src_row[r];
-          d.out[r + (int64_t)(jb + u) * a.ldout] = src >= 0 ? stage[u][src] : 0.0;
+        for (int u = 0; u < 4; ++u) {
+          const int j = jb + u0 + u;
+          bool in = u0 + u < nc;
+          if (in && d.box != nullptr && j >= d.box_from && j < d.box_to) {
+            const ColBox b = d.box[j];
+            in = h >= b.h0 && h <= b.h1 && w >= b.w0 && w <= b.w1;
+          }
+          v[u] = in ? d.in[r + (int64_t)j * a.ldin] : 0.0;
         }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (u0 + u < nc) stage[(u0 + u) * stride + r + r / 32] = v[u];
+      }
+    }
+    __syncthreads();
+    for (int64_t r = tid; r < a.ldout; r += 64 * kEwWaves) {
+      const int src = a.src_row[r];
+      const double* from = stage + max(src, 0) + max(src, 0) / 32;
+      for (int u = 0; u < nc; ++u) d.out[r + (int64_t)(jb + u) * a.ldout] = src >= 0 ? from[u * stride] : 0.0;
+    }
     __syncthreads();
   }
 }
@@ -389,13 +419,22 @@ __global__ __launch_bounds__(64 * kEwWaves) void permute_rows_lds_kernel(const S
 // Common launch plumbing: output handles, descriptor table, grid with a few thousand blocks.
 template <class Launch>
 static int run_row_layer(nnvhip_ctx* c, int64_t count, nnvhip_star* const* in, nnvhip_star** out, int64_t Nout,
-                         int64_t rows_per_block, int min_cols_per_chunk, Launch launch) {
+                         int64_t rows_per_block, int min_cols_per_chunk, Launch launch, bool reads_windows = false) {
   if (count > 65535) NNV_FAIL(NNVHIP_ERR_SHAPE, "at most 65535 sets per call");
   for (int64_t i = 0; i < count; ++i) {
     if (in[i]->N != in[0]->N || in[i]->ld != in[0]->ld)
       NNV_FAIL(NNVHIP_ERR_SHAPE, "sets of one array must have the same dimension");
   }
-  NNV_TRY(ensure_dense_batch(c, count, in));  // these passes read every column
+  // These passes read every column.  (reads_windows: the launch knows how to read a set of which nothing is missing but the zeros
+  // around its images' windows.)
+  auto only_zeros_missing = [&](const nnvhip_star* s) {
+    return reads_windows && s->cs.win_pending() && !s->cs.in_pixels() && !s->rows_pending && s->stored_cols() == s->n + 1 && !s->cs.pending &&
+           s->cs.zero_to <= 1 && !s->cs.delta_pending() && s->cs.win_rows == s->N;
+  };
+  std::vector<nnvhip_star*> whole;
+  for (int64_t i = 0; i < count; ++i)
+    if (!only_zeros_missing(in[i])) whole.push_back(in[i]);
+  if (!whole.empty()) NNV_TRY(ensure_dense_batch(c, (int64_t)whole.size(), whole.data()));
   std::vector<nnvhip_star*> outs;
   bool contig = false;
   int64_t cols = 0;
@@ -409,6 +448,15 @@ static int run_row_layer(nnvhip_ctx* c, int64_t count, nnvhip_star* const* in, n
       descs[i].out = outs[i]->V;
       descs[i].ncols = (int32_t)(in[i]->n + 1);
       descs[i].pad_ = 0;
+      descs[i].box = nullptr;
+      if (only_zeros_missing(in[i])) {
+        const ColSource& cs = in[i]->cs;
+        descs[i].box = cs.win_box;
+        descs[i].box_from = (int32_t)cs.win_from;
+        descs[i].box_to = (int32_t)cs.win_to;
+        descs[i].H = cs.win_H;
+        descs[i].HW = cs.win_H * cs.win_W;
+      }
       max_cols = std::max<int64_t>(max_cols, in[i]->n + 1);
     }
     const SetDesc* table = nullptr;
@@ -889,13 +937,14 @@ int nnvhip_permute_rows(nnvhip_ctx* c, int64_t N, const int32_t* src_row, int64_
   a.src_row = perm->as<int32_t>();
   a.ldin = in[0]->ld;
   if (ld <= kPermLdsRows)
-    return run_row_layer(c, count, in, out, N, int64_t(1) << 30, 4 * kPermCols,
+    return run_row_layer(c, count, in, out, N, int64_t(1) << 30, perm_columns((int)N),
                          [&](dim3 grid, const SetDesc* table, const SetDesc& one, int32_t cpc, int64_t ldout) {
                            a.cols_per_chunk = cpc;
                            a.ldout = ldout;
-                           NNV_LAUNCH(c, c->kernel_timing, permute_rows_lds_kernel, grid, dim3(64 * kEwWaves), 0, table, one,
-                                              a, (int)N);
-                         });
+                           const int step = perm_columns((int)N);
+                           NNV_LAUNCH(c, c->kernel_timing, permute_rows_lds_kernel, grid, dim3(64 * kEwWaves),
+                                      sizeof(double) * step * perm_stride((int)N), table, one, a, (int)N, step);
+                         }, true);
   return run_row_layer(c, count, in, out, N, kEwRows, 4 * kEwWaves,
                        [&](dim3 grid, const SetDesc* table, const SetDesc& one, int32_t cpc, int64_t ldout) {
                          a.cols_per_chunk = cpc;
