@@ -455,9 +455,14 @@ bool conv_window_takes(const nnvhip_conv2d* cv, int64_t H, int64_t W, int64_t Ho
 static int conv_window_tile(const nnvhip_conv2d* cv) { return cv->Cout <= 16 ? 16 : cv->Cout <= 32 ? 32 : 64; }
 
 int conv_window_parts(const nnvhip_conv2d* cv, int64_t Ho, int64_t Wo, int64_t dense, int eh, int ew) {
-  // about 1024 blocks for a set by itself, no part with less than a tile of columns
+  // A set by itself: blocks that fill the 1024 places of four to a CU once, or, where positions are too many for that to come
+  // out nearly even, twice; about one more a position writes stamps.  No part with less than a tile of columns.  (15 x 15
+  // positions, 288 taps into 64 channels: 4 parts 77.9 us, 5 - 1360 blocks - 79.4, 8 - 2032 - 74.6, 12 85.0; 7 x 7 positions, 576
+  // taps: 14 parts 90.0, 18 - 992 blocks - 81.6, 21 - 1088 - 92.4, 32 92.8.)
+  const int64_t a_part = Ho * Wo * ceil_div(cv->Cout, conv_window_tile(cv)), places = 1024;
+  int64_t want = (places - Ho * Wo) / a_part;
+  if (want < 1 || (double)(want * a_part + Ho * Wo) < 0.93 * (double)places) want = std::max<int64_t>(want, (2 * places - Ho * Wo) / a_part);
   const double cols = (double)(dense - 1) * eh * ew / (double)(Ho * Wo);
-  const int64_t want = ceil_div(1024, Ho * Wo * ceil_div(cv->Cout, conv_window_tile(cv)));
   return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(want, 32), (int64_t)(cols / 32.0)));
 }
 
