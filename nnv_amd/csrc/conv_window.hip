@@ -79,7 +79,7 @@ constexpr int kConvWinCols = 128;   // columns of a position listed at a time
 // instructions they are for columns: where a listed row lies in an image and which of the filter's positions it belongs to are
 // one word, a column's window is one bit per position, made once a tile, and an element that is not wanted is read from a zero
 // instead of being dropped later (a row of padding meets zeros, so its weights need not be).  32 x 32 x 3 network, second to
-// fourth layer: 38, 129 and 151 us with columns, 26, 97 and 108 with pixels through the same instructions, 22, 85 and 91 now.
+// fourth layer: 38, 129 and 151 us with columns, 26, 97 and 108 with pixels through the same instructions, 22, 85 and 91 with these.
 template <int TM, int TN, int WR, int WC, int S_LANES, bool PIXELS>
 __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_kernel(const ConvWinSet* __restrict__ table, ConvWinSet one, ConvWinArgs a) {
   constexpr int NT = 64 * WR * WC, NW = WR * WC;
@@ -370,6 +370,10 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
+      // A wave without columns, and a stage of padding, leave the matrix cores to the other blocks: a part has 30 to 60 columns, and
+      // half of its second tile is often empty.  64 channels: 74.6 -> 70.5 and 80.8 -> 75.3 us; with 32 a stage's four
+      // instructions do not pay for the branch (22.0 -> 22.7).
+      const bool some_col = c0 + wc * (TN / WC) < n;
       Regs g0, g1;
       load_tiles(0, g0);
       load_tiles(KT, g1);
@@ -379,7 +383,8 @@ __global__ __launch_bounds__(64 * WR * WC, TM == 16 ? 3 : 4) void conv_window_ke
       auto step = [&](int t, Regs& next, Regs& far) {
         const int cur = t & 1;
         load_tiles(KT * min(t + 2, nk - 1), far);
-        mfma_tile_k16<FM, FN, KT>(&Ws[cur][wr * (TM / WR)], LDA_S, &Vs[cur][(wc * (TN / WC)) * LDB_S], LDB_S, lane, acc);
+        if (TM < 64 || (some_col && KT * t < nrow))
+          mfma_tile_k16<FM, FN, KT>(&Ws[cur][wr * (TM / WR)], LDA_S, &Vs[cur][(wc * (TN / WC)) * LDB_S], LDB_S, lane, acc);
         store_tiles(cur ^ 1, next);
         __syncthreads();
       };
@@ -458,7 +463,7 @@ int conv_window_parts(const nnvhip_conv2d* cv, int64_t Ho, int64_t Wo, int64_t d
   // A set by itself: blocks that fill the 1024 places of four to a CU once, or, where positions are too many for that to come
   // out nearly even, twice; about one more a position writes stamps.  No part with less than a tile of columns.  (15 x 15
   // positions, 288 taps into 64 channels: 4 parts 77.9 us, 5 - 1360 blocks - 79.4, 8 - 2032 - 74.6, 12 85.0; 7 x 7 positions, 576
-  // taps: 14 parts 90.0, 18 - 992 blocks - 81.6, 21 - 1088 - 92.4, 32 92.8.)
+  // taps: 14 parts 90.0, 19 - 992 blocks - 81.6, 21 - 1088 - 92.4, 32 92.8.)
   const int64_t a_part = Ho * Wo * ceil_div(cv->Cout, conv_window_tile(cv)), places = 1024;
   int64_t want = (places - Ho * Wo) / a_part;
   if (want < 1 || (double)(want * a_part + Ho * Wo) < 0.93 * (double)places) want = std::max<int64_t>(want, (2 * places - Ho * Wo) / a_part);
