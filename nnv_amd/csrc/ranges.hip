@@ -907,15 +907,20 @@ struct RowSumArgs {
 // 6.6 -> 5.4.  (Fewer rows to a block, for a block on every CU, cost more
 // than they bring: a load then touches twice as many lines.  1024 x 1024: 12.9 us with 4 rows, 6.5 with 8, 8.2 with 16.)
 constexpr int kRowSumRows = 8;  // output rows per block
+// E: sums of the GEMM's tiles a thread asks for ahead (512 outputs of 3136 inputs behind 77 tiles: 16.1 us with one, 14.0 with four)
+template <int E>
 __global__ __launch_bounds__(1024) void fc_rowsum_kernel(RowSumArgs a) {
   constexpr int R = kRowSumRows;
   constexpr int kGroups = 64 / R;      // input rows a wave takes at a time, R lanes each
   constexpr int kStep = 16 * kGroups;  // ... and the block
-  constexpr int kEarly = 1024 / (4 * R);
+  constexpr int kEarly = E * (1024 / (4 * R));
   __shared__ double red[16][3][R];
   __shared__ double skey[4 * R];
-  __shared__ double early[1024];
-  const int rb = blockIdx.x;
+  __shared__ double early[E * 1024];
+  // neighbouring row blocks on one XCD (workgroups are dealt to the eight in turn): they read the two halves of a line
+  // (784 inputs of a box into 1024 outputs 9.0 -> 6.8 us)
+  const int rb = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (rb * R >= a.Mp) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -923,8 +928,12 @@ __global__ __launch_bounds__(1024) void fc_rowsum_kernel(RowSumArgs a) {
   const int row = rb * R + rl;
   const double* wrow = a.W + row;
   const bool with_centre = a.centre_mode == 1;
-  double pv = 0.0, c_in = 0.0, c_bias = 0.0;
-  if (a.part != nullptr && tid / (4 * R) < a.chunks) pv = a.part[(int64_t)(tid / R) * a.ld + rb * R + tid % R];  // (chunk * 4 + sum)
+  double pv[E], c_in = 0.0, c_bias = 0.0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int t = e * 1024 + tid;
+    pv[e] = a.part != nullptr && t / (4 * R) < a.chunks ? a.part[(int64_t)(t / R) * a.ld + rb * R + t % R] : 0.0;  // (chunk * 4 + sum)
+  }
   if (tid < R) {
     if (a.centre_mode == 0) c_in = a.centre[row];
     else if (a.bias != nullptr) c_bias = a.bias[row];
@@ -973,7 +982,8 @@ __global__ __launch_bounds__(1024) void fc_rowsum_kernel(RowSumArgs a) {
     red[wave][1][rl] = sn;
     red[wave][2][rl] = cacc;
   }
-  early[tid] = pv;
+#pragma unroll
+  for (int e = 0; e < E; ++e) early[e * 1024 + tid] = pv[e];
   __syncthreads();
   if (tid < 4 * R) {  // sum q of a row: the GEMM tiles' chunks in order, then the gathered columns' term
     const int q = tid / R, r8 = tid % R;
@@ -1038,10 +1048,14 @@ int launch_fc_rowsum(nnvhip_ctx* ctx, const nnvhip_fc* fc, nnvhip_star* out, int
   a.ld = out->ld;
   a.lb = rb->as<double>();
   a.ub = a.lb + out->ld;
-  const unsigned blocks = (unsigned)(fc->Mp / kRowSumRows);
+  const unsigned blocks = (unsigned)round_up(fc->Mp / kRowSumRows, 8);
   // algorithmic bytes: W once, the finished ranges (timed with the gather passes it stands in for)
   const double bytes = 8.0 * (double)fc->Mp * (double)fc->K + 16.0 * (double)fc->Mp;
-  NNV_LAUNCH(ctx, ctx->kernel_timing, fc_rowsum_kernel, dim3(blocks), dim3(1024), 0, a);
+  // (more than 32 tiles: up to 128 of their sums asked for ahead)
+  if (chunks > 32)
+    NNV_LAUNCH(ctx, ctx->kernel_timing, fc_rowsum_kernel<4>, dim3(blocks), dim3(1024), 0, a);
+  else
+    NNV_LAUNCH(ctx, ctx->kernel_timing, fc_rowsum_kernel<1>, dim3(blocks), dim3(1024), 0, a);
   NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 5, bytes));
   NNV_HIP_TRY(hipGetLastError());
   out->rbuf = rb;
@@ -1461,7 +1475,17 @@ int compute_ranges(nnvhip_ctx* ctx, int64_t count, nnvhip_star* const* s, RangeC
   bool scan = false;
   for (int64_t i = 0; i < nset; ++i) scan = scan || !(descs[i].n == 0 && (descs[i].chunks2 > 0 || descs[i].part3 != nullptr));
   if (!scan)
-    for (int64_t i = 0; i < nset; ++i) descs[i].chunks = 0;
+    for (int64_t i = 0; i < nset; ++i) {
+      RangeDesc& d = descs[i];
+      d.chunks = 0;
+      // (the producer's chunks are then all there is: few rows of them take the kernel for that)
+      if (d.chunks2_at == 0 && d.part3 == nullptr && ld <= 64 && d.chunks2 >= kManyChunks) {
+        d.part = const_cast<double*>(d.part2);
+        d.chunks = d.chunks2;
+        d.part2 = nullptr;
+        d.chunks2 = 0;
+      }
+    }
   // an array of sets has blocks to spare for the last step: two rows per lane, read 16 bytes at a time
   bool wide_final = ceil_div(ld, 64) * nset >= 4096;
   {
