@@ -392,6 +392,7 @@ int nnvhip_create(int device, nnvhip_ctx** out) {
   c->no_sum_shortcuts = getenv("NNVHIP_NO_SUM_SHORTCUTS") != nullptr;
   c->no_host_pool = getenv("NNVHIP_NO_HOST_POOL") != nullptr;
   if (const char* e = getenv("NNVHIP_WEIGHT_CACHE_MB")) c->weight_cache_budget = (int64_t)atoll(e) << 20;
+  c->waiting.reserve(nnvhip_ctx::kWaitingCopies);  // (a constructor that adds one allocates nothing)
   NNV_HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   NNV_HIP_TRY(hipEventCreate(&c->ev0));
   NNV_HIP_TRY(hipEventCreate(&c->ev1));

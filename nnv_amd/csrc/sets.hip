@@ -167,8 +167,8 @@ int nnvhip_star_create(nnvhip_ctx* c, int64_t N, int64_t n, const double* V, con
 // Star(lb, ub) for every column of two N x count matrices.  A box's generators are scaled unit vectors, and the handle
 // says which (oh_idx, oh_scale): only the centres go to memory (vcols = 1), back to back, and whoever reads the whole
 // matrix has the columns written then (ensure_dense).  Everything the call puts on the device - centres, half-widths,
-// predicate bounds, index lists - is laid out in pinned memory and travels in one copy (pieces of kBoxPiece entries,
-// so that the staging ring stays at 16 MB whatever the array's size); no kernel runs.  (Writing the matrices took 133 us for 100 boxes of 784 dimensions, 1.54 ms for 1024 of them, 6.4 GB nobody read; seven small
+// predicate bounds, index lists - is laid out in pinned memory and travels from there together (nnvhip_ctx::copy_staged; pieces of kBoxPiece entries,
+// so that the staging ring stays at 16 MB whatever the array's size).  (Writing the matrices took 133 us for 100 boxes of 784 dimensions, 1.54 ms for 1024 of them, 6.4 GB nobody read; seven small
 // copies and kernels took 60 us of a single set's reach.)
 constexpr int64_t kBoxPiece = int64_t(1) << 20;
 // Host arrays of 1.5 MB and more are worth waking the context's workers for (some 20 us); several parts to a thread, so that
