@@ -158,6 +158,9 @@ NNVHIP_API int nnvhip_debug_relu_bounds(nnvhip_ctx* ctx, int64_t* appended_in_pl
  * NNVHIP_ERR_OOM past that, as it does where the device has no more; 0: no such limit.  The context also forgets that it
  * ever ran out of memory. */
 NNVHIP_API int nnvhip_debug_pool_limit(nnvhip_ctx* ctx, int64_t bytes);
+/* Test hook (no counterpart in the reference): the next `launches` launches that fetch bounds or tables from pinned memory are
+ * refused with NNVHIP_ERR_HIP instead of being made. */
+NNVHIP_API int nnvhip_debug_fail_copies(nnvhip_ctx* ctx, int64_t launches);
 /* Which way the sets of the layer calls went since the context was created, for tests of the dispatch rules: sets[r] =
  * how many took route r (NNVHIP_ROUTES entries).  A set counts where a kernel of the route was launched for it. */
 enum {

@@ -29,7 +29,7 @@ SYMBOLS = [
     "nnvhip_star_fetch_rows", "nnvhip_relu_apply_lists", "nnvhip_probe_mfma_peak",
     "nnvhip_estimate_ranges_static", "nnvhip_debug_mailbox_pack", "nnvhip_debug_mailbox_unpack",
     "nnvhip_debug_set_relu_call_number", "nnvhip_reach_layers", "nnvhip_reach_is_one_launch", "nnvhip_relu_reduce_mem",
-    "nnvhip_set_switch", "nnvhip_hint_next_fc", "nnvhip_debug_counters", "nnvhip_debug_relu_bounds", "nnvhip_debug_routes", "nnvhip_debug_pool_limit", "nnvhip_debug_staging", "nnvhip_weight_cache_stats", "nnvhip_weight_cache_release", "nnvhip_debug_weak_weight_hash",
+    "nnvhip_set_switch", "nnvhip_hint_next_fc", "nnvhip_debug_counters", "nnvhip_debug_relu_bounds", "nnvhip_debug_routes", "nnvhip_debug_pool_limit", "nnvhip_debug_fail_copies", "nnvhip_debug_staging", "nnvhip_weight_cache_stats", "nnvhip_weight_cache_release", "nnvhip_debug_weak_weight_hash",
 ]
 
 
@@ -131,6 +131,7 @@ def load():
         "nnvhip_debug_relu_bounds": [p, pi64, pi64],
         "nnvhip_debug_routes": [p, C.POINTER(i64)],
         "nnvhip_debug_pool_limit": [p, i64],
+        "nnvhip_debug_fail_copies": [p, i64],
         "nnvhip_debug_staging": [p, pi64, pi64],
         "nnvhip_weight_cache_stats": [p, pi64, pi64, pi64],
         "nnvhip_weight_cache_release": [p, pi64],
@@ -292,6 +293,10 @@ class Context:
     def debug_pool_limit(self, nbytes):
         """At most nbytes of device memory for the pool (0: no limit), see nnvhip_debug_pool_limit."""
         check(self.lib.nnvhip_debug_pool_limit(self.handle, int(nbytes)))
+
+    def debug_fail_copies(self, launches):
+        """The next launches that fetch staged bounds or tables fail, see nnvhip_debug_fail_copies."""
+        check(self.lib.nnvhip_debug_fail_copies(self.handle, int(launches)))
 
     def routes(self):
         """{route: sets that took it} since the context was created (nnvhip_debug_routes)."""

@@ -281,6 +281,10 @@ static int launch_copy_staged(nnvhip_ctx* c, const StagedPieces& p, int count) {
   uint32_t most = 0;
   for (int i = 0; i < count; ++i) most = std::max(most, p.words[i]);
   if (most == 0) return NNVHIP_OK;
+  if (c->failing_copies > 0) {
+    --c->failing_copies;
+    NNV_FAIL(NNVHIP_ERR_HIP, "launch of copy_staged_kernel refused (nnvhip_debug_fail_copies)");
+  }
   hipLaunchKernelGGL(copy_staged_kernel, dim3((most + 1023) / 1024, (unsigned)count), dim3(256), 0, c->stream, p);
   NNV_HIP_TRY(hipGetLastError());
   return NNVHIP_OK;
@@ -297,6 +301,7 @@ int nnvhip_ctx::copy_staged(const BufRef& dev, size_t at, const void* staged, si
   // waits for more of them, or for the next call that is not another constructor (25 images of 28 x 28 and their reach: 675 us
   // with a copy each, 690 with a launch each, 574 so).
   if (may_wait && copied_last) {
+    if (waiting.size() == kWaitingCopies) NNV_TRY(flush_copies());  // (their launch failed when the last of them came)
     waiting.push_back(WaitingCopy{dev, at, staged, (uint32_t)(bytes / 4)});
     return waiting.size() < kWaitingCopies ? NNVHIP_OK : flush_copies();
   }
@@ -316,9 +321,10 @@ int nnvhip_ctx::flush_copies() {
     p.out[i] = reinterpret_cast<uint32_t*>(static_cast<char*>(waiting[i].dev->ptr) + waiting[i].at);
     p.words[i] = waiting[i].words;
   }
-  const int st = launch_copy_staged(this, p, (int)waiting.size());
+  // (after a launch that failed they go on waiting: their sets' constructors have returned, so nothing else may run before them)
+  NNV_TRY(launch_copy_staged(this, p, (int)waiting.size()));
   waiting.clear();  // (released blocks are used again behind the launch, on the same stream)
-  return st;
+  return NNVHIP_OK;
 }
 
 int nnvhip_ctx::upload(const void* host, size_t bytes, BufRef* out) {
@@ -412,6 +418,7 @@ int nnvhip_destroy(nnvhip_ctx* c) {
   c->drain_deferred();
   if (c->live_handles != 0)
     NNV_FAIL(NNVHIP_ERR_ARG, "context still has %lld live handles", (long long)c->live_handles);
+  c->waiting.clear();  // (no handle is left that could read them)
   NNV_TRY(nnvhip::enter_ctx(c));
   c->trim();
   for (void* mem : c->free_stars) ::operator delete(mem);
@@ -647,6 +654,12 @@ int nnvhip_debug_pool_limit(nnvhip_ctx* c, int64_t bytes) {
   if (!c || bytes < 0) NNV_FAIL(NNVHIP_ERR_ARG, "null context or negative limit");
   c->pool_limit = bytes;
   c->pixel_limit = c->device_bytes / 8;
+  return NNVHIP_OK;
+}
+
+int nnvhip_debug_fail_copies(nnvhip_ctx* c, int64_t launches) {
+  if (!c || launches < 0) NNV_FAIL(NNVHIP_ERR_ARG, "null context or negative count");
+  c->failing_copies = launches;
   return NNVHIP_OK;
 }
 

@@ -477,8 +477,9 @@ struct nnvhip_ctx {
   };
   std::vector<WaitingCopy> waiting;
   bool copied_last = false;  // nothing but constructors has come in since a copy was launched at once
+  int64_t failing_copies = 0;  // so many launches are refused (nnvhip_debug_fail_copies)
   int copy_staged(const nnvhip::BufRef& dev, size_t at, const void* staged, size_t bytes, bool may_wait = false);
-  int flush_copies();
+  int flush_copies();  // (what could not be launched goes on waiting: the next entry point tries again)
   // Copies a host table to a fresh device buffer through the pinned ring (async on the stream).
   int upload(const void* host, size_t bytes, nnvhip::BufRef* out);
   // A descriptor table that only the launches of the current call read.  Small ones stay in the pinned

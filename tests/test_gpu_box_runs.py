@@ -1,6 +1,6 @@
 """Sets made one after the other: their bounds are fetched several sets at a time (the first at once, up to sixteen later ones with the
 next call that is not a constructor).  Whatever comes in between - sets that are dropped at once, sizes that differ, a set too
-large for it, a staging ring that wraps - every set has its own centre and generators, to the bit."""
+large for it, a staging ring that wraps, a launch that fails - every set has its own centre and generators, to the bit."""
 import numpy as np
 import pytest
 
@@ -66,3 +66,50 @@ def test_bounds_in_any_layout(nnv):
     for lb in (a[:, 3], a.T[2], a[1, ::3], np.arange(5), ro, a[:, :1]):
         lbf = np.asarray(lb, dtype=np.float64)
         _check(nnv.Star(lb, lb + 2), lbf.reshape(-1), lbf.reshape(-1) + 2)
+
+
+def _boxes(ctx, nnv, rs, count):
+    made = []
+    for n in rs.choice([1, 16, 17, 300], count):
+        lb = rs.randn(int(n))
+        ub = lb + rs.rand(lb.size)
+        made.append((nnv.Star(lb, ub, ctx=ctx), lb, ub))
+    return made
+
+
+def test_bounds_whose_copy_could_not_be_launched_go_on_waiting(nnv):
+    """The constructors have returned: every later call fails until the bounds are there, and then all is as if nothing had been."""
+    from nnv_amd import _lib
+    ctx, rs = _lib.Context(0), np.random.RandomState(3)
+    for count in (2, 6, 16):   # one at once, the others wait
+        made = _boxes(ctx, nnv, rs, count)
+        ctx.debug_fail_copies(2)
+        with pytest.raises(_lib.NNVHipError):
+            made[-1][0].estimateRanges()
+        with pytest.raises(_lib.NNVHipError):
+            ctx.synchronize()
+        for S, lb, ub in made:
+            _check(S, lb, ub)
+
+
+def test_a_constructor_that_cannot_launch_the_waiting_copies_fails_alone(nnv):
+    from nnv_amd import _lib
+    ctx, rs = _lib.Context(0), np.random.RandomState(4)
+    made = _boxes(ctx, nnv, rs, 16)   # fifteen wait
+    ctx.debug_fail_copies(2)
+    for _ in range(2):                # the sixteenth that waits, and one that finds sixteen waiting
+        with pytest.raises(_lib.NNVHipError):
+            _boxes(ctx, nnv, rs, 1)
+    made += _boxes(ctx, nnv, rs, 20)
+    for S, lb, ub in made:
+        _check(S, lb, ub)
+
+
+def test_a_context_goes_with_copies_that_cannot_be_launched(nnv):
+    from nnv_amd import _lib
+    ctx = _lib.Context(0)
+    made = _boxes(ctx, nnv, np.random.RandomState(5), 5)
+    del made
+    ctx.debug_fail_copies(100)
+    _lib.check(ctx.lib.nnvhip_destroy(ctx.handle))
+    ctx.handle = None
