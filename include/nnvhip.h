@@ -174,6 +174,8 @@ enum {
   NNVHIP_ROUTE_CHAIN,              /* whole reach in one launch, layers' matrices through memory */
   NNVHIP_ROUTE_CHAIN_LDS,          /* ... sets in the LDS throughout */
   NNVHIP_ROUTE_FC_SKINNY,          /* FC layer of few outputs straight behind a ReLU step */
+  NNVHIP_ROUTE_SUMS_PRODUCT,       /* a matrix product of an FC layer's range sums is formed ... */
+  NNVHIP_ROUTE_SUMS_PRODUCT_READ,  /* ... and left on the layer's output */
   NNVHIP_ROUTES
 };
 NNVHIP_API int nnvhip_debug_routes(nnvhip_ctx* ctx, int64_t* sets);

@@ -98,7 +98,10 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
   std::vector<int64_t> mm_slot;  // which pair of the product's columns holds a set's sums
   bool mm_plb_zero = true;       // every gathered column of every set has predicate lower bound 0
   int st = NNVHIP_OK;
-  if (count >= 64 && !c->eager_cols && !c->dense_affine) {
+  // Few outputs straight behind a ReLU step: one launch that takes the step's rows and unit vectors as it recorded them, and
+  // leaves all range sums itself
+  const bool skinny = !c->dense_affine && fc_skinny_takes(fc, count, in);
+  if (count >= 64 && !skinny && !c->eager_cols && !c->dense_affine) {
     std::vector<GatherSet> es((size_t)count);
     bool ok = true, any = false;
     for (int64_t i = 0; i < count; ++i) {
@@ -176,8 +179,6 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
                          in[0]->rows_pending && in[0]->cls != nullptr && in[0]->pre_ub != nullptr;
     // (skinny layers keep the gather pass: a handful of 16-row blocks would not cover the chip)
     bool rowsum = (box_in || relu_in) && fc->Mp >= 128 && fc->K < (int64_t(1) << 31);
-    // Few outputs straight behind a ReLU step: one launch that takes the step's rows and unit vectors as it recorded them
-    const bool skinny = !dense_only && fc_skinny_takes(fc, count, in);
     // sets whose implicit unit-vector columns take part in the contraction after all get them written out
     // (which also runs a pending row reset)
     std::vector<nnvhip_star*> full;
@@ -1019,6 +1020,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
           if (chunk_off[count] > 0) st = c->alloc(sizeof(double) * 4 * ldo * chunk_off[count], &sums);
         }
         if (st == NNVHIP_OK && use_mm) {
+          c->routes[NNVHIP_ROUTE_SUMS_PRODUCT_READ] += count;
           if (mm_early) mm_sums = mm_early;  // queued at the start of the call, from the same lists
           else {
             bool zero = true;

@@ -207,10 +207,12 @@ __global__ __launch_bounds__(64 * NW) void fc_skinny_kernel(const SkinnySet* __r
 // columns of the set that are contracted: those the step's input had
 static int64_t leading_columns(const nnvhip_star* s) { return s->oh_from > 0 ? s->oh_from : s->n + 1; }
 
+// (finite weights: an infinite one times the zero of a reset row is NaN, and the rows left out count then)
+bool fc_skinny_layer(const nnvhip_fc* fc) { return fc->Mp <= 32 && fc->finite && fc->K < (int64_t(1) << 30); }
+
 bool fc_skinny_takes(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in) {
-  // (matrices of a shared-product call take the same way whether somebody has had them written or not: ColSource::delta.  And
-  // finite weights: an infinite one times the zero of a reset row is NaN, and the rows left out count then)
-  if (fc->Mp > 32 || !fc->finite || fc->K >= (int64_t(1) << 30) || count > 65535) return false;
+  // (matrices of a shared-product call take the same way whether somebody has had them written or not: ColSource::delta)
+  if (!fc_skinny_layer(fc) || count > 65535) return false;
   int64_t empty = 0;
   double gathered = 0.0;
   for (int64_t i = 0; i < count; ++i) {

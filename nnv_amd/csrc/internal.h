@@ -1011,6 +1011,7 @@ int finalize_fused_ranges(nnvhip_ctx* ctx, nnvhip_star* s, const BufRef& part, i
 // fc_skinny.hip: a fully connected layer of few outputs over sets a ReLU step has just made, in one launch that needs neither the
 // step's rows reset nor its unit vectors in memory.  Whether all sets of a call take it, how many chunks of range sums it
 // leaves of a set, and the launch (part[i]: room for set i's chunks of [4][Mp]).
+bool fc_skinny_layer(const nnvhip_fc* fc);  // ... the part of the rule that the layer decides
 bool fc_skinny_takes(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in);
 int fc_skinny_waves(const nnvhip_fc* fc, int64_t count, nnvhip_star* const* in);  // ... of a block, which its chunks depend on
 int64_t fc_skinny_chunks(const nnvhip_star* in, int waves);

@@ -1140,6 +1140,7 @@ __global__ __launch_bounds__(256) void crossing_ub_vectors_kernel(const AheadSet
 int launch_range_sums_mm_ahead(nnvhip_ctx* ctx, const nnvhip_fc* fc, int64_t count, const AheadSet* sets, int64_t N, BufRef* out) {
   const int64_t Kp = fc->Kp;
   if (count >= (int64_t(1) << 30) || N > Kp) NNV_FAIL(NNVHIP_ERR_ARG, "internal: range sums ahead of their layer out of range");
+  ctx->routes[NNVHIP_ROUTE_SUMS_PRODUCT] += count;
   NNV_TRY(ensure_split_weights(ctx, fc));
   BufRef X, tab;
   NNV_TRY(ctx->alloc(sizeof(double) * Kp * 2 * count, &X));
@@ -1154,6 +1155,7 @@ int launch_range_sums_mm_ahead(nnvhip_ctx* ctx, const nnvhip_fc* fc, int64_t cou
 int launch_range_sums_mm(nnvhip_ctx* ctx, const nnvhip_fc* fc, int64_t count, const GatherSet* sets, BufRef* out,
                          std::vector<int64_t>* slot, bool plb_zero) {
   const int64_t Mp = fc->Mp, Kp = fc->Kp;
+  ctx->routes[NNVHIP_ROUTE_SUMS_PRODUCT] += count;
   NNV_TRY(ensure_split_weights(ctx, fc));
   // Sets that gather the same columns with the same scales under the same bounds (the boxes of one shape,
   // nnvhip_star_from_box) have the same sums: one pair of columns serves them all.  Only runs of a few distinct

@@ -91,3 +91,26 @@ def test_infinite_weight_takes_the_dense_product(nnv):
     assert S.ctx.routes()["fc_skinny"] == before
     with np.errstate(invalid="ignore"):
         assert np.array_equal(np.isnan(np.array(out.V)), np.isnan(W @ np.array(mid.V)))
+
+
+@pytest.mark.parametrize("hint", [True, False])
+def test_no_product_of_range_sums_is_formed_for_it(nnv, hint):
+    """An inner layer of few outputs over an array large enough for one: the kernel sums its columns itself.  The layer behind it
+    is not of few outputs; its product is formed once, whether the ReLU step is told of the layer or not, and read."""
+    rs = np.random.RandomState(17)
+    count, widths = 64, [40, 256, 24, 240]
+    fcs = [nnv.layers.FullyConnectedLayer(rs.randn(m, k) / np.sqrt(k), 0.1 * rs.randn(m)) for k, m in zip(widths, widths[1:])]
+    opts = ("relax-star-area", [], 1, None, "linprog")
+    x = rs.rand(40, count)
+    s = fcs[0].reach(nnv.Star.from_boxes(np.asfortranarray(x - 0.3), np.asfortranarray(x + 0.3)), *opts)
+    ctx = s[0].ctx
+    for layer, formed, skinny in ((fcs[1], 0, count), (fcs[2], count, 0)):
+        was = ctx.routes()
+        if hint:
+            ctx.hint_next_fc(layer._weights(ctx))
+        mid = nnv.layers.ReluLayer().reach(s, *opts)
+        s = layer.reach(mid, *opts)
+        now = ctx.routes()
+        assert [now[k] - was[k] for k in ("sums_product", "sums_product_read", "fc_skinny")] == [formed, formed, skinny]
+        for i in (0, count - 1):
+            _check(mid[i], s[i], np.asarray(layer.Weights), np.asarray(layer.Bias).reshape(-1), (layer.OutputSize, i))
