@@ -114,3 +114,24 @@ def test_no_product_of_range_sums_is_formed_for_it(nnv, hint):
         assert [now[k] - was[k] for k in ("sums_product", "sums_product_read", "fc_skinny")] == [formed, formed, skinny]
         for i in (0, count - 1):
             _check(mid[i], s[i], np.asarray(layer.Weights), np.asarray(layer.Bias).reshape(-1), (layer.OutputSize, i))
+
+
+@pytest.mark.parametrize("last", [10, 40])
+def test_a_reach_forms_no_product_that_nobody_reads(nnv, last):
+    """The last layer writes its columns whoever forms their sums: the ReLU step in front of it is not told of it."""
+    rs = np.random.RandomState(last)
+    count, widths = 64, [40, 256, 240, last]
+    layers = []
+    for k, m in zip(widths, widths[1:]):
+        layers += [{"type": "fc", "W": rs.randn(m, k) / np.sqrt(k), "b": 0.1 * rs.randn(m)}, {"type": "relu"}]
+    net = nnv.NN.from_config(layers[:-1])
+    x = rs.rand(40, count)
+    S = nnv.Star.from_boxes(np.asfortranarray(x - 0.3), np.asfortranarray(x + 0.3))
+    ctx = S[0].ctx
+    was = ctx.routes()
+    out = net.reach(S, {"reachMethod": "relax-star-area", "relaxFactor": 1})
+    now = ctx.routes()
+    # the first layer's, over the boxes, and the second's
+    assert [now[k] - was[k] for k in ("sums_product", "sums_product_read")] == [2 * count, 2 * count]
+    for i in (0, count - 1):
+        _check(net.reachSet[3][i], out[i], layers[-2]["W"], layers[-2]["b"], i)
