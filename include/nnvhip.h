@@ -176,6 +176,12 @@ enum {
   NNVHIP_ROUTE_FC_SKINNY,          /* FC layer of few outputs straight behind a ReLU step */
   NNVHIP_ROUTE_SUMS_PRODUCT,       /* a matrix product of an FC layer's range sums is formed ... */
   NNVHIP_ROUTE_SUMS_PRODUCT_READ,  /* ... and left on the layer's output */
+  NNVHIP_ROUTE_FC_ROWSUM,          /* FC layer whose gathered columns are summed straight from the weights */
+  NNVHIP_ROUTE_FC_ROWSUM_MANY,     /* ... behind more than 32 tiles of contracted columns */
+  NNVHIP_ROUTE_FC_SCALED,          /* FC layer over an array, shared rows of weights times the set's own scales */
+  NNVHIP_ROUTE_PERMUTE_WINDOW,     /* row permutation that reads images inside their windows */
+  NNVHIP_ROUTE_COPIES_FETCHED,     /* (pieces, not sets) staged bounds or tables fetched by a kernel ... */
+  NNVHIP_ROUTE_COPIES_TOGETHER,    /* ... that had waited for others */
   NNVHIP_ROUTES
 };
 NNVHIP_API int nnvhip_debug_routes(nnvhip_ctx* ctx, int64_t* sets);

@@ -301,7 +301,8 @@ class Context:
     def routes(self):
         """{route: sets that took it} since the context was created (nnvhip_debug_routes)."""
         names = ("conv_window", "conv_window_parts", "fc_window", "rowmap_window", "rowmap_box", "pool_window", "conv_pixels", "chain", "chain_lds", "fc_skinny",
-                 "sums_product", "sums_product_read")
+                 "sums_product", "sums_product_read", "fc_rowsum", "fc_rowsum_many", "fc_scaled", "permute_window", "copies_fetched",
+                 "copies_together")
         v = (C.c_int64 * len(names))()
         check(self.lib.nnvhip_debug_routes(self.handle, v))
         return dict(zip(names, v))

@@ -287,6 +287,7 @@ static int launch_copy_staged(nnvhip_ctx* c, const StagedPieces& p, int count) {
   }
   hipLaunchKernelGGL(copy_staged_kernel, dim3((most + 1023) / 1024, (unsigned)count), dim3(256), 0, c->stream, p);
   NNV_HIP_TRY(hipGetLastError());
+  c->routes[NNVHIP_ROUTE_COPIES_FETCHED] += count;
   return NNVHIP_OK;
 }
 
@@ -323,6 +324,7 @@ int nnvhip_ctx::flush_copies() {
   }
   // (after a launch that failed they go on waiting: their sets' constructors have returned, so nothing else may run before them)
   NNV_TRY(launch_copy_staged(this, p, (int)waiting.size()));
+  routes[NNVHIP_ROUTE_COPIES_TOGETHER] += (int64_t)waiting.size();
   waiting.clear();  // (released blocks are used again behind the launch, on the same stream)
   return NNVHIP_OK;
 }

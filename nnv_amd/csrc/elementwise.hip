@@ -456,6 +456,7 @@ static int run_row_layer(nnvhip_ctx* c, int64_t count, nnvhip_star* const* in, n
         descs[i].box_to = (int32_t)cs.win_to;
         descs[i].H = cs.win_H;
         descs[i].HW = cs.win_H * cs.win_W;
+        ++c->routes[NNVHIP_ROUTE_PERMUTE_WINDOW];
       }
       max_cols = std::max<int64_t>(max_cols, in[i]->n + 1);
     }

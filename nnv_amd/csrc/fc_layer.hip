@@ -894,6 +894,7 @@ int nnvhip_affine_fc(nnvhip_ctx* c, const nnvhip_fc* fc, int64_t count, nnvhip_s
           double flop[4] = {0.0, 0.0, 0.0, 0.0};
           int64_t off = 0;
           for (int64_t i = 0; i < count && st == NNVHIP_OK; ++i) {
+            if (scaled && shared && !filled[i]) ++c->routes[NNVHIP_ROUTE_FC_SCALED];
             for (int64_t j = 0; j < dense[i] && !filled[i]; j += 128) {
               const int64_t valid = std::min<int64_t>(128, dense[i] - j);
               const bool gather = shared && j < 128 * nfull_of(i);

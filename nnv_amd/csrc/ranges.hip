@@ -1058,6 +1058,8 @@ int launch_fc_rowsum(nnvhip_ctx* ctx, const nnvhip_fc* fc, nnvhip_star* out, int
     NNV_LAUNCH(ctx, ctx->kernel_timing, fc_rowsum_kernel<1>, dim3(blocks), dim3(1024), 0, a);
   NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 5, bytes));
   NNV_HIP_TRY(hipGetLastError());
+  ++ctx->routes[NNVHIP_ROUTE_FC_ROWSUM];
+  if (chunks > 32) ++ctx->routes[NNVHIP_ROUTE_FC_ROWSUM_MANY];
   out->rbuf = rb;
   out->lb = a.lb;
   out->ub = a.ub;

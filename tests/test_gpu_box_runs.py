@@ -28,6 +28,9 @@ def _check(S, lb, ub):
 def test_runs_of_constructors(nnv, count):
     rs = np.random.RandomState(count)
     made = []
+    ctx = nnv.default_context()
+    ctx.synchronize()        # (nothing waits, and the first of the run goes at once)
+    was = ctx.routes()
     for i in range(count):
         n = int(rs.choice([1, 2, 15, 16, 17, 300, 784]))
         lb = rs.randn(n)
@@ -39,8 +42,34 @@ def test_runs_of_constructors(nnv, count):
         made.append((S, lb.copy(), ub.copy()))
         lb += 1.0            # the caller's arrays are its own again
         ub -= 7.0
+    ctx.synchronize()
+    now = ctx.routes()
+    assert [now[k] - was[k] for k in ("copies_fetched", "copies_together")] == [count, count - 1]
     for S, lb, ub in made:
         _check(S, lb, ub)
+
+
+@pytest.mark.parametrize("n,fetched", [(7280, 3), (7281, 0)])
+def test_the_largest_piece_a_kernel_fetches(nnv, n, fetched):
+    """256 KB: 262080 bytes of centre, half-widths, bounds and index list on one side of the line, 262656 on the other."""
+    rs = np.random.RandomState(n)
+    ctx = nnv.default_context()
+    ctx.synchronize()
+    was = ctx.routes()["copies_fetched"]
+    made = []
+    for _ in range(3):
+        lb = rs.randn(n)
+        ub = lb + 0.5 + rs.rand(n)
+        made.append((nnv.Star(lb, ub), lb, ub))
+    ctx.synchronize()
+    assert ctx.routes()["copies_fetched"] == was + fetched
+    for S, lb, ub in made:
+        l, u = S.estimateRanges()
+        tol = 4 * np.finfo(float).eps * (np.abs(lb) + np.abs(ub))
+        assert np.all(np.abs(l - lb) <= tol) and np.all(np.abs(u - ub) <= tol)
+        rows = S._h.fetch_rows([0, n - 1])
+        assert rows[0, 1] == 0.5 * (ub[0] - lb[0]) and rows[1, n] == 0.5 * (ub[-1] - lb[-1]) and np.count_nonzero(rows[:, 1:]) == 2
+        assert np.array_equal(S.predicate_lb, -np.ones(n)) and np.array_equal(S.predicate_ub, np.ones(n))
 
 
 def test_large_and_small_in_turn_past_the_end_of_the_ring(nnv):
