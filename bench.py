@@ -5,7 +5,8 @@
 
 A step is one full ``NN.reach`` of a benchmark configuration with the input set(s) and the weights
 already resident in HBM; it ends with the output set(s) and their estimated output bounds resident in
-HBM.  Without ``--config`` all five configurations are measured in one run and ONE JSON line is printed:
+HBM.  Without ``--config`` all five configurations are measured in one run.  ONE JSON line is printed on standard
+output, under 2000 characters; standard error has the whole report, as one line too, with the tables the line leaves out:
 
   headline       configuration 5 (the 1024 sub-boxes of config 2's input box, reached as one array on
                  config 2's network) - the largest single-GPU workload: ``value``, ``ms_per_step``,
@@ -45,6 +46,7 @@ HBM_PEAK_GBS = 8000.0
 MIN_WARM_SECONDS = 0.3
 
 
+KERNEL_GROUPS = 14   # timed groups of the library (nnvhip_kernel_time)
 # kernels whose launches a timed group of the library covers (nnvhip_kernel_time), by the group's label below
 GROUP_KERNELS = {
     "gemm_f64_kernel": ("gemm_f64_kernel", "gemm_gather_kernel"),
@@ -52,6 +54,7 @@ GROUP_KERNELS = {
     "conv2d_fast_kernel": ("conv2d_fast_kernel", "conv2d_fast_stamps_kernel", "conv2d_f64_kernel"),
     "conv_window_kernel": ("conv_window_kernel",),
     "fc_window_kernel": ("fc_window_kernel",),
+    "fc_skinny_kernel": ("fc_skinny_kernel",),
     "gather_columns_kernel": ("gather_columns_kernel", "gather_skinny_kernel", "fc_rowsum_kernel", "conv_stamp_kernel", "conv_stamp_rows_kernel"),
     "ranges_partial_kernel": ("ranges_partial_kernel", "ranges_window_kernel"),
     "relu_classify_kernel": ("relu_classify_kernel", "relu_classify_rank_kernel", "relu_count_kernel", "relu_compact_kernel"),
@@ -251,13 +254,13 @@ def measure(k, args, ctx, exact_steps, extras):
         return acc / reps
 
     # a small FC / ReLU network is reached by ONE launch (nnvhip_reach_layers): time that kernel on the step's own path
-    for grp in range(13):
+    for grp in range(KERNEL_GROUPS):
         ctx.kernel_time(grp)
     ctx.set_timing(2)
     for _ in range(reps):
         step()
     ctx.set_timing(0)
-    step_groups = [ctx.kernel_time(grp) for grp in range(13)]
+    step_groups = [ctx.kernel_time(grp) for grp in range(KERNEL_GROUPS)]
     chain_ms, chain_launches, chain_bytes = step_groups[8]
 
     per_layer = timed_pass(1)          # NN.reachTime-style device time per layer (layer-by-layer calls)
@@ -265,7 +268,7 @@ def measure(k, args, ctx, exact_steps, extras):
     # a network with convolutions keeps its images in another layout where it is reached in one call: its kernels are
     # those of the step
     if any(grp[1] for grp in (step_groups[1], step_groups[12])) and not chain_launches:
-        for grp in range(13):
+        for grp in range(KERNEL_GROUPS):
             ctx.kernel_time(grp)
 
         def group_time(grp):
@@ -284,6 +287,7 @@ def measure(k, args, ctx, exact_steps, extras):
     dlt_ms, dlt_launches, dlt_bytes = group_time(10)
     fcw_ms, fcw_launches, fcw_work = group_time(11)
     cvw_ms, cvw_launches, cvw_work = group_time(12)
+    skn_ms, skn_launches, skn_work = group_time(13)
 
     # algorithmic (unpadded, dense) flop of the launches the kernel timers cover
     gemm_flop = conv_flop = 0.0
@@ -357,9 +361,9 @@ def measure(k, args, ctx, exact_steps, extras):
     groups = []
     # (the dense count of the FC layers is quoted with the one of the FC kernel groups that takes longest, that of the
     # convolutions likewise)
-    fc_longest = max(seg_ms, gemm_ms, fcw_ms)
+    fc_longest = max(seg_ms, gemm_ms, fcw_ms, skn_ms)
     for name, ms_, n_, work in (("gemm_seg_kernel", seg_ms, seg_launches, seg_work), ("gemm_f64_kernel", gemm_ms, gemm_launches, gemm_work),
-                                ("fc_window_kernel", fcw_ms, fcw_launches, fcw_work)):
+                                ("fc_window_kernel", fcw_ms, fcw_launches, fcw_work), ("fc_skinny_kernel", skn_ms, skn_launches, skn_work)):
         if n_:
             groups.append((ms_, mfma_roofline(name, work, gemm_flop if ms_ == fc_longest else 0.0, ms_, n_)))
     for name, ms_, n_, work in (("conv2d_fast_kernel", conv_ms, conv_launches, conv_work), ("conv_window_kernel", cvw_ms, cvw_launches, cvw_work)):
@@ -573,6 +577,28 @@ def measure(k, args, ctx, exact_steps, extras):
     }
 
 
+def brief(report):
+    """The report without its tables: what was measured, on what, and the kernel that takes longest of each workload."""
+    def top(r):
+        return {k: r[k] for k in ("kernel", "bound", "achieved", "peak", "unit", "frac", "traffic", "measured_mfma_TFLOPs", "measured_copy_GBps") if k in r}
+
+    out = {k: report[k] for k in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling", "vs_baseline",
+                                  "dtype", "data")}
+    out["config"] = {k: report["config"][k] for k in ("workload", "reach_method", "relax_factor", "switches", "sets", "updates_per_step")}
+    out["roofline"] = top(report["roofline"])
+    if report["cpu_baseline"]:
+        out["cpu_baseline"] = {k: v for k, v in report["cpu_baseline"].items() if k != "sample"}
+    for k in ("value_is", "value_all_sets_written", "ms_per_step_all_sets_written"):
+        out[k] = report[k]
+    for k, ms in (("host_to_host", "ms_per_step"), ("spec_check", "ms")):
+        if report[k]:
+            out[k + "_ms"] = report[k][ms]
+    if report["per_config"]:
+        out["per_config"] = [{"workload": r["config"]["workload"], "ms_per_step": round(r["ms_per_step"], 5), "kernel": r["roofline"]["kernel"], "frac": r["roofline"]["frac"]}
+                             for r in report["per_config"]]
+    return out
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -644,7 +670,7 @@ def main():
         cpu["device_over_cpu_all_sets_written"] = round(head["all_sets_written"]["value"] / cpu["value"], 1)
         cpu["device_over_cpu_sets_described"] = round(head["value"] / cpu["value"], 1)
 
-    print(json.dumps({
+    report = {
         "metric": "generator_neuron_updates_per_s", "value": head["value"], "unit": "updates/s", "n_gpus": 1,
         "steps": head["steps"], "warmup": head["warmup"], "ms_per_step": head["ms_per_step"], "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "f64", "data": "synthetic",
@@ -657,7 +683,10 @@ def main():
         "ms_per_step_all_sets_written": head["all_sets_written"]["ms_per_step"] if head["all_sets_written"] else None,
         "spec_check": head["spec_check"], "host_to_host": head["host_to_host"],
         "all_sets_written": head["all_sets_written"], "layers": head["layers"], "per_config": per_config,
-    }))
+    }
+    # the whole report goes to standard error; the line on standard output is short enough to be kept whole by whoever logs it
+    print(json.dumps(report), file=sys.stderr, flush=True)
+    print(json.dumps(brief(report)))
 
 
 if __name__ == "__main__":

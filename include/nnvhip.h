@@ -105,7 +105,8 @@ NNVHIP_API int nnvhip_set_eager_relu(nnvhip_ctx* ctx, int enabled);
  * whole-reach kernel of small fully connected networks (nnvhip_reach_layers); 9: the tile kernel that
  * contracts kept rows only, for arrays of sets and wide single sets (work: 2*Mp*kept*columns per set); 10: outputs
  * that start from a product shared by many sets (work: bytes); 11: the contraction of an FC layer inside its images'
- * windows; 12: the convolution by output position (work of both: flop of the kept rows' products inside the windows).
+ * windows; 12: the convolution by output position (work of both: flop of the kept rows' products inside the windows);
+ * 13: FC layer of at most 32 outputs straight behind a ReLU step (work: 2*Mp*kept*contracted columns per set).
  * Returns accumulated kernel time,
  * launch count and work since the last reset.  Work is the flop executed for 0 and 1 (GEMM:
  * 2*Mp*Kp*ncols over the columns and rows the launch contracts, M and K padded to 16; conv:

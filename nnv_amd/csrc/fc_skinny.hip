@@ -292,7 +292,7 @@ int launch_fc_skinny(nnvhip_ctx* ctx, const nnvhip_fc* fc, int64_t count, nnvhip
     NNV_LAUNCH(ctx, ctx->kernel_timing, (fc_skinny_kernel<2, 4>), grid, dim3(256), 0, table, sets[0], W, bias);
   else
     NNV_LAUNCH(ctx, ctx->kernel_timing, (fc_skinny_kernel<2, 8>), grid, dim3(512), 0, table, sets[0], W, bias);
-  NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 0, flop));
+  NNV_TRY(ctx->kernel_timer_end(ctx->kernel_timing, 13, flop));
   NNV_HIP_TRY(hipGetLastError());
   ctx->routes[NNVHIP_ROUTE_FC_SKINNY] += count;
   return NNVHIP_OK;

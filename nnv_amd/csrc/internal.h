@@ -447,7 +447,8 @@ struct nnvhip_ctx {
   // add only the rows in which a set differs from it (delta_tiles_kernel; work = bytes written)
   // [11] FC contraction inside the images' windows (fc_window_kernel), [12] convolution by output position
   // (conv_window_kernel); work = flop of the kept rows' products inside the bounds on the columns' windows
-  static constexpr int kKernelGroups = 13;
+  // [13] FC layer of few outputs straight behind a ReLU step (fc_skinny_kernel); work = flop over the kept rows
+  static constexpr int kKernelGroups = 14;
   double kern_ms[kKernelGroups] = {};
   int64_t kern_launches[kKernelGroups] = {};
   double kern_flop[kKernelGroups] = {};
