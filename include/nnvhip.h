@@ -380,8 +380,9 @@ NNVHIP_API int nnvhip_set_switch(nnvhip_ctx* ctx, const char* name, int enabled)
  * layer's range estimate that needs nothing but the classes (the sums over the columns the step appends), so that
  * the device works on it while the host reads the step's counts and sets the FC call up; nnvhip_affine_fc finds it
  * on the sets and does not form it again.  Results are the same to the bit with and without the hint; a hint that
- * does not come true (another layer follows, other sets are passed) costs the product and nothing else.  The hint
- * is consumed by the next nnvhip_relu_relax call; fc == NULL withdraws it. */
+ * does not come true (another layer follows, other sets are passed, or it is the last one and writes its columns at once,
+ * nnvhip_set_eager_columns) costs the product and nothing else.  For a layer of at most 32 outputs nothing is queued: it
+ * sums its columns in its own launch.  The hint is consumed by the next nnvhip_relu_relax call; fc == NULL withdraws it. */
 NNVHIP_API int nnvhip_hint_next_fc(nnvhip_ctx* ctx, const nnvhip_fc* fc);
 enum { NNVHIP_LAYER_FC = 0, NNVHIP_LAYER_CONV2D = 1, NNVHIP_LAYER_RELU = 2 };
 NNVHIP_API int nnvhip_reach_layers(nnvhip_ctx* ctx, int64_t n_layers, const int32_t* kind, const void* const* layer,

@@ -461,9 +461,16 @@ static int conv_window_tile(const nnvhip_conv2d* cv) { return cv->Cout <= 16 ? 1
 
 int conv_window_parts(const nnvhip_conv2d* cv, int64_t Ho, int64_t Wo, int64_t dense, int eh, int ew) {
   // A set by itself: blocks that fill the 1024 places of four to a CU once, or, where positions are too many for that to come
-  // out nearly even, twice; about one more a position writes stamps.  No part with less than a tile of columns.  (15 x 15
-  // positions, 288 taps into 64 channels: 4 parts 77.9 us, 5 - 1360 blocks - 79.4, 8 - 2032 - 74.6, 12 85.0; 7 x 7 positions, 576
-  // taps: 14 parts 90.0, 19 - 992 blocks - 81.6, 21 - 1088 - 92.4, 32 92.8.)
+  // out nearly even, twice; about one more a position writes stamps.  No part with less than a tile of columns, which is what
+  // decides where a set has no more than some 1000 columns.  (15 x 15 positions, 288 taps into 64 channels: 4 parts 77.9 us, 5 -
+  // 1360 blocks - 79.4, 8 - 2032 - 74.6, 12 85.0; 7 x 7 positions, 576 taps: 14 parts 90.0, 19 - 980 blocks - 81.6, 21 - 1088 -
+  // 92.4, 32 92.8.)  Where "nearly even" lies: those 980 blocks are 0.96 of the places, and one round; three parts of the 15 x 15
+  // would be 900, 0.88, and neither 4 nor 5 is as fast as two rounds.  All layers by position of other networks of four
+  // convolutions, us, with 1024 blocks whatever they come out to -> with this -> with 768 places: 32 x 32 x 3 into 16, 16 channels
+  // 67.6 -> 65.1 -> 71.8; 16, 32 84.5 -> 80.1 -> 83.1; 32, 48 150.5 -> 149.2 -> 164.0; 5 x 5 taps into 16, 48 133.8 -> 136.8 -> 136.2;
+  // 28 x 28 x 3 into 24, 24 81.0 -> 75.3 -> 78.3; 24 x 24 x 3 into 16, 32 41.9 -> 39.4 -> 42.0; smaller ones within 2 % of one another
+  // (16-channel tiles too do best with four blocks to a CU).  Arrays take the same parts set by set: 3 sets of 24 x 24 and 8 of
+  // 28 x 28 are within 2 % in all three.
   const int64_t a_part = Ho * Wo * ceil_div(cv->Cout, conv_window_tile(cv)), places = 1024;
   int64_t want = (places - Ho * Wo) / a_part;
   if (want < 1 || (double)(want * a_part + Ho * Wo) < 0.93 * (double)places) want = std::max<int64_t>(want, (2 * places - Ho * Wo) / a_part);

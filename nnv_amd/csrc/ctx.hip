@@ -291,7 +291,8 @@ static int launch_copy_staged(nnvhip_ctx* c, const StagedPieces& p, int count) {
   return NNVHIP_OK;
 }
 
-// Small pieces are fetched by a kernel: the runtime hands most copies to the copy engines, which the queue then waits for.
+// Small pieces are fetched by a kernel: the runtime hands copies of 64 KB and more to the copy engines, which the queue then waits
+// for (kStagedByKernel has the figures).
 int nnvhip_ctx::copy_staged(const BufRef& dev, size_t at, const void* staged, size_t bytes, bool may_wait) {
   char* const to = static_cast<char*>(dev->ptr) + at;
   if (bytes > kStagedByKernel || bytes % 4 != 0) {

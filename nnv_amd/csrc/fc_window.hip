@@ -128,13 +128,14 @@ __global__ __launch_bounds__(kSortThreads) void fc_window_setup_kernel(const FcW
   sort_windows(S.ncols - 1, a.buckets, S.order, nullptr, a.sort_run, blockIdx.x, [&](int j) { return window_bucket(S.box[j], a); });
 }
 
+__device__ double g_win_zero[1];  // what an element outside its image's window is read from (never written)
+
 // TM x TN output tile per block of WR x WC waves.  Column tiles are dealt to the XCDs (blockIdx.x % 8) with all their row
 // tiles, which read the same images.  The last column tile of a set is its centre: the sum of the partial products.
 // PIXELS: every set's images are kept pixel by pixel (ColSource::pix).  A listed row then has a place in the image beside its number
 // and its position.  As one kernel for both ways, with lists of half the length and eight registers more, a CU held one block of
 // 64 x 64 less and unions of windows went through several lists: 25 images of 28 x 28 x 1 and of 40 x 40 x 1, column by column, 119 and
 // 245 us, 101 and 213 apart (101 and 206 before there were pixels); pixel by pixel 115 and 232, 101 and 204 now.
-__device__ double g_win_zero[1];  // (never written)
 constexpr int kWinRows = 2048, kWinPixelRows = 1536;  // rows a stage list holds; a union with more kept rows is walked in several lists
 template <int TM, int TN, int WR, int WC, int KT, bool PIXELS>
 __global__ __launch_bounds__(64 * WR * WC, TN == 64 ? 6 : 4) void fc_window_kernel(const FcWinSet* __restrict__ table, FcWinSet one, FcWinArgs a) {

@@ -73,8 +73,8 @@ __global__ __launch_bounds__(kSegNT, 4) void gemm_seg_kernel(const double* __res
     if (ok) pb_reg = src[sc - 1];
   }
   // SCALED: the rows of B are those of the weights as they are, and what a column is multiplied by is the set's own: the factors of
-  // the lane's columns (one multiplication per operand and column ahead of FM matrix instructions).  Asked for before the row list, whose arrival the first transfers wait for:
-  // nothing in the K loop waits for them.
+  // the lane's columns (one multiplication per operand and column ahead of FM matrix instructions).  Asked for before the row list,
+  // whose arrival the first transfers wait for: nothing in the K loop waits for them.
   static_assert(!SCALED || GATHER, "only gathered rows come without their scales");
   double fac[FN];
 #pragma unroll

@@ -468,7 +468,12 @@ struct nnvhip_ctx {
   // Copies `bytes` of the staging ring to a buffer, `at` bytes from its start (all aligned to 16 bytes; async on the stream).
   // may_wait: the copy may be put off until the next entry point (enter_ctx) so that several travel together; the buffer
   // is held until then.
-  static constexpr size_t kStagedByKernel = size_t(256) << 10;  // larger ones go to a copy engine
+  // Larger ones go to a copy engine.  A copy and the kernel that reads it, us, behind nothing and behind 55 us of queued work,
+  // with hipMemcpyAsync / with copy_staged_kernel: 4 and 16 KB 14 / 14 and 69 / 69 (the runtime's own kernel), 64 KB 19 / 16 and
+  // 83 / 70 (from here on it takes a copy engine, and the queue waits for it), 128 KB 20 / 17 and 85 / 72, 256 KB 23 / 20 and 87 / 75,
+  // 512 KB 28 / 26 and 92 / 81, 1 MB 38 / 38 and 101 / 94.  What is won shrinks beyond 256 KB, and sixteen pieces of that size that
+  // wait for one another fill the ring's first 4 MB.
+  static constexpr size_t kStagedByKernel = size_t(256) << 10;
   static constexpr size_t kWaitingCopies = 16;
   struct WaitingCopy {
     nnvhip::BufRef dev;
