@@ -1044,8 +1044,8 @@ int relu_relax(nnvhip_ctx* ctx, int order, int64_t count, nnvhip_star* const* in
   // Queued here, the product runs while the host reads the counts, makes the handles and sets the layer call up.  (A layer of few
   // outputs sums its columns itself, fc_skinny.hip: no product for it.  That saves the device the work and the buffers, a pass
   // no time - 100 sets through 784-1024-24-300-10: 1840 us with and without.  Where it does not - most sets keep no row - it forms
-  // the product in its call: 700 us with 32 in the place of 24 and a wide box, 690 where it was queued here, which runs of one
-  // build differ by too.)
+  // the product in its call: 700 us with 784-1024-512-32-300-10 and wide boxes, 690 where it was queued here, no more than
+  // two runs of the same code differ by.)
   BufRef ahead_mm;
   if (next_fc != nullptr && given == nullptr && lazy_rows && count >= 64 && !ctx->eager_cols && !ctx->dense_affine &&
       next_fc->K == N && next_fc->ctx == ctx && !fc_skinny_layer(next_fc)) {
